@@ -47,7 +47,6 @@ namespace {
 
 constexpr int kIpt = 8;                 // elements per thread in the LDS sort
 constexpr int kTeamIpt = 8;             // entries per lane of the wave-per-item tier
-constexpr int kMaxDigitRun = 16;        // longest run of equal top digits ordered in place
 static_assert(kWave * kTeamIpt >= kMaxCutTeam, "wave tier capacity");
 constexpr int kCap = kBlock * kIpt;     // LDS chunk capacity (2048)
 constexpr int kHistWords = 8192;        // LDS histogram words (32 KB)
@@ -62,6 +61,7 @@ __device__ __forceinline__ void load_ln_table(double* s_inv, double* s_logc) {
 
 // ------------------------------------------------------------- args -----
 constexpr int kMaxTiers = 7;
+constexpr int kTfMax = 4096;  // entries of the fp32 x ln x table
 struct DataArgs {
   const float* X;
   const uint32_t* K;
@@ -78,6 +78,7 @@ struct DataArgs {
   int igF;           // fixed-point shift of the x ln x terms (per fit)
   const int64_t* T;  // T[x] = xlnx_fixed(x, igF) for x <= Tmax (classification)
   int64_t Tmax;
+  const float* Tf;   // x ln x in fp32 for x < kTfMax (bounds of the random-forest search)
   // Joint build of several extra-trees forests in one set of level steps:
   // the data of batch tree t is forests[forest_of_tree[t]], whose D0 / R
   // are its mandatory and retry draws; C is the joint class width in every
@@ -740,7 +741,7 @@ __device__ void eval_hist_bucket(const uint32_t* skey, const uint32_t* saux, con
 
 // Sort a chunk (keys relative to kbase, span < 2^bits) held in LDS buffer 0
 // and evaluate it.
-template <int MAXC, int TASK, int TEAM, int IPT, bool DIGIT = false, class LX = LnCtx>
+template <int MAXC, int TASK, int TEAM, int IPT, class LX = LnCtx>
 __device__ void sort_and_eval(int n, int bits, uint32_t kbase, const NodeCtx& nc,
                               TeamLds<MAXC, TASK, TEAM, IPT>& L, const LX& lx) {
   constexpr int kSpan = TeamLds<MAXC, TASK, TEAM, IPT>::SPAN;
@@ -748,14 +749,6 @@ __device__ void sort_and_eval(int n, int bits, uint32_t kbase, const NodeCtx& nc
     lds_count_sort<IPT, TEAM>(L.u.srt.k[0], L.u.srt.v[0], L.u.srt.k[1], L.u.srt.v[1], n, 1 << bits,
                               reinterpret_cast<uint32_t*>(L.u.srt.cnt), L.w);
     eval_sorted_chunk<MAXC, TASK, TEAM, IPT>(L.u.srt.k[1], L.u.srt.v[1], n, kbase, nc, L, lx);
-    return;
-  }
-  // Wide key spans: one counting pass on the top digit, then short runs
-  // ordered in place; radix passes when a run is long (clustered keys).
-  if (DIGIT && bits > 8 &&
-      lds_digit_sort<IPT, TEAM>(L.u.srt.k[0], L.u.srt.v[0], L.u.srt.k[1], L.u.srt.v[1], n, bits, kSpan, kMaxDigitRun,
-                                reinterpret_cast<uint32_t*>(L.u.srt.cnt), L.w)) {
-    eval_sorted_chunk<MAXC, TASK, TEAM, IPT>(L.u.srt.k[0], L.u.srt.v[0], n, kbase, nc, L, lx);
     return;
   }
   int cur = 0;
@@ -1033,166 +1026,55 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
   if (t == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
 }
 
-// Wave-team (TEAM = 64) and workgroup (TEAM = 256) tiers, node-major: one
-// team per node walks the node's draws in order.  The node's statistics, row
-// ids and payloads are read once; the key gather of the next draw is in
-// flight while the current draw is sorted and walked.  Same results as
-// k_search_rf<.., TEAM, false> item by item.
-template <int MAXC, int TASK, int TEAM>
-__global__ void __launch_bounds__(kBlock) k_search_rf_team(DataArgs d, LevelArgs lv, ItemArgs it) {
-  constexpr int IPT = TEAM == kWave ? kTeamIpt : kIpt;
-  constexpr int NT = kBlock / TEAM;
-  resolve_level(lv, d.C);
-  resolve_items(it);
-  if ((int64_t)blockIdx.x * NT >= it.n_groups) return;  // no node for this workgroup
-  // LDS copy of T's head for wave teams (still 2 workgroups per CU); the
-  // workgroup teams keep their registers for occupancy instead
-  constexpr int kTL = (TASK == 0 && TEAM == kWave) ? 1024 : 0;
-  __shared__ double s_inv[128], s_logc[128];
-  __shared__ int64_t s_T[kTL > 0 ? kTL : 1];
-  __shared__ TeamLds<MAXC, TASK, TEAM, IPT> s_team[NT];
-  load_tables(s_inv, s_logc);
-  const int64_t nTL = kTL > 0 ? load_t_prefix<kTL>(s_T, d.T, d.Tmax) : 0;
-  __syncthreads();
-  const auto lx = [&]() {
-    if constexpr (kTL > 0)
-      return LnCtxL{s_inv, s_logc, d.T, d.Tmax, d.igF, s_T, nTL};
-    else
-      return LnCtx{s_inv, s_logc, d.T, d.Tmax, d.igF};
-  }();
-  const int team = TEAM == kWave ? (int)(threadIdx.x / kWave) : 0;
-  TeamLds<MAXC, TASK, TEAM, IPT>& L = s_team[team];
-  const int t = team_tid<TEAM>();
-  unsigned long long my_bytes = 0;
-  for (int64_t grp = (int64_t)blockIdx.x * NT + team; grp < it.n_groups; grp += (int64_t)gridDim.x * NT) {
-    const uint32_t o = it.list ? it.list[grp] : (uint32_t)grp;
-    const uint32_t i = lv.open_idx[o];
-    const uint32_t tg = (uint32_t)lv.tree_global[lv.tree[i]];
-    const uint32_t nid = lv.id[i];
-    NodeCtx nc;
-    const bool pure = node_context<MAXC, TASK, TEAM, IPT>(d, lv, i, nc, L, lx);
-    if (pure) {
-      // Every boundary of a pure node has gain exactly 0: no positive split.
-      if (t == 0)
-        for (int jj = 0; jj < it.per_group; ++jj) {
-          const int j = it.j0 + jj;
-          const int64_t ridx = (int64_t)o * it.D + j;
-          it.res_score[ridx] = 0.0f;
-          it.res_thr[ridx] = 0.0f;
-          it.res_feat[ridx] = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)j) % (uint32_t)d.F);
-        }
-      team_sync<TEAM>();
-      continue;
-    }
-    const int m = lv.m[i];
-    const int64_t st = lv.start[i];
-    uint32_t rows[IPT], kn[IPT];
-#pragma unroll
-    for (int q = 0; q < IPT; ++q) {
-      const int e = t + q * TEAM;
-      if (e < m) {
-        rows[q] = lv.row[st + e];
-        L.aux[e] = lv.aux[st + e];
-        if (TASK == 1) L.y[e] = lv.ey[st + e];
-      }
-    }
-    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)it.j0) % (uint32_t)d.F);
-#pragma unroll
-    for (int q = 0; q < IPT; ++q)
-      if (t + q * TEAM < m) kn[q] = d.K[(int64_t)f_nx * d.N + rows[q]];
-    for (int jj = 0; jj < it.per_group; ++jj) {
-      const int j = it.j0 + jj;
-      const int64_t ridx = (int64_t)o * it.D + j;
-      const int f = f_nx;
-      uint32_t key[IPT];
-#pragma unroll
-      for (int q = 0; q < IPT; ++q) key[q] = kn[q];
-      if (jj + 1 < it.per_group) {
-        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + 1)) % (uint32_t)d.F);
-#pragma unroll
-        for (int q = 0; q < IPT; ++q)
-          if (t + q * TEAM < m) kn[q] = d.K[(int64_t)f_nx * d.N + rows[q]];
-      }
-      if (t == 0) {
-        for (int c = 0; c < MAXC; ++c) L.cr.run[c] = 0;
-        L.cr.run_n = 0;
-        L.cr.run_s = 0;
-        L.cr.last_key = 0;
-        L.cr.best_g = 0.0;
-        L.cr.best_key = kNone;
-        L.cr.best_prev = kNone;
-      }
-      uint32_t kmin = kNone, kmax = 0;
-#pragma unroll
-      for (int q = 0; q < IPT; ++q) {
-        const int e = t + q * TEAM;
-        if (e < m) {
-          kmin = min(kmin, key[q]);
-          kmax = max(kmax, key[q]);
-        }
-      }
-      kmin = team_reduce_min<TEAM>(kmin, L.w);
-      kmax = team_reduce_max<TEAM>(kmax, L.w);
-#pragma unroll
-      for (int q = 0; q < IPT; ++q) {
-        const int e = t + q * TEAM;
-        if (e < m) {
-          L.u.srt.k[0][e] = key[q] - kmin;
-          L.u.srt.v[0][e] = (uint16_t)e;
-        }
-      }
-      team_sync<TEAM>();
-      sort_and_eval<MAXC, TASK, TEAM, IPT, true>(m, bit_length(kmax - kmin), kmin, nc, L, lx);
-      team_sync<TEAM>();
-      if (t == 0) rf_write_result<MAXC, TASK, TEAM, IPT>(d, it, ridx, f, L.cr);
-      team_sync<TEAM>();
-    }
-    if (t == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
-  }
-  if (t == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
-}
-
 // ------------------------------------- chunk-parallel big-node search ---
 // Items (node, feature draw) above the workgroup's LDS capacity.  The keys of
-// an item (dense ranks of the drawn feature) are split into nb coarse buckets
-// of consecutive keys, bucket = key >> shift, sized so that a bucket holds
-// about kV2Target entries: one wave-sized chunk.  Every bucket of every item
-// of a level is then evaluated in parallel:
-//   1. k_v2_hist     per (item, tile): bucket counts and max key; the
-//                    gathered keys are kept in entry order for the scatter
-//   2. k_v2_scan     per item: bucket offsets, last key before each bucket,
-//                    task lists
-//   3. k_v2_scatter  per (item, tile): entries into bucket order, staged in
-//                    LDS so that each bucket's run is written contiguously
-//   4. k_v2_ctot     per bucket: class totals (regression: weight and target
-//                    sums) of the bucket's entries
-//   5. k_v2_carry    per item: totals before each bucket
-//   6. k_v2_eval     per bucket, one wave each: LDS sort + scored walk from
-//                    the carry
-//   7. k_v2_spill    per overfull bucket (ties, clustered keys): fine
-//                    sub-buckets walked in order by one workgroup
-//   8. k_v2_reduce   per item: best bucket -> (score, threshold)
-// Entry order inside a bucket does not matter: the walk sorts by key and
-// scores only boundaries between distinct keys from integer prefix sums.
-constexpr int kV2Tile = 16384;   // entries per histogram tile
+// an item (dense ranks of the drawn feature) are split into nb buckets of
+// consecutive keys, bucket = key / width, of about 64 entries each.  The gain
+// is a convex function of what lies left of a boundary, so a bucket's class
+// counts (regression: weights and target sums) bound the gain of every
+// boundary inside it; only buckets whose bound reaches the best bucket edge
+// of the node's draws are sorted and walked:
+//   1. k_v2_hist     per (item, tile): class counts (weight, target sums) of
+//                    every bucket; the gathered keys are kept in entry order
+//   2. k_v2_bound    per item: totals before each bucket, the gain at each
+//                    bucket's lower edge, the bound of the bucket; the best
+//                    edge over a node's draws
+//   3. k_v2_select   per item: the buckets that can still hold the node's
+//                    best split, with a scratch slot each
+//   4. k_v2_collect  per (item, tile): entries of selected buckets into their
+//                    slots, last key before each selected bucket
+//   5. k_v2_eval     per selected bucket, one wave each: LDS sort + scored
+//                    walk from the totals before it
+//   6. k_v2_spill    per selected bucket above a wave's capacity (clustered
+//                    keys, capped bucket counts): fine sub-buckets walked in
+//                    order by one workgroup
+//   7. k_v2_reduce   per item: best bucket -> (score, threshold)
+// A draw whose best candidate is pruned reports a lower score (or none), and
+// never one of the node's best score: every bucket that could reach it, ties
+// in fp32 included, is walked.  Entry order inside a bucket does not matter:
+// the walk sorts by key and scores only boundaries between distinct keys from
+// integer prefix sums.
+constexpr int kV2Tile = 16384;   // entries per tile
 constexpr int kXcds = 8;          // XCDs of an MI355X, one L2 each
-constexpr int kScatterTile = 4096;  // entries per scatter tile (classification)
 constexpr int kV2MaxB = 4096;    // buckets per item
 constexpr int kV2Ipt = kIpt;     // entries per lane of the bucket evaluator
-constexpr int kV2Target = kDefBucketTarget;  // entries per bucket aimed at (default)
 constexpr int kV2WaveCap = kWave * kV2Ipt;  // bucket capacity of a wave (512)
+// LDS words of a tile's bucket table: three workgroups per CU.  A bucket
+// takes a word per class (regression: a weight and two 64-bit sums).
+constexpr int kV2HistWords = 12288;
+constexpr int kV2RegWords = 5;
 
 struct V2Item {
   int32_t f;
   int32_t m;
   int64_t start;  // first entry of the node
-  int64_t soff;   // first scratch slot of the item
+  int64_t soff;   // first slot of the item's gathered keys
   int32_t boff;   // first bucket slot of the item
   int32_t nb;     // buckets
   uint32_t width;  // bucket = key / width (v2_bucket)
   uint32_t magic;  // floor(2^32 / width)
   uint32_t node;  // level node index
-  int32_t sgrp;   // buckets per super-bucket of the two-pass scatter (0: one pass)
+  int32_t grp;    // node of the phase (its best bucket edge: nbest[grp])
   int64_t ridx;   // result slot (open position * D + draw)
   // node context (as node_context computes it)
   int64_t n_w;    // sum of weights
@@ -1209,6 +1091,12 @@ __device__ __forceinline__ uint32_t v2_bucket(uint32_t key, const V2Item& it) {
   return q;
 }
 
+// Fixed-point mean of a regression node: its targets are centred on it, which
+// makes the bounds tight (the gain does not depend on the centre).
+__device__ __forceinline__ int64_t v2_centre(const V2Item& it) {
+  return d2ll_rn((double)it.ssum / (double)it.n_w);
+}
+
 struct V2Tile {
   uint32_t item;
   uint32_t e0;
@@ -1223,89 +1111,55 @@ struct V2Args {
   const V2Item* items;
   int64_t n_items;
   const V2Tile* tiles;
-  // per bucket
-  uint32_t* bcount;
-  uint32_t* bmax;
-  uint32_t* bcls;   // [bucket * C + c] (classification)
-  uint32_t* bwn;    // weight sum (regression)
-  int64_t* bsum;    // target sum (regression)
-  uint32_t* bbase;  // scratch offset within the item
-  uint32_t* bcur;
-  uint32_t* bsup;   // two-pass scatter: write cursor of each super-bucket [boff + s]
-  uint32_t* carry_cls;
-  int64_t* carry_n;
-  int64_t* carry_s;
-  uint32_t* carry_last;
+  // per bucket: k_v2_hist's counts, overwritten by k_v2_bound with the totals
+  // before the bucket
+  uint32_t* bcls;   // classification [boff * C + c * nb + b]
+  uint32_t* bn;     // weights
+  int64_t* bpos;    // regression: sums of the targets above / below the node's
+  int64_t* bneg;    // centre; then bpos: target sum before the bucket
+  float* bub;       // bound of the scores inside the bucket (-1: empty)
+  uint32_t* nbest;  // per node of the phase: best edge score (float bits)
+  float best_cap;   // edges above this count as this (retry phase)
+  double max_dev;   // regression: largest |fixed target|
+  uint32_t* bslot;  // scratch slot of a selected bucket (kNone: not selected)
+  uint32_t* bnext;  // selected bucket whose lower neighbour this is (kNone: none)
+  uint32_t* bcur;   // entries collected
+  uint32_t* carry_last;  // last key before the bucket
+  uint32_t* isel;   // per item: selected buckets
   double* res_g;
   uint32_t* res_key;
   uint32_t* res_prev;
-  // scratch, item-major, bucket order
+  uint32_t* gkey;   // keys in entry order, item-major
+  // scratch slots of the selected buckets
   uint32_t* skey;
   uint32_t* saux;
   int64_t* sy;
-  uint32_t* skey2;  // overfull buckets: fine sub-bucket order
-  uint32_t* gkey;   // keys in entry order (histogram -> scatter; aliases skey2)
+  uint32_t* skey2;  // k_v2_spill: fine sub-bucket order (skey2 aliases gkey)
   uint32_t* saux2;
   int64_t* sy2;
-  uint32_t* tkey;   // two-pass scatter: keys in super-bucket order (aux, y in saux2, sy2)
   // task lists
   V2Task* tasks;
   V2Task* spill;
-  unsigned int* counters;  // [0] tasks, [1] spill
+  unsigned int* counters;  // [0] tasks, [1] spill, [2] scratch slots
 };
 
-// Exclusive max-scan over a team (one wave, or the 256-thread workgroup with
-// kWaves words in s_w).
-template <int TEAM>
-__device__ __forceinline__ uint32_t team_excl_max(uint32_t v, uint32_t* s_w) {
-  const int lane = threadIdx.x & (kWave - 1);
-  uint32_t inc = v;
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t y = __shfl_up(inc, off, kWave);
-    if (lane >= off) inc = max(inc, y);
-  }
-  uint32_t exc = __shfl_up(inc, 1, kWave);
-  if (lane == 0) exc = 0;
-  if constexpr (TEAM == kWave) {
-    return exc;
-  } else {
-    const int w = threadIdx.x / kWave;
-    if (lane == kWave - 1) s_w[w] = inc;
-    __syncthreads();
-    uint32_t pre = 0;
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) pre = (i < w) ? max(pre, s_w[i]) : pre;
-    __syncthreads();
-    return max(pre, exc);
-  }
-}
-
-// Items with at most kV2SmallB buckets take one wave in the per-item passes
-// (offsets, carries); larger ones a workgroup.
-constexpr int kV2SmallB = 256;
-
-// The item of a per-item team: list[team], teams of TEAM threads.
-template <int TEAM>
-__device__ __forceinline__ int64_t v2_team_item(const uint32_t* list, int64_t n_list) {
-  const int64_t k = TEAM == kWave ? (int64_t)blockIdx.x * kWaves + threadIdx.x / kWave : (int64_t)blockIdx.x;
-  return k < n_list ? (int64_t)list[k] : -1;
-}
-
 // Tiles are issued feature-major and split in eighths across the XCDs (see
-// big_pipeline): a larger grid of smaller bucket tables was slower, since
-// more tiles in flight gather from more columns of K at once.
+// big_pipeline).  The bucket table lives in dynamic LDS: [c * nb + b] class
+// counts, or nb sums above, nb sums below, nb weights.
 template <int TASK>
 __global__ void __launch_bounds__(kBlock) k_v2_hist(DataArgs d, LevelArgs lv, V2Args a) {
-  __shared__ uint32_t s_cnt[kV2MaxB];
-  __shared__ uint32_t s_max[kV2MaxB];
+  extern __shared__ uint64_t s_tab[];
   const V2Tile tl = a.tiles[blockIdx.x];
   const V2Item it = a.items[tl.item];
   const int t = threadIdx.x;
-  for (int b = t; b < it.nb; b += kBlock) {
-    s_cnt[b] = 0;
-    s_max[b] = 0;
-  }
+  const int nb = it.nb;
+  uint32_t* s_cls = reinterpret_cast<uint32_t*>(s_tab);
+  unsigned long long* s_pos = reinterpret_cast<unsigned long long*>(s_tab);
+  unsigned long long* s_neg = s_pos + nb;
+  uint32_t* s_n = reinterpret_cast<uint32_t*>(s_neg + nb);
+  const int words = TASK == 0 ? nb * d.C : nb * kV2RegWords;
+  for (int b = t; b < words; b += kBlock) s_cls[b] = 0;
+  const int64_t mu = TASK == 1 ? v2_centre(it) : 0;
   __syncthreads();
   const uint32_t* Kf = d.K + (int64_t)it.f * d.N;
   const int n = min(kV2Tile, it.m - (int)tl.e0);
@@ -1313,328 +1167,486 @@ __global__ void __launch_bounds__(kBlock) k_v2_hist(DataArgs d, LevelArgs lv, V2
   uint32_t* gkey = a.gkey + it.soff + tl.e0;
   constexpr int U = 8;
   for (int base = 0; base < n; base += kBlock * U) {
-    uint32_t rows[U];
-#pragma unroll
-    for (int q = 0; q < U; ++q) {
-      const int e = base + t + q * kBlock;
-      if (e < n) rows[q] = lv.row[e0 + e];
-    }
+    uint32_t rows[U], aux[U], keys[U];
+    int64_t y[TASK == 1 ? U : 1];
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       const int e = base + t + q * kBlock;
       if (e < n) {
-        const uint32_t key = Kf[rows[q]];
-        gkey[e] = key;
-        const uint32_t b = v2_bucket(key, it);
-        atomicAdd(&s_cnt[b], 1u);
-        atomicMax(&s_max[b], key);
+        rows[q] = lv.row[e0 + e];
+        aux[q] = lv.aux[e0 + e];
+        if (TASK == 1) y[q] = lv.ey[e0 + e];
       }
     }
-  }
-  __syncthreads();
-  for (int b = t; b < it.nb; b += kBlock) {
-    const uint32_t c = s_cnt[b];
-    if (!c) continue;
-    const int64_t gb = (int64_t)it.boff + b;
-    atomicAdd(&a.bcount[gb], c);
-    atomicMax(&a.bmax[gb], s_max[b]);
-  }
-}
-
-// One team per item: offsets, last key before each bucket, task lists.
-template <int TEAM>
-__global__ void __launch_bounds__(kBlock) k_v2_scan(V2Args a, const uint32_t* list, int64_t n_list) {
-  __shared__ uint32_t s_w[kWaves];
-  __shared__ uint32_t s_base[kWaves][2];
-  const int64_t k = v2_team_item<TEAM>(list, n_list);
-  if (k < 0) return;  // team-uniform; wave teams have no workgroup barrier
-  const V2Item it = a.items[k];
-  const int t = team_tid<TEAM>();
-  uint32_t* sb = s_base[TEAM == kWave ? threadIdx.x / kWave : 0];
-  constexpr int PER = (TEAM == kWave ? kV2SmallB : kV2MaxB) / TEAM;  // buckets per thread
-  const int b0 = t * PER;
-  const int64_t gb0 = (int64_t)it.boff + b0;
-  uint32_t cnt[PER], mx[PER];
-  uint32_t lcnt = 0, lmax = 0, n_norm = 0, n_spill = 0;
 #pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const bool ok = b0 + q < it.nb;
-    cnt[q] = ok ? a.bcount[gb0 + q] : 0u;
-    mx[q] = ok ? a.bmax[gb0 + q] : 0u;
-    lcnt += cnt[q];
-    if (cnt[q]) {
-      lmax = max(lmax, mx[q]);
-      if (cnt[q] > (uint32_t)kV2WaveCap) ++n_spill;
-      else ++n_norm;
-    }
-  }
-  uint32_t off = team_excl_scan<TEAM>(lcnt, s_w, nullptr);
-  uint32_t last = team_excl_max<TEAM>(lmax, s_w);
-  uint32_t tot_norm = 0, tot_spill = 0;
-  const uint32_t pn = team_excl_scan<TEAM>(n_norm, s_w, &tot_norm);
-  const uint32_t ps = team_excl_scan<TEAM>(n_spill, s_w, &tot_spill);
-  if (t == 0) {
-    sb[0] = tot_norm ? atomicAdd(&a.counters[0], tot_norm) : 0u;
-    sb[1] = tot_spill ? atomicAdd(&a.counters[1], tot_spill) : 0u;
-  }
-  team_sync<TEAM>();
-  uint32_t in = sb[0] + pn, is = sb[1] + ps;
+    for (int q = 0; q < U; ++q)
+      if (base + t + q * kBlock < n) keys[q] = Kf[rows[q]];
 #pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    if (b0 + q >= it.nb) break;
-    const int64_t gb = gb0 + q;
-    a.bbase[gb] = off;
-    a.bcur[gb] = off;
-    if (it.sgrp > 0 && (b0 + q) % it.sgrp == 0) a.bsup[(int64_t)it.boff + (b0 + q) / it.sgrp] = off;
-    a.carry_last[gb] = last;
-    off += cnt[q];
-    if (!cnt[q]) continue;
-    last = max(last, mx[q]);
-    const V2Task tk{(uint32_t)k, (uint32_t)(b0 + q)};
-    if (cnt[q] > (uint32_t)kV2WaveCap)
-      a.spill[is++] = tk;
-    else
-      a.tasks[in++] = tk;
-  }
-}
-
-// Entries of one tile into bucket order.  Each entry takes a rank inside its
-// bucket from an LDS counter, the tile reserves one run per bucket in the
-// item's scratch, and the entries are staged in LDS in (bucket, rank) order
-// so that consecutive threads write consecutive slots of a run.
-// Items of at most kV2FewB (kV2MidB) buckets take the scatter variants with
-// small bucket tables (less LDS: three workgroups per CU instead of two).
-//
-// Items with more than kV2MidB buckets hold about one entry per bucket in a
-// tile, or a fraction of one, so a one-pass scatter writes runs of about one
-// entry: every write touches its own cache line.  They go in two passes
-// over the same tiles (MODE 1, then MODE 2): first into kV2Super
-// super-buckets of sgrp consecutive buckets each (runs of tens of entries,
-// into tkey / saux2 / sy2), then each tile of that super-bucket order into
-// its buckets -- a tile now spans one or two super-buckets, so its runs are
-// long again.
-// Entry order inside a bucket is not used by the evaluation (it sorts).
-constexpr int kV2FewB = 512;
-constexpr int kV2MidB = 1024;
-constexpr int kV2Super = 64;
-
-template <int TASK, int MAXB, int MODE = 0>
-__global__ void __launch_bounds__(kBlock) k_v2_scatter(DataArgs d, LevelArgs lv, V2Args a) {
-  constexpr int TILE = TASK == 0 ? kScatterTile : 2048;
-  constexpr int U = TILE / kBlock;
-  __shared__ uint32_t s_cnt[MAXB];
-  __shared__ uint32_t s_gpos[MAXB];
-  __shared__ uint32_t s_key[TILE];
-  __shared__ uint32_t s_aux[TILE];
-  __shared__ uint16_t s_b[TILE];
-  __shared__ int64_t s_y[TASK == 1 ? TILE : 1];
-  __shared__ uint32_t s_w[kWaves];
-  const V2Tile tl = a.tiles[blockIdx.x];
-  const V2Item it = a.items[tl.item];
-  const int t = threadIdx.x;
-  const int n = min(TILE, it.m - (int)tl.e0);
-  // input: keys in entry order (MODE 0 / 1) or in super-bucket order (MODE 2)
-  const uint32_t* gkey = (MODE == 2 ? a.tkey : a.gkey) + it.soff + tl.e0;
-  const uint32_t* gaux = MODE == 2 ? a.saux2 + it.soff + tl.e0 : lv.aux + it.start + tl.e0;
-  const int64_t* gy = MODE == 2 ? a.sy2 + it.soff + tl.e0 : lv.ey + it.start + tl.e0;
-  // table slots: bucket (MODE 0), super-bucket (MODE 1), bucket - b_lo (MODE 2)
-  int b_lo = 0, n_slots = it.nb;
-  if (MODE == 1) n_slots = (it.nb + it.sgrp - 1) / it.sgrp;
-  if (MODE == 2) {
-    const int s_first = (int)v2_bucket(gkey[0], it) / it.sgrp;
-    const int s_last = (int)v2_bucket(gkey[n - 1], it) / it.sgrp;
-    b_lo = s_first * it.sgrp;
-    n_slots = min(it.nb, (s_last + 1) * it.sgrp) - b_lo;
-  }
-  auto slot_of = [&](uint32_t key) -> int {
-    const int b = (int)v2_bucket(key, it);
-    return MODE == 1 ? b / it.sgrp : b - b_lo;
-  };
-  for (int b = t; b < n_slots; b += kBlock) s_cnt[b] = 0;
-  __syncthreads();
-  uint32_t keys[U], auxv[U], rank[U];
-  int64_t yv[U];
-#pragma unroll
-  for (int q = 0; q < U; ++q) {
-    const int e = t + q * kBlock;
-    if (e < n) {
-      keys[q] = gkey[e];
-      auxv[q] = gaux[e];
-      if (TASK == 1) yv[q] = gy[e];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < U; ++q) {
-    const int e = t + q * kBlock;
-    if (e < n) rank[q] = atomicAdd(&s_cnt[slot_of(keys[q])], 1u);
-  }
-  __syncthreads();
-  {
-    // slots in chunks of PER per thread (several rounds for a MODE 2 table)
-    constexpr int PER = MAXB / kBlock > 0 ? MAXB / kBlock : 1;
-    uint32_t* cur = MODE == 1 ? a.bsup : a.bcur;
-    const int64_t cbase = (int64_t)it.boff + (MODE == 2 ? b_lo : 0);
-    const int b0 = t * PER;
-    uint32_t c[PER], loc = 0;
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      c[q] = b0 + q < n_slots ? s_cnt[b0 + q] : 0u;
-      loc += c[q];
-    }
-    uint32_t off = team_excl_scan<256>(loc, s_w, nullptr);
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      if (b0 + q >= n_slots) break;
-      s_cnt[b0 + q] = off;  // local offset of the slot's run
-      s_gpos[b0 + q] = c[q] ? atomicAdd(&cur[cbase + b0 + q], c[q]) : 0u;
-      off += c[q];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < U; ++q) {
-    const int e = t + q * kBlock;
-    if (e < n) {
-      const int b = slot_of(keys[q]);
-      const uint32_t li = s_cnt[b] + rank[q];
-      s_key[li] = keys[q];
-      s_aux[li] = auxv[q];
-      s_b[li] = (uint16_t)b;
-      if (TASK == 1) s_y[li] = yv[q];
-    }
-  }
-  __syncthreads();
-  uint32_t* okey = MODE == 1 ? a.tkey : a.skey;
-  uint32_t* oaux = MODE == 1 ? a.saux2 : a.saux;
-  int64_t* oy = MODE == 1 ? a.sy2 : a.sy;
-  for (int i = t; i < n; i += kBlock) {
-    const uint32_t b = s_b[i];
-    const int64_t pos = it.soff + s_gpos[b] + (uint32_t)i - s_cnt[b];
-    okey[pos] = s_key[i];
-    oaux[pos] = s_aux[i];
-    if (TASK == 1) oy[pos] = s_y[i];
-  }
-}
-
-// One workgroup per tile of kV2CTile buckets of an item, one wave per
-// bucket: class totals (regression: weight and target sums) of each
-// bucket's entries.
-constexpr int kV2CTile = 64;
-
-template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock) k_v2_ctot(DataArgs d, V2Args a) {
-  __shared__ uint32_t s_c[kWaves][MAXC];
-  const int lane = threadIdx.x & (kWave - 1);
-  const V2Tile tl = a.tiles[blockIdx.x];
-  const V2Item it = a.items[tl.item];
-  const int b_end = min(it.nb, (int)tl.e0 + kV2CTile);
-  for (int b = (int)tl.e0 + threadIdx.x / kWave; b < b_end; b += kWaves) {
-    const int64_t gb = (int64_t)it.boff + b;
-    const uint32_t n = a.bcount[gb];
-    const int64_t e0 = it.soff + a.bbase[gb];
-    if constexpr (TASK == 0) {
-      uint32_t* sc = s_c[threadIdx.x / kWave];
-      if (lane < MAXC) sc[lane] = 0u;
-      team_sync<kWave>();
-      constexpr int U = 4;
-      for (uint32_t e = lane; e < n; e += kWave * U) {
-        uint32_t x[U];
-#pragma unroll
-        for (int q = 0; q < U; ++q) x[q] = e + q * kWave < n ? a.saux[e0 + e + q * kWave] : 0u;
-#pragma unroll
-        for (int q = 0; q < U; ++q)
-          if (e + q * kWave < n) atomicAdd(&sc[x[q] >> 16], x[q] & 0xFFFFu);
-      }
-      team_sync<kWave>();
-      if (lane < d.C) a.bcls[gb * d.C + lane] = sc[lane];
-      team_sync<kWave>();
-    } else {
-      int64_t wn = 0, ws = 0;
-      for (uint32_t e = lane; e < n; e += kWave) {
-        const int64_t w = (int64_t)(a.saux[e0 + e] & 0xFFFFu);
-        wn += w;
-        ws += w * a.sy[e0 + e];
-      }
-#pragma unroll
-      for (int off = kWave / 2; off > 0; off >>= 1) {
-        wn += __shfl_xor(wn, off, kWave);
-        ws += __shfl_xor(ws, off, kWave);
-      }
-      if (lane == 0) {
-        a.bwn[gb] = (uint32_t)wn;
-        a.bsum[gb] = ws;
-      }
-    }
-  }
-}
-
-// One team per item: totals before each bucket.
-template <int TASK, int TEAM>
-__global__ void __launch_bounds__(kBlock) k_v2_carry(DataArgs d, V2Args a, const uint32_t* list, int64_t n_list) {
-  __shared__ uint32_t s_w[8 * kWaves + kWaves];
-  __shared__ int64_t s_w64[kWaves];
-  const int64_t ki = v2_team_item<TEAM>(list, n_list);
-  if (ki < 0) return;  // team-uniform; wave teams have no workgroup barrier
-  const V2Item it = a.items[ki];
-  const int t = team_tid<TEAM>();
-  const int C = d.C;
-  constexpr int PER = (TEAM == kWave ? kV2SmallB : kV2MaxB) / TEAM;
-  const int b0 = t * PER;
-  const int64_t gb0 = (int64_t)it.boff + b0;
-  if constexpr (TASK == 0) {
-    int64_t lw = 0;
-    for (int q = 0; q < PER && b0 + q < it.nb; ++q)
-      for (int c = 0; c < C; ++c) lw += a.bcls[(gb0 + q) * C + c];
-    int64_t run_n = team_excl_scan_i64<TEAM>(lw, s_w64, nullptr);
-    for (int q = 0; q < PER && b0 + q < it.nb; ++q) {
-      a.carry_n[gb0 + q] = run_n;
-      for (int c = 0; c < C; ++c) run_n += a.bcls[(gb0 + q) * C + c];
-    }
-    for (int c0 = 0; c0 < C; c0 += 8) {
-      uint32_t v[8], tot[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        v[k] = 0;
-        if (c0 + k < C)
-          for (int q = 0; q < PER && b0 + q < it.nb; ++q) v[k] += a.bcls[(gb0 + q) * C + c0 + k];
-      }
-      team_excl_scan_vec<TEAM, 8>(v, s_w, tot);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (c0 + k >= C) continue;
-        uint32_t r = v[k];
-        for (int q = 0; q < PER && b0 + q < it.nb; ++q) {
-          const int64_t gb = gb0 + q;
-          a.carry_cls[gb * C + c0 + k] = r;
-          r += a.bcls[gb * C + c0 + k];
+    for (int q = 0; q < U; ++q) {
+      const int e = base + t + q * kBlock;
+      if (e < n) {
+        gkey[e] = keys[q];
+        const uint32_t b = v2_bucket(keys[q], it);
+        const uint32_t w = aux[q] & 0xFFFFu;
+        if (TASK == 0) {
+          atomicAdd(&s_cls[(aux[q] >> 16) * (uint32_t)nb + b], w);
+        } else {
+          const int64_t dy = y[q] - mu;
+          atomicAdd(&s_n[b], w);
+          atomicAdd(dy < 0 ? &s_neg[b] : &s_pos[b], (unsigned long long)((int64_t)w * dy));
         }
       }
     }
-  } else {
-    int64_t lw = 0, ls = 0;
-    for (int q = 0; q < PER && b0 + q < it.nb; ++q) {
-      lw += a.bwn[gb0 + q];
-      ls += a.bsum[gb0 + q];
+  }
+  __syncthreads();
+  const bool only = it.m <= kV2Tile;  // the item's only tile: plain stores
+  if (TASK == 0) {
+    uint32_t* g = a.bcls + (int64_t)it.boff * d.C;
+    for (int i = t; i < words; i += kBlock) {
+      const uint32_t v = s_cls[i];
+      if (only) g[i] = v;
+      else if (v) atomicAdd(&g[i], v);
     }
-    int64_t run_n = team_excl_scan_i64<TEAM>(lw, s_w64, nullptr);
-    int64_t run_s = team_excl_scan_i64<TEAM>(ls, s_w64, nullptr);
-    for (int q = 0; q < PER && b0 + q < it.nb; ++q) {
-      const int64_t gb = gb0 + q;
-      a.carry_n[gb] = run_n;
-      a.carry_s[gb] = run_s;
-      run_n += a.bwn[gb];
-      run_s += a.bsum[gb];
+  } else {
+    for (int b = t; b < nb; b += kBlock) {
+      const int64_t gb = (int64_t)it.boff + b;
+      const uint32_t w = s_n[b];
+      if (only) {
+        a.bn[gb] = w;
+        a.bpos[gb] = (int64_t)s_pos[b];
+        a.bneg[gb] = (int64_t)s_neg[b];
+      } else if (w) {
+        atomicAdd(&a.bn[gb], w);
+        atomicAdd(reinterpret_cast<unsigned long long*>(&a.bpos[gb]), s_pos[b]);
+        atomicAdd(reinterpret_cast<unsigned long long*>(&a.bneg[gb]), s_neg[b]);
+      }
     }
   }
 }
 
+// Largest distance (in units of x) between x ln x and its chord over an
+// interval of s that starts at a: at most s / e (a = 0), and s^2 / 8 times the
+// largest curvature 1 / a.
+__device__ __forceinline__ double chord_gap(double a, double s) {
+  const double e = s * 0.36787944117144233;
+  return a > 0.0 ? fmin(e, s * s / (8.0 * a)) : e;
+}
+
+// Units of the fixed-point entropy sums that cover the difference between the
+// fixed-point terms and the double arithmetic of the bounds: each term is at
+// most 2^62 / (2C + 2) units and off by 7e-16 of that (its series) and half a
+// unit, a few tens of terms and roundings of 1.1e-16 each.
+constexpr double kBoundUnits = 131072.0;
+
+// Value of the lane below (lane 0: `first`), and of the last lane.
+__device__ __forceinline__ double lane_below(double v, double first) {
+  const double y = __shfl_up(v, 1, kWave);
+  return (threadIdx.x & (kWave - 1)) == 0 ? first : y;
+}
+__device__ __forceinline__ double wave_last_f64(double v) {
+  return __builtin_bit_cast(double, wave_last_i64(__builtin_bit_cast(int64_t, v)));
+}
+
+// variance_gain takes the difference of two rounded means: it is off by up to
+// 2^-50 of their size, so a computed gain g and the real one f, both sums over
+// the node, satisfy |sqrt g - sqrt f| <= e = sqrt(N) / 2 * 2^-50 max|y|, hence
+// g <= f (1 + t) + e^2 (1 + 1 / t), and the same with f and g exchanged.  The
+// bounds take t = 1e-6; this is the second term.
+__device__ __forceinline__ double reg_gain_error(double N, double y_max) {
+  const double e = y_max * 8.8817841970012523e-16;
+  return 0.25 * N * e * e * 1.1e6;
+}
+
+// Upper bound of the variance criterion over left weights [n0, n1] and left
+// target sums [lo, hi], for a node of weight N, target sum S and largest
+// deviation M: f(n, s) = s^2 / n + (S - s)^2 / (N - n) is convex, so its
+// maximum over the box is at a corner; a side that may be empty has a mean of
+// at most M, so its term is at most |sum| M.
+__device__ __forceinline__ double reg_box_bound(double n0, double n1, double lo, double hi, double N, double S,
+                                                double M) {
+  const double a = lo * lo, b = hi * hi, c = (S - lo) * (S - lo), e = (S - hi) * (S - hi);
+  if (n0 > 0.0 && n1 < N) {
+    const double l0 = 1.0 / n0, l1 = 1.0 / n1, r0 = 1.0 / (N - n0), r1 = 1.0 / (N - n1);
+    const double f0 = fmax(a * l0 + c * r0, b * l0 + e * r0);
+    const double f1 = fmax(a * l1 + c * r1, b * l1 + e * r1);
+    return fmax(f0, f1) - S * S / N;
+  }
+  const double left = n0 > 0.0 ? fmax(a, b) / n0 : fmax(fabs(lo), fabs(hi)) * M;
+  const double right = n1 < N ? fmax(c, e) / (N - n1) : fmax(fabs(S - lo), fabs(S - hi)) * M;
+  return left + right;
+}
+
+// One wave per item, 64 buckets at a time.  Per bucket: totals before it (in
+// place of the counts), the gain at its lower edge, and a bound of every gain
+// inside it.  Classification: with phi_c(x) = T(x) + T(n_c - x) and
+// psi(x) = T(x) + T(n - x), both convex, the gain sum is
+// P + sum_c phi_c(l_c) - psi(sum_c l_c).  Between the bucket's ends each phi_c
+// tilted by the chord slope of psi stays below the larger of its ends, and psi
+// less its own chord stays above -chord_gap, so
+//   gain <= edge + sum_c max(0, phi_c(end) - phi_c(start) - slope s_c) + gap.
+template <int MAXC, int TASK>
+__global__ void __launch_bounds__(kBlock) k_v2_bound(DataArgs d, LevelArgs lv, V2Args a) {
+  __shared__ double s_inv[128], s_logc[128];
+  load_tables(s_inv, s_logc);
+  __syncthreads();
+  const int64_t k = (int64_t)blockIdx.x * kWaves + threadIdx.x / kWave;
+  if (k >= a.n_items) return;  // wave-uniform; no workgroup barrier follows
+  const V2Item it = a.items[k];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int nb = it.nb;
+  float best = 0.0f;
+  if constexpr (TASK == 0) {
+    // x ln x in double from the reduction table in LDS: the counts of a big
+    // node spread over an 8 MB table of terms, and 4 reads per class and
+    // bucket of it took 0.45 ms per phase of a 32-tree 1M-row level.
+    auto xl = [&](uint32_t x) { return xlnx(x, s_inv, s_logc); };
+    const int C = d.C;
+    uint32_t* cls = a.bcls + (int64_t)it.boff * C;
+    uint32_t run[MAXC], ncl[MAXC];
+    double phi_row[MAXC];  // phi_c before the row
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+      run[c] = 0;
+      ncl[c] = c < C ? lv.cls[(int64_t)it.node * C + c] : 0u;
+      phi_row[c] = c < C ? xl(ncl[c]) : 0.0;
+    }
+    const uint32_t n_w = (uint32_t)it.n_w;
+    const double P = ldexp_d((double)it.P, -d.igF);
+    const double margin = ldexp_d(kBoundUnits, -d.igF);
+    uint32_t run_n = 0;
+    double psi_row = xl(n_w);  // psi before the row
+    for (int b0 = 0; b0 < nb; b0 += kWave) {
+      const int b = b0 + lane;
+      const bool ok = b < nb;
+      uint32_t v[MAXC], sw = 0;
+#pragma unroll
+      for (int c = 0; c < MAXC; ++c) {
+        v[c] = c < C && ok ? cls[c * nb + b] : 0u;
+        sw += v[c];
+      }
+      // values at the bucket's end; its start is the end of the lane below
+      const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
+      run_n = wave_last(lb);
+      const double psb = xl(lb) + xl(n_w - lb);
+      const double psa = lane_below(psb, psi_row);
+      psi_row = wave_last_f64(psb);
+      const double slope = sw ? (psb - psa) / (double)sw : 0.0;
+      double phi = 0.0, slack = 0.0;
+#pragma unroll
+      for (int c = 0; c < MAXC; ++c) {
+        if (c < C) {
+          const uint32_t l = run[c] + wave_incl_scan(v[c]);
+          run[c] = wave_last(l);
+          const double pb = xl(l) + xl(ncl[c] - l);
+          const double pa = lane_below(pb, phi_row[c]);
+          phi_row[c] = wave_last_f64(pb);
+          phi += pa;
+          slack += fmax(0.0, (pb - pa) - slope * (double)v[c]);
+          if (ok) cls[c * nb + b] = l - v[c];
+        }
+      }
+      slack += chord_gap((double)la, (double)sw) + chord_gap((double)(n_w - lb), (double)sw);
+      const double edge = P + phi - psa;
+      float ub = -1.0f;
+      if (sw) {
+        // nats to bits per unit weight, as ig_from_fixed
+        ub = (float)((edge + slack * (1.0 + 1e-9) + margin) * it.inv * (1.0 + 1e-12));
+        if (la > 0) best = fmaxf(best, (float)((edge - margin) * it.inv * (1.0 - 1e-12)));
+        if (it.width == 1) {  // one key: no boundary but the lower edge
+          const LnCtx lx{s_inv, s_logc, d.T, d.Tmax, d.igF};
+          int64_t e = it.P - lx.t(la) - lx.t(n_w - la);
+#pragma unroll
+          for (int c = 0; c < MAXC; ++c)
+            if (c < C) {
+              const uint32_t l = cls[c * nb + b];  // stored above by this lane
+              e += lx.t(l) + lx.t(ncl[c] - l);
+            }
+          const double g = la > 0 ? ig_from_fixed(e, d.igF, it.inv) : 0.0;
+          a.res_g[(int64_t)it.boff + b] = g;
+          ub = fmaxf((float)g, 0.0f);
+        }
+      }
+      if (ok) {
+        a.bn[(int64_t)it.boff + b] = la;
+        a.bub[(int64_t)it.boff + b] = it.P > 0 ? ub : -1.0f;  // P = 0: pure node, every gain is 0
+      }
+    }
+  } else {
+    const int64_t mu = v2_centre(it);
+    const double M = a.max_dev + fabs((double)mu), E = reg_gain_error((double)it.n_w, a.max_dev);
+    const double N = (double)it.n_w, S = (double)(it.ssum - mu * it.n_w);
+    uint32_t run_n = 0;
+    int64_t run_s = 0;  // centred sum before the row
+    for (int b0 = 0; b0 < nb; b0 += kWave) {
+      const int b = b0 + lane;
+      const bool ok = b < nb;
+      const int64_t gb = (int64_t)it.boff + b;
+      const uint32_t w = ok ? a.bn[gb] : 0u;
+      const int64_t sp = ok ? a.bpos[gb] : 0, sn = ok ? a.bneg[gb] : 0;
+      const uint32_t inc = wave_incl_scan(w);
+      const uint32_t la = run_n + inc - w;
+      run_n += wave_last(inc);
+      const int64_t is = wave_incl_scan_i64(sp + sn);
+      const int64_t sa = run_s + is - (sp + sn);
+      run_s += wave_last_i64(is);
+      const int64_t su = sa + mu * (int64_t)la;  // uncentred target sum before the bucket
+      float ub = -1.0f;
+      if (w) {
+        const double u = reg_box_bound((double)la, (double)(la + w), (double)(sa + sn), (double)(sa + sp), N, S, M);
+        ub = (float)ldexp_d(u * (1.0 + 2e-6) + E, -2 * d.shift);
+        if (la > 0) {
+          const double g = variance_gain(la, su, it.n_w - la, it.ssum - su, 0);
+          best = fmaxf(best, (float)ldexp_d(g, -2 * d.shift));
+          if (it.width == 1) {
+            a.res_g[gb] = g;
+            ub = (float)ldexp_d(g, -2 * d.shift);
+          }
+        } else if (it.width == 1) {
+          ub = 0.0f;
+        }
+      }
+      if (ok) {
+        a.bn[gb] = la;
+        a.bpos[gb] = su;
+        a.bub[gb] = ub;
+      }
+    }
+  }
+  // scores are at least 0: their bits order as unsigned words
+  const uint32_t bits = wave_max_u32(__float_as_uint(best));
+  if (lane == 0 && bits) atomicMax(&a.nbest[it.grp], bits);
+}
+
+// One wave per item: selects the buckets whose bound reaches the node's best
+// edge, from the last bucket down (a bucket that precedes a selected one keeps
+// its largest key).  A selected bucket of one key (width 1) is its lower edge:
+// its result is complete here and its entries are not collected (kDone).
+constexpr uint32_t kDone = kNone - 1u;
+// The slots and list places of a workgroup's items are taken by two atomics:
+// with one per item and row, the waves queued on those words (1.1 ms of a
+// phase of 172,000 items; 4M x 64 regression).
+constexpr int kSelectWaves = 16;
+template <int TASK>
+__global__ void __launch_bounds__(kSelectWaves * kWave) k_v2_select(DataArgs d, V2Args a) {
+  __shared__ unsigned int s_cnt[kSelectWaves][3];
+  __shared__ unsigned int s_base[3];
+  const int wv = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t k = (int64_t)blockIdx.x * kSelectWaves + wv;
+  const bool live = k < a.n_items;
+  V2Item it{};
+  if (live) it = a.items[k];
+  const int nb = live ? it.nb : 0;
+  const int64_t g0 = it.boff;
+  const float thr = live ? fminf(__uint_as_float(a.nbest[it.grp]), a.best_cap) : 0.0f;
+  auto weight = [&](int b) {
+    return (b + 1 < nb ? a.bn[g0 + b + 1] : (uint32_t)it.n_w) - a.bn[g0 + b];
+  };
+  unsigned int n_small = 0, n_big = 0, n_slot = 0;
+  for (int b0 = 0; b0 < nb; b0 += kWave) {
+    const int b = b0 + lane;
+    const float u = b < nb ? a.bub[g0 + b] : -1.0f;
+    const bool sel = u > 0.0f && u >= thr;
+    if (!__ballot(sel)) continue;
+    const uint32_t w = sel ? weight(b) : 0u;
+    n_small += (unsigned int)__popcll(__ballot(sel && w <= (uint32_t)kV2WaveCap));
+    n_big += (unsigned int)__popcll(__ballot(w > (uint32_t)kV2WaveCap));
+    n_slot += wave_last(wave_incl_scan(w));
+  }
+  const unsigned int n_sel = n_small + n_big;
+  if (live && lane == 0) a.isel[k] = n_sel;
+  const bool one_key = it.width == 1;
+  if (lane == 0) {
+    s_cnt[wv][0] = one_key ? 0u : n_small;
+    s_cnt[wv][1] = one_key ? 0u : n_big;
+    s_cnt[wv][2] = one_key ? 0u : n_slot;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    unsigned int sum = 0;
+    for (int i = 0; i < kSelectWaves; ++i) {
+      const unsigned int c = s_cnt[i][threadIdx.x];
+      s_cnt[i][threadIdx.x] = sum;
+      sum += c;
+    }
+    s_base[threadIdx.x] = sum ? atomicAdd(&a.counters[threadIdx.x], sum) : 0u;
+  }
+  __syncthreads();
+  if (!n_sel) return;
+  uint32_t at_small = s_base[0] + s_cnt[wv][0], at_big = s_base[1] + s_cnt[wv][1], at_slot = s_base[2] + s_cnt[wv][2];
+  uint32_t next = kNone;  // the selected bucket next above the row, if it is the next non-empty one
+  for (int b0 = (nb - 1) / kWave * kWave; b0 >= 0; b0 -= kWave) {
+    const int b = b0 + lane;
+    const bool ok = b < nb;
+    const int64_t gb = g0 + b;
+    const float u = ok ? a.bub[gb] : -1.0f;
+    const bool full = u >= 0.0f;
+    const bool sel = u > 0.0f && u >= thr;
+    if (one_key) {
+      if (sel) {
+        const uint32_t lo = a.bn[gb];
+        int p = b - 1;  // the key before: the bucket in which the weight before b ends
+        while (a.bn[g0 + p] == lo) --p;
+        a.res_key[gb] = (uint32_t)b;
+        a.res_prev[gb] = (uint32_t)p;
+      }
+      if (ok) {
+        a.bslot[gb] = sel ? kDone : kNone;
+        a.bnext[gb] = kNone;
+      }
+      continue;
+    }
+    const uint64_t m_full = __ballot(full), m_sel = __ballot(sel);
+    // next non-empty bucket above this one
+    const uint64_t above = lane == 63 ? 0ull : m_full >> (lane + 1);
+    uint32_t nx = next;
+    if (above) {
+      const int l = lane + 1 + (int)__ffsll((unsigned long long)above) - 1;
+      nx = (m_sel >> l) & 1ull ? (uint32_t)(g0 + b0 + l) : kNone;
+    }
+    uint32_t slot = kNone;
+    if (m_sel) {
+      const uint32_t w = sel ? weight(b) : 0u;
+      const bool big = w > (uint32_t)kV2WaveCap;
+      const uint64_t m_big = __ballot(big), m_small = m_sel & ~m_big;
+      const uint32_t winc = wave_incl_scan(w);
+      const uint64_t below = (1ull << lane) - 1ull;
+      if (sel) {
+        const V2Task tk{(uint32_t)k, (uint32_t)b};
+        if (big) a.spill[at_big + (uint32_t)__popcll(m_big & below)] = tk;
+        else a.tasks[at_small + (uint32_t)__popcll(m_small & below)] = tk;
+        a.bcur[gb] = 0;
+        a.carry_last[gb] = 0;
+        slot = at_slot + winc - w;
+      }
+      at_small += (uint32_t)__popcll(m_small);
+      at_big += (uint32_t)__popcll(m_big);
+      at_slot += wave_last(winc);
+    }
+    if (ok) {
+      a.bslot[gb] = slot;
+      a.bnext[gb] = full ? nx : kNone;
+    }
+    if (m_full) {
+      const int l = (int)__ffsll((unsigned long long)m_full) - 1;
+      next = (m_sel >> l) & 1ull ? (uint32_t)(g0 + b0 + l) : kNone;
+    }
+  }
+}
+
+// Entries of the selected buckets into their scratch slots (the tiles of
+// k_v2_hist; a tile of an item without a selected bucket ends at once).  A
+// pass over the tile's keys appends the few selected entries to a list in LDS;
+// the list then takes ranks per bucket in LDS and one run per bucket in the
+// slots, so that a bucket's cursor sees one atomic per tile.  Bound by reading
+// the keys (4 B per entry).
+constexpr int kCollectCap = 4096;
+template <int TASK>
+__global__ void __launch_bounds__(kBlock) k_v2_collect(DataArgs d, LevelArgs lv, V2Args a) {
+  extern __shared__ uint64_t s_tab[];
+  __shared__ uint16_t s_list[kCollectCap];
+  __shared__ unsigned int s_n;
+  const V2Tile tl = a.tiles[blockIdx.x];
+  if (!a.isel[tl.item]) return;
+  const V2Item it = a.items[tl.item];
+  if (it.width == 1) return;
+  const int t = threadIdx.x;
+  uint32_t* s_cnt = reinterpret_cast<uint32_t*>(s_tab);  // entries taken, then first position
+  uint32_t* s_max = s_cnt + it.nb;                       // largest key (buckets below a selected one)
+  uint8_t* s_flag = reinterpret_cast<uint8_t*>(s_max + it.nb);  // 1: selected, 2: below a selected one
+  for (int b = t; b < it.nb; b += kBlock) {
+    s_cnt[b] = 0;
+    s_max[b] = 0;
+    s_flag[b] = (uint8_t)((a.bslot[(int64_t)it.boff + b] != kNone ? 1 : 0) |
+                          (a.bnext[(int64_t)it.boff + b] != kNone ? 2 : 0));
+  }
+  if (t == 0) s_n = 0;
+  __syncthreads();
+  const int n = min(kV2Tile, it.m - (int)tl.e0);
+  const int64_t e0 = it.start + tl.e0;
+  const uint32_t* gkey = a.gkey + it.soff + tl.e0;
+  const int lane = t & (kWave - 1);
+  auto flush = [&]() {
+    __syncthreads();
+    const int m = (int)s_n;
+    constexpr int R = kCollectCap / kBlock;
+    uint32_t key[R], rank[R], bk[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = t + r * kBlock;
+      if (i < m) {
+        key[r] = gkey[s_list[i]];
+        bk[r] = v2_bucket(key[r], it);
+        rank[r] = atomicAdd(&s_cnt[bk[r]], 1u);
+      }
+    }
+    __syncthreads();
+    for (int b = t; b < it.nb; b += kBlock) {
+      const uint32_t c = s_cnt[b];
+      if (c) s_cnt[b] = a.bslot[(int64_t)it.boff + b] + atomicAdd(&a.bcur[(int64_t)it.boff + b], c);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = t + r * kBlock;
+      if (i < m) {
+        const int64_t e = e0 + s_list[i];
+        const uint32_t pos = s_cnt[bk[r]] + rank[r];
+        a.skey[pos] = key[r];
+        a.saux[pos] = lv.aux[e];
+        if (TASK == 1) a.sy[pos] = lv.ey[e];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (t + r * kBlock < m) s_cnt[bk[r]] = 0;
+    if (t == 0) s_n = 0;
+    __syncthreads();
+  };
+  constexpr int U = 8;
+  for (int base = 0; base < n; base += kBlock * U) {
+    uint32_t keys[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int e = base + t + q * kBlock;
+      keys[q] = e < n ? gkey[e] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int e = base + t + q * kBlock;
+      uint32_t fl = 0;
+      if (e < n) {
+        const uint32_t b = v2_bucket(keys[q], it);
+        fl = s_flag[b];
+        if (fl & 2u) atomicMax(&s_max[b], keys[q]);
+      }
+      const uint64_t sel = __ballot(fl & 1u);
+      if (sel) {
+        unsigned int at = 0;
+        if (lane == 0) at = atomicAdd(&s_n, (unsigned int)__popcll(sel));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (fl & 1u) s_list[at + (unsigned int)__popcll(sel & ((1ull << lane) - 1ull))] = (uint16_t)e;
+      }
+    }
+    __syncthreads();
+    const bool full = s_n > (unsigned int)(kCollectCap - kBlock * U);
+    if (full) flush();  // workgroup-uniform
+    else __syncthreads();
+  }
+  flush();
+  for (int b = t; b < it.nb; b += kBlock)
+    if (s_flag[b] & 2u) atomicMax(&a.carry_last[a.bnext[(int64_t)it.boff + b]], s_max[b]);
+}
+
 template <int MAXC, int TASK, int IPT>
-__device__ __forceinline__ void v2_carry(const DataArgs& d, const V2Args& a, int64_t gb,
+__device__ __forceinline__ void v2_carry(const DataArgs& d, const V2Args& a, const V2Item& it, int64_t gb,
                                          TeamLds<MAXC, TASK, 256, IPT>& L) {
   if (threadIdx.x == 0) {
-    for (int c = 0; c < MAXC; ++c) L.cr.run[c] = (TASK == 0 && c < d.C) ? a.carry_cls[gb * d.C + c] : 0u;
-    L.cr.run_n = a.carry_n[gb];
-    L.cr.run_s = TASK == 1 ? a.carry_s[gb] : 0;
+    for (int c = 0; c < MAXC; ++c)
+      L.cr.run[c] = (TASK == 0 && c < d.C) ? a.bcls[(int64_t)it.boff * d.C + (int64_t)c * it.nb + (gb - it.boff)] : 0u;
+    L.cr.run_n = a.bn[gb];
+    L.cr.run_s = TASK == 1 ? a.bpos[gb] : 0;
     L.cr.last_key = a.carry_last[gb];
     L.cr.best_g = 0.0;
     L.cr.best_key = kNone;
@@ -1667,7 +1679,7 @@ __device__ __forceinline__ NodeCtx v2_node(const DataArgs& d, const LevelArgs& l
 template <int TASK, int IPT>
 struct V2Pre {
   int64_t gb, e0;
-  uint32_t node, kbase, bmax;
+  uint32_t node, kbase, width;
   int n;
   int64_t n_w, P, ssum;
   double inv;
@@ -1692,13 +1704,13 @@ __device__ __forceinline__ void v2_prefetch(const DataArgs& d, const LevelArgs& 
   P.P = it.P;
   P.ssum = it.ssum;
   P.inv = it.inv;
-  P.n = (int)a.bcount[P.gb];
-  P.e0 = it.soff + a.bbase[P.gb];
-  P.bmax = a.bmax[P.gb];
-  P.carry_n = a.carry_n[P.gb];
-  P.carry_s = TASK == 1 ? a.carry_s[P.gb] : 0;
+  P.width = it.width;
+  P.n = (int)a.bcur[P.gb];
+  P.e0 = a.bslot[P.gb];
+  P.carry_n = a.bn[P.gb];
+  P.carry_s = TASK == 1 ? a.bpos[P.gb] : 0;
   P.carry_last = a.carry_last[P.gb];
-  P.carry_c = (TASK == 0 && lane < d.C) ? a.carry_cls[P.gb * d.C + lane] : 0u;
+  P.carry_c = (TASK == 0 && lane < d.C) ? a.bcls[(int64_t)it.boff * d.C + (int64_t)lane * it.nb + tk.b] : 0u;
   P.ncls = (TASK == 0 && lane < d.C) ? lv.cls[(int64_t)P.node * d.C + lane] : 0u;
 #pragma unroll
   for (int k = 0; k < IPT; ++k) {
@@ -1712,7 +1724,8 @@ __device__ __forceinline__ void v2_prefetch(const DataArgs& d, const LevelArgs& 
 }
 
 template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock, MAXC <= 16 ? 3 : 1) k_v2_eval(DataArgs d, LevelArgs lv, V2Args a, int64_t n_tasks) {
+__global__ void __launch_bounds__(kBlock, MAXC <= 16 ? 3 : 1) k_v2_eval(DataArgs d, LevelArgs lv, V2Args a) {
+  const int64_t n_tasks = a.counters[0];
   static_assert(TASK == 0, "regression buckets go through k_v2_eval_reg");
   constexpr int IPT = kV2Ipt;
   __shared__ double s_inv[128], s_logc[128];
@@ -1759,7 +1772,7 @@ __global__ void __launch_bounds__(kBlock, MAXC <= 16 ? 3 : 1) k_v2_eval(DataArgs
     }
     const int64_t gb = cur.gb;
     const uint32_t kbase = cur.kbase;
-    const int bits = bit_length(cur.bmax - kbase);
+    const int bits = bit_length(cur.width - 1u);
     team_sync<kWave>();
     const int64_t qn = q + stride;
     if (qn < n_tasks) v2_prefetch<TASK, IPT>(d, lv, a, qn, cur);
@@ -1844,7 +1857,8 @@ __device__ void eval_sorted_reg_wave(const uint32_t* keys, const uint16_t* vals,
 // k_v2_eval for regression: one wave per bucket, the same task order, sorts
 // and walk, with the payloads written to LDS only once the bucket is sorted.
 template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock, 3) k_v2_eval_reg(DataArgs d, LevelArgs lv, V2Args a, int64_t n_tasks) {
+__global__ void __launch_bounds__(kBlock, 3) k_v2_eval_reg(DataArgs d, LevelArgs lv, V2Args a) {
+  const int64_t n_tasks = a.counters[0];
   static_assert(TASK == 1, "regression only");
   constexpr int IPT = kV2Ipt;
   constexpr int kSpan = RegWaveLds<IPT>::SPAN;
@@ -1887,7 +1901,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_v2_eval_reg(DataArgs d, LevelArgs
     }
     const int64_t gb = cur.gb;
     const uint32_t kbase = cur.kbase;
-    const int bits = bit_length(cur.bmax - kbase);
+    const int bits = bit_length(cur.width - 1u);
     team_sync<kWave>();
     const int64_t qn = q + stride;
     if (qn < n_tasks) v2_prefetch<TASK, IPT>(d, lv, a, qn, cur);
@@ -1927,7 +1941,9 @@ __global__ void __launch_bounds__(kBlock, 3) k_v2_eval_reg(DataArgs d, LevelArgs
 // range, packed into LDS-sized chunks or read through an LDS histogram
 // (a single sub-bucket above the capacity: heavy ties), walked in order.
 template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock) k_v2_spill(DataArgs d, LevelArgs lv, V2Args a, int64_t n_spill) {
+__global__ void __launch_bounds__(kBlock) k_v2_spill(DataArgs d, LevelArgs lv, V2Args a) {
+  const int64_t n_spill = a.counters[1];
+  if ((int64_t)blockIdx.x >= n_spill) return;
   constexpr int IPT = kIpt;
   constexpr int CAP = kCap;
   __shared__ double s_inv[128], s_logc[128];
@@ -1941,12 +1957,12 @@ __global__ void __launch_bounds__(kBlock) k_v2_spill(DataArgs d, LevelArgs lv, V
     const V2Task tk = a.spill[q];
     const V2Item it = a.items[tk.item];
     const int64_t gb = (int64_t)it.boff + tk.b;
-    const int n = (int)a.bcount[gb];
-    const int64_t e0 = it.soff + a.bbase[gb];
+    const int n = (int)a.bcur[gb];
+    const int64_t e0 = a.bslot[gb];
     const uint32_t klo = tk.b * it.width;
-    const uint32_t span = a.bmax[gb] - klo + 1u;
+    const uint32_t span = min(it.width, d.S[it.f] - klo);
     const NodeCtx nc = v2_node(d, lv, it, L);
-    v2_carry<MAXC, TASK, IPT>(d, a, gb, L);
+    v2_carry<MAXC, TASK, IPT>(d, a, it, gb, L);
     __syncthreads();
     if (n <= CAP) {
       // within the workgroup's LDS chunk: one sort and walk
@@ -2059,9 +2075,10 @@ __global__ void __launch_bounds__(kBlock) k_v2_reduce(DataArgs d, V2Args a, Item
   if (k >= a.n_items) return;
   const V2Item bi = a.items[k];
   BestCand b{0.0, kNone, kNone};
-  for (int q = lane; q < bi.nb; q += kWave) {
+  const int nb = a.isel[k] ? bi.nb : 0;
+  for (int q = lane; q < nb; q += kWave) {
     const int64_t gb = (int64_t)bi.boff + q;
-    if (!a.bcount[gb]) continue;
+    if (a.bslot[gb] == kNone) continue;
     const uint32_t key = a.res_key[gb];
     if (key != kNone && cand_better(a.res_g[gb], key, b.g, b.key)) b = BestCand{a.res_g[gb], key, a.res_prev[gb]};
   }
@@ -2081,7 +2098,7 @@ __global__ void __launch_bounds__(kBlock) k_v2_reduce(DataArgs d, V2Args a, Item
 
 // Item table of a phase: one item per (big group, draw).
 __global__ void k_v2_items(DataArgs d, LevelArgs lv, const uint32_t* groups, int64_t n_groups, int per_group, int j0,
-                           int D, int nb_cap, int target, V2Item* items) {
+                           int D, int nb_cap, int target, const float* res_score, uint32_t* nbest, V2Item* items) {
   const int64_t n = n_groups * per_group;
   for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
     const uint32_t o = groups[k / per_group];
@@ -2104,7 +2121,12 @@ __global__ void k_v2_items(DataArgs d, LevelArgs lv, const uint32_t* groups, int
     b.soff = 0;
     b.boff = 0;
     b.node = i;
-    b.sgrp = 0;
+    b.grp = (int)(k / per_group);
+    if (j == j0) {  // the node's best score so far: the draws before this phase
+      float best = 0.0f;
+      for (int q = 0; q < j0; ++q) best = fmaxf(best, res_score[(int64_t)o * D + q]);
+      nbest[b.grp] = __float_as_uint(best);
+    }
     b.ridx = (int64_t)o * D + j;
     b.n_w = lv.count[i];
     b.P = 0;
@@ -2439,7 +2461,7 @@ __device__ __forceinline__ BestCand seg_best(BestCand b) {
 }
 
 template <int MAXC, int TASK, int SEG>
-__global__ void __launch_bounds__(kBlock, SEG == 64 ? 4 : 1) k_search_rf_seg(DataArgs d, LevelArgs lv, ItemArgs it) {
+__global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs lv, ItemArgs it) {
   constexpr int NPW = kWave / SEG;  // nodes per wave
   resolve_level(lv, d.C);
   resolve_items(it);
@@ -2603,6 +2625,650 @@ __global__ void __launch_bounds__(kBlock, SEG == 64 ? 4 : 1) k_search_rf_seg(Dat
     }
   }
   if (sl == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+}
+
+// ------------------------------------ RF split search by bucket bounds ---
+// Nodes of 33 .. 2048 entries.  A wave takes one (node, draw) at a time with
+// the node's keys in registers, spreads them over power-of-two wide key
+// buckets, counts classes (regression: weights and centred target sums) per
+// bucket in LDS, and bounds the gain of every boundary inside a bucket from
+// the counts on both sides of it (k_v2_bound has the inequality).  Only
+// buckets whose bound reaches the node's best candidate so far -- over the
+// bucket edges of this draw and everything earlier draws found -- are ordered
+// and scored exactly; with about 8 entries a bucket that is one bucket in a
+// hundred, so the sort and the scored walk of all entries (310 wave
+// instructions per 64 entries at 10 classes) are replaced by a histogram (14)
+// and a fixed 300 or so per draw.  The bounds are in fp32 with a margin for
+// their rounding; scored candidates use the exact fixed-point sums, and a
+// candidate whose fp32 score could equal the node's best is always scored.
+// A surviving bucket above 64 entries is split again over its own key range
+// (entries below it are counted as the totals before it); one of a single key
+// has no boundary but its lower edge.
+constexpr uint32_t kEdge = 0xFFFFFFFEu;  // previous key not in the list (lower edge of a bucket)
+
+// Best candidate of a draw: exact gain, key, key before it.
+struct DrawBest {
+  double g;
+  uint32_t key, prev;
+};
+
+template <int MAXC, int TASK, int LOGB, int IPT>
+struct BoundLds {
+  static constexpr int NB = 1 << LOGB;
+  // classification: bucket words [p * nb + b], two classes of 16 bits a word
+  // (nb = NB), or one of 32 bits for node weights above 65535 (nb = NB / 2)
+  static constexpr int PAIRS = (MAXC + 1) / 2;
+  static constexpr int TAB = IPT > 8 ? kTfMax : kTfMax / 2;  // staged x ln x terms
+  uint32_t hist[TASK == 0 ? NB * PAIRS : NB];
+  int64_t pos[TASK == 1 ? NB : 1], neg[TASK == 1 ? NB : 1];
+  uint32_t below[TASK == 0 ? MAXC : 1];
+  int64_t below_s[1];
+  uint32_t ncls[TASK == 0 ? MAXC : 1];
+  uint32_t lkey[kWave], laux[kWave];
+  int64_t ly[TASK == 1 ? kWave : 1];
+  uint32_t stk_k[IPT + 1];
+  uint32_t stk_b[IPT + 1];
+};
+
+// Value of the lane below (lane 0: `first`) through DPP wave_shr:1.
+__device__ __forceinline__ float lane_below_f32(float v, float first) {
+  return __uint_as_float(dpp_u32<0x138>(__float_as_uint(v), __float_as_uint(first)));
+}
+__device__ __forceinline__ float wave_last_f32(float v) { return __uint_as_float(wave_last(__float_as_uint(v))); }
+
+// fp32 chord_gap.
+__device__ __forceinline__ float chord_gap_f32(float a, float s) {
+  const float e = s * 0.36788f;
+  return a > 0.0f ? fminf(e, s * s * 0.125001f / a) : e;
+}
+
+// A node as one wave works on it.
+struct BoundNode {
+  int m;
+  int64_t n;
+  int64_t P;      // classification
+  int64_t ssum;   // regression
+  double inv;     // classification: 1 / (n ln 2)
+  float Pn, margin;  // classification: P and the rounding margin, nats
+  int64_t mu;     // regression: centre
+  double M;       // regression: largest |target - centre|
+  double E;       // regression: reg_gain_error
+  bool packed;
+};
+
+// Exact scores of the boundaries of a run of buckets holding cnt <= 64
+// entries (in L.lkey / laux / ly), with the totals before bucket b of the
+// bucket table.
+template <int MAXC, int TASK, int LOGB, int IPT>
+__device__ __forceinline__ void bound_run(const DataArgs& d, const BoundNode& nd, BoundLds<MAXC, TASK, LOGB, IPT>& L,
+                                          int cnt, int b, int nb, DrawBest& best) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool valid = lane < cnt;
+  const uint32_t key = valid ? L.lkey[lane] : kNone;
+  const uint32_t pay = valid ? L.laux[lane] : 0u;
+  const uint32_t w = pay & 0xFFFFu;
+  BestCand c{0.0, kNone, kNone};
+  if constexpr (TASK == 0) {
+    const LnCtx lx{g_ln_table.inv, g_ln_table.logc, d.T, d.Tmax, d.igF};
+    const uint32_t lab = pay >> 16;
+    auto before = [&](uint32_t cl) -> uint32_t {
+      return nd.packed ? (L.hist[(cl >> 1) * nb + b] >> ((cl & 1u) << 4)) & 0xFFFFu : L.hist[cl * nb + b];
+    };
+    // totals before the run, one class per lane
+    const uint32_t rc = lane < d.C ? before((uint32_t)lane) : 0u;
+    int64_t s0 = lane < d.C ? lx.t(rc) + lx.t(L.ncls[lane] - rc) : 0;
+    s0 = wave_last_i64(wave_incl_scan_i64(s0));
+    const uint32_t n0 = wave_last(wave_incl_scan(rc));
+    uint32_t rank = 0, pre = 0, nw = 0;
+    for (int x = 0; x < cnt; ++x) {
+      const uint32_t kx = (uint32_t)__builtin_amdgcn_readlane((int)key, x);
+      const uint32_t px = (uint32_t)__builtin_amdgcn_readlane((int)pay, x);
+      const uint32_t lt = kx < key || (kx == key && x < lane) ? 1u : 0u;
+      const uint32_t wx = lt ? px & 0xFFFFu : 0u;
+      rank += lt;
+      nw += wx;
+      pre += (px >> 16) == lab ? wx : 0u;
+    }
+    if (!valid) rank = (uint32_t)lane;
+    int64_t dd = 0, tq = 0;
+    const uint32_t nl = n0 + nw;
+    if (valid) {
+      const uint32_t l = before(lab) + pre, tc = L.ncls[lab];
+      dd = (lx.t(l + w) - lx.t(l)) + (lx.t(tc - l - w) - lx.t(tc - l));
+      tq = lx.t(nl) + lx.t((uint32_t)nd.n - nl);
+    }
+    // running sums in key order, then back to the entry's lane
+    const uint32_t ks = ds_permute_u32(rank, key);
+    const uint32_t dlo = ds_permute_u32(rank, (uint32_t)(uint64_t)dd);
+    const uint32_t dhi = ds_permute_u32(rank, (uint32_t)((uint64_t)dd >> 32));
+    const int64_t ds = (int64_t)(((uint64_t)dhi << 32) | dlo);
+    const int64_t ex = wave_incl_scan_i64(ds) - ds;
+    const int64_t sum = __shfl(ex, (int)rank, kWave);
+    const uint32_t pk = __shfl(ks, (int)rank > 0 ? (int)rank - 1 : 0, kWave);
+    if (valid && nl > 0 && (rank == 0 || pk < key)) {
+      const int64_t pq = nd.P + s0 + sum - tq;
+      if (pq > 0) {
+        const double g = ig_from_fixed(pq, d.igF, nd.inv);
+        if (cand_better(g, key, best.g, best.key)) c = BestCand{g, key, rank == 0 ? kEdge : pk};
+      }
+    }
+  } else {
+    const int64_t y = valid ? L.ly[lane] : 0;
+    uint32_t rank = 0;
+    for (int x = 0; x < cnt; ++x) {
+      const uint32_t kx = (uint32_t)__builtin_amdgcn_readlane((int)key, x);
+      rank += kx < key || (kx == key && x < lane) ? 1u : 0u;
+    }
+    if (!valid) rank = (uint32_t)lane;
+    const uint32_t ks = ds_permute_u32(rank, key);
+    const uint32_t ws = ds_permute_u32(rank, w);
+    const int64_t wy = (int64_t)w * y;
+    const uint32_t ylo = ds_permute_u32(rank, (uint32_t)(uint64_t)wy);
+    const uint32_t yhi = ds_permute_u32(rank, (uint32_t)((uint64_t)wy >> 32));
+    const int64_t ys = (int64_t)(((uint64_t)yhi << 32) | ylo);
+    const int64_t pn = (int64_t)(L.hist[b] + wave_incl_scan(ws) - ws);
+    const int64_t ps = L.pos[b] + wave_incl_scan_i64(ys) - ys;
+    const uint32_t pk = dpp_u32<0x138>(ks, 0u);
+    if (lane < cnt && pn > 0 && (lane == 0 || pk < ks)) {
+      const double g = variance_gain(pn, ps, nd.n - pn, nd.ssum - ps, 0);
+      if (g > 0.0 && cand_better(g, ks, best.g, best.key)) c = BestCand{g, ks, lane == 0 ? kEdge : pk};
+    }
+  }
+  if (__ballot(c.key != kNone)) {
+    c = wave_best(c);
+    best = DrawBest{c.g, c.key, c.prev};
+  }
+}
+
+// The lower edge of bucket b (a single key, `key`) alone.
+template <int MAXC, int TASK, int LOGB, int IPT>
+__device__ __forceinline__ void bound_edge(const DataArgs& d, const BoundNode& nd, BoundLds<MAXC, TASK, LOGB, IPT>& L,
+                                           uint32_t key, int b, int nb, DrawBest& best) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double g = 0.0;
+  if constexpr (TASK == 0) {
+    const LnCtx lx{g_ln_table.inv, g_ln_table.logc, d.T, d.Tmax, d.igF};
+    uint32_t rc = 0;
+    if (lane < d.C)
+      rc = nd.packed ? (L.hist[(lane >> 1) * nb + b] >> ((lane & 1) << 4)) & 0xFFFFu : L.hist[lane * nb + b];
+    int64_t s0 = lane < d.C ? lx.t(rc) + lx.t(L.ncls[lane] - rc) : 0;
+    s0 = wave_last_i64(wave_incl_scan_i64(s0));
+    const uint32_t n0 = wave_last(wave_incl_scan(rc));
+    if (n0 == 0) return;
+    const int64_t pq = nd.P + s0 - (lx.t(n0) + lx.t((uint32_t)nd.n - n0));
+    if (pq > 0) g = ig_from_fixed(pq, d.igF, nd.inv);
+  } else {
+    const int64_t pn = (int64_t)L.hist[b], ps = L.pos[b];
+    if (pn == 0) return;
+    g = variance_gain(pn, ps, nd.n - pn, nd.ssum - ps, 0);
+  }
+  if (g > 0.0 && cand_better(g, key, best.g, best.key)) best = DrawBest{g, key, kEdge};
+}
+
+// One draw of a node.  thr: lower bound of the node's best gain that matters
+// here (nats / fixed-point units squared, as float / double); returns the
+// draw's best in `best` (none when no candidate of it can be the node's best)
+// and raises thr by what it found.
+template <int MAXC, int TASK, int LOGB, int IPT>
+__device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& nd, const float* s_tf,
+                                           BoundLds<MAXC, TASK, LOGB, IPT>& L, const uint32_t (&key)[IPT],
+                                           const uint32_t (&aux)[IPT], const int64_t (&y)[TASK == 1 ? IPT : 1],
+                                           double& thr, DrawBest& best) {
+  using LdsT = BoundLds<MAXC, TASK, LOGB, IPT>;
+  constexpr int NB = LdsT::NB;
+  constexpr int NR = NB / kWave > 0 ? NB / kWave : 1;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int m = nd.m;
+  uint32_t kmin = kNone, kmax = 0;
+#pragma unroll
+  for (int q = 0; q < IPT; ++q) {
+    if (q * kWave >= m) break;
+    if (lane + q * kWave < m) {
+      kmin = min(kmin, key[q]);
+      kmax = max(kmax, key[q]);
+    }
+  }
+  kmin = wave_min_u32(kmin);
+  kmax = wave_max_u32(kmax);
+  best = DrawBest{0.0, kNone, kNone};
+  if (kmin == kmax) return;  // one value: no boundary
+  const int lognb = nd.packed || TASK == 1 ? LOGB : LOGB - 1;
+  const int nb = 1 << lognb;
+  int sp = 1;
+  uint32_t k0 = kmin;
+  int sb = bit_length(kmax - kmin);
+  bool first = true;
+  for (;;) {
+    const int shift = max(0, sb - lognb);
+    const uint32_t nbk = 1u << (sb - shift);  // buckets of the range
+    // ---- bucket table
+    if constexpr (TASK == 0) {
+      const int words = nd.packed ? (d.C + 1) / 2 : d.C;
+      for (int i = lane; i < words * nb; i += kWave) L.hist[i] = 0;
+      if (lane < MAXC) L.below[lane] = 0;
+    } else {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        L.hist[r * kWave + lane] = 0;
+        L.pos[r * kWave + lane] = 0;
+        L.neg[r * kWave + lane] = 0;
+      }
+      if (lane == 0) {
+        L.below[0] = 0;
+        L.below_s[0] = 0;
+      }
+    }
+    team_sync<kWave>();
+#pragma unroll
+    for (int q = 0; q < IPT; ++q) {
+      if (q * kWave >= m) break;
+      if (lane + q * kWave < m) {
+        const uint32_t b = (key[q] - k0) >> shift;
+        const bool in = key[q] >= k0 && b < nbk, lower = key[q] < k0;
+        const uint32_t w = aux[q] & 0xFFFFu;
+        if constexpr (TASK == 0) {
+          const uint32_t c = aux[q] >> 16;
+          const uint32_t p = nd.packed ? c >> 1 : c;
+          const uint32_t v = nd.packed ? w << ((c & 1u) << 4) : w;
+          if (in) atomicAdd(&L.hist[p * (uint32_t)nb + b], v);
+          else if (lower) atomicAdd(&L.below[p], v);
+        } else {
+          const int64_t dy = y[q] - nd.mu;
+          const unsigned long long wy = (unsigned long long)((int64_t)w * dy);
+          if (in) {
+            atomicAdd(&L.hist[b], w);
+            atomicAdd(reinterpret_cast<unsigned long long*>(dy < 0 ? &L.neg[b] : &L.pos[b]), wy);
+          } else if (lower) {
+            atomicAdd(&L.below[0], w);
+            atomicAdd(reinterpret_cast<unsigned long long*>(&L.below_s[0]), wy);
+          }
+        }
+      }
+    }
+    team_sync<kWave>();
+    // ---- edges and bounds, 64 buckets at a time
+    float ubf[NR];
+    double ubd[TASK == 1 ? NR : 1];
+    uint32_t wgt[NR];
+    if constexpr (TASK == 0) {
+      const bool big_n = nd.n >= LdsT::TAB;
+      auto tf = [&](uint32_t x) -> float {
+        if (big_n) return x > 1 ? (float)x * __logf((float)x) : 0.0f;
+        return s_tf[x];
+      };
+      constexpr int PAIRS = LdsT::PAIRS;
+      const uint32_t n = (uint32_t)nd.n;
+      const int words = nd.packed ? (d.C + 1) / 2 : d.C;
+      float eb = 0.0f;
+      if (nd.packed) {
+        uint32_t run[PAIRS];
+        uint32_t run_n = 0;
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) {
+          run[p] = p < words ? __builtin_amdgcn_readfirstlane(L.below[p]) : 0u;
+          run_n += (run[p] & 0xFFFFu) + (run[p] >> 16);
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          ubf[r] = -1.0f;
+          wgt[r] = 0;
+          if ((uint32_t)(r * kWave) >= nbk) break;
+          const int b = r * kWave + lane;
+          uint32_t v[PAIRS], sw = 0;
+#pragma unroll
+          for (int p = 0; p < PAIRS; ++p) {
+            v[p] = p < words ? L.hist[p * nb + b] : 0u;
+            sw += (v[p] & 0xFFFFu) + (v[p] >> 16);
+          }
+          const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
+          const float psb = tf(lb) + tf(n - lb);
+          const float psa = lane_below_f32(psb, tf(run_n) + tf(n - run_n));
+          run_n = wave_last(lb);
+          const float slope = sw ? (psb - psa) / (float)sw : 0.0f;
+          float phi = 0.0f, slack = 0.0f;
+#pragma unroll
+          for (int p = 0; p < PAIRS; ++p) {
+            if (p < words) {
+              const uint32_t inc = run[p] + wave_incl_scan(v[p]);
+              const uint32_t n0 = L.ncls[2 * p], n1 = 2 * p + 1 < d.C ? L.ncls[2 * p + 1] : 0u;
+              const uint32_t l0 = inc & 0xFFFFu, l1 = inc >> 16;
+              const float b0 = tf(l0) + tf(n0 - l0), b1 = tf(l1) + tf(n1 - l1);
+              const uint32_t r0 = run[p] & 0xFFFFu, r1 = run[p] >> 16;
+              const float a0 = lane_below_f32(b0, tf(r0) + tf(n0 - r0));
+              const float a1 = lane_below_f32(b1, tf(r1) + tf(n1 - r1));
+              run[p] = wave_last(inc);
+              phi += a0 + a1;
+              slack += fmaxf(0.0f, (b0 - a0) - slope * (float)(v[p] & 0xFFFFu)) +
+                       fmaxf(0.0f, (b1 - a1) - slope * (float)(v[p] >> 16));
+              L.hist[p * nb + b] = inc - v[p];
+            }
+          }
+          slack += chord_gap_f32((float)la, (float)sw) + chord_gap_f32((float)(n - lb), (float)sw);
+          const float edge = nd.Pn + phi - psa;
+          if (sw) {
+            ubf[r] = edge + (shift ? slack : 0.0f) + nd.margin;  // shift 0: one key, only the edge
+            if (la > 0) eb = fmaxf(eb, edge - nd.margin);
+            else if (!shift) ubf[r] = -1.0f;
+          }
+          wgt[r] = sw;
+        }
+      } else {
+        // node weight above 65535: 32-bit counts, half the buckets
+        uint32_t run_n = 0;
+        for (int c = 0; c < words; ++c) run_n += __builtin_amdgcn_readfirstlane(L.below[c]);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          ubf[r] = -1.0f;
+          wgt[r] = 0;
+          if ((uint32_t)(r * kWave) >= nbk) break;
+          const int b = r * kWave + lane;
+          const bool ok = b < nb;
+          uint32_t sw = 0;
+          for (int c = 0; c < words; ++c) sw += ok ? L.hist[c * nb + b] : 0u;
+          const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
+          const float psb = tf(lb) + tf(n - lb);
+          const float psa = lane_below_f32(psb, tf(run_n) + tf(n - run_n));
+          run_n = wave_last(lb);
+          const float slope = sw ? (psb - psa) / (float)sw : 0.0f;
+          float phi = 0.0f, slack = 0.0f;
+          for (int c = 0; c < words; ++c) {
+            const uint32_t v = ok ? L.hist[c * nb + b] : 0u;
+            const uint32_t r0 = __builtin_amdgcn_readfirstlane(L.below[c]);
+            const uint32_t n0 = L.ncls[c];
+            const uint32_t l = r0 + wave_incl_scan(v);
+            const float b0 = tf(l) + tf(n0 - l);
+            const float a0 = lane_below_f32(b0, tf(r0) + tf(n0 - r0));
+            phi += a0;
+            slack += fmaxf(0.0f, (b0 - a0) - slope * (float)v);
+            if (ok) L.hist[c * nb + b] = l - v;
+            if (lane == 0) L.below[c] = wave_last(l);
+            team_sync<kWave>();
+          }
+          slack += chord_gap_f32((float)la, (float)sw) + chord_gap_f32((float)(n - lb), (float)sw);
+          const float edge = nd.Pn + phi - psa;
+          if (sw) {
+            ubf[r] = edge + (shift ? slack : 0.0f) + nd.margin;
+            if (la > 0) eb = fmaxf(eb, edge - nd.margin);
+            else if (!shift) ubf[r] = -1.0f;
+          }
+          wgt[r] = sw;
+        }
+      }
+      eb = __uint_as_float(wave_max_u32(__float_as_uint(fmaxf(eb, 0.0f))));
+      thr = fmax(thr, (double)eb);
+    } else {
+      const double N = (double)nd.n, S = (double)(nd.ssum - nd.mu * nd.n);
+      uint32_t run_n = __builtin_amdgcn_readfirstlane(L.below[0]);
+      int64_t run_s = L.below_s[0];
+      double eb = 0.0;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        ubd[r] = -1.0;
+        wgt[r] = 0;
+        if ((uint32_t)(r * kWave) >= nbk) break;
+        const int b = r * kWave + lane;
+        const uint32_t w = L.hist[b];
+        const int64_t sp_ = L.pos[b], sn_ = L.neg[b];
+        const uint32_t lb = run_n + wave_incl_scan(w), la = lb - w;
+        run_n = wave_last(lb);
+        const int64_t se = run_s + wave_incl_scan_i64(sp_ + sn_), sa = se - (sp_ + sn_);
+        run_s = wave_last_i64(se);
+        L.hist[b] = la;
+        L.pos[b] = sa + nd.mu * (int64_t)la;  // uncentred target sum before the bucket
+        if (w) {
+          double edge = 0.0;
+          if (la > 0) {
+            const double s = (double)sa, t = S - s;
+            edge = s * s / (double)la + t * t / (N - (double)la) - S * S / N;
+            eb = fmax(eb, edge * (1.0 - 2e-6) - nd.E);
+          }
+          if (shift)
+            ubd[r] = reg_box_bound((double)la, (double)lb, (double)(sa + sn_), (double)(sa + sp_), N, S, nd.M) *
+                         (1.0 + 2e-6) + nd.E;
+          else if (la > 0)
+            ubd[r] = edge * (1.0 + 2e-6) + nd.E;
+        }
+        wgt[r] = w;
+      }
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) eb = fmax(eb, __shfl_xor(eb, off, kWave));
+      thr = fmax(thr, eb);
+    }
+    team_sync<kWave>();
+    // ---- surviving buckets
+    const float thr_f = (float)(thr * (1.0 - 1e-6));
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if ((uint32_t)(r * kWave) >= nbk) break;
+      bool sv;
+      if constexpr (TASK == 0) sv = wgt[r] && ubf[r] >= thr_f && ubf[r] > 0.0f;
+      else sv = wgt[r] && ubd[r] >= thr * (1.0 - 1e-6) && ubd[r] > 0.0;
+      uint64_t mask = __ballot(sv);
+      while (mask) {
+        const int i = (int)__ffsll((unsigned long long)mask) - 1;
+        int e = i;  // last bucket of the run
+        uint32_t wsum = (uint32_t)__builtin_amdgcn_readlane((int)wgt[r], i);
+        mask &= mask - 1;
+        while (e + 1 < kWave && ((mask >> (e + 1)) & 1ull)) {
+          const uint32_t wn = (uint32_t)__builtin_amdgcn_readlane((int)wgt[r], e + 1);
+          if (wsum + wn > (uint32_t)kWave) break;
+          wsum += wn;
+          ++e;
+          mask &= mask - 1;
+        }
+        const int b = r * kWave + i;
+        const uint32_t klo = k0 + ((uint32_t)b << shift);
+        const uint32_t kspan = (uint32_t)(e - i + 1) << shift;
+        if (!shift && wsum > (uint32_t)kWave) {
+          bound_edge<MAXC, TASK, LOGB, IPT>(d, nd, L, klo, b, nb, best);
+          continue;
+        }
+        int cnt = 0;
+#pragma unroll
+        for (int q = 0; q < IPT; ++q) {
+          if (q * kWave >= m) break;
+          const bool in = lane + q * kWave < m && key[q] - klo < kspan && key[q] >= klo;
+          const uint64_t bal = __ballot(in);
+          if (bal) {
+            const int at = cnt + (int)__popcll(bal & ((1ull << lane) - 1ull));
+            if (in && at < kWave) {
+              L.lkey[at] = key[q];
+              L.laux[at] = aux[q];
+              if constexpr (TASK == 1) L.ly[at] = y[q];
+            }
+            cnt += (int)__popcll(bal);
+          }
+        }
+        team_sync<kWave>();
+        if (cnt > kWave) {
+          // one bucket above 64 entries (runs are merged by weight): split it
+          // again; at most IPT disjoint ranges of more than 64 entries exist
+          if (lane == 0) {
+            L.stk_k[sp] = klo;
+            L.stk_b[sp] = (uint32_t)shift;
+          }
+          ++sp;
+        } else {
+          bound_run<MAXC, TASK, LOGB, IPT>(d, nd, L, cnt, b, nb, best);
+        }
+        team_sync<kWave>();
+      }
+    }
+    if (best.key != kNone)
+      thr = fmax(thr, (TASK == 0 ? best.g * (double)nd.n * kLn2 : best.g) * (1.0 - 1e-6));
+    if (sp <= 1) break;
+    --sp;
+    team_sync<kWave>();
+    k0 = __builtin_amdgcn_readfirstlane(L.stk_k[sp]);
+    sb = (int)__builtin_amdgcn_readfirstlane(L.stk_b[sp]);
+    first = false;
+  }
+  (void)first;
+  if (best.prev == kEdge) {  // largest key below the best candidate's
+    uint32_t p = 0;
+#pragma unroll
+    for (int q = 0; q < IPT; ++q) {
+      if (q * kWave >= m) break;
+      if (lane + q * kWave < m && key[q] < best.key) p = max(p, key[q]);
+    }
+    best.prev = wave_max_u32(p);
+  }
+}
+
+// WPN waves per node: 1 (a wave walks its node's draws in order, the next
+// draw's key gather in flight) or 4 (a workgroup per node, its waves take the
+// draws in turn and share the best bound found).
+template <int MAXC, int TASK, int IPT, int LOGB, int WPN>
+__global__ void __launch_bounds__(kBlock) k_search_rf_bound(DataArgs d, LevelArgs lv, ItemArgs it) {
+  constexpr int NPB = kWaves / WPN;  // nodes per workgroup
+  resolve_level(lv, d.C);
+  resolve_items(it);
+  if ((int64_t)blockIdx.x * NPB >= it.n_groups) return;  // no node for this workgroup
+  constexpr int kTab = BoundLds<MAXC, TASK, LOGB, IPT>::TAB;
+  __shared__ float s_tf[TASK == 0 ? kTab : 1];
+  __shared__ BoundLds<MAXC, TASK, LOGB, IPT> s_l[kWaves];
+  __shared__ unsigned long long s_best;  // WPN > 1: bits of the shared bound
+  if (TASK == 0)
+    for (int i = threadIdx.x; i < kTab; i += kBlock) s_tf[i] = d.Tf[i];
+  __syncthreads();
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  BoundLds<MAXC, TASK, LOGB, IPT>& L = s_l[wv];
+  const int lane = threadIdx.x & (kWave - 1);
+  unsigned long long my_bytes = 0;
+  for (int64_t g0 = (int64_t)blockIdx.x * NPB; g0 < it.n_groups; g0 += (int64_t)gridDim.x * NPB) {
+    const int64_t grp = g0 + (WPN == 1 ? wv : 0);
+    const bool live = grp < it.n_groups;
+    if (WPN == 1 && !live) break;  // wave-uniform; one-wave teams have no workgroup barrier
+    const uint32_t o = __builtin_amdgcn_readfirstlane(it.list ? it.list[grp] : (uint32_t)grp);
+    const uint32_t i = __builtin_amdgcn_readfirstlane(lv.open_idx[o]);
+    const uint32_t tg = (uint32_t)__builtin_amdgcn_readfirstlane(lv.tree_global[lv.tree[i]]);
+    const uint32_t nid = __builtin_amdgcn_readfirstlane(lv.id[i]);
+    BoundNode nd;
+    nd.m = __builtin_amdgcn_readfirstlane(lv.m[i]);
+    nd.n = __builtin_amdgcn_readfirstlane(lv.count[i]);
+    nd.packed = nd.n <= 65535;
+    nd.P = 0;
+    nd.ssum = 0;
+    nd.mu = 0;
+    nd.M = 0.0;
+    nd.E = 0.0;
+    bool pure = false;
+    const int first_draw = WPN == 1 ? 0 : wv;
+    if constexpr (TASK == 0) {
+      const uint32_t my = lane < d.C ? lv.cls[(int64_t)i * d.C + lane] : 0u;
+      if (lane < MAXC) L.ncls[lane] = my;
+      pure = (int64_t)wave_max_u32(my) == nd.n;
+      const LnCtx lx{g_ln_table.inv, g_ln_table.logc, d.T, d.Tmax, d.igF};
+      const int64_t tn_fixed = lx.t((uint64_t)nd.n);
+      nd.P = tn_fixed - wave_last_i64(wave_incl_scan_i64(lane < d.C ? lx.t(my) : 0));
+      nd.inv = 1.0 / ((double)nd.n * kLn2);
+      nd.Pn = (float)ldexp_d((double)nd.P, -d.igF);
+      // fp32 terms of at most T(n) nats: (4 C + 16) roundings of 2^-24 of
+      // twice that, doubled
+      const float tn = (float)ldexp_d((double)tn_fixed, -d.igF);
+      nd.margin = tn * (float)(4 * d.C + 16) * 2.4e-7f + 1e-6f;
+    } else {
+      nd.ssum = lv.sum[i];
+      nd.mu = d2ll_rn((double)nd.ssum / (double)nd.n);
+    }
+    const int m = nd.m;
+    const int64_t st = lv.start[i];
+    if (pure) {
+      // Every boundary of a pure node has gain exactly 0: no positive split.
+      if (lane == 0)
+        for (int jj = first_draw; jj < it.per_group; jj += WPN) {
+          const int j = it.j0 + jj;
+          const int64_t ridx = (int64_t)o * it.D + j;
+          it.res_score[ridx] = 0.0f;
+          it.res_thr[ridx] = 0.0f;
+          it.res_feat[ridx] = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)j) % (uint32_t)d.F);
+        }
+      continue;  // workgroup-uniform with WPN > 1
+    }
+    uint32_t rows[IPT], aux[IPT], kn[IPT];
+    int64_t y[TASK == 1 ? IPT : 1];
+#pragma unroll
+    for (int q = 0; q < IPT; ++q) {
+      rows[q] = 0;
+      aux[q] = 0;
+      const int e = lane + q * kWave;
+      if (q * kWave < m && e < m) {
+        rows[q] = lv.row[st + e];
+        aux[q] = lv.aux[st + e];
+        if constexpr (TASK == 1) y[q] = lv.ey[st + e];
+      }
+    }
+    if constexpr (TASK == 1) {
+      double M = 0.0;
+#pragma unroll
+      for (int q = 0; q < IPT; ++q)
+        if (q * kWave < m && lane + q * kWave < m) M = fmax(M, fabs((double)(y[q] - nd.mu)));
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) M = fmax(M, __shfl_xor(M, off, kWave));
+      nd.M = M * (1.0 + 1e-12);
+      nd.E = reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
+    }
+    // The node's best score so far (retry phase: the mandatory draws, at most
+    // 1e-3) as a bound in the units of `thr`.
+    double thr = 0.0;
+    float best_score = 0.0f;
+    for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
+    auto to_units = [&](float s) {
+      return (TASK == 0 ? (double)s * (double)nd.n * kLn2 : ldexp_d((double)s, 2 * d.shift)) * (1.0 - 1e-6);
+    };
+    thr = to_units(best_score);
+    // Retry draws count in order until one scores above 1e-3 (k_decide2): a
+    // candidate may be dropped for one of a later draw only up to that score.
+    const double cap = it.j0 > 0 && WPN > 1 ? to_units(1e-3f) : __builtin_inf();
+    if (WPN > 1) {
+      __syncthreads();
+      if (threadIdx.x == 0) s_best = __builtin_bit_cast(unsigned long long, thr);
+      __syncthreads();
+    }
+    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + first_draw)) % (uint32_t)d.F);
+    if (WPN == 1) {
+#pragma unroll
+      for (int q = 0; q < IPT; ++q)
+        if (q * kWave < m && lane + q * kWave < m) kn[q] = d.K[(int64_t)f_nx * d.N + rows[q]];
+    }
+    for (int jj = first_draw; jj < it.per_group; jj += WPN) {
+      const int j = it.j0 + jj;
+      const int64_t ridx = (int64_t)o * it.D + j;
+      // in order: once a retry draw passed 1e-3 the later ones are not looked at
+      if (WPN == 1 && it.j0 > 0 && (double)best_score > 1e-3) break;
+      const int f = f_nx;
+      uint32_t key[IPT];
+#pragma unroll
+      for (int q = 0; q < IPT; ++q) {
+        key[q] = 0;
+        if (q * kWave < m && lane + q * kWave < m) key[q] = WPN == 1 ? kn[q] : d.K[(int64_t)f * d.N + rows[q]];
+      }
+      if (jj + WPN < it.per_group) {
+        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + WPN)) % (uint32_t)d.F);
+        if (WPN == 1) {
+#pragma unroll
+          for (int q = 0; q < IPT; ++q)
+            if (q * kWave < m && lane + q * kWave < m) kn[q] = d.K[(int64_t)f_nx * d.N + rows[q]];
+        }
+      }
+      DrawBest best;
+      if (WPN > 1) thr = fmin(__builtin_bit_cast(double, *(volatile unsigned long long*)&s_best), cap);
+      bound_draw<MAXC, TASK, LOGB, IPT>(d, nd, s_tf, L, key, aux, y, thr, best);
+      if (WPN > 1 && lane == 0) atomicMax(&s_best, __builtin_bit_cast(unsigned long long, thr));
+      float score = 0.0f;
+      if (best.key != kNone) score = (float)(TASK == 0 ? best.g : ldexp_d(best.g, -2 * d.shift));
+      best_score = fmaxf(best_score, score);
+      if (lane == 0) {
+        const float* sv = d.SV + d.SVoff[f];
+        it.res_score[ridx] = score;
+        it.res_thr[ridx] = best.key != kNone ? midpoint(sv[best.prev], sv[best.key]) : 0.0f;
+        it.res_feat[ridx] = f;
+      }
+    }
+    if (lane == 0 && (WPN == 1 || wv == 0))
+      my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
+  }
+  if (lane == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
 }
 
 // ERT, one wave per item (any node size; lanes stride over the entries).
@@ -4472,9 +5138,9 @@ void launch_search(int algorithm, int tier, int grid, hipStream_t s, const DataA
     switch (tier) {
       case 0: hipLaunchKernelGGL((k_search_rf_seg<MAXC, TASK, 16>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       case 1: hipLaunchKernelGGL((k_search_rf_seg<MAXC, TASK, 32>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 2: hipLaunchKernelGGL((k_search_rf_seg<MAXC, TASK, 64>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 3: hipLaunchKernelGGL((k_search_rf_team<MAXC, TASK, 64>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 4: hipLaunchKernelGGL((k_search_rf_team<MAXC, TASK, 256>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 2: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 1, 6, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 3: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 8, 6, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 4: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 32, MAXC <= 16 ? 8 : 7, 4>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       default: hipLaunchKernelGGL((k_search_rf<MAXC, TASK, 256, true>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
     }
   } else {
@@ -4521,31 +5187,33 @@ void launch_partition_chunks(hipStream_t s, const DataArgs& d, const LevelArgs& 
 // Scratch and bookkeeping of the big-node pipeline, reused across levels.
 struct BigState {
   DevBuf<V2Item> items;
-  DevBuf<V2Tile> htiles, stiles, ctiles;
-  DevBuf<uint32_t> bcount, bmax, bcls, bwn, bbase, bcur, bsup, carry_cls, carry_last, res_key, res_prev;
-  DevBuf<int64_t> bsum, carry_n, carry_s;
+  DevBuf<V2Tile> htiles;
+  DevBuf<uint32_t> bcls, bn, bslot, bnext, bcur, carry_last, res_key, res_prev, isel, nbest;
+  DevBuf<int64_t> bpos, bneg;
+  DevBuf<float> bub;
   DevBuf<double> res_g;
-  DevBuf<uint32_t> skey, saux, skey2, saux2, tkey;
+  DevBuf<uint32_t> skey, saux, skey2, saux2;
   DevBuf<int64_t> sy, sy2;
   DevBuf<V2Task> tasks, spill;
   DevBuf<unsigned int> ctr;
-  DevBuf<uint32_t> lists;  // item indices: small items (wave teams), then the rest
   std::vector<V2Item> host_items;
-  std::vector<V2Tile> host_htiles, host_stiles, host_ctiles, host_stiles_mid, host_stiles_many;
-  std::vector<uint32_t> host_lists;
-  std::vector<int64_t> host_fcount;   // histogram tiles: items per feature
+  std::vector<V2Tile> host_htiles;
+  std::vector<int64_t> host_fcount;   // tiles: items per feature
   std::vector<uint32_t> host_forder;  // batch items in feature order
   std::vector<V2Tile> host_forder_tiles;
-  int target = kV2Target;  // entries per bucket aimed at
+  int target = kDefBucketTarget;  // bucket_target of the fit
+  double max_dev = 0.0;           // regression: largest |fixed target|
 };
 
+// Entries per bucket aimed at: a sixth of bucket_target (64 by default).
+// Finer buckets give tighter bounds (fewer entries to sort) and larger tables.
+constexpr int kV2TargetDiv = 6;
+
 // Chunk-parallel search of the big items of one phase (see k_v2_*): items in
-// batches of at most kV2Batch scratch entries.  A batch's scratch is about
-// 20 B (classification) to 36 B (regression) per entry, so 1.5 Gi entries
-// hold a whole level of a 200-tree 1M-row fit in one batch at 32-58 GB of
-// the 288 GB of HBM (fewer, larger launches and host round trips than
-// 384 Mi-entry batches: headline fit 1231 -> 1221 ms, 4M x 64 regression
-// fit 3.98 -> 3.76 s with the side stream of the other tiers).
+// batches of at most kV2Batch scratch slots (a slot per unit of bootstrap
+// weight, the bound of a bucket's entries).  A batch's scratch is 16 B
+// (classification) to 40 B (regression) per slot, so 1.5 Gi slots hold most
+// of a level of a 200-tree 1M-row fit in one batch.
 constexpr int64_t kV2Batch = (int64_t)1536 << 20;
 
 template <int MAXC, int TASK>
@@ -4553,42 +5221,37 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
                   int64_t n_groups, hipStream_t s, int num_cu) {
   const int64_t n_all = n_groups * it.per_group;
   if (n_all == 0) return;
-  const int nb_cap = kV2MaxB;
   const int C = d.C;
+  const int bucket_words = TASK == 0 ? C : kV2RegWords;
+  const int nb_cap = std::min(kV2MaxB, kV2HistWords / bucket_words);
   B.items.reserve(n_all);
+  B.nbest.reserve(n_groups);
   hipLaunchKernelGGL(k_v2_items, dim3(grid_for(n_all)), dim3(kBlock), 0, s, d, lv, groups, n_groups, it.per_group,
-                     it.j0, it.D, nb_cap, B.target, B.items.p);
+                     it.j0, it.D, nb_cap, std::max(1, B.target / kV2TargetDiv), (const float*)it.res_score, B.nbest.p,
+                     B.items.p);
   B.host_items.resize(n_all);
   DTE_HIP(hipMemcpyAsync(B.host_items.data(), B.items.p, sizeof(V2Item) * n_all, hipMemcpyDeviceToHost, s));
   DTE_HIP(hipStreamSynchronize(s));
-  constexpr int kSTile = TASK == 0 ? kScatterTile : 2048;
   int64_t k0 = 0;
   while (k0 < n_all) {
-    int64_t k1 = k0, el = 0, nb = 0;
+    int64_t k1 = k0, el = 0, slots = 0, nb = 0;
+    int nb_max = 0;
     B.host_htiles.clear();
-    B.host_stiles.clear();
-    B.host_stiles_mid.clear();
-    B.host_stiles_many.clear();
-    B.host_ctiles.clear();
-    B.host_lists.clear();
-    while (k1 < n_all && (k1 == k0 || el + B.host_items[k1].m <= kV2Batch)) {
+    while (k1 < n_all && (k1 == k0 || slots + B.host_items[k1].n_w <= kV2Batch)) {
       V2Item& bi = B.host_items[k1];
       bi.boff = (int32_t)nb;
       bi.soff = el;
-      const uint32_t li = (uint32_t)(k1 - k0);
-      auto& st = bi.nb <= kV2FewB ? B.host_stiles : (bi.nb <= kV2MidB ? B.host_stiles_mid : B.host_stiles_many);
-      bi.sgrp = bi.nb > kV2MidB ? (bi.nb + kV2Super - 1) / kV2Super : 0;  // two-pass scatter
-      for (int e0 = 0; e0 < bi.m; e0 += kSTile) st.push_back(V2Tile{li, (uint32_t)e0});
-      for (int b0 = 0; b0 < bi.nb; b0 += kV2CTile) B.host_ctiles.push_back(V2Tile{li, (uint32_t)b0});
       el += bi.m;
+      slots += bi.n_w;
       nb += bi.nb;
+      nb_max = std::max(nb_max, (int)bi.nb);
       ++k1;
     }
     const int64_t n_items = k1 - k0;
-    // Histogram tiles feature-major: the tiles in flight gather from a few
-    // feature columns of K at a time instead of from all of them, so the
-    // columns stay in the caches.  The histogram's results do not depend on
-    // the tile order (per-bucket counts and maxima, keys stored per entry).
+    // Tiles feature-major: the tiles in flight gather from a few feature
+    // columns of K at a time instead of from all of them, so the columns stay
+    // in the caches.  The results do not depend on the tile order (counts,
+    // keys stored per entry).
     B.host_fcount.assign((size_t)d.F + 1, 0);
     for (int64_t k = k0; k < k1; ++k) ++B.host_fcount[(size_t)B.host_items[k].f + 1];
     for (int f = 0; f < d.F; ++f) B.host_fcount[(size_t)f + 1] += B.host_fcount[(size_t)f];
@@ -4611,168 +5274,119 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
         }
       B.host_forder_tiles.clear();
     }
-    // scatter tiles of items with few buckets first, then the rest
-    const int64_t n_sfew = (int64_t)B.host_stiles.size();
-    B.host_stiles.insert(B.host_stiles.end(), B.host_stiles_mid.begin(), B.host_stiles_mid.end());
-    const int64_t n_smid = (int64_t)B.host_stiles.size();
-    B.host_stiles.insert(B.host_stiles.end(), B.host_stiles_many.begin(), B.host_stiles_many.end());
-    const int64_t n_sall = (int64_t)B.host_stiles.size();
-    for (int64_t k = k0; k < k1; ++k)
-      if (B.host_items[k].nb <= kV2SmallB) B.host_lists.push_back((uint32_t)(k - k0));
-    const int64_t n_small = (int64_t)B.host_lists.size();
-    for (int64_t k = k0; k < k1; ++k)
-      if (B.host_items[k].nb > kV2SmallB) B.host_lists.push_back((uint32_t)(k - k0));
-    const int64_t n_large = n_items - n_small;
-    B.lists.reserve(n_items);
-    DTE_HIP(hipMemcpyAsync(B.lists.p, B.host_lists.data(), 4 * n_items, hipMemcpyHostToDevice, s));
     DTE_HIP(hipMemcpyAsync(B.items.p, B.host_items.data() + k0, sizeof(V2Item) * n_items, hipMemcpyHostToDevice, s));
     B.htiles.reserve(B.host_htiles.size());
-    B.stiles.reserve(B.host_stiles.size());
-    B.ctiles.reserve(B.host_ctiles.size());
-    DTE_HIP(hipMemcpyAsync(B.ctiles.p, B.host_ctiles.data(), sizeof(V2Tile) * B.host_ctiles.size(),
-                           hipMemcpyHostToDevice, s));
     DTE_HIP(hipMemcpyAsync(B.htiles.p, B.host_htiles.data(), sizeof(V2Tile) * B.host_htiles.size(),
                            hipMemcpyHostToDevice, s));
-    DTE_HIP(hipMemcpyAsync(B.stiles.p, B.host_stiles.data(), sizeof(V2Tile) * B.host_stiles.size(),
-                           hipMemcpyHostToDevice, s));
-    B.bcount.reserve(nb);
-    B.bmax.reserve(nb);
-    B.bbase.reserve(nb);
+    B.bn.reserve(nb);
+    B.bub.reserve(nb);
+    B.bslot.reserve(nb);
+    B.bnext.reserve(nb);
     B.bcur.reserve(nb);
-    B.bsup.reserve(nb);
-    B.carry_n.reserve(nb);
     B.carry_last.reserve(nb);
     B.res_g.reserve(nb);
     B.res_key.reserve(nb);
     B.res_prev.reserve(nb);
     B.tasks.reserve(nb);
     B.spill.reserve(nb);
-    B.ctr.reserve(2);
+    B.isel.reserve(n_items);
+    B.ctr.reserve(3);
     if (TASK == 0) {
       B.bcls.reserve((size_t)nb * C);
-      B.carry_cls.reserve((size_t)nb * C);
     } else {
-      B.bwn.reserve(nb);
-      B.bsum.reserve(nb);
-      B.carry_s.reserve(nb);
+      B.bpos.reserve(nb);
+      B.bneg.reserve(nb);
     }
-    B.skey.reserve(el);
-    B.saux.reserve(el);
-    B.skey2.reserve(el);
-    B.saux2.reserve(el);
-    if (n_sall > n_smid) B.tkey.reserve(el);
+    B.skey.reserve(slots);
+    B.saux.reserve(slots);
+    B.skey2.reserve(slots);
+    B.saux2.reserve(slots);
     if (TASK == 1) {
-      B.sy.reserve(el);
-      B.sy2.reserve(el);
+      B.sy.reserve(slots);
+      B.sy2.reserve(slots);
     }
-    DTE_HIP(hipMemsetAsync(B.bcount.p, 0, 4 * nb, s));
-    DTE_HIP(hipMemsetAsync(B.bmax.p, 0, 4 * nb, s));
-    DTE_HIP(hipMemsetAsync(B.ctr.p, 0, 8, s));
+    if (TASK == 0) {
+      DTE_HIP(hipMemsetAsync(B.bcls.p, 0, 4 * (size_t)nb * C, s));
+    } else {
+      DTE_HIP(hipMemsetAsync(B.bn.p, 0, 4 * nb, s));
+      DTE_HIP(hipMemsetAsync(B.bpos.p, 0, 8 * nb, s));
+      DTE_HIP(hipMemsetAsync(B.bneg.p, 0, 8 * nb, s));
+    }
+    DTE_HIP(hipMemsetAsync(B.ctr.p, 0, 12, s));
     V2Args a{};
     a.items = B.items.p;
     a.n_items = n_items;
-    a.bcount = B.bcount.p;
-    a.bmax = B.bmax.p;
+    a.tiles = B.htiles.p;
     a.bcls = B.bcls.p;
-    a.bwn = B.bwn.p;
-    a.bsum = B.bsum.p;
-    a.bbase = B.bbase.p;
+    a.bn = B.bn.p;
+    a.bpos = B.bpos.p;
+    a.bneg = B.bneg.p;
+    a.bub = B.bub.p;
+    a.nbest = B.nbest.p;
+    // Retry draws are taken in order until one scores above 1e-3 (k_decide2):
+    // a draw may be dropped for a later one only while it scores at most that.
+    a.best_cap = it.j0 > 0 ? 1e-3f : __builtin_inff();
+    a.max_dev = B.max_dev;
+    a.bslot = B.bslot.p;
+    a.bnext = B.bnext.p;
     a.bcur = B.bcur.p;
-    a.bsup = B.bsup.p;
-    a.carry_cls = B.carry_cls.p;
-    a.carry_n = B.carry_n.p;
-    a.carry_s = B.carry_s.p;
     a.carry_last = B.carry_last.p;
+    a.isel = B.isel.p;
     a.res_g = B.res_g.p;
     a.res_key = B.res_key.p;
     a.res_prev = B.res_prev.p;
+    a.gkey = B.skey2.p;
     a.skey = B.skey.p;
     a.saux = B.saux.p;
     a.sy = B.sy.p;
     a.skey2 = B.skey2.p;
-    a.gkey = B.skey2.p;
     a.saux2 = B.saux2.p;
     a.sy2 = B.sy2.p;
-    a.tkey = B.tkey.p;
     a.tasks = B.tasks.p;
     a.spill = B.spill.p;
     a.counters = B.ctr.p;
-    a.tiles = B.htiles.p;
+    const dim3 tiles((unsigned)B.host_htiles.size());
+    const dim3 waves((unsigned)((n_items + kWaves - 1) / kWaves));
     {
-      Timer tm("chunk_hist", 0.0, s);
-      hipLaunchKernelGGL(k_v2_hist<TASK>, dim3((unsigned)B.host_htiles.size()), dim3(kBlock), 0, s, d, lv, a);
+      // Algorithmic bytes of the batch's items (12 B per entry, 20 B for
+      // regression) belong to the kernel that reads every entry.
+      Timer tm("chunk_hist", profiling_enabled() ? (double)el * (TASK == 0 ? 12.0 : 20.0) : 0.0, s);
+      hipLaunchKernelGGL(k_v2_hist<TASK>, tiles, dim3(kBlock), (unsigned)(4 * bucket_words * nb_max), s, d, lv, a);
     }
     {
-      Timer tm("chunk_scan", 0.0, s);
-      if (n_small)
-        hipLaunchKernelGGL(k_v2_scan<kWave>, dim3((unsigned)((n_small + kWaves - 1) / kWaves)), dim3(kBlock), 0, s,
-                           a, B.lists.p, n_small);
-      if (n_large)
-        hipLaunchKernelGGL(k_v2_scan<256>, dim3((unsigned)n_large), dim3(kBlock), 0, s, a, B.lists.p + n_small,
-                           n_large);
-    }
-    a.tiles = B.stiles.p;
-    {
-      Timer tm("chunk_scatter", 0.0, s);
-      if (n_sfew)
-        hipLaunchKernelGGL((k_v2_scatter<TASK, kV2FewB>), dim3((unsigned)n_sfew), dim3(kBlock), 0, s, d, lv, a);
-      a.tiles = B.stiles.p + n_sfew;
-      if (n_smid > n_sfew)
-        hipLaunchKernelGGL((k_v2_scatter<TASK, kV2MidB>), dim3((unsigned)(n_smid - n_sfew)), dim3(kBlock), 0, s, d,
-                           lv, a);
-      a.tiles = B.stiles.p + n_smid;
-      if (n_sall > n_smid) {
-        // many buckets: super-buckets, then buckets, over the same tiles
-        hipLaunchKernelGGL((k_v2_scatter<TASK, kV2Super, 1>), dim3((unsigned)(n_sall - n_smid)), dim3(kBlock), 0, s,
-                           d, lv, a);
-        hipLaunchKernelGGL((k_v2_scatter<TASK, kV2MaxB, 2>), dim3((unsigned)(n_sall - n_smid)), dim3(kBlock), 0, s,
-                           d, lv, a);
-      }
-    }
-    a.tiles = B.ctiles.p;
-    {
-      Timer tm("chunk_ctot", 0.0, s);
-      hipLaunchKernelGGL((k_v2_ctot<MAXC, TASK>), dim3((unsigned)B.host_ctiles.size()), dim3(kBlock), 0, s, d, a);
+      Timer tm("chunk_bound", 0.0, s);
+      hipLaunchKernelGGL((k_v2_bound<MAXC, TASK>), waves, dim3(kBlock), 0, s, d, lv, a);
+      hipLaunchKernelGGL(k_v2_select<TASK>, dim3((unsigned)((n_items + kSelectWaves - 1) / kSelectWaves)),
+                         dim3(kSelectWaves * kWave), 0, s, d, a);
     }
     {
-      Timer tm("chunk_carry", 0.0, s);
-      if (n_small)
-        hipLaunchKernelGGL((k_v2_carry<TASK, kWave>), dim3((unsigned)((n_small + kWaves - 1) / kWaves)), dim3(kBlock),
-                           0, s, d, a, B.lists.p, n_small);
-      if (n_large)
-        hipLaunchKernelGGL((k_v2_carry<TASK, 256>), dim3((unsigned)n_large), dim3(kBlock), 0, s, d, a,
-                           B.lists.p + n_small, n_large);
+      Timer tm("chunk_collect", 0.0, s);
+      hipLaunchKernelGGL(k_v2_collect<TASK>, tiles, dim3(kBlock), (unsigned)(9 * nb_max), s, d, lv, a);
     }
-    unsigned int nt[2];
-    DTE_HIP(hipMemcpyAsync(nt, B.ctr.p, 8, hipMemcpyDeviceToHost, s));
-    DTE_HIP(hipStreamSynchronize(s));
-    // Algorithmic bytes of the batch's items (12 B per entry, 20 B for
-    // regression) belong to the evaluation kernel, where every entry is read
-    // and scored; the other pipeline kernels are the price of bucketing.
-    if (nt[0]) {
-      Timer tm("chunk_eval", profiling_enabled() ? (double)el * (TASK == 0 ? 12.0 : 20.0) : 0.0, s);
-      // Two full rounds of the three workgroups a CU holds: grid-stride
-      // over similar buckets, so no partial last round (8 per CU, 2.67
-      // rounds, was 4.5 % slower).
-      const dim3 grid((unsigned)std::min<int64_t>((nt[0] + kWaves - 1) / kWaves, (int64_t)num_cu * 6));
+    {
+      Timer tm("chunk_eval", 0.0, s);
+      // at most two full rounds of the three workgroups a CU holds,
+      // grid-stride over similar buckets (no partial last round)
+      const dim3 grid((unsigned)std::min<int64_t>((nb + kWaves - 1) / kWaves, (int64_t)num_cu * 6));
       if constexpr (TASK == 1)
-        hipLaunchKernelGGL((k_v2_eval_reg<MAXC, TASK>), grid, dim3(kBlock), 0, s, d, lv, a, (int64_t)nt[0]);
+        hipLaunchKernelGGL((k_v2_eval_reg<MAXC, TASK>), grid, dim3(kBlock), 0, s, d, lv, a);
       else
-        hipLaunchKernelGGL((k_v2_eval<MAXC, TASK>), grid, dim3(kBlock), 0, s, d, lv, a, (int64_t)nt[0]);
+        hipLaunchKernelGGL((k_v2_eval<MAXC, TASK>), grid, dim3(kBlock), 0, s, d, lv, a);
     }
-    if (nt[1]) {
+    {
       Timer tm("chunk_spill", 0.0, s);
-      hipLaunchKernelGGL((k_v2_spill<MAXC, TASK>), dim3((unsigned)std::min<int64_t>(nt[1], (int64_t)num_cu * 4)),
-                         dim3(kBlock), 0, s, d, lv, a, (int64_t)nt[1]);
+      hipLaunchKernelGGL((k_v2_spill<MAXC, TASK>), dim3((unsigned)std::min<int64_t>(nb, (int64_t)num_cu * 4)),
+                         dim3(kBlock), 0, s, d, lv, a);
     }
-    hipLaunchKernelGGL(k_v2_reduce<TASK>, dim3((unsigned)((n_items + kWaves - 1) / kWaves)), dim3(kBlock), 0, s, d,
-                       a, it);
+    hipLaunchKernelGGL(k_v2_reduce<TASK>, waves, dim3(kBlock), 0, s, d, a, it);
     if (it.bytes) {
       // algorithmic bytes of the batch: 12 (20) bytes per entry
       const unsigned long long by = (unsigned long long)el * (TASK == 0 ? 12ull : 20ull);
       hipLaunchKernelGGL(k_add_u64, dim3(1), dim3(1), 0, s, it.bytes, by);
     }
     k0 = k1;
+    // the host tables are refilled for the next batch
+    if (k0 < n_all) DTE_HIP(hipStreamSynchronize(s));
   }
 }
 
@@ -4877,7 +5491,9 @@ constexpr int64_t kTMaxCap = (int64_t)1 << 26;
 // needs a scratch slab of this many entries per workgroup.
 constexpr int64_t kGraphMaxM = 65536;
 
-__global__ void k_build_T(int64_t* T, int64_t tmax, int F) {
+__global__ void k_build_T(int64_t* T, int64_t tmax, int F, float* Tf) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < kTfMax) Tf[t] = (float)xlnx((uint64_t)t, g_ln_table.inv, g_ln_table.logc);
   for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x <= tmax; x += (int64_t)gridDim.x * blockDim.x)
     T[x] = xlnx_fixed((uint64_t)x, F, g_ln_table.inv, g_ln_table.logc);
 }
@@ -4888,11 +5504,13 @@ struct FitData {
   DevBuf<uint32_t> label;  // classification
   DevBuf<int64_t> yfix;    // regression: fixed-point targets
   int shift = 0;
+  double max_fixed = 0.0;  // regression: largest |fixed-point target|
   DevBuf<uint32_t> K;      // dense ranks (random forest)
   DevBuf<float> SV;
   DevBuf<int64_t> SVoff;
   DevBuf<uint32_t> Sdev;
   DevBuf<int64_t> Ttab;    // fixed-point x ln x terms T[0..Tmax]
+  DevBuf<float> Tf;        // x ln x in fp32, x < kTfMax
   DataArgs d{};
 };
 
@@ -4931,6 +5549,7 @@ void prepare_data(FitData& fd, const float* X_dev_in, const float* y_host, int64
     double mx = 0;
     for (int64_t i = 0; i < N; ++i) mx = std::max(mx, std::fabs((double)y_host[i]));
     shift = fixed_shift(mx, N);
+    fd.max_fixed = std::ldexp(mx, shift) + 1.0;
     std::vector<int64_t> yf(N);
     for (int64_t i = 0; i < N; ++i) yf[i] = std::llrint(std::ldexp((double)y_host[i], shift));
     yfix.alloc(N);
@@ -4974,8 +5593,11 @@ void prepare_data(FitData& fd, const float* X_dev_in, const float* y_host, int64
     // Counts of a fit never exceed the root's total weight N.
     d.Tmax = task == 0 ? std::min<int64_t>(N, kTMaxCap) : 0;
     Ttab.alloc(d.Tmax + 1);
-    hipLaunchKernelGGL(k_build_T, dim3(grid_for(d.Tmax + 1)), dim3(kBlock), 0, s, Ttab.p, d.Tmax, d.igF);
+    fd.Tf.alloc(kTfMax);
+    hipLaunchKernelGGL(k_build_T, dim3(grid_for(std::max<int64_t>(d.Tmax + 1, kTfMax))), dim3(kBlock), 0, s, Ttab.p,
+                       d.Tmax, d.igF, fd.Tf.p);
     d.T = Ttab.p;
+    d.Tf = fd.Tf.p;
   }
 }
 
@@ -5280,6 +5902,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   const int cut_team = p.cut_team ? p.cut_team : kDefCutTeam;
   const int cut_block = std::max(cut_team, std::min(kCap, p.cut_block ? p.cut_block : kDefCutBlock));
   bigst.target = p.bucket_target ? p.bucket_target : kDefBucketTarget;
+  bigst.max_dev = fd.max_fixed;
   Cuts cuts{};
   if (algorithm == DTE_RANDOM_FOREST) {
     const int c16 = (task == 1 || C <= 16) ? 16 : 0;
