@@ -2638,12 +2638,16 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs 
 // and scored exactly; with about 8 entries a bucket that is one bucket in a
 // hundred, so the sort and the scored walk of all entries (310 wave
 // instructions per 64 entries at 10 classes) are replaced by a histogram (14)
-// and a fixed 300 or so per draw.  The bounds are in fp32 with a margin for
+// and a fixed 400 or so per draw.  The bounds are in fp32 with a margin for
 // their rounding; scored candidates use the exact fixed-point sums, and a
 // candidate whose fp32 score could equal the node's best is always scored.
 // A surviving bucket above 64 entries is split again over its own key range
 // (entries below it are counted as the totals before it); one of a single key
 // has no boundary but its lower edge.
+//
+// Bound by VALU issue, so the register budget decides (a first version with
+// 184 VGPRs ran two waves per SIMD).  Node weights stay within 16 bits (fit_batch's cuts), so that two classes
+// share a word and the table of terms answers every lookup.
 constexpr uint32_t kEdge = 0xFFFFFFFEu;  // previous key not in the list (lower edge of a bucket)
 
 // Best candidate of a draw: exact gain, key, key before it.
@@ -2652,20 +2656,26 @@ struct DrawBest {
   uint32_t key, prev;
 };
 
+// Entries of a run of surviving buckets, for one wave.
+struct BoundList {
+  uint32_t key[kWave], aux[kWave];
+  int64_t y[kWave];
+};
+
 template <int MAXC, int TASK, int LOGB, int IPT>
 struct BoundLds {
   static constexpr int NB = 1 << LOGB;
-  // classification: bucket words [p * nb + b], two classes of 16 bits a word
-  // (nb = NB), or one of 32 bits for node weights above 65535 (nb = NB / 2)
   static constexpr int PAIRS = (MAXC + 1) / 2;
-  static constexpr int TAB = IPT > 8 ? kTfMax : kTfMax / 2;  // staged x ln x terms
+  static constexpr int TAB = kTfMax / 2;  // staged x ln x terms
+  // classification: [p * NB + b], classes 2p and 2p + 1 in the halves of a
+  // word; regression: weights.  Counts, then totals before the bucket.
   uint32_t hist[TASK == 0 ? NB * PAIRS : NB];
   int64_t pos[TASK == 1 ? NB : 1], neg[TASK == 1 ? NB : 1];
-  uint32_t below[TASK == 0 ? MAXC : 1];
+  uint16_t wgt[NB];  // bucket weights
+  uint32_t below[TASK == 0 ? PAIRS : 1];
   int64_t below_s[1];
   uint32_t ncls[TASK == 0 ? MAXC : 1];
-  uint32_t lkey[kWave], laux[kWave];
-  int64_t ly[TASK == 1 ? kWave : 1];
+  BoundList list;
   uint32_t stk_k[IPT + 1];
   uint32_t stk_b[IPT + 1];
 };
@@ -2679,13 +2689,16 @@ __device__ __forceinline__ float wave_last_f32(float v) { return __uint_as_float
 // fp32 chord_gap.
 __device__ __forceinline__ float chord_gap_f32(float a, float s) {
   const float e = s * 0.36788f;
-  return a > 0.0f ? fminf(e, s * s * 0.125001f / a) : e;
+  return a > 0.0f ? fminf(e, s * s * 0.125001f * __builtin_amdgcn_rcpf(a) * 1.00001f) : e;
 }
 
 // A node as one wave works on it.
 struct BoundNode {
   int m;
   int64_t n;
+  const uint32_t* row;  // the node's entries (wave-uniform bases: the loads
+  const uint32_t* aux;  // take a scalar base and a 32-bit lane offset)
+  const int64_t* ey;
   int64_t P;      // classification
   int64_t ssum;   // regression
   double inv;     // classification: 1 / (n ln 2)
@@ -2693,30 +2706,77 @@ struct BoundNode {
   int64_t mu;     // regression: centre
   double M;       // regression: largest |target - centre|
   double E;       // regression: reg_gain_error
-  bool packed;
 };
+
+// f(q, e) for the steps q of a team of TEAM lanes over a node's m entries, q
+// unrolled behind a wave-uniform test; e = lane + TEAM q, clamped to the last
+// entry (no lane is masked off: loads of several steps stay in flight
+// together).  Keys of lanes past m are kNone and fall in no range.
+template <int IPT, int TEAM, class F>
+__device__ __forceinline__ void for_entries(int m, F&& f) {
+  const uint32_t t = TEAM == kWave ? threadIdx.x & (kWave - 1) : threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < IPT; ++q)
+    if (q * TEAM < m) f(q, min(t + (uint32_t)(q * TEAM), (uint32_t)(m - 1)));
+}
+
+// Keys of a draw; kNone past the node's entries.
+template <int IPT, int TEAM>
+__device__ __forceinline__ void gather_keys(const uint32_t* Kf, int m, const uint32_t (&rows)[IPT],
+                                            uint32_t (&key)[IPT]) {
+  for_entries<IPT, TEAM>(m, [&](int q, uint32_t) {
+    uint32_t r = rows[q];
+    asm volatile("" : "+v"(r));  // 32-bit here: else every row is kept as a 64-bit pair
+    key[q] = Kf[r];
+  });
+}
+template <int IPT, int TEAM>
+__device__ __forceinline__ void mask_keys(int m, uint32_t (&key)[IPT]) {
+  const uint32_t t = TEAM == kWave ? threadIdx.x & (kWave - 1) : threadIdx.x;
+  for_entries<IPT, TEAM>(m, [&](int q, uint32_t) {
+    if (t + (uint32_t)(q * TEAM) >= (uint32_t)m) key[q] = kNone;
+  });
+}
+
+// A node's payloads.
+template <int TASK, int IPT>
+struct BoundPay {
+  uint32_t a[IPT];
+  int64_t t[TASK == 1 ? IPT : 1];
+};
+
+// Payloads of a list whose aux words hold entry numbers.
+template <int TASK>
+__device__ __forceinline__ void bound_list_payload(const BoundNode& nd, BoundList& W, int cnt) {
+  const int lane = threadIdx.x & (kWave - 1);
+  if (lane < cnt) {
+    const uint32_t x = W.aux[lane];
+    W.aux[lane] = nd.aux[x];
+    if constexpr (TASK == 1) W.y[lane] = nd.ey[x];
+  }
+  team_sync<kWave>();
+}
 
 // Exact scores of the boundaries of a run of buckets holding cnt <= 64
 // entries (in L.lkey / laux / ly), with the totals before bucket b of the
 // bucket table.
-template <int MAXC, int TASK, int LOGB, int IPT>
-__device__ __forceinline__ void bound_run(const DataArgs& d, const BoundNode& nd, BoundLds<MAXC, TASK, LOGB, IPT>& L,
-                                          int cnt, int b, int nb, DrawBest& best) {
+template <int TASK, int LOGB, class LdsT>
+__device__ __forceinline__ void bound_run(const DataArgs& d, const BoundNode& nd, const LdsT& L, const BoundList& W,
+                                          int cnt, int b, DrawBest& best) {
+  constexpr int NB = 1 << LOGB;
   const int lane = threadIdx.x & (kWave - 1);
   const bool valid = lane < cnt;
-  const uint32_t key = valid ? L.lkey[lane] : kNone;
-  const uint32_t pay = valid ? L.laux[lane] : 0u;
+  const uint32_t key = valid ? W.key[lane] : kNone;
+  const uint32_t pay = valid ? W.aux[lane] : 0u;
   const uint32_t w = pay & 0xFFFFu;
   BestCand c{0.0, kNone, kNone};
   if constexpr (TASK == 0) {
-    const LnCtx lx{g_ln_table.inv, g_ln_table.logc, d.T, d.Tmax, d.igF};
+    const int64_t* T = d.T;
     const uint32_t lab = pay >> 16;
-    auto before = [&](uint32_t cl) -> uint32_t {
-      return nd.packed ? (L.hist[(cl >> 1) * nb + b] >> ((cl & 1u) << 4)) & 0xFFFFu : L.hist[cl * nb + b];
-    };
+    auto before = [&](uint32_t cl) -> uint32_t { return (L.hist[(cl >> 1) * NB + b] >> ((cl & 1u) << 4)) & 0xFFFFu; };
     // totals before the run, one class per lane
     const uint32_t rc = lane < d.C ? before((uint32_t)lane) : 0u;
-    int64_t s0 = lane < d.C ? lx.t(rc) + lx.t(L.ncls[lane] - rc) : 0;
+    int64_t s0 = lane < d.C ? T[rc] + T[L.ncls[lane] - rc] : 0;
     s0 = wave_last_i64(wave_incl_scan_i64(s0));
     const uint32_t n0 = wave_last(wave_incl_scan(rc));
     uint32_t rank = 0, pre = 0, nw = 0;
@@ -2734,8 +2794,8 @@ __device__ __forceinline__ void bound_run(const DataArgs& d, const BoundNode& nd
     const uint32_t nl = n0 + nw;
     if (valid) {
       const uint32_t l = before(lab) + pre, tc = L.ncls[lab];
-      dd = (lx.t(l + w) - lx.t(l)) + (lx.t(tc - l - w) - lx.t(tc - l));
-      tq = lx.t(nl) + lx.t((uint32_t)nd.n - nl);
+      dd = (T[l + w] - T[l]) + (T[tc - l - w] - T[tc - l]);
+      tq = T[nl] + T[(uint32_t)nd.n - nl];
     }
     // running sums in key order, then back to the entry's lane
     const uint32_t ks = ds_permute_u32(rank, key);
@@ -2753,7 +2813,7 @@ __device__ __forceinline__ void bound_run(const DataArgs& d, const BoundNode& nd
       }
     }
   } else {
-    const int64_t y = valid ? L.ly[lane] : 0;
+    const int64_t y = valid ? W.y[lane] : 0;
     uint32_t rank = 0;
     for (int x = 0; x < cnt; ++x) {
       const uint32_t kx = (uint32_t)__builtin_amdgcn_readlane((int)key, x);
@@ -2781,21 +2841,19 @@ __device__ __forceinline__ void bound_run(const DataArgs& d, const BoundNode& nd
 }
 
 // The lower edge of bucket b (a single key, `key`) alone.
-template <int MAXC, int TASK, int LOGB, int IPT>
-__device__ __forceinline__ void bound_edge(const DataArgs& d, const BoundNode& nd, BoundLds<MAXC, TASK, LOGB, IPT>& L,
-                                           uint32_t key, int b, int nb, DrawBest& best) {
+template <int TASK, int LOGB, class LdsT>
+__device__ __forceinline__ void bound_edge(const DataArgs& d, const BoundNode& nd, const LdsT& L, uint32_t key, int b, DrawBest& best) {
+  constexpr int NB = 1 << LOGB;
   const int lane = threadIdx.x & (kWave - 1);
   double g = 0.0;
   if constexpr (TASK == 0) {
-    const LnCtx lx{g_ln_table.inv, g_ln_table.logc, d.T, d.Tmax, d.igF};
-    uint32_t rc = 0;
-    if (lane < d.C)
-      rc = nd.packed ? (L.hist[(lane >> 1) * nb + b] >> ((lane & 1) << 4)) & 0xFFFFu : L.hist[lane * nb + b];
-    int64_t s0 = lane < d.C ? lx.t(rc) + lx.t(L.ncls[lane] - rc) : 0;
+    const int64_t* T = d.T;
+    const uint32_t rc = lane < d.C ? (L.hist[(lane >> 1) * NB + b] >> ((lane & 1) << 4)) & 0xFFFFu : 0u;
+    int64_t s0 = lane < d.C ? T[rc] + T[L.ncls[lane] - rc] : 0;
     s0 = wave_last_i64(wave_incl_scan_i64(s0));
     const uint32_t n0 = wave_last(wave_incl_scan(rc));
     if (n0 == 0) return;
-    const int64_t pq = nd.P + s0 - (lx.t(n0) + lx.t((uint32_t)nd.n - n0));
+    const int64_t pq = nd.P + s0 - (T[n0] + T[(uint32_t)nd.n - n0]);
     if (pq > 0) g = ig_from_fixed(pq, d.igF, nd.inv);
   } else {
     const int64_t pn = (int64_t)L.hist[b], ps = L.pos[b];
@@ -2806,46 +2864,39 @@ __device__ __forceinline__ void bound_edge(const DataArgs& d, const BoundNode& n
 }
 
 // One draw of a node.  thr: lower bound of the node's best gain that matters
-// here (nats / fixed-point units squared, as float / double); returns the
-// draw's best in `best` (none when no candidate of it can be the node's best)
-// and raises thr by what it found.
+// here (nats, or fixed-point units squared); returns the draw's best in
+// `best` (none when no candidate of it can be the node's best) and raises thr
+// by what it found.
 template <int MAXC, int TASK, int LOGB, int IPT>
-__device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& nd, const float* s_tf,
-                                           BoundLds<MAXC, TASK, LOGB, IPT>& L, const uint32_t (&key)[IPT],
-                                           const uint32_t (&aux)[IPT], const int64_t (&y)[TASK == 1 ? IPT : 1],
-                                           double& thr, DrawBest& best) {
+__device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& nd,
+                                           const float* s_tf, BoundLds<MAXC, TASK, LOGB, IPT>& L,
+                                           const uint32_t (&key)[IPT], const BoundPay<TASK, IPT>& pay, double& thr,
+                                           DrawBest& best) {
   using LdsT = BoundLds<MAXC, TASK, LOGB, IPT>;
   constexpr int NB = LdsT::NB;
-  constexpr int NR = NB / kWave > 0 ? NB / kWave : 1;
+  constexpr int NR = NB / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const int m = nd.m;
   uint32_t kmin = kNone, kmax = 0;
-#pragma unroll
-  for (int q = 0; q < IPT; ++q) {
-    if (q * kWave >= m) break;
-    if (lane + q * kWave < m) {
-      kmin = min(kmin, key[q]);
-      kmax = max(kmax, key[q]);
-    }
-  }
+  for_entries<IPT, kWave>(m, [&](int q, uint32_t) {
+    kmin = min(kmin, key[q]);
+    kmax = max(kmax, key[q] + 1u);  // kNone wraps to 0
+  });
   kmin = wave_min_u32(kmin);
-  kmax = wave_max_u32(kmax);
+  kmax = wave_max_u32(kmax) - 1u;
   best = DrawBest{0.0, kNone, kNone};
   if (kmin == kmax) return;  // one value: no boundary
-  const int lognb = nd.packed || TASK == 1 ? LOGB : LOGB - 1;
-  const int nb = 1 << lognb;
   int sp = 1;
   uint32_t k0 = kmin;
   int sb = bit_length(kmax - kmin);
-  bool first = true;
   for (;;) {
-    const int shift = max(0, sb - lognb);
+    const int shift = max(0, sb - LOGB);
     const uint32_t nbk = 1u << (sb - shift);  // buckets of the range
     // ---- bucket table
     if constexpr (TASK == 0) {
-      const int words = nd.packed ? (d.C + 1) / 2 : d.C;
-      for (int i = lane; i < words * nb; i += kWave) L.hist[i] = 0;
-      if (lane < MAXC) L.below[lane] = 0;
+      const int words = (d.C + 1) / 2;
+      for (int i = lane; i < words * NB; i += kWave) L.hist[i] = 0;
+      if (lane < LdsT::PAIRS) L.below[lane] = 0;
     } else {
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
@@ -2859,37 +2910,31 @@ __device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& n
       }
     }
     team_sync<kWave>();
-#pragma unroll
-    for (int q = 0; q < IPT; ++q) {
-      if (q * kWave >= m) break;
-      if (lane + q * kWave < m) {
-        const uint32_t b = (key[q] - k0) >> shift;
-        const bool in = key[q] >= k0 && b < nbk, lower = key[q] < k0;
-        const uint32_t w = aux[q] & 0xFFFFu;
-        if constexpr (TASK == 0) {
-          const uint32_t c = aux[q] >> 16;
-          const uint32_t p = nd.packed ? c >> 1 : c;
-          const uint32_t v = nd.packed ? w << ((c & 1u) << 4) : w;
-          if (in) atomicAdd(&L.hist[p * (uint32_t)nb + b], v);
-          else if (lower) atomicAdd(&L.below[p], v);
-        } else {
-          const int64_t dy = y[q] - nd.mu;
-          const unsigned long long wy = (unsigned long long)((int64_t)w * dy);
-          if (in) {
-            atomicAdd(&L.hist[b], w);
-            atomicAdd(reinterpret_cast<unsigned long long*>(dy < 0 ? &L.neg[b] : &L.pos[b]), wy);
-          } else if (lower) {
-            atomicAdd(&L.below[0], w);
-            atomicAdd(reinterpret_cast<unsigned long long*>(&L.below_s[0]), wy);
-          }
+    for_entries<IPT, kWave>(m, [&](int q, uint32_t e) {
+      const uint32_t b = (key[q] - k0) >> shift;
+      const bool in = key[q] >= k0 && b < nbk, lower = key[q] < k0;
+      const uint32_t a = pay.a[q];
+      const uint32_t w = a & 0xFFFFu;
+      if constexpr (TASK == 0) {
+        const uint32_t p = a >> 17;                 // class / 2
+        const uint32_t v = w << ((a >> 12) & 16u);  // odd class: high half
+        if (in) atomicAdd(&L.hist[p * (uint32_t)NB + b], v);
+        else if (lower) atomicAdd(&L.below[p], v);
+      } else {
+        const int64_t dy = pay.t[q] - nd.mu;
+        const unsigned long long wy = (unsigned long long)((int64_t)w * dy);
+        if (in) {
+          atomicAdd(&L.hist[b], w);
+          atomicAdd(reinterpret_cast<unsigned long long*>(dy < 0 ? &L.neg[b] : &L.pos[b]), wy);
+        } else if (lower) {
+          atomicAdd(&L.below[0], w);
+          atomicAdd(reinterpret_cast<unsigned long long*>(&L.below_s[0]), wy);
         }
       }
-    }
+    });
     team_sync<kWave>();
     // ---- edges and bounds, 64 buckets at a time
-    float ubf[NR];
-    double ubd[TASK == 1 ? NR : 1];
-    uint32_t wgt[NR];
+    uint64_t mask[NR];
     if constexpr (TASK == 0) {
       const bool big_n = nd.n >= LdsT::TAB;
       auto tf = [&](uint32_t x) -> float {
@@ -2898,113 +2943,75 @@ __device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& n
       };
       constexpr int PAIRS = LdsT::PAIRS;
       const uint32_t n = (uint32_t)nd.n;
-      const int words = nd.packed ? (d.C + 1) / 2 : d.C;
+      const int words = (d.C + 1) / 2;
       float eb = 0.0f;
-      if (nd.packed) {
-        uint32_t run[PAIRS];
-        uint32_t run_n = 0;
+      float ub[NR];
+      uint32_t run[PAIRS];
+      uint32_t run_n = 0;
+#pragma unroll
+      for (int p = 0; p < PAIRS; ++p) {
+        run[p] = p < words ? __builtin_amdgcn_readfirstlane(L.below[p]) : 0u;
+        run_n += (run[p] & 0xFFFFu) + (run[p] >> 16);
+      }
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        ub[r] = -1.0f;
+        if ((uint32_t)(r * kWave) >= nbk) break;
+        const int b = r * kWave + lane;
+        uint32_t sw = 0;
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p)
+          if (p < words) {
+            const uint32_t v = L.hist[p * NB + b];
+            sw += (v & 0xFFFFu) + (v >> 16);
+          }
+        const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
+        const float psb = tf(lb) + tf(n - lb);
+        const float psa = lane_below_f32(psb, tf(run_n) + tf(n - run_n));
+        run_n = wave_last(lb);
+        const float slope = sw ? (psb - psa) / (float)sw : 0.0f;
+        float phi = 0.0f, slack = 0.0f;
 #pragma unroll
         for (int p = 0; p < PAIRS; ++p) {
-          run[p] = p < words ? __builtin_amdgcn_readfirstlane(L.below[p]) : 0u;
-          run_n += (run[p] & 0xFFFFu) + (run[p] >> 16);
-        }
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          ubf[r] = -1.0f;
-          wgt[r] = 0;
-          if ((uint32_t)(r * kWave) >= nbk) break;
-          const int b = r * kWave + lane;
-          uint32_t v[PAIRS], sw = 0;
-#pragma unroll
-          for (int p = 0; p < PAIRS; ++p) {
-            v[p] = p < words ? L.hist[p * nb + b] : 0u;
-            sw += (v[p] & 0xFFFFu) + (v[p] >> 16);
-          }
-          const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
-          const float psb = tf(lb) + tf(n - lb);
-          const float psa = lane_below_f32(psb, tf(run_n) + tf(n - run_n));
-          run_n = wave_last(lb);
-          const float slope = sw ? (psb - psa) / (float)sw : 0.0f;
-          float phi = 0.0f, slack = 0.0f;
-#pragma unroll
-          for (int p = 0; p < PAIRS; ++p) {
-            if (p < words) {
-              const uint32_t inc = run[p] + wave_incl_scan(v[p]);
-              const uint32_t n0 = L.ncls[2 * p], n1 = 2 * p + 1 < d.C ? L.ncls[2 * p + 1] : 0u;
-              const uint32_t l0 = inc & 0xFFFFu, l1 = inc >> 16;
-              const float b0 = tf(l0) + tf(n0 - l0), b1 = tf(l1) + tf(n1 - l1);
-              const uint32_t r0 = run[p] & 0xFFFFu, r1 = run[p] >> 16;
-              const float a0 = lane_below_f32(b0, tf(r0) + tf(n0 - r0));
-              const float a1 = lane_below_f32(b1, tf(r1) + tf(n1 - r1));
-              run[p] = wave_last(inc);
-              phi += a0 + a1;
-              slack += fmaxf(0.0f, (b0 - a0) - slope * (float)(v[p] & 0xFFFFu)) +
-                       fmaxf(0.0f, (b1 - a1) - slope * (float)(v[p] >> 16));
-              L.hist[p * nb + b] = inc - v[p];
-            }
-          }
-          slack += chord_gap_f32((float)la, (float)sw) + chord_gap_f32((float)(n - lb), (float)sw);
-          const float edge = nd.Pn + phi - psa;
-          if (sw) {
-            ubf[r] = edge + (shift ? slack : 0.0f) + nd.margin;  // shift 0: one key, only the edge
-            if (la > 0) eb = fmaxf(eb, edge - nd.margin);
-            else if (!shift) ubf[r] = -1.0f;
-          }
-          wgt[r] = sw;
-        }
-      } else {
-        // node weight above 65535: 32-bit counts, half the buckets
-        uint32_t run_n = 0;
-        for (int c = 0; c < words; ++c) run_n += __builtin_amdgcn_readfirstlane(L.below[c]);
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          ubf[r] = -1.0f;
-          wgt[r] = 0;
-          if ((uint32_t)(r * kWave) >= nbk) break;
-          const int b = r * kWave + lane;
-          const bool ok = b < nb;
-          uint32_t sw = 0;
-          for (int c = 0; c < words; ++c) sw += ok ? L.hist[c * nb + b] : 0u;
-          const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
-          const float psb = tf(lb) + tf(n - lb);
-          const float psa = lane_below_f32(psb, tf(run_n) + tf(n - run_n));
-          run_n = wave_last(lb);
-          const float slope = sw ? (psb - psa) / (float)sw : 0.0f;
-          float phi = 0.0f, slack = 0.0f;
-          for (int c = 0; c < words; ++c) {
-            const uint32_t v = ok ? L.hist[c * nb + b] : 0u;
-            const uint32_t r0 = __builtin_amdgcn_readfirstlane(L.below[c]);
-            const uint32_t n0 = L.ncls[c];
-            const uint32_t l = r0 + wave_incl_scan(v);
-            const float b0 = tf(l) + tf(n0 - l);
+          if (p < words) {
+            const uint32_t v = L.hist[p * NB + b];
+            const uint32_t inc = run[p] + wave_incl_scan(v);
+            const uint32_t n0 = L.ncls[2 * p], n1 = PAIRS > 1 || MAXC > 1 ? L.ncls[2 * p + 1] : 0u;
+            const uint32_t l0 = inc & 0xFFFFu, l1 = inc >> 16;
+            const float b0 = tf(l0) + tf(n0 - l0), b1 = tf(l1) + tf(n1 - l1);
+            const uint32_t r0 = run[p] & 0xFFFFu, r1 = run[p] >> 16;
             const float a0 = lane_below_f32(b0, tf(r0) + tf(n0 - r0));
-            phi += a0;
-            slack += fmaxf(0.0f, (b0 - a0) - slope * (float)v);
-            if (ok) L.hist[c * nb + b] = l - v;
-            if (lane == 0) L.below[c] = wave_last(l);
-            team_sync<kWave>();
+            const float a1 = lane_below_f32(b1, tf(r1) + tf(n1 - r1));
+            run[p] = wave_last(inc);
+            phi += a0 + a1;
+            slack += fmaxf(0.0f, (b0 - a0) - slope * (float)(v & 0xFFFFu)) +
+                     fmaxf(0.0f, (b1 - a1) - slope * (float)(v >> 16));
+            L.hist[p * NB + b] = inc - v;
           }
-          slack += chord_gap_f32((float)la, (float)sw) + chord_gap_f32((float)(n - lb), (float)sw);
-          const float edge = nd.Pn + phi - psa;
-          if (sw) {
-            ubf[r] = edge + (shift ? slack : 0.0f) + nd.margin;
-            if (la > 0) eb = fmaxf(eb, edge - nd.margin);
-            else if (!shift) ubf[r] = -1.0f;
-          }
-          wgt[r] = sw;
         }
+        slack += chord_gap_f32((float)la, (float)sw) + chord_gap_f32((float)(n - lb), (float)sw);
+        const float edge = nd.Pn + phi - psa;
+        if (sw) {
+          ub[r] = edge + (shift ? slack : 0.0f) + nd.margin;  // shift 0: one key, only the edge
+          if (la > 0) eb = fmaxf(eb, edge - nd.margin);
+          else if (!shift) ub[r] = -1.0f;
+        }
+        L.wgt[b] = (uint16_t)sw;
       }
-      eb = __uint_as_float(wave_max_u32(__float_as_uint(fmaxf(eb, 0.0f))));
+      eb = __uint_as_float(wave_max_u32(__float_as_uint(eb)));
       thr = fmax(thr, (double)eb);
+      const float thr_f = (float)(thr * (1.0 - 1e-6));
+#pragma unroll
+      for (int r = 0; r < NR; ++r) mask[r] = __ballot(ub[r] >= thr_f && ub[r] > 0.0f);
     } else {
       const double N = (double)nd.n, S = (double)(nd.ssum - nd.mu * nd.n);
       uint32_t run_n = __builtin_amdgcn_readfirstlane(L.below[0]);
       int64_t run_s = L.below_s[0];
       double eb = 0.0;
+      double ub[NR];
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
-        ubd[r] = -1.0;
-        wgt[r] = 0;
+        ub[r] = -1.0;
         if ((uint32_t)(r * kWave) >= nbk) break;
         const int b = r * kWave + lane;
         const uint32_t w = L.hist[b];
@@ -3023,73 +3030,68 @@ __device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& n
             eb = fmax(eb, edge * (1.0 - 2e-6) - nd.E);
           }
           if (shift)
-            ubd[r] = reg_box_bound((double)la, (double)lb, (double)(sa + sn_), (double)(sa + sp_), N, S, nd.M) *
-                         (1.0 + 2e-6) + nd.E;
+            ub[r] = reg_box_bound((double)la, (double)lb, (double)(sa + sn_), (double)(sa + sp_), N, S, nd.M) *
+                        (1.0 + 2e-6) + nd.E;
           else if (la > 0)
-            ubd[r] = edge * (1.0 + 2e-6) + nd.E;
+            ub[r] = edge * (1.0 + 2e-6) + nd.E;
         }
-        wgt[r] = w;
+        L.wgt[b] = (uint16_t)w;
       }
 #pragma unroll
       for (int off = kWave / 2; off > 0; off >>= 1) eb = fmax(eb, __shfl_xor(eb, off, kWave));
       thr = fmax(thr, eb);
+      const double thr_d = thr * (1.0 - 1e-6);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) mask[r] = __ballot(ub[r] >= thr_d && ub[r] > 0.0);
     }
     team_sync<kWave>();
     // ---- surviving buckets
-    const float thr_f = (float)(thr * (1.0 - 1e-6));
-#pragma unroll
     for (int r = 0; r < NR; ++r) {
-      if ((uint32_t)(r * kWave) >= nbk) break;
-      bool sv;
-      if constexpr (TASK == 0) sv = wgt[r] && ubf[r] >= thr_f && ubf[r] > 0.0f;
-      else sv = wgt[r] && ubd[r] >= thr * (1.0 - 1e-6) && ubd[r] > 0.0;
-      uint64_t mask = __ballot(sv);
-      while (mask) {
-        const int i = (int)__ffsll((unsigned long long)mask) - 1;
+      uint64_t mk = mask[0];
+#pragma unroll
+      for (int x = 1; x < NR; ++x) mk = r == x ? mask[x] : mk;
+      while (mk) {
+        const int i = (int)__ffsll((unsigned long long)mk) - 1;
         int e = i;  // last bucket of the run
-        uint32_t wsum = (uint32_t)__builtin_amdgcn_readlane((int)wgt[r], i);
-        mask &= mask - 1;
-        while (e + 1 < kWave && ((mask >> (e + 1)) & 1ull)) {
-          const uint32_t wn = (uint32_t)__builtin_amdgcn_readlane((int)wgt[r], e + 1);
+        const int b = r * kWave + i;
+        uint32_t wsum = __builtin_amdgcn_readfirstlane((uint32_t)L.wgt[b]);
+        mk &= mk - 1;
+        while (e + 1 < kWave && ((mk >> (e + 1)) & 1ull)) {
+          const uint32_t wn = __builtin_amdgcn_readfirstlane((uint32_t)L.wgt[b + (e - i) + 1]);
           if (wsum + wn > (uint32_t)kWave) break;
           wsum += wn;
           ++e;
-          mask &= mask - 1;
+          mk &= mk - 1;
         }
-        const int b = r * kWave + i;
         const uint32_t klo = k0 + ((uint32_t)b << shift);
         const uint32_t kspan = (uint32_t)(e - i + 1) << shift;
         if (!shift && wsum > (uint32_t)kWave) {
-          bound_edge<MAXC, TASK, LOGB, IPT>(d, nd, L, klo, b, nb, best);
+          bound_edge<TASK, LOGB>(d, nd, L, klo, b, best);
           continue;
         }
         int cnt = 0;
-#pragma unroll
-        for (int q = 0; q < IPT; ++q) {
-          if (q * kWave >= m) break;
-          const bool in = lane + q * kWave < m && key[q] - klo < kspan && key[q] >= klo;
+        for_entries<IPT, kWave>(m, [&](int q, uint32_t x) {
+          const bool in = key[q] >= klo && key[q] - klo < kspan;
           const uint64_t bal = __ballot(in);
-          if (bal) {
-            const int at = cnt + (int)__popcll(bal & ((1ull << lane) - 1ull));
-            if (in && at < kWave) {
-              L.lkey[at] = key[q];
-              L.laux[at] = aux[q];
-              if constexpr (TASK == 1) L.ly[at] = y[q];
-            }
-            cnt += (int)__popcll(bal);
+          const int at = cnt + (int)__popcll(bal & ((1ull << lane) - 1ull));
+          if (in && at < kWave) {
+            L.list.key[at] = key[q];
+            L.list.aux[at] = x;  // entry, its payload below
           }
-        }
+          cnt += (int)__popcll(bal);
+        });
         team_sync<kWave>();
         if (cnt > kWave) {
           // one bucket above 64 entries (runs are merged by weight): split it
-          // again; at most IPT disjoint ranges of more than 64 entries exist
+          // again; fewer than IPT disjoint ranges of more than 64 entries exist
           if (lane == 0) {
             L.stk_k[sp] = klo;
             L.stk_b[sp] = (uint32_t)shift;
           }
           ++sp;
         } else {
-          bound_run<MAXC, TASK, LOGB, IPT>(d, nd, L, cnt, b, nb, best);
+          bound_list_payload<TASK>(nd, L.list, cnt);
+          bound_run<TASK, LOGB>(d, nd, L, L.list, cnt, b, best);
         }
         team_sync<kWave>();
       }
@@ -3101,174 +3103,585 @@ __device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& n
     team_sync<kWave>();
     k0 = __builtin_amdgcn_readfirstlane(L.stk_k[sp]);
     sb = (int)__builtin_amdgcn_readfirstlane(L.stk_b[sp]);
-    first = false;
   }
-  (void)first;
   if (best.prev == kEdge) {  // largest key below the best candidate's
     uint32_t p = 0;
-#pragma unroll
-    for (int q = 0; q < IPT; ++q) {
-      if (q * kWave >= m) break;
-      if (lane + q * kWave < m && key[q] < best.key) p = max(p, key[q]);
-    }
+    for_entries<IPT, kWave>(m, [&](int q, uint32_t) {
+      if (key[q] < best.key) p = max(p, key[q]);
+    });
     best.prev = wave_max_u32(p);
   }
 }
 
-// WPN waves per node: 1 (a wave walks its node's draws in order, the next
-// draw's key gather in flight) or 4 (a workgroup per node, its waves take the
-// draws in turn and share the best bound found).
-template <int MAXC, int TASK, int IPT, int LOGB, int WPN>
-__global__ void __launch_bounds__(kBlock) k_search_rf_bound(DataArgs d, LevelArgs lv, ItemArgs it) {
-  constexpr int NPB = kWaves / WPN;  // nodes per workgroup
+// Node context of a bounded search; returns whether the node is pure.  ncls:
+// class totals (LDS).  WG: entries of the node spread over the workgroup
+// (256 per step), else over a wave.
+template <int MAXC, int TASK>
+__device__ __forceinline__ bool bound_node(const DataArgs& d, const LevelArgs& lv, uint32_t i, uint32_t* ncls,
+                                           BoundNode& nd) {
+  const int lane = threadIdx.x & (kWave - 1);
+  nd.m = __builtin_amdgcn_readfirstlane(lv.m[i]);
+  nd.n = __builtin_amdgcn_readfirstlane(lv.count[i]);
+  const int64_t st = lv.start[i];
+  nd.row = lv.row + st;
+  nd.aux = lv.aux + st;
+  nd.ey = TASK == 1 ? lv.ey + st : nullptr;
+  nd.P = 0;
+  nd.ssum = 0;
+  nd.mu = 0;
+  nd.M = 0.0;
+  nd.E = 0.0;
+  if constexpr (TASK == 0) {
+    const uint32_t my = lane < d.C ? lv.cls[(int64_t)i * d.C + lane] : 0u;
+    if (lane < MAXC) ncls[lane] = my;
+    const int64_t tn_fixed = d.T[nd.n];
+    nd.P = tn_fixed - wave_last_i64(wave_incl_scan_i64(lane < d.C ? d.T[my] : 0));
+    nd.inv = 1.0 / ((double)nd.n * kLn2);
+    nd.Pn = (float)ldexp_d((double)nd.P, -d.igF);
+    // fp32 terms of at most T(n) nats: (4 C + 16) roundings of 2^-24 of
+    // twice that, doubled
+    const float tn = (float)ldexp_d((double)tn_fixed, -d.igF);
+    nd.margin = tn * (float)(4 * d.C + 16) * 2.4e-7f + 1e-6f;
+    return (int64_t)wave_max_u32(my) == nd.n;
+  } else {
+    nd.ssum = lv.sum[i];
+    nd.mu = d2ll_rn((double)nd.ssum / (double)nd.n);
+    return false;
+  }
+}
+
+// A score in the units of the bounds, rounded down.
+template <int TASK>
+__device__ __forceinline__ double bound_units(const DataArgs& d, const BoundNode& nd, float s) {
+  return (TASK == 0 ? (double)s * (double)nd.n * kLn2 : ldexp_d((double)s, 2 * d.shift)) * (1.0 - 1e-6);
+}
+
+template <int TASK>
+__device__ __forceinline__ void bound_write(const DataArgs& d, const ItemArgs& it, int64_t ridx, int f,
+                                            const DrawBest& best, float score) {
+  const float* sv = d.SV + d.SVoff[f];
+  it.res_score[ridx] = score;
+  it.res_thr[ridx] = best.key != kNone ? midpoint(sv[best.prev], sv[best.key]) : 0.0f;
+  it.res_feat[ridx] = f;
+}
+
+// Every boundary of a pure node has gain exactly 0: no positive split.
+__device__ __forceinline__ void bound_pure(const DataArgs& d, const ItemArgs& it, uint32_t o, uint32_t tg,
+                                           uint32_t nid) {
+  for (int jj = 0; jj < it.per_group; ++jj) {
+    const int j = it.j0 + jj;
+    const int64_t ridx = (int64_t)o * it.D + j;
+    it.res_score[ridx] = 0.0f;
+    it.res_thr[ridx] = 0.0f;
+    it.res_feat[ridx] = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)j) % (uint32_t)d.F);
+  }
+}
+
+// Nodes of up to 64 IPT entries, one wave per node: the draws in order, the
+// next draw's key gather in flight.
+template <int MAXC, int TASK, int IPT>
+__global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_bound(DataArgs d, LevelArgs lv, ItemArgs it) {
+  constexpr int LOGB = 6;
+  using LdsT = BoundLds<MAXC, TASK, LOGB, IPT>;
   resolve_level(lv, d.C);
   resolve_items(it);
-  if ((int64_t)blockIdx.x * NPB >= it.n_groups) return;  // no node for this workgroup
-  constexpr int kTab = BoundLds<MAXC, TASK, LOGB, IPT>::TAB;
-  __shared__ float s_tf[TASK == 0 ? kTab : 1];
-  __shared__ BoundLds<MAXC, TASK, LOGB, IPT> s_l[kWaves];
-  __shared__ unsigned long long s_best;  // WPN > 1: bits of the shared bound
+  if ((int64_t)blockIdx.x * kWaves >= it.n_groups) return;  // no node for this workgroup
+  __shared__ float s_tf[TASK == 0 ? LdsT::TAB : 1];
+  __shared__ LdsT s_l[kWaves];
   if (TASK == 0)
-    for (int i = threadIdx.x; i < kTab; i += kBlock) s_tf[i] = d.Tf[i];
+    for (int i = threadIdx.x; i < LdsT::TAB; i += kBlock) s_tf[i] = d.Tf[i];
   __syncthreads();
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  BoundLds<MAXC, TASK, LOGB, IPT>& L = s_l[wv];
+  LdsT& L = s_l[wv];
   const int lane = threadIdx.x & (kWave - 1);
   unsigned long long my_bytes = 0;
-  for (int64_t g0 = (int64_t)blockIdx.x * NPB; g0 < it.n_groups; g0 += (int64_t)gridDim.x * NPB) {
-    const int64_t grp = g0 + (WPN == 1 ? wv : 0);
-    const bool live = grp < it.n_groups;
-    if (WPN == 1 && !live) break;  // wave-uniform; one-wave teams have no workgroup barrier
+  for (int64_t grp = (int64_t)blockIdx.x * kWaves + wv; grp < it.n_groups; grp += (int64_t)gridDim.x * kWaves) {
     const uint32_t o = __builtin_amdgcn_readfirstlane(it.list ? it.list[grp] : (uint32_t)grp);
     const uint32_t i = __builtin_amdgcn_readfirstlane(lv.open_idx[o]);
     const uint32_t tg = (uint32_t)__builtin_amdgcn_readfirstlane(lv.tree_global[lv.tree[i]]);
     const uint32_t nid = __builtin_amdgcn_readfirstlane(lv.id[i]);
     BoundNode nd;
-    nd.m = __builtin_amdgcn_readfirstlane(lv.m[i]);
-    nd.n = __builtin_amdgcn_readfirstlane(lv.count[i]);
-    nd.packed = nd.n <= 65535;
-    nd.P = 0;
-    nd.ssum = 0;
-    nd.mu = 0;
-    nd.M = 0.0;
-    nd.E = 0.0;
-    bool pure = false;
-    const int first_draw = WPN == 1 ? 0 : wv;
-    if constexpr (TASK == 0) {
-      const uint32_t my = lane < d.C ? lv.cls[(int64_t)i * d.C + lane] : 0u;
-      if (lane < MAXC) L.ncls[lane] = my;
-      pure = (int64_t)wave_max_u32(my) == nd.n;
-      const LnCtx lx{g_ln_table.inv, g_ln_table.logc, d.T, d.Tmax, d.igF};
-      const int64_t tn_fixed = lx.t((uint64_t)nd.n);
-      nd.P = tn_fixed - wave_last_i64(wave_incl_scan_i64(lane < d.C ? lx.t(my) : 0));
-      nd.inv = 1.0 / ((double)nd.n * kLn2);
-      nd.Pn = (float)ldexp_d((double)nd.P, -d.igF);
-      // fp32 terms of at most T(n) nats: (4 C + 16) roundings of 2^-24 of
-      // twice that, doubled
-      const float tn = (float)ldexp_d((double)tn_fixed, -d.igF);
-      nd.margin = tn * (float)(4 * d.C + 16) * 2.4e-7f + 1e-6f;
-    } else {
-      nd.ssum = lv.sum[i];
-      nd.mu = d2ll_rn((double)nd.ssum / (double)nd.n);
+    if (bound_node<MAXC, TASK>(d, lv, i, L.ncls, nd)) {
+      if (lane == 0) bound_pure(d, it, o, tg, nid);
+      continue;
     }
     const int m = nd.m;
-    const int64_t st = lv.start[i];
-    if (pure) {
-      // Every boundary of a pure node has gain exactly 0: no positive split.
-      if (lane == 0)
-        for (int jj = first_draw; jj < it.per_group; jj += WPN) {
-          const int j = it.j0 + jj;
-          const int64_t ridx = (int64_t)o * it.D + j;
-          it.res_score[ridx] = 0.0f;
-          it.res_thr[ridx] = 0.0f;
-          it.res_feat[ridx] = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)j) % (uint32_t)d.F);
-        }
-      continue;  // workgroup-uniform with WPN > 1
-    }
-    uint32_t rows[IPT], aux[IPT], kn[IPT];
-    int64_t y[TASK == 1 ? IPT : 1];
-#pragma unroll
-    for (int q = 0; q < IPT; ++q) {
-      rows[q] = 0;
-      aux[q] = 0;
-      const int e = lane + q * kWave;
-      if (q * kWave < m && e < m) {
-        rows[q] = lv.row[st + e];
-        aux[q] = lv.aux[st + e];
-        if constexpr (TASK == 1) y[q] = lv.ey[st + e];
-      }
-    }
+    uint32_t rows[IPT], kn[IPT];
+    BoundPay<TASK, IPT> pay;
+    for_entries<IPT, kWave>(m, [&](int q, uint32_t e) {
+      rows[q] = nd.row[e];
+      pay.a[q] = nd.aux[e];
+      if constexpr (TASK == 1) pay.t[q] = nd.ey[e];
+    });
     if constexpr (TASK == 1) {
       double M = 0.0;
-#pragma unroll
-      for (int q = 0; q < IPT; ++q)
-        if (q * kWave < m && lane + q * kWave < m) M = fmax(M, fabs((double)(y[q] - nd.mu)));
+      for_entries<IPT, kWave>(m, [&](int q, uint32_t) { M = fmax(M, fabs((double)(pay.t[q] - nd.mu))); });
 #pragma unroll
       for (int off = kWave / 2; off > 0; off >>= 1) M = fmax(M, __shfl_xor(M, off, kWave));
       nd.M = M * (1.0 + 1e-12);
       nd.E = reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
     }
-    // The node's best score so far (retry phase: the mandatory draws, at most
-    // 1e-3) as a bound in the units of `thr`.
-    double thr = 0.0;
+    // the node's best score so far: the draws before this phase
     float best_score = 0.0f;
     for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
-    auto to_units = [&](float s) {
-      return (TASK == 0 ? (double)s * (double)nd.n * kLn2 : ldexp_d((double)s, 2 * d.shift)) * (1.0 - 1e-6);
-    };
-    thr = to_units(best_score);
-    // Retry draws count in order until one scores above 1e-3 (k_decide2): a
-    // candidate may be dropped for one of a later draw only up to that score.
-    const double cap = it.j0 > 0 && WPN > 1 ? to_units(1e-3f) : __builtin_inf();
-    if (WPN > 1) {
-      __syncthreads();
-      if (threadIdx.x == 0) s_best = __builtin_bit_cast(unsigned long long, thr);
-      __syncthreads();
+    double thr = bound_units<TASK>(d, nd, best_score);
+    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)it.j0) % (uint32_t)d.F);
+    {
+      gather_keys<IPT, kWave>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
     }
-    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + first_draw)) % (uint32_t)d.F);
-    if (WPN == 1) {
-#pragma unroll
-      for (int q = 0; q < IPT; ++q)
-        if (q * kWave < m && lane + q * kWave < m) kn[q] = d.K[(int64_t)f_nx * d.N + rows[q]];
-    }
-    for (int jj = first_draw; jj < it.per_group; jj += WPN) {
+    for (int jj = 0; jj < it.per_group; ++jj) {
       const int j = it.j0 + jj;
-      const int64_t ridx = (int64_t)o * it.D + j;
-      // in order: once a retry draw passed 1e-3 the later ones are not looked at
-      if (WPN == 1 && it.j0 > 0 && (double)best_score > 1e-3) break;
+      // once a retry draw passed 1e-3 the later ones are not looked at (k_decide2)
+      if (it.j0 > 0 && (double)best_score > 1e-3) break;
       const int f = f_nx;
       uint32_t key[IPT];
 #pragma unroll
-      for (int q = 0; q < IPT; ++q) {
-        key[q] = 0;
-        if (q * kWave < m && lane + q * kWave < m) key[q] = WPN == 1 ? kn[q] : d.K[(int64_t)f * d.N + rows[q]];
-      }
-      if (jj + WPN < it.per_group) {
-        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + WPN)) % (uint32_t)d.F);
-        if (WPN == 1) {
-#pragma unroll
-          for (int q = 0; q < IPT; ++q)
-            if (q * kWave < m && lane + q * kWave < m) kn[q] = d.K[(int64_t)f_nx * d.N + rows[q]];
-        }
+      for (int q = 0; q < IPT; ++q) key[q] = kn[q];
+      mask_keys<IPT, kWave>(m, key);
+      if (jj + 1 < it.per_group) {
+        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + 1)) % (uint32_t)d.F);
+        gather_keys<IPT, kWave>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
       }
       DrawBest best;
-      if (WPN > 1) thr = fmin(__builtin_bit_cast(double, *(volatile unsigned long long*)&s_best), cap);
-      bound_draw<MAXC, TASK, LOGB, IPT>(d, nd, s_tf, L, key, aux, y, thr, best);
-      if (WPN > 1 && lane == 0) atomicMax(&s_best, __builtin_bit_cast(unsigned long long, thr));
+      bound_draw<MAXC, TASK, LOGB, IPT>(d, nd, s_tf, L, key, pay, thr, best);
       float score = 0.0f;
       if (best.key != kNone) score = (float)(TASK == 0 ? best.g : ldexp_d(best.g, -2 * d.shift));
       best_score = fmaxf(best_score, score);
-      if (lane == 0) {
-        const float* sv = d.SV + d.SVoff[f];
-        it.res_score[ridx] = score;
-        it.res_thr[ridx] = best.key != kNone ? midpoint(sv[best.prev], sv[best.key]) : 0.0f;
-        it.res_feat[ridx] = f;
-      }
+      if (lane == 0) bound_write<TASK>(d, it, (int64_t)o * it.D + j, f, best, score);
     }
-    if (lane == 0 && (WPN == 1 || wv == 0))
-      my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
+    if (lane == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
   }
   if (lane == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+}
+
+// Nodes of up to 2048 entries, one workgroup per node and draw at a time: 256
+// buckets (128 above 16 classes), bounded 64 to a wave; every wave scores the
+// surviving buckets of its own 64.  The entries of those buckets come from
+// all waves through a list per wave, in rounds of at most kTeamList of them.
+constexpr int kTeamIpt2 = kCap / kBlock;  // entries per thread
+constexpr int kTeamList = 128;
+constexpr int kTeamStack = kCap / kWave + 1;  // disjoint ranges of more than 64 entries
+
+template <int MAXC, int TASK, int LOGB>
+struct BoundTeamLds {
+  static constexpr int NB = 1 << LOGB;
+  static constexpr int PAIRS = (MAXC + 1) / 2;
+  uint32_t hist[TASK == 0 ? NB * PAIRS : NB];
+  int64_t pos[TASK == 1 ? NB : 1], neg[TASK == 1 ? NB : 1];
+  uint16_t wgt[NB];
+  uint32_t below[TASK == 0 ? PAIRS : 1];
+  int64_t below_s[1];
+  uint32_t ncls[TASK == 0 ? MAXC : 1];
+  uint32_t tot[kWaves][TASK == 0 ? PAIRS : 1];  // of a wave's buckets
+  uint32_t tot_n[kWaves];
+  int64_t tot_s[kWaves];
+  uint32_t w[kWaves], w2[kWaves];
+  double eb[kWaves];
+  unsigned long long mask[kWaves];
+  unsigned int cnt[kWaves];
+  uint32_t lkey[kWaves][kTeamList];
+  uint16_t lidx[kWaves][kTeamList];
+  BoundList list[kWaves];
+  DrawBest best[kWaves];
+  uint32_t stk_k[kTeamStack], stk_b[kTeamStack];
+  int sp;
+};
+
+template <int MAXC, int TASK, int LOGB>
+__global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataArgs d, LevelArgs lv, ItemArgs it) {
+  using LdsT = BoundTeamLds<MAXC, TASK, LOGB>;
+  constexpr int IPT = kTeamIpt2;
+  constexpr int NB = LdsT::NB, PAIRS = LdsT::PAIRS;
+  constexpr int NW = NB / kWave;  // waves with buckets
+  resolve_level(lv, d.C);
+  resolve_items(it);
+  if ((int64_t)blockIdx.x >= it.n_groups) return;  // no node for this workgroup
+  __shared__ float s_tf[TASK == 0 ? kTfMax : 1];
+  __shared__ LdsT L;
+  const int t = threadIdx.x;
+  const int lane = t & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(t / kWave);
+  if (TASK == 0)
+    for (int i = t; i < kTfMax; i += kBlock) s_tf[i] = d.Tf[i];
+  unsigned long long my_bytes = 0;
+  for (int64_t grp = blockIdx.x; grp < it.n_groups; grp += gridDim.x) {
+    const uint32_t o = __builtin_amdgcn_readfirstlane(it.list ? it.list[grp] : (uint32_t)grp);
+    const uint32_t i = __builtin_amdgcn_readfirstlane(lv.open_idx[o]);
+    const uint32_t tg = (uint32_t)__builtin_amdgcn_readfirstlane(lv.tree_global[lv.tree[i]]);
+    const uint32_t nid = __builtin_amdgcn_readfirstlane(lv.id[i]);
+    BoundNode nd;
+    __syncthreads();  // the previous node's class totals are read no more
+    if (bound_node<MAXC, TASK>(d, lv, i, L.ncls, nd)) {  // workgroup-uniform
+      if (t == 0) bound_pure(d, it, o, tg, nid);
+      continue;
+    }
+    const int m = nd.m;
+    uint32_t rows[IPT], kn[IPT];
+    BoundPay<TASK, IPT> pay;
+    auto entries = [&](auto&& f) { for_entries<IPT, kBlock>(m, f); };
+    entries([&](int q, uint32_t e) {
+      rows[q] = nd.row[e];
+      pay.a[q] = nd.aux[e];
+      if constexpr (TASK == 1) pay.t[q] = nd.ey[e];
+    });
+    if constexpr (TASK == 1) {
+      double M = 0.0;
+      entries([&](int q, uint32_t) { M = fmax(M, fabs((double)(pay.t[q] - nd.mu))); });
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) M = fmax(M, __shfl_xor(M, off, kWave));
+      if (lane == 0) L.eb[wv] = M;
+      __syncthreads();
+      for (int x = 0; x < kWaves; ++x) M = fmax(M, L.eb[x]);
+      nd.M = M * (1.0 + 1e-12);
+      nd.E = reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
+    }
+    float best_score = 0.0f;
+    for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
+    double thr = bound_units<TASK>(d, nd, best_score);
+    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)it.j0) % (uint32_t)d.F);
+    {
+      gather_keys<IPT, kBlock>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
+    }
+    for (int jj = 0; jj < it.per_group; ++jj) {
+      const int j = it.j0 + jj;
+      if (it.j0 > 0 && (double)best_score > 1e-3) break;
+      const int f = f_nx;
+      uint32_t key[IPT];
+#pragma unroll
+      for (int q = 0; q < IPT; ++q) key[q] = kn[q];
+      mask_keys<IPT, kBlock>(m, key);
+      if (jj + 1 < it.per_group) {
+        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + 1)) % (uint32_t)d.F);
+        gather_keys<IPT, kBlock>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
+      }
+      uint32_t kmin = kNone, kmax = 0;
+      entries([&](int q, uint32_t) {
+        kmin = min(kmin, key[q]);
+        kmax = max(kmax, key[q] + 1u);  // kNone wraps to 0
+      });
+      kmin = wave_min_u32(kmin);
+      kmax = wave_max_u32(kmax);
+      if (lane == 0) {
+        L.w[wv] = kmin;
+        L.w2[wv] = kmax;
+      }
+      if (t == 0) L.sp = 0;
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < kWaves; ++x) {
+        kmin = min(kmin, L.w[x]);
+        kmax = max(kmax, L.w2[x]);
+      }
+      kmin = __builtin_amdgcn_readfirstlane(kmin);
+      kmax = __builtin_amdgcn_readfirstlane(kmax) - 1u;
+      DrawBest best{0.0, kNone, kNone};
+      uint32_t k0 = kmin;
+      int sb = bit_length(kmax - kmin);
+      bool more = kmin != kmax;  // one value: no boundary
+      while (more) {
+        const int shift = max(0, sb - LOGB);
+        const uint32_t nbk = 1u << (sb - shift);  // buckets of the range
+        // ---- bucket table
+        if constexpr (TASK == 0) {
+          const int words = (d.C + 1) / 2;
+          for (int x = t; x < words * NB; x += kBlock) L.hist[x] = 0;
+          if (t < PAIRS) L.below[t] = 0;
+        } else {
+          for (int x = t; x < NB; x += kBlock) {
+            L.hist[x] = 0;
+            L.pos[x] = 0;
+            L.neg[x] = 0;
+          }
+          if (t == 0) {
+            L.below[0] = 0;
+            L.below_s[0] = 0;
+          }
+        }
+        __syncthreads();
+        entries([&](int q, uint32_t) {
+          const uint32_t b = (key[q] - k0) >> shift;
+          const bool in = key[q] >= k0 && b < nbk, lower = key[q] < k0;
+          const uint32_t a = pay.a[q];
+          const uint32_t w = a & 0xFFFFu;
+          if constexpr (TASK == 0) {
+            const uint32_t p = a >> 17;                 // class / 2
+            const uint32_t v = w << ((a >> 12) & 16u);  // odd class: high half
+            if (in) atomicAdd(&L.hist[p * (uint32_t)NB + b], v);
+            else if (lower) atomicAdd(&L.below[p], v);
+          } else {
+            const int64_t dy = pay.t[q] - nd.mu;
+            const unsigned long long wy = (unsigned long long)((int64_t)w * dy);
+            if (in) {
+              atomicAdd(&L.hist[b], w);
+              atomicAdd(reinterpret_cast<unsigned long long*>(dy < 0 ? &L.neg[b] : &L.pos[b]), wy);
+            } else if (lower) {
+              atomicAdd(&L.below[0], w);
+              atomicAdd(reinterpret_cast<unsigned long long*>(&L.below_s[0]), wy);
+            }
+          }
+        });
+        __syncthreads();
+        // ---- edges and bounds of the wave's 64 buckets
+        const int b = wv * kWave + lane;
+        const bool mine = wv < NW && (uint32_t)(wv * kWave) < nbk;
+        double ub = -1.0, eb = 0.0;
+        if constexpr (TASK == 0) {
+          const bool big_n = nd.n >= kTfMax;
+          auto tf = [&](uint32_t x) -> float {
+            if (big_n) return x > 1 ? (float)x * __logf((float)x) : 0.0f;
+            return s_tf[x];
+          };
+          const uint32_t n = (uint32_t)nd.n;
+          const int words = (d.C + 1) / 2;
+          uint32_t inc[PAIRS], sw = 0;
+          if (mine) {
+#pragma unroll
+            for (int p = 0; p < PAIRS; ++p) {
+              inc[p] = 0;
+              if (p < words) {
+                const uint32_t v = L.hist[p * NB + b];
+                sw += (v & 0xFFFFu) + (v >> 16);
+                inc[p] = wave_incl_scan(v);
+                if (lane == kWave - 1) L.tot[wv][p] = inc[p];
+              }
+            }
+            const uint32_t si = wave_incl_scan(sw);
+            if (lane == kWave - 1) L.tot_n[wv] = si;
+          }
+          __syncthreads();
+          if (mine) {
+            uint32_t run_n = 0;
+#pragma unroll
+            for (int p = 0; p < PAIRS; ++p)
+              if (p < words) {
+                const uint32_t bl = L.below[p];
+                run_n += (bl & 0xFFFFu) + (bl >> 16);
+              }
+            for (int x = 0; x < wv; ++x) run_n += L.tot_n[x];
+            const uint32_t lb = run_n + wave_incl_scan(sw), la = lb - sw;
+            const float psb = tf(lb) + tf(n - lb);
+            const float psa = lane_below_f32(psb, tf(run_n) + tf(n - run_n));
+            const float slope = sw ? (psb - psa) / (float)sw : 0.0f;
+            float phi = 0.0f, slack = 0.0f;
+#pragma unroll
+            for (int p = 0; p < PAIRS; ++p) {
+              if (p < words) {
+                uint32_t run = L.below[p];
+                for (int x = 0; x < wv; ++x) run += L.tot[x][p];
+                const uint32_t v = L.hist[p * NB + b];
+                const uint32_t e = run + inc[p];
+                const uint32_t n0 = L.ncls[2 * p], n1 = MAXC > 1 ? L.ncls[2 * p + 1] : 0u;
+                const uint32_t l0 = e & 0xFFFFu, l1 = e >> 16;
+                const float b0 = tf(l0) + tf(n0 - l0), b1 = tf(l1) + tf(n1 - l1);
+                const uint32_t r0 = run & 0xFFFFu, r1 = run >> 16;
+                const float a0 = lane_below_f32(b0, tf(r0) + tf(n0 - r0));
+                const float a1 = lane_below_f32(b1, tf(r1) + tf(n1 - r1));
+                phi += a0 + a1;
+                slack += fmaxf(0.0f, (b0 - a0) - slope * (float)(v & 0xFFFFu)) +
+                         fmaxf(0.0f, (b1 - a1) - slope * (float)(v >> 16));
+                L.hist[p * NB + b] = e - v;
+              }
+            }
+            slack += chord_gap_f32((float)la, (float)sw) + chord_gap_f32((float)(n - lb), (float)sw);
+            const float edge = nd.Pn + phi - psa;
+            float ebf = 0.0f;
+            if (sw) {
+              if (shift || la > 0) ub = (double)(edge + (shift ? slack : 0.0f) + nd.margin);
+              if (la > 0) ebf = fmaxf(0.0f, edge - nd.margin);
+            }
+            L.wgt[b] = (uint16_t)sw;
+            eb = (double)__uint_as_float(wave_max_u32(__float_as_uint(ebf)));
+          }
+        } else {
+          uint32_t w = 0;
+          int64_t sp_ = 0, sn_ = 0, si = 0;
+          uint32_t wi = 0;
+          if (mine) {
+            w = L.hist[b];
+            sp_ = L.pos[b];
+            sn_ = L.neg[b];
+            wi = wave_incl_scan(w);
+            si = wave_incl_scan_i64(sp_ + sn_);
+            if (lane == kWave - 1) {
+              L.tot_n[wv] = wi;
+              L.tot_s[wv] = si;
+            }
+          }
+          __syncthreads();
+          if (mine) {
+            uint32_t run_n = L.below[0];
+            int64_t run_s = L.below_s[0];
+            for (int x = 0; x < wv; ++x) {
+              run_n += L.tot_n[x];
+              run_s += L.tot_s[x];
+            }
+            const double N = (double)nd.n, S = (double)(nd.ssum - nd.mu * nd.n);
+            const uint32_t lb = run_n + wi, la = lb - w;
+            const int64_t sa = run_s + si - (sp_ + sn_);
+            L.hist[b] = la;
+            L.pos[b] = sa + nd.mu * (int64_t)la;  // uncentred target sum before the bucket
+            L.wgt[b] = (uint16_t)w;
+            if (w) {
+              double edge = 0.0;
+              if (la > 0) {
+                const double s = (double)sa, q = S - s;
+                edge = s * s / (double)la + q * q / (N - (double)la) - S * S / N;
+                eb = fmax(0.0, edge * (1.0 - 2e-6) - nd.E);
+              }
+              if (shift)
+                ub = reg_box_bound((double)la, (double)lb, (double)(sa + sn_), (double)(sa + sp_), N, S, nd.M) *
+                         (1.0 + 2e-6) + nd.E;
+              else if (la > 0)
+                ub = edge * (1.0 + 2e-6) + nd.E;
+            }
+#pragma unroll
+            for (int off = kWave / 2; off > 0; off >>= 1) eb = fmax(eb, __shfl_xor(eb, off, kWave));
+          }
+        }
+        if (lane == 0) L.eb[wv] = eb;
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < kWaves; ++x) thr = fmax(thr, L.eb[x]);
+        const double thr_d = thr * (1.0 - 1e-6);
+        uint64_t mk = __ballot(ub >= thr_d && ub > 0.0);
+        // ---- surviving buckets, in rounds of at most kTeamList entries a wave
+        for (;;) {
+          uint64_t sel = 0;
+          uint32_t wsel = 0;
+          while (mk) {
+            const int x = (int)__ffsll((unsigned long long)mk) - 1;
+            const int bx = wv * kWave + x;
+            const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)L.wgt[bx]);
+            if (w > (uint32_t)kWave) {
+              // more than a list: a single key has only its edge, a wider
+              // bucket is split again
+              const uint32_t klo = k0 + ((uint32_t)bx << shift);
+              if (!shift) {
+                bound_edge<TASK, LOGB>(d, nd, L, klo, bx, best);
+              } else if (lane == 0) {
+                const int at = atomicAdd(&L.sp, 1);
+                L.stk_k[at] = klo;
+                L.stk_b[at] = (uint32_t)shift;
+              }
+            } else {
+              if (wsel + w > (uint32_t)kTeamList) break;
+              wsel += w;
+              sel |= 1ull << x;
+            }
+            mk &= mk - 1;
+          }
+          if (lane == 0) {
+            L.mask[wv] = sel;
+            L.cnt[wv] = 0;
+            L.w[wv] = mk != 0;
+          }
+          __syncthreads();
+          uint64_t any = 0;
+          bool left = false;
+#pragma unroll
+          for (int x = 0; x < NW; ++x) {
+            any |= L.mask[x];
+            left = left || L.w[x];
+          }
+          if (any) {  // workgroup-uniform
+            entries([&](int q, uint32_t e) {
+              const uint32_t bx = (key[q] - k0) >> shift;
+              if (key[q] >= k0 && bx < nbk && ((L.mask[bx / kWave] >> (bx & (kWave - 1))) & 1ull)) {
+                const unsigned int at = atomicAdd(&L.cnt[bx / kWave], 1u);
+                L.lkey[bx / kWave][at] = key[q];
+                L.lidx[bx / kWave][at] = (uint16_t)e;
+              }
+            });
+          }
+          __syncthreads();
+          if (sel) {
+            const int nl = (int)L.cnt[wv];
+            uint32_t lk[kTeamList / kWave], lx[kTeamList / kWave];
+#pragma unroll
+            for (int x = 0; x < kTeamList / kWave; ++x) {
+              const bool in = lane + x * kWave < nl;
+              lk[x] = in ? L.lkey[wv][lane + x * kWave] : 0u;
+              lx[x] = in ? L.lidx[wv][lane + x * kWave] : 0u;
+            }
+            BoundList& W = L.list[wv];
+            while (sel) {
+              const int x0 = (int)__ffsll((unsigned long long)sel) - 1;
+              int x1 = x0;  // last bucket of the run
+              const int bx = wv * kWave + x0;
+              uint32_t wsum = __builtin_amdgcn_readfirstlane((uint32_t)L.wgt[bx]);
+              sel &= sel - 1;
+              while (x1 + 1 < kWave && ((sel >> (x1 + 1)) & 1ull)) {
+                const uint32_t wn = __builtin_amdgcn_readfirstlane((uint32_t)L.wgt[wv * kWave + x1 + 1]);
+                if (wsum + wn > (uint32_t)kWave) break;
+                wsum += wn;
+                ++x1;
+                sel &= sel - 1;
+              }
+              const uint32_t klo = k0 + ((uint32_t)bx << shift);
+              const uint32_t kspan = (uint32_t)(x1 - x0 + 1) << shift;
+              int cnt = 0;
+#pragma unroll
+              for (int x = 0; x < kTeamList / kWave; ++x) {
+                const bool in = lane + x * kWave < nl && lk[x] >= klo && lk[x] - klo < kspan;
+                const uint64_t bal = __ballot(in);
+                const int at = cnt + (int)__popcll(bal & ((1ull << lane) - 1ull));
+                if (in) {
+                  W.key[at] = lk[x];
+                  W.aux[at] = lx[x];
+                }
+                cnt += (int)__popcll(bal);
+              }
+              team_sync<kWave>();
+              bound_list_payload<TASK>(nd, W, cnt);
+              bound_run<TASK, LOGB>(d, nd, L, W, cnt, bx, best);
+              team_sync<kWave>();
+            }
+          }
+          __syncthreads();
+          if (!left) break;  // workgroup-uniform
+        }
+        if (best.key != kNone)
+          thr = fmax(thr, (TASK == 0 ? best.g * (double)nd.n * kLn2 : best.g) * (1.0 - 1e-6));
+        // ---- next range (every thread takes the same one)
+        const int sp = L.sp;
+        more = sp > 0;
+        if (more) {
+          k0 = __builtin_amdgcn_readfirstlane(L.stk_k[sp - 1]);
+          sb = (int)__builtin_amdgcn_readfirstlane(L.stk_b[sp - 1]);
+        }
+        __syncthreads();
+        if (more && t == 0) L.sp = sp - 1;
+      }
+      // ---- the draw's best over the waves
+      if (lane == 0) L.best[wv] = best;
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < kWaves; ++x)
+        if (L.best[x].key != kNone && cand_better(L.best[x].g, L.best[x].key, best.g, best.key)) best = L.best[x];
+      if (best.prev == kEdge) {  // largest key below the best candidate's
+        uint32_t p = 0;
+        entries([&](int q, uint32_t) {
+          if (key[q] < best.key) p = max(p, key[q]);
+        });
+        p = wave_max_u32(p);
+        if (lane == 0) L.w[wv] = p;
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < kWaves; ++x) p = max(p, L.w[x]);
+        best.prev = p;
+      }
+      float score = 0.0f;
+      if (best.key != kNone) {
+        score = (float)(TASK == 0 ? best.g : ldexp_d(best.g, -2 * d.shift));
+        thr = fmax(thr, (TASK == 0 ? best.g * (double)nd.n * kLn2 : best.g) * (1.0 - 1e-6));
+      }
+      best_score = fmaxf(best_score, score);
+      if (t == 0) bound_write<TASK>(d, it, (int64_t)o * it.D + j, f, best, score);
+      __syncthreads();  // L.best, L.w are rewritten by the next draw
+    }
+    if (t == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
+  }
+  if (t == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
 }
 
 // ERT, one wave per item (any node size; lanes stride over the entries).
@@ -4740,7 +5153,7 @@ __global__ void __launch_bounds__(kBlock) k_boot_compact(const uint32_t* mult, c
                                                          const uint32_t* label, const int64_t* yfix, int C,
                                                          uint32_t* row, uint32_t* aux, int64_t* ey,
                                                          uint32_t* root_cls, int64_t* root_sum, uint64_t* root_hash,
-                                                         uint32_t* overflow) {
+                                                         uint32_t* w_max) {
   __shared__ uint32_t s_cls[32 * kBlock];  // [class * kBlock + thread]
   const int tr = blockIdx.y;
   const uint32_t* mt = mult + (int64_t)tr * N;
@@ -4750,10 +5163,11 @@ __global__ void __launch_bounds__(kBlock) k_boot_compact(const uint32_t* mult, c
     for (int c = 0; c < C; ++c) s_cls[c * kBlock + t] = 0;
   uint64_t hsh = 0;
   int64_t sm = 0;
+  uint32_t wm = 0;
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < N; r += (int64_t)gridDim.x * blockDim.x) {
     const uint32_t w = mt[r];
     if (!w) continue;
-    if (w > 0xFFFFu) atomicOr(overflow, 1u);
+    wm = max(wm, w);
     const uint32_t p = pt[r];
     const uint32_t lab = label ? label[r] : 0u;
     row[p] = (uint32_t)r;
@@ -4777,7 +5191,9 @@ __global__ void __launch_bounds__(kBlock) k_boot_compact(const uint32_t* mult, c
     hsh += __shfl_xor(hsh, off, kWave);
     sm += __shfl_xor(sm, off, kWave);
   }
+  wm = wave_max_u32(wm);
   if ((threadIdx.x & (kWave - 1)) == 0) {
+    atomicMax(w_max, wm);
     atomicAdd((unsigned long long*)&root_hash[tr], (unsigned long long)hsh);
     if (yfix) atomicAdd((unsigned long long*)&root_sum[tr], (unsigned long long)sm);
   }
@@ -5138,9 +5554,9 @@ void launch_search(int algorithm, int tier, int grid, hipStream_t s, const DataA
     switch (tier) {
       case 0: hipLaunchKernelGGL((k_search_rf_seg<MAXC, TASK, 16>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       case 1: hipLaunchKernelGGL((k_search_rf_seg<MAXC, TASK, 32>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 2: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 1, 6, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 3: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 8, 6, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 4: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 32, MAXC <= 16 ? 8 : 7, 4>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 2: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 3: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 8>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 4: hipLaunchKernelGGL((k_search_rf_bound_team<MAXC, TASK, MAXC <= 16 ? 8 : 7>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       default: hipLaunchKernelGGL((k_search_rf<MAXC, TASK, 256, true>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
     }
   } else {
@@ -5666,6 +6082,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
 
   // ---- root entries.
   int64_t E = 0;
+  uint32_t w_max = 1;  // largest entry weight
   std::vector<int64_t> root_start(T), root_m(T);
   DevBuf<uint32_t> rowA, auxA, rowB, auxB;
   DevBuf<int64_t> eyA, eyB;
@@ -5706,13 +6123,14 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       eyA.alloc(E);
       eyB.alloc(E);
     }
-    DevBuf<uint32_t> overflow(1);
-    DTE_HIP(hipMemsetAsync(overflow.p, 0, 4, s));
+    DevBuf<uint32_t> w_max_dev(1);
+    DTE_HIP(hipMemsetAsync(w_max_dev.p, 0, 4, s));
     hipLaunchKernelGGL(k_boot_compact, dim3(grid_for(N, kBlock, kBootCompactBlocks), T), dim3(kBlock), 0, s, mult.p,
                        pos.p, N,
                        label, yfix, C, rowA.p, auxA.p, eyA.p, root_cls.p, root_sum.p, root_hash.p,
-                       overflow.p);
-    if (read_one(overflow.p, s)) fail(DTE_ERR_INTERNAL, "bootstrap multiplicity above 65535");
+                       w_max_dev.p);
+    w_max = read_one(w_max_dev.p, s);
+    if (w_max > 0xFFFFu) fail(DTE_ERR_INTERNAL, "bootstrap multiplicity above 65535");
   } else {
     E = 0;
     for (int t = 0; t < T; ++t) {
@@ -5899,15 +6317,20 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   // path above its LDS capacity).
   // Nodes above the workgroup's LDS capacity go through the chunk-parallel
   // pipeline (the plain driver keeps one workgroup per node throughout).
-  const int cut_team = p.cut_team ? p.cut_team : kDefCutTeam;
-  const int cut_block = std::max(cut_team, std::min(kCap, p.cut_block ? p.cut_block : kDefCutBlock));
+  // k_search_rf_bound counts two classes in a word: its nodes weigh at most
+  // 65535 (a bootstrap's multiplicities hardly ever pass 15, so this bites at
+  // no node size; the pipeline takes any weight).
+  const int m_packed = (int)std::max<int64_t>(1, 65535 / (int64_t)std::max<uint32_t>(w_max, 1));
+  const int cut_team = std::min(m_packed, p.cut_team ? p.cut_team : kDefCutTeam);
+  const int cut_block =
+      std::min(m_packed, std::max(cut_team, std::min(kCap, p.cut_block ? p.cut_block : kDefCutBlock)));
   bigst.target = p.bucket_target ? p.bucket_target : kDefBucketTarget;
   bigst.max_dev = fd.max_fixed;
   Cuts cuts{};
   if (algorithm == DTE_RANDOM_FOREST) {
     const int c16 = (task == 1 || C <= 16) ? 16 : 0;
     const int c32 = (task == 1 || C <= 32) ? 32 : 0;
-    cuts = Cuts{{c16, std::max(c16, c32), 64, cut_team, cut_block, 0x7FFFFFFF}, 6};
+    cuts = Cuts{{c16, std::max(c16, c32), std::min(64, cut_team), cut_team, cut_block, 0x7FFFFFFF}, 6};
   } else {
     // segment tiers need a lane per class
     const int c16 = (task == 1 || C <= 16) ? 16 : 0;
