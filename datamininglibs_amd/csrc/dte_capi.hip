@@ -323,35 +323,6 @@ void profile_add_bytes(const char* name, double bytes) {
 using namespace dte;
 
 namespace {
-struct HostModel {
-  std::vector<int64_t> ts;
-  std::vector<int32_t> feature, left;
-  std::vector<float> thr, value;
-  std::vector<uint32_t> cls;
-};
-
-HostModel pull_model(const Forest& f) {
-  hipStream_t s = library_stream(f.device);
-  HostModel m;
-  const int64_t n = f.n_nodes;
-  m.ts.resize(f.n_trees + 1);
-  DTE_HIP(hipMemcpyAsync(m.ts.data(), f.tree_start.p, 8 * (f.n_trees + 1), hipMemcpyDeviceToHost, s));
-  m.feature.resize(n);
-  m.left.resize(n);
-  m.thr.resize(n);
-  m.value.resize(n);
-  DTE_HIP(hipMemcpyAsync(m.feature.data(), f.feature.p, 4 * n, hipMemcpyDeviceToHost, s));
-  DTE_HIP(hipMemcpyAsync(m.left.data(), f.left.p, 4 * n, hipMemcpyDeviceToHost, s));
-  DTE_HIP(hipMemcpyAsync(m.thr.data(), f.threshold.p, 4 * n, hipMemcpyDeviceToHost, s));
-  DTE_HIP(hipMemcpyAsync(m.value.data(), f.value.p, 4 * n, hipMemcpyDeviceToHost, s));
-  if (f.task == 0) {
-    m.cls.resize((size_t)n * f.n_classes);
-    DTE_HIP(hipMemcpyAsync(m.cls.data(), f.class_counts.p, 4 * m.cls.size(), hipMemcpyDeviceToHost, s));
-  }
-  DTE_HIP(hipStreamSynchronize(s));
-  return m;
-}
-
 int64_t count_leaves(const std::vector<int32_t>& feature) {
   int64_t n = 0;
   for (auto v : feature) n += v < 0;
@@ -615,44 +586,7 @@ int dte_forest_export(const dte_forest* forest, dte_node* nodes, int64_t nodes_c
     if (!forest || !nodes || !probs) fail(DTE_ERR_INVALID_ARGUMENT, "NULL pointer argument");
     const Forest& f = forest->f;
     DTE_HIP(hipSetDevice(f.device));
-    HostModel m = pull_model(f);
-    const int64_t n = f.n_nodes;
-    const int T = f.n_trees;
-    const int P = f.task == 0 ? f.n_classes : 1;
-    if (nodes_cap < n) fail(DTE_ERR_INVALID_ARGUMENT, "nodes_cap too small");
-    if (probs_cap < count_leaves(m.feature) * P) fail(DTE_ERR_INVALID_ARGUMENT, "probs_cap too small");
-    // canonical index -> export index: roots first (gpudte_algorithm.cc:349-357),
-    // then every tree's remaining nodes in level order.
-    std::vector<int64_t> ex(n);
-    int64_t next = T;
-    for (int t = 0; t < T; ++t) {
-      ex[m.ts[t]] = t;
-      for (int64_t g = m.ts[t] + 1; g < m.ts[t + 1]; ++g) ex[g] = next++;
-    }
-    std::vector<int64_t> inv(n);
-    for (int64_t g = 0; g < n; ++g) inv[ex[g]] = g;
-    int64_t pcur = 0;
-    for (int64_t e = 0; e < n; ++e) {
-      const int64_t g = inv[e];
-      dte_node& d = nodes[e];
-      if (m.feature[g] >= 0) {
-        d.child_start = (int32_t)ex[m.left[g]];
-        d.child_count = 2;
-        d.probability_start = -1;
-        d.attribute = m.feature[g];
-        d.split_point = m.thr[g];
-      } else {
-        d.child_start = -1;
-        d.child_count = 0;
-        d.probability_start = (int32_t)pcur;
-        d.attribute = -1;
-        d.split_point = -1.0f;
-        if (f.task == 0)
-          for (int c = 0; c < P; ++c) probs[pcur++] = (float)m.cls[g * P + c];
-        else
-          probs[pcur++] = m.value[g];
-      }
-    }
+    export_forest(f, nodes, nodes_cap, probs, probs_cap, library_stream(f.device));
   });
 }
 

@@ -225,6 +225,11 @@ std::vector<Forest*> fit_joint(const float* const* X_dev, const float* const* y_
                                const int32_t* n_features, const dte_params* params, int n, hipStream_t stream);
 void predict_forest(const Forest& f, const float* X_dev, int64_t n_rows, int64_t ld,
                     int row_major, int32_t* votes_dev, float* sums_dev, hipStream_t stream);
+// Reference model layout (dte_forest_export) into host arrays.
+void export_forest(const Forest& f, dte_node* nodes, int64_t nodes_cap, float* probs, int64_t probs_cap,
+                   hipStream_t stream);
+// Exclusive scan of n words into out[0 .. n] (out[n] = total).
+void scan_u32_ext(const uint32_t* in, int64_t n, uint32_t* out, hipStream_t s, std::vector<DevBuf<uint32_t>>& tmp);
 // In place: int32 vote counts -> the same values as float.
 void votes_to_float(int32_t* votes, int64_t n, hipStream_t stream);
 // Out-of-bag evaluation (dte_oob_evaluate): pairs evaluated, correct pairs
