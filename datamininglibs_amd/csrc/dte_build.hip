@@ -5293,34 +5293,6 @@ __global__ void k_finalize(FinalArgs a) {
   }
 }
 
-__global__ void k_predict_nodes(int64_t n, int C, int task, const int32_t* feature, const float* thr,
-                                const int32_t* left, const uint32_t* cls, const float* value, PNode* out) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    PNode p;
-    p.feature = feature[i];
-    p.pad = 0;
-    if (p.feature >= 0) {
-      p.thr = thr[i];
-      p.left = left[i];
-    } else if (task == 0) {
-      // vote = argmax, strict > from 0: lowest class on ties (gpudte.cu:341-351)
-      int best = 0;
-      uint32_t bv = 0;
-      for (int c = 0; c < C; ++c)
-        if (cls[i * C + c] > bv) {
-          bv = cls[i * C + c];
-          best = c;
-        }
-      p.thr = 0.0f;
-      p.left = best;
-    } else {
-      p.thr = value[i];
-      p.left = 0;
-    }
-    out[i] = p;
-  }
-}
-
 // ---------------------------------------- device-described level step --
 // Partition tiers: 16- and 32-lane segments, a wave, a workgroup per node.
 constexpr Cuts kPartCuts{{16, 32, 512, 0x7FFFFFFF, 0, 0}, 4};
@@ -6041,8 +6013,10 @@ struct JointSpec {
 // open nodes in chunks of at most 512, one workgroup per node walking its
 // feature draws in order, a host round trip after every chunk; the same
 // device functions compute every result, so both modes give the same bits.
+// whole: the trees are a forest of their own (else part of one, without
+// predict records).
 Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_params& p, hipStream_t s,
-                  bool plain, const JointSpec* J = nullptr) {
+                  bool plain, const JointSpec* J = nullptr, bool whole = true) {
   const auto fit_t0 = std::chrono::steady_clock::now();
   const int task = p.task;
   const int algorithm = p.algorithm;
@@ -7194,7 +7168,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   fa.f_sum = fo->sum_fixed.p;
   fa.f_value = fo->value.p;
   hipLaunchKernelGGL(k_finalize, dim3(grid_for(n_nodes)), dim3(kBlock), 0, s, fa);
-  build_predict_nodes(*fo, s);
+  if (whole) build_predict_nodes(*fo, *std::max_element(per_tree.begin(), per_tree.end()), s);
   DTE_HIP(hipStreamSynchronize(s));
   return fo;
 }
@@ -7265,7 +7239,12 @@ Forest* merge_forests(std::vector<std::unique_ptr<Forest>>& parts, hipStream_t s
     off += m;
     t_off += q->n_trees;
   }
-  build_predict_nodes(*fo, s);
+  std::vector<int64_t> ts(T + 1);
+  DTE_HIP(hipMemcpyAsync(ts.data(), fo->tree_start.p, 8 * ts.size(), hipMemcpyDeviceToHost, s));
+  DTE_HIP(hipStreamSynchronize(s));
+  int64_t max_tree = 1;
+  for (int t = 0; t < T; ++t) max_tree = std::max(max_tree, ts[t + 1] - ts[t]);
+  build_predict_nodes(*fo, max_tree, s);
   DTE_HIP(hipStreamSynchronize(s));
   return guard.release();
 }
@@ -7279,7 +7258,8 @@ Forest* fit_forest(const float* X_dev_in, const float* y_host, int64_t N, int32_
   std::vector<std::unique_ptr<Forest>> parts;
   for (int t0 = 0; t0 < p.n_trees; t0 += kPlainTrees)
     parts.emplace_back(
-        fit_batch(fd, p.tree_offset + t0, std::min(kPlainTrees, p.n_trees - t0), N, F, p, s, true));
+        fit_batch(fd, p.tree_offset + t0, std::min(kPlainTrees, p.n_trees - t0), N, F, p, s, true, nullptr,
+                  p.n_trees <= kPlainTrees));
   if (parts.size() == 1) return parts[0].release();
   return merge_forests(parts, s);
 }
@@ -7371,7 +7351,7 @@ std::vector<Forest*> fit_joint(const float* const* X, const float* const* y, con
     profile_host("joint_prepare_host", ms(h0, now()));
   }
   const auto h1 = now();
-  std::unique_ptr<Forest> all(fit_batch(*fds[0], 0, T, N[0], F[0], pj, s, false, &J));
+  std::unique_ptr<Forest> all(fit_batch(*fds[0], 0, T, N[0], F[0], pj, s, false, &J, false));
   const auto h2 = now();
   if (prof) profile_host("joint_build_host", ms(h1, h2));
   // one forest per input, from its trees' node range
@@ -7398,7 +7378,11 @@ std::vector<Forest*> fit_joint(const float* const* X, const float* const* y, con
     fo->n_leaves = (nn + jf.T) / 2;
     fo->has_stats = true;
     std::vector<int64_t> tsf(jf.T + 1);
-    for (int q = 0; q <= jf.T; ++q) tsf[q] = ts[jf.t0 + q] - off;
+    int64_t max_tree = 1;
+    for (int q = 0; q <= jf.T; ++q) {
+      tsf[q] = ts[jf.t0 + q] - off;
+      if (q) max_tree = std::max(max_tree, tsf[q] - tsf[q - 1]);
+    }
     fo->tree_start.alloc(jf.T + 1);
     DTE_HIP(hipMemcpyAsync(fo->tree_start.p, tsf.data(), 8 * (size_t)(jf.T + 1), hipMemcpyHostToDevice, s));
     fo->feature.alloc(nn);
@@ -7419,7 +7403,7 @@ std::vector<Forest*> fit_joint(const float* const* X, const float* const* y, con
                  fo->feature.p, fo->left.p, fo->depth.p, fo->count.p, fo->n_entries.p,
                  fo->threshold.p, fo->score.p, fo->value.p, fo->rowhash.p, fo->class_counts.p, fo->sum_fixed.p};
     hipLaunchKernelGGL(k_slice_nodes, dim3(grid_for(nn)), dim3(kBlock), 0, s, sa);
-    build_predict_nodes(*fo, s);
+    build_predict_nodes(*fo, max_tree, s);
     DTE_HIP(hipStreamSynchronize(s));  // tsf goes out of scope
     out.push_back(std::move(fo));
   }
@@ -7428,13 +7412,6 @@ std::vector<Forest*> fit_joint(const float* const* X, const float* const* y, con
   std::vector<Forest*> res;
   for (auto& f : out) res.push_back(f.release());
   return res;
-}
-
-void build_predict_nodes(Forest& f, hipStream_t s) {
-  PoolSuspend own;
-  f.pnodes.alloc(f.n_nodes);
-  hipLaunchKernelGGL(k_predict_nodes, dim3(grid_for(f.n_nodes)), dim3(kBlock), 0, s, f.n_nodes, f.n_classes,
-                     f.task, f.feature.p, f.threshold.p, f.left.p, f.class_counts.p, f.value.p, f.pnodes.p);
 }
 
 }  // namespace dte

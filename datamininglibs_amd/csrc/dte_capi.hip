@@ -323,6 +323,12 @@ void profile_add_bytes(const char* name, double bytes) {
 using namespace dte;
 
 namespace {
+int64_t largest_tree(const std::vector<int64_t>& ts) {
+  int64_t m = 1;
+  for (size_t t = 1; t < ts.size(); ++t) m = std::max(m, ts[t] - ts[t - 1]);
+  return m;
+}
+
 int64_t count_leaves(const std::vector<int32_t>& feature) {
   int64_t n = 0;
   for (auto v : feature) n += v < 0;
@@ -573,7 +579,7 @@ int dte_forest_info_get(const dte_forest* forest, dte_forest_info* out) {
     out->n_nodes = f.n_nodes;
     out->n_leaves = f.n_leaves;
     out->n_probabilities = out->n_leaves * (f.task == 0 ? f.n_classes : 1);
-    out->device_bytes = (int64_t)(f.pnodes.bytes() + f.tree_start.bytes() + f.feature.bytes() + f.left.bytes() +
+    out->device_bytes = (int64_t)(f.pairs.bytes() + f.pair_base.bytes() + f.pnodes.bytes() + f.tree_start.bytes() + f.feature.bytes() + f.left.bytes() +
                                   f.depth.bytes() + f.count.bytes() + f.n_entries.bytes() + f.threshold.bytes() +
                                   f.score.bytes() + f.value.bytes() + f.rowhash.bytes() +
                                   f.class_counts.bytes() + f.sum_fixed.bytes());
@@ -681,7 +687,7 @@ int dte_forest_import(const dte_node* nodes, int64_t n_nodes, const float* probs
     DTE_HIP(hipMemcpyAsync(f.threshold.p, thr.data(), 4 * n, hipMemcpyHostToDevice, s));
     DTE_HIP(hipMemcpyAsync(f.value.p, value.data(), 4 * n, hipMemcpyHostToDevice, s));
     if (task == 0) DTE_HIP(hipMemcpyAsync(f.class_counts.p, cls.data(), 4 * cls.size(), hipMemcpyHostToDevice, s));
-    build_predict_nodes(f, s);
+    build_predict_nodes(f, largest_tree(ts), s);
     DTE_HIP(hipStreamSynchronize(s));
     *out = guard.release();
   });
@@ -921,7 +927,7 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
       up(f.sum_fixed, n, o);
       o += 8 * n;
     }
-    build_predict_nodes(f, s);
+    build_predict_nodes(f, largest_tree(ts), s);
     DTE_HIP(hipStreamSynchronize(s));
     *out = guard.release();
   });
@@ -991,11 +997,9 @@ int dte_predict(const dte_forest* forest, const float* samples, int64_t n_rows, 
     DTE_HIP(hipMemcpyAsync(X.p, samples, sizeof(float) * n_rows * f.n_features, hipMemcpyHostToDevice, s));
     if (f.task == 0) {
       DevBuf<int32_t> v((size_t)n_rows * f.n_classes);
-      predict_forest(f, X.p, n_rows, n_rows, 0, v.p, nullptr, s);
-      std::vector<int32_t> h((size_t)n_rows * f.n_classes);
-      DTE_HIP(hipMemcpyAsync(h.data(), v.p, 4 * h.size(), hipMemcpyDeviceToHost, s));
+      predict_forest(f, X.p, n_rows, n_rows, 0, v.p, nullptr, s, true);
+      DTE_HIP(hipMemcpyAsync(out, v.p, v.bytes(), hipMemcpyDeviceToHost, s));
       DTE_HIP(hipStreamSynchronize(s));
-      for (size_t i = 0; i < h.size(); ++i) out[i] = (float)h[i];
     } else {
       DevBuf<float> v(n_rows);
       predict_forest(f, X.p, n_rows, n_rows, 0, nullptr, v.p, s);
@@ -1030,8 +1034,7 @@ int dte_predict_noalloc(const dte_forest* forest, const float* samples, int64_t 
     void* o = base + x_bytes;
     DTE_HIP(hipMemcpyAsync(X, samples, 4 * n_rows * F, hipMemcpyHostToDevice, s));
     if (f.task == 0) {
-      predict_forest(f, X, n_rows, n_rows, 0, static_cast<int32_t*>(o), nullptr, s);  // clears the votes itself
-      votes_to_float(static_cast<int32_t*>(o), n_rows * W, s);
+      predict_forest(f, X, n_rows, n_rows, 0, static_cast<int32_t*>(o), nullptr, s, true);  // clears them itself
     } else {
       predict_forest(f, X, n_rows, n_rows, 0, nullptr, static_cast<float*>(o), s);
     }

@@ -167,12 +167,20 @@ struct Timer {
   }
 };
 
-// Predict-side node record: 16 bytes, one 128-bit load per visited node.
-//   internal: feature >= 0, thr, left child index (right = left + 1)
-//   leaf:     feature = -1, thr = regression leaf value, left = vote class
+// Predict-side records.  Packed (dte_predict.hip: build_predict_nodes): 8
+// bytes a node, (threshold bits, pair of the children << fbits | feature + 1)
+// or (leaf payload, 0), siblings side by side in a 16-byte pair; the payload is
+// the vote class or the bits of the regression value.  Wide, for trees whose
+// pairs and features do not fit a link of 32 bits: 16 bytes a node in
+// canonical order,
+//   internal: feature >= 0, thr bits, left child index (right = left + 1)
+//   leaf:     feature = -1, thr = payload
+struct PPair {
+  uint32_t w[4];
+};
 struct PNode {
   int32_t feature;
-  float thr;
+  uint32_t thr;
   int32_t left;
   int32_t pad;
 };
@@ -198,7 +206,10 @@ struct Forest {
   int32_t tree_offset = 0;
   int64_t fit_rows = 0;
   DevBuf<int64_t> tree_start;  // n_trees + 1
-  DevBuf<PNode> pnodes;        // n_nodes
+  DevBuf<PPair> pairs;         // packed predict records (empty: wide ones)
+  DevBuf<int64_t> pair_base;   // packed: first pair of each tree
+  int pair_fbits = 0;          // packed: feature bits of a link
+  DevBuf<PNode> pnodes;        // wide predict records (n_nodes), or empty
   // Build diagnostics (absent for imported forests).
   bool has_stats = false;
   DevBuf<int32_t> feature, left, depth, count, n_entries;
@@ -218,20 +229,20 @@ struct FitInput {
 // Entry points implemented in dte_build.hip / dte_predict.hip.
 Forest* fit_forest(const float* X_dev, const float* y_host, int64_t n_rows, int32_t n_features,
                    const dte_params& p, hipStream_t stream);
-void build_predict_nodes(Forest& f, hipStream_t stream);
+void build_predict_nodes(Forest& f, int64_t max_tree, hipStream_t stream);
 // Several extra-trees forests of one task in one build: every level step
 // serves the open nodes of all forests (see dte_fit_many).
 std::vector<Forest*> fit_joint(const float* const* X_dev, const float* const* y_host, const int64_t* n_rows,
                                const int32_t* n_features, const dte_params* params, int n, hipStream_t stream);
+// float_votes: the vote counts as floats in votes_dev's words.
 void predict_forest(const Forest& f, const float* X_dev, int64_t n_rows, int64_t ld,
-                    int row_major, int32_t* votes_dev, float* sums_dev, hipStream_t stream);
+                    int row_major, int32_t* votes_dev, float* sums_dev, hipStream_t stream,
+                    bool float_votes = false);
 // Reference model layout (dte_forest_export) into host arrays.
 void export_forest(const Forest& f, dte_node* nodes, int64_t nodes_cap, float* probs, int64_t probs_cap,
                    hipStream_t stream);
 // Exclusive scan of n words into out[0 .. n] (out[n] = total).
 void scan_u32_ext(const uint32_t* in, int64_t n, uint32_t* out, hipStream_t s, std::vector<DevBuf<uint32_t>>& tmp);
-// In place: int32 vote counts -> the same values as float.
-void votes_to_float(int32_t* votes, int64_t n, hipStream_t stream);
 // Out-of-bag evaluation (dte_oob_evaluate): pairs evaluated, correct pairs
 // (classification) or the sum of squared errors (regression).
 void oob_evaluate(const Forest& f, const float* X_dev, const float* targets, int64_t n_rows, int perm_feature,

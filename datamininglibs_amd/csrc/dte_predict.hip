@@ -2,16 +2,18 @@
 // source/gpudte.cu:311-359) and the host launch loop of
 // GpuDteAlgorithm<T>::Predict (gpudte_algorithm.cc:292-311):
 //
-//  * nodes are 16-byte records (feature, threshold, left / leaf payload), one
-//    128-bit load per visited node;
+//  * nodes are 8-byte records, sibling pairs side by side, three levels of a
+//    subtree in one cache line (build_predict_nodes); a visit loads the pair
+//    of children while the node's feature value is read and compared;
 //  * classification: every (row, tree) pair is walked exactly once (FIX of
 //    the truncated grid, gpudte_algorithm.cc:297-305) and votes are integer
-//    atomics, so the result is order-free;
+//    sums, so the result is order-free;
 //  * regression: every row's trees are summed in tree order (fixed fp32
 //    order instead of float atomics, gpudte.cu:354-357).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "dte_internal.h"
@@ -19,169 +21,359 @@
 namespace dte {
 namespace {
 
-constexpr int kRowsPerBlock = 64;
 constexpr int kWave = 64;
+constexpr int kWalkThreads = 512;  // a block's rows in LDS serve eight waves
 
-// One visited node = one wide load.  Left alone, the compiler splits the
-// record into dword loads and sinks the threshold's load past the feature's
-// LDS lookup: two memory round trips per level instead of one.  The empty
-// asm statement (no instruction) takes the three fields as operands, so
-// their loads stay together and merge into one.
-__device__ __forceinline__ PNode load_node(const PNode* __restrict__ nodes, int64_t i) {
-  const int4 v = reinterpret_cast<const int4*>(nodes)[i];
-  asm volatile("" : : "v"(v.x), "v"(v.y), "v"(v.z));
-  return PNode{v.x, __int_as_float(v.y), v.z, v.w};
-}
+// ------------------------------------------------------ node layout ----
+// Bound by the rate of cache lines that come over the fabric for the deep
+// levels (16-byte records in level order: a line per visited level, 79 GB for
+// 200 M walks of 60 M nodes, 16.0 ms).  Here a tree's pairs are grouped by
+// clusters of three levels -- the pair at depth 1, 4, 7, .. and up to six
+// pairs below it, 16 B each -- in slots of 1, 2, 4 or 8 pairs aligned to
+// their size, so that a cluster never straddles a 128-byte line and a walk
+// touches one line per three levels.  The root shares a line with the cluster
+// below it.
+constexpr int kClusterLevels = 3;
 
-__device__ __forceinline__ int walk(const PNode* __restrict__ nodes, int64_t root, const float* __restrict__ X,
-                                    int64_t row, int64_t ld, int row_major, float* leaf_value) {
-  PNode nd = load_node(nodes, root);
-  while (nd.feature >= 0) {
-    const float x = row_major ? X[row * ld + nd.feature] : X[(int64_t)nd.feature * ld + row];
-    nd = load_node(nodes, nd.left + side_of(x, nd.thr));
+// Slot class of a cluster of s pairs: 2^class slots of a pair.
+__device__ __forceinline__ int slot_class(int s) { return s <= 1 ? 0 : s <= 2 ? 1 : s <= 4 ? 2 : 3; }
+
+// Tree of canonical node g.
+__device__ __forceinline__ int tree_of(int64_t g, int T, const int64_t* __restrict__ ts) {
+  int lo = 0, hi = T - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (ts[mid] <= g) lo = mid;
+    else hi = mid - 1;
   }
-  *leaf_value = nd.thr;
-  return nd.left;
+  return lo;
 }
 
-// Block = 64 rows x 4 tree lanes; each wave walks every 4th tree for its
-// row, votes are gathered in LDS and flushed with one atomic per class.
-__global__ void __launch_bounds__(kBlock) k_predict_cls(const PNode* __restrict__ nodes,
-                                                        const int64_t* __restrict__ tree_start, int T,
-                                                        const float* __restrict__ X, int64_t n_rows, int64_t ld,
-                                                        int row_major, int C, int trees_per_block,
-                                                        int32_t* __restrict__ votes) {
-  extern __shared__ uint32_t s_votes[];  // kRowsPerBlock * C
-  const int lane = threadIdx.x & (kRowsPerBlock - 1);
-  const int group = threadIdx.x / kRowsPerBlock;
-  const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + lane;
-  const int t0 = blockIdx.y * trees_per_block;
-  const int t1 = min(T, t0 + trees_per_block);
-  for (int i = threadIdx.x; i < kRowsPerBlock * C; i += kBlock) s_votes[i] = 0;
-  __syncthreads();
-  if (row < n_rows) {
-    for (int t = t0 + group; t < t1; t += kBlock / kRowsPerBlock) {
-      float v;
-      const int cls = walk(nodes, tree_start[t], X, row, ld, row_major, &v);
-      atomicAdd(&s_votes[lane * C + cls], 1u);
+// The pairs of a cluster, by their first nodes (-1: not there): the head pair,
+// the pairs below its two nodes, and the pairs below those.
+struct Cluster {
+  int32_t head, mid[2], low[4];
+  int n;  // pairs
+};
+__device__ __forceinline__ Cluster cluster_at(int32_t head, const int32_t* __restrict__ feature,
+                                              const int32_t* __restrict__ left) {
+  Cluster c;
+  c.head = head;
+  c.n = 1;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    c.mid[k] = feature[head + k] >= 0 ? left[head + k] : -1;
+    c.n += c.mid[k] >= 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      c.low[2 * k + j] = c.mid[k] >= 0 && feature[c.mid[k] + j] >= 0 ? left[c.mid[k] + j] : -1;
+      c.n += c.low[2 * k + j] >= 0;
     }
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kRowsPerBlock * C; i += kBlock) {
-    const int r = i / C;
-    const int64_t gr = (int64_t)blockIdx.x * kRowsPerBlock + r;
-    const uint32_t v = s_votes[i];
-    if (gr < n_rows && v) atomicAdd(&votes[gr * C + (i % C)], (int32_t)v);
+  return c;
+}
+
+// Every internal node at a depth divisible by three heads the cluster of its
+// children: its slot class and number among the tree's clusters of that class.
+// One atomic per wave, tree and class.
+__global__ void __launch_bounds__(kBlock) k_cluster_count(int64_t n, int T, const int64_t* __restrict__ ts,
+                                                          const int32_t* __restrict__ feature,
+                                                          const int32_t* __restrict__ left,
+                                                          const int32_t* __restrict__ depth, uint32_t* code,
+                                                          unsigned int* cnt) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t n_up = (n + kBlock - 1) / kBlock * kBlock;
+  for (int64_t g = blockIdx.x * (int64_t)kBlock + threadIdx.x; g < n_up; g += (int64_t)gridDim.x * kBlock) {
+    int key = -1;  // 4 * tree + class
+    int32_t first = 0;
+    if (g < n && feature[g] >= 0 && depth[g] % kClusterLevels == 0) {
+      first = left[g];
+      // the root's cluster has a line of its own, behind the root pair
+      if (depth[g] > 0) key = 4 * tree_of(g, T, ts) + slot_class(cluster_at(first, feature, left).n);
+    }
+    uint64_t todo = __ballot(key >= 0);
+    while (todo) {
+      const int l = (int)__ffsll((unsigned long long)todo) - 1;
+      const int k = __shfl(key, l, kWave);
+      const uint64_t same = __ballot(key == k);
+      unsigned int at = 0;
+      if (lane == l) at = atomicAdd(&cnt[k], (unsigned int)__popcll(same));
+      at = __shfl(at, l, kWave);
+      if (key == k) code[first] = (at + (unsigned int)__popcll(same & ((1ull << lane) - 1ull))) * 4u + (unsigned)(k & 3);
+      todo &= ~same;
+    }
   }
 }
 
-// The same with the block's R rows staged in LDS first (coalesced reads of
-// X, feature-major or row-major), so that every visit reads its feature
-// value from LDS: block = R rows x (256 / R) tree lanes.
+// Bases (in pairs) of the trees and of their slot classes: 8 pairs for the
+// root and its cluster, then the slots of 8, 4, 2 and 1 pairs.
+__global__ void __launch_bounds__(kBlock) k_cluster_bases(int T, const unsigned int* __restrict__ cnt,
+                                                          int64_t* __restrict__ tbase,
+                                                          uint32_t* __restrict__ cbase) {
+  __shared__ int64_t s_sum[kBlock];
+  const int t = threadIdx.x;
+  int64_t run = 0;
+  for (int t0 = 0; t0 < T; t0 += kBlock) {
+    const int i = t0 + t;
+    int64_t size = 0;
+    if (i < T) {
+      const unsigned int* c = cnt + 4 * (int64_t)i;
+      uint32_t at = 8;
+      cbase[4 * (int64_t)i + 3] = at;
+      at += 8u * c[3];
+      cbase[4 * (int64_t)i + 2] = at;
+      at += 4u * c[2];
+      cbase[4 * (int64_t)i + 1] = at;
+      at += 2u * c[1];
+      cbase[4 * (int64_t)i] = at;
+      at += c[0];
+      size = (at + 7u) & ~7u;
+    }
+    s_sum[t] = size;
+    __syncthreads();
+    for (int off = 1; off < kBlock; off <<= 1) {
+      const int64_t v = t >= off ? s_sum[t - off] : 0;
+      __syncthreads();
+      s_sum[t] += v;
+      __syncthreads();
+    }
+    if (i < T) tbase[i] = run + s_sum[t] - size;
+    run += s_sum[kBlock - 1];
+    __syncthreads();
+  }
+}
+
+// vote = argmax, strict > from 0: lowest class on ties (gpudte.cu:341-351)
+__device__ __forceinline__ int vote_of(const uint32_t* __restrict__ cls, int C) {
+  int best = 0;
+  uint32_t bv = 0;
+  for (int c = 0; c < C; ++c)
+    if (cls[c] > bv) {
+      bv = cls[c];
+      best = c;
+    }
+  return best;
+}
+
+// Record of node g: (threshold, link) or, for a leaf, (payload, 0); link =
+// pair of the children << fbits | feature + 1.
+__device__ __forceinline__ uint2 leaf_record(int64_t g, int C, int task, const uint32_t* __restrict__ cls,
+                                             const float* __restrict__ value) {
+  return make_uint2(task == 0 ? (uint32_t)vote_of(cls + g * C, C) : __float_as_uint(value[g]), 0u);
+}
+
+__global__ void __launch_bounds__(kBlock) k_cluster_write(int64_t n, int T, const int64_t* __restrict__ ts,
+                                                          const int32_t* __restrict__ feature,
+                                                          const int32_t* __restrict__ left,
+                                                          const int32_t* __restrict__ depth,
+                                                          const float* __restrict__ thr,
+                                                          const uint32_t* __restrict__ cls,
+                                                          const float* __restrict__ value, int C, int task, int fbits,
+                                                          const uint32_t* __restrict__ code,
+                                                          const int64_t* __restrict__ tbase,
+                                                          const uint32_t* __restrict__ cbase, uint4* __restrict__ out) {
+  for (int64_t g = blockIdx.x * (int64_t)kBlock + threadIdx.x; g < n; g += (int64_t)gridDim.x * kBlock) {
+    if (depth[g] % kClusterLevels != 0) continue;
+    const int32_t f = feature[g];
+    const bool root = depth[g] == 0;
+    if (f < 0 && !root) continue;
+    const int t = tree_of(g, T, ts);
+    const uint32_t* cb = cbase + 4 * (int64_t)t;
+    uint4* tree = out + tbase[t];
+    if (root) {
+      const uint2 r = f < 0 ? leaf_record(g, C, task, cls, value)
+                            : make_uint2(__float_as_uint(thr[g]), 1u << fbits | (uint32_t)(f + 1));
+      tree[0] = make_uint4(r.x, r.y, 0u, 0u);
+      if (f < 0) continue;
+    }
+    const Cluster c = cluster_at(left[g], feature, left);
+    auto slot = [&](int32_t first) { return cb[code[first] & 3u] + ((code[first] >> 2) << (code[first] & 3u)); };
+    const uint32_t at = root ? 1u : slot(c.head);
+    // breadth-first places of the pairs in the cluster's slots
+    uint32_t next = at + 1u, mid[2], low[4];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      mid[k] = next;
+      next += c.mid[k] >= 0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      low[k] = next;
+      next += c.low[k] >= 0;
+    }
+    auto record = [&](int32_t i, uint32_t child) {
+      const int32_t cf = feature[i];
+      return cf < 0 ? leaf_record(i, C, task, cls, value)
+                    : make_uint2(__float_as_uint(thr[i]), child << fbits | (uint32_t)(cf + 1));
+    };
+    auto put = [&](uint32_t where, uint2 l, uint2 r) { tree[where] = make_uint4(l.x, l.y, r.x, r.y); };
+    put(at, record(c.head, mid[0]), record(c.head + 1, mid[1]));
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (c.mid[k] >= 0) put(mid[k], record(c.mid[k], low[2 * k]), record(c.mid[k] + 1, low[2 * k + 1]));
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (c.low[k] >= 0) {  // below it: heads of other clusters
+        const int32_t i = c.low[k];
+        put(low[k], record(i, feature[i] >= 0 ? slot(left[i]) : 0u),
+            record(i + 1, feature[i + 1] >= 0 ? slot(left[i + 1]) : 0u));
+      }
+  }
+}
+
+// Canonical order, 16-byte records: trees too large for a link of 32 bits.
+__global__ void __launch_bounds__(kBlock) k_wide_nodes(int64_t n, int C, int task, const int32_t* feature,
+                                                       const float* thr, const int32_t* left, const uint32_t* cls,
+                                                       const float* value, PNode* out) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    PNode p;
+    p.feature = feature[i];
+    p.pad = 0;
+    if (p.feature >= 0) {
+      p.thr = __float_as_uint(thr[i]);
+      p.left = left[i];
+    } else {
+      p.thr = leaf_record(i, C, task, cls, value).x;
+      p.left = 0;
+    }
+    out[i] = p;
+  }
+}
+
+// ------------------------------------------------------------- walks ----
+struct Trees {
+  const uint4* pairs;        // packed: sibling pairs
+  const int64_t* tbase;      // packed: first pair of each tree
+  int fbits;
+  const PNode* wide;         // wide: canonical records
+  const int64_t* tree_start;
+  int T;
+};
+
+// Leaf payload of a row in tree t: its values at xr[feature * xs].  visit(f,
+// depth, &x) may replace the value read.
+template <bool PACKED, class Visit>
+__device__ __forceinline__ uint32_t walk(const Trees& tr, int t, const float* xr, int64_t xs, Visit&& visit) {
+  uint32_t depth = 0;
+  if constexpr (PACKED) {
+    const uint4* tree = tr.pairs + tr.tbase[t];
+    const uint32_t fmask = (1u << tr.fbits) - 1u;
+    uint2 nd = *reinterpret_cast<const uint2*>(tree);
+    while (nd.y & fmask) {
+      const uint4 kids = tree[nd.y >> tr.fbits];  // in flight beside the feature value
+      const int f = (int)(nd.y & fmask) - 1;
+      float x = xr[f * xs];
+      visit(f, depth, x);
+      const bool right = side_of(x, __uint_as_float(nd.x)) != 0;
+      nd = right ? make_uint2(kids.z, kids.w) : make_uint2(kids.x, kids.y);
+      ++depth;
+    }
+    return nd.x;
+  } else {
+    PNode nd = tr.wide[tr.tree_start[t]];
+    while (nd.feature >= 0) {
+      float x = xr[nd.feature * xs];
+      visit(nd.feature, depth, x);
+      nd = tr.wide[(int64_t)nd.left + side_of(x, __uint_as_float(nd.thr))];
+      ++depth;
+    }
+    return nd.thr;
+  }
+}
+
+// Stages a block's R rows of F features in LDS, F + 1 floats apart.
 template <int R>
-__global__ void __launch_bounds__(kBlock) k_predict_cls_lds(const PNode* __restrict__ nodes,
-                                                            const int64_t* __restrict__ tree_start, int T,
-                                                            const float* __restrict__ X, int64_t n_rows, int64_t ld,
-                                                            int row_major, int C, int F, int trees_per_block,
-                                                            int32_t* __restrict__ votes) {
-  extern __shared__ uint32_t s_mem[];
-  uint32_t* s_votes = s_mem;                            // R * C
-  float* s_x = reinterpret_cast<float*>(s_mem + R * C);  // R rows of F + 1 floats
+__device__ __forceinline__ void stage_rows(const float* __restrict__ X, int64_t row0, int nr, int64_t ld,
+                                           int row_major, int F, float* s_x) {
   const int FP = F + 1;
-  const int lane = threadIdx.x % R;
-  const int group = threadIdx.x / R;
-  const int64_t row0 = (int64_t)blockIdx.x * R;
-  const int nr = (int)min<int64_t>(R, n_rows - row0);
-  const int t0 = blockIdx.y * trees_per_block;
-  const int t1 = min(T, t0 + trees_per_block);
-  for (int i = threadIdx.x; i < R * C; i += kBlock) s_votes[i] = 0;
   if (row_major) {
-    for (int i = threadIdx.x; i < nr * F; i += kBlock) {
+    for (int i = threadIdx.x; i < nr * F; i += kWalkThreads) {
       const int r = i / F, f = i - r * F;
       s_x[r * FP + f] = X[(row0 + r) * ld + f];
     }
   } else {
-    for (int i = threadIdx.x; i < R * F; i += kBlock) {
+    for (int i = threadIdx.x; i < R * F; i += kWalkThreads) {
       const int f = i / R, r = i - f * R;
       if (r < nr) s_x[r * FP + f] = X[(int64_t)f * ld + row0 + r];
     }
   }
+}
+
+// What a block does with its votes: it adds them to others' (several tree
+// chunks), or it alone covers its rows' trees and stores them.
+enum VoteMode { kVoteAdd = 0, kVoteInt = 1, kVoteFloat = 2 };
+
+// A block's R rows x (512 / R) tree lanes; R = 0: rows read from X, 64 rows
+// x 8 tree lanes.
+template <int R, bool PACKED>
+__global__ void __launch_bounds__(kWalkThreads) k_predict_cls(Trees tr, const float* __restrict__ X, int64_t n_rows,
+                                                              int64_t ld, int row_major, int C, int F,
+                                                              int trees_per_block, int mode, void* __restrict__ out) {
+  extern __shared__ uint32_t s_mem[];
+  constexpr int RB = R ? R : 64;
+  uint32_t* s_votes = s_mem;                              // RB * C
+  float* s_x = reinterpret_cast<float*>(s_mem + RB * C);  // R rows of F + 1 floats
+  const int lane = threadIdx.x % RB;
+  const int group = threadIdx.x / RB;
+  const int64_t row0 = (int64_t)blockIdx.x * RB;
+  const int nr = (int)min<int64_t>(RB, n_rows - row0);
+  const int t0 = blockIdx.y * trees_per_block;
+  const int t1 = min(tr.T, t0 + trees_per_block);
+  for (int i = threadIdx.x; i < RB * C; i += kWalkThreads) s_votes[i] = 0;
+  if (R) stage_rows<RB>(X, row0, nr, ld, row_major, F, s_x);
   __syncthreads();
   if (lane < nr) {
-    const float* xr = s_x + lane * FP;
-    for (int t = t0 + group; t < t1; t += kBlock / R) {
-      PNode nd = load_node(nodes, tree_start[t]);
-      while (nd.feature >= 0) nd = load_node(nodes, nd.left + side_of(xr[nd.feature], nd.thr));
-      atomicAdd(&s_votes[lane * C + nd.left], 1u);
-    }
+    const float* xr = R ? s_x + lane * (F + 1) : row_major ? X + (row0 + lane) * ld : X + row0 + lane;
+    const int64_t xs = R || row_major ? 1 : ld;
+    for (int t = t0 + group; t < t1; t += kWalkThreads / RB)
+      atomicAdd(&s_votes[lane * C + walk<PACKED>(tr, t, xr, xs, [](int, uint32_t, float&) {})], 1u);
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < R * C; i += kBlock) {
-    const int r = i / C;
+  for (int i = threadIdx.x; i < nr * C; i += kWalkThreads) {
     const uint32_t v = s_votes[i];
-    if (r < nr && v) atomicAdd(&votes[(row0 + r) * C + (i % C)], (int32_t)v);
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) k_predict_reg(const PNode* __restrict__ nodes,
-                                                        const int64_t* __restrict__ tree_start, int T,
-                                                        const float* __restrict__ X, int64_t n_rows, int64_t ld,
-                                                        int row_major, float* __restrict__ sums) {
-  for (int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; row < n_rows;
-       row += (int64_t)gridDim.x * blockDim.x) {
-    float acc = 0.0f;
-    for (int t = 0; t < T; ++t) {
-      float v;
-      walk(nodes, tree_start[t], X, row, ld, row_major, &v);
-      acc = acc + v;
+    const int64_t o = row0 * C + i;
+    if (mode == kVoteFloat) {
+      static_cast<float*>(out)[o] = (float)v;
+    } else if (mode == kVoteInt) {
+      static_cast<int32_t*>(out)[o] = (int32_t)v;
+    } else if (v) {
+      atomicAdd(static_cast<int32_t*>(out) + o, (int32_t)v);
     }
-    sums[row] = acc;
   }
 }
 
-// Regression with a block's R rows staged in LDS.  Trees go in chunks of
-// kRegChunk: the 256 / R tree lanes of a row write the chunk's leaf values
-// to LDS, then one lane per row adds them in tree order, so every row's sum
-// is formed in the same order as the one-thread-per-row kernel.
-constexpr int kRegChunk = 32;
-template <int R>
-__global__ void __launch_bounds__(kBlock) k_predict_reg_lds(const PNode* __restrict__ nodes,
-                                                            const int64_t* __restrict__ tree_start, int T,
-                                                            const float* __restrict__ X, int64_t n_rows, int64_t ld,
-                                                            int row_major, int F, float* __restrict__ sums) {
+// Regression: trees go in chunks of as many as the block has tree lanes (at
+// least 32); the lanes of a row write the chunk's leaf values to LDS, then
+// one lane per row adds them in tree order, so every row's sum is formed in
+// that order whatever R is.
+constexpr int reg_chunk(int R) { return kWalkThreads / (R ? R : 64) > 32 ? kWalkThreads / (R ? R : 64) : 32; }
+
+template <int R, bool PACKED>
+__global__ void __launch_bounds__(kWalkThreads) k_predict_reg(Trees tr, const float* __restrict__ X, int64_t n_rows,
+                                                              int64_t ld, int row_major, int F,
+                                                              float* __restrict__ sums) {
   extern __shared__ float s_mem_f[];
-  float* s_val = s_mem_f;              // R x kRegChunk leaf values
-  float* s_x = s_mem_f + R * kRegChunk;  // R rows of F + 1 floats
-  const int FP = F + 1;
-  const int lane = threadIdx.x % R;
-  const int group = threadIdx.x / R;
-  const int64_t row0 = (int64_t)blockIdx.x * R;
-  const int nr = (int)min<int64_t>(R, n_rows - row0);
-  if (row_major) {
-    for (int i = threadIdx.x; i < nr * F; i += kBlock) {
-      const int r = i / F, f = i - r * F;
-      s_x[r * FP + f] = X[(row0 + r) * ld + f];
-    }
-  } else {
-    for (int i = threadIdx.x; i < R * F; i += kBlock) {
-      const int f = i / R, r = i - f * R;
-      if (r < nr) s_x[r * FP + f] = X[(int64_t)f * ld + row0 + r];
-    }
-  }
+  constexpr int RB = R ? R : 64;
+  constexpr int CH = reg_chunk(R);
+  float* s_val = s_mem_f;              // RB x CH leaf values, CH + 1 apart
+  float* s_x = s_mem_f + RB * (CH + 1);  // R rows of F + 1 floats
+  const int lane = threadIdx.x % RB;
+  const int group = threadIdx.x / RB;
+  const int64_t row0 = (int64_t)blockIdx.x * RB;
+  const int nr = (int)min<int64_t>(RB, n_rows - row0);
+  if (R) stage_rows<RB>(X, row0, nr, ld, row_major, F, s_x);
   __syncthreads();
-  const float* xr = s_x + lane * FP;
+  const float* xr = R ? s_x + lane * (F + 1) : row_major ? X + (row0 + lane) * ld : X + row0 + lane;
+  const int64_t xs = R || row_major ? 1 : ld;
   float acc = 0.0f;
-  for (int c0 = 0; c0 < T; c0 += kRegChunk) {
-    const int c1 = min(T, c0 + kRegChunk);
+  for (int c0 = 0; c0 < tr.T; c0 += CH) {
+    const int c1 = min(tr.T, c0 + CH);
     if (lane < nr)
-      for (int t = c0 + group; t < c1; t += kBlock / R) {
-        PNode nd = load_node(nodes, tree_start[t]);
-        while (nd.feature >= 0) nd = load_node(nodes, nd.left + side_of(xr[nd.feature], nd.thr));
-        s_val[lane * kRegChunk + (t - c0)] = nd.thr;
-      }
+      for (int t = c0 + group; t < c1; t += kWalkThreads / RB)
+        s_val[lane * (CH + 1) + (t - c0)] = __uint_as_float(walk<PACKED>(tr, t, xr, xs, [](int, uint32_t, float&) {}));
     __syncthreads();
     if (group == 0 && lane < nr)
-      for (int t = c0; t < c1; ++t) acc = acc + s_val[lane * kRegChunk + (t - c0)];
+      for (int t = c0; t < c1; ++t) acc = acc + s_val[lane * (CH + 1) + (t - c0)];
     __syncthreads();
   }
   if (group == 0 && lane < nr) sums[row0 + lane] = acc;
@@ -221,99 +413,46 @@ __global__ void __launch_bounds__(kBagThreads) k_inbag_bits_lds(uint32_t* bits, 
 // draw per visit keyed by (tree, row, depth) (gpurf.cu:356-438).
 // Classification counts the pairs whose tree vote equals the label;
 // regression sums the squared errors of the leaf values.
-template <int TASK>
-__global__ void __launch_bounds__(kBlock) k_oob(const PNode* __restrict__ nodes, const int64_t* __restrict__ tree_start,
-                                                const float* __restrict__ X, int64_t N, const uint32_t* __restrict__ bits,
-                                                int64_t words, const uint32_t* __restrict__ label,
-                                                const float* __restrict__ y, int32_t tree0, uint64_t seed, int perm,
-                                                unsigned long long* counts, double* sse) {
-  const int t = blockIdx.y;
-  const uint32_t tg = (uint32_t)(tree0 + t);
-  const uint32_t* bt = bits + (int64_t)t * words;
-  const int64_t root = tree_start[t];
-  unsigned long long n_pairs = 0, n_ok = 0;
-  double e2 = 0.0;
-  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < N; r += (int64_t)gridDim.x * blockDim.x) {
-    if ((bt[r >> 5] >> (r & 31)) & 1u) continue;  // in the bag
-    PNode nd = load_node(nodes, root);
-    uint32_t depth = 0;
-    while (nd.feature >= 0) {
-      int64_t src = r;
-      if (nd.feature == perm) src = rand_u32(seed, kStreamImp, tg, (uint32_t)r, depth) % (uint32_t)N;
-      nd = load_node(nodes, nd.left + side_of(X[(int64_t)nd.feature * N + src], nd.thr));
-      ++depth;
-    }
-    ++n_pairs;
-    if (TASK == 0) {
-      n_ok += (uint32_t)nd.left == label[r] ? 1ull : 0ull;
-    } else {
-      const double e = (double)nd.thr - (double)y[r];
-      e2 += e * e;
-    }
-  }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    n_pairs += __shfl_xor(n_pairs, off, kWave);
-    n_ok += __shfl_xor(n_ok, off, kWave);
-    if (TASK == 1) e2 += __shfl_xor(e2, off, kWave);
-  }
-  if ((threadIdx.x & (kWave - 1)) == 0 && n_pairs) {
-    atomicAdd(&counts[0], n_pairs);
-    if (TASK == 0) atomicAdd(&counts[1], n_ok);
-    else atomicAdd(sse, e2);
-  }
-}
-
-// The same pairs with a block's R rows staged in LDS (feature-major X read
-// coalesced), R rows x 256 / R tree lanes, trees [t0, t1) of the block's
-// chunk; the permuted feature still reads its drawn row from X.
-template <int TASK, int R>
-__global__ void __launch_bounds__(kBlock) k_oob_lds(const PNode* __restrict__ nodes,
-                                                    const int64_t* __restrict__ tree_start, int T,
-                                                    const float* __restrict__ X, int64_t N, int F,
-                                                    const uint32_t* __restrict__ bits, int64_t words,
-                                                    const uint32_t* __restrict__ label, const float* __restrict__ y,
-                                                    int32_t tree0, uint64_t seed, int perm, int trees_per_block,
-                                                    unsigned long long* counts, double* sse) {
+//
+// R rows staged in LDS x 512 / R tree lanes, trees [t0, t1) of the block's
+// chunk (R = 0: rows read from X, 64 x 8); the permuted feature always reads
+// its drawn row from X.
+template <int TASK, int R, bool PACKED>
+__global__ void __launch_bounds__(kWalkThreads) k_oob(Trees tr, const float* __restrict__ X, int64_t N, int F,
+                                                      const uint32_t* __restrict__ bits, int64_t words,
+                                                      const uint32_t* __restrict__ label, const float* __restrict__ y,
+                                                      int32_t tree0, uint64_t seed, int perm, int trees_per_block,
+                                                      unsigned long long* counts, double* sse) {
   extern __shared__ float s_x[];  // R rows of F + 1 floats
-  const int FP = F + 1;
-  const int lane = threadIdx.x % R;
-  const int group = threadIdx.x / R;
-  const int64_t row0 = (int64_t)blockIdx.x * R;
-  const int nr = (int)min<int64_t>(R, N - row0);
+  constexpr int RB = R ? R : 64;
+  const int lane = threadIdx.x % RB;
+  const int group = threadIdx.x / RB;
+  const int64_t row0 = (int64_t)blockIdx.x * RB;
+  const int nr = (int)min<int64_t>(RB, N - row0);
   const int t0 = blockIdx.y * trees_per_block;
-  const int t1 = min(T, t0 + trees_per_block);
-  for (int i = threadIdx.x; i < R * F; i += kBlock) {
-    const int f = i / R, r = i - f * R;
-    if (r < nr) s_x[r * FP + f] = X[(int64_t)f * N + row0 + r];
-  }
+  const int t1 = min(tr.T, t0 + trees_per_block);
+  if (R) stage_rows<RB>(X, row0, nr, N, 0, F, s_x);
   __syncthreads();
   unsigned long long n_pairs = 0, n_ok = 0;
   double e2 = 0.0;
   if (lane < nr) {
     const int64_t r = row0 + lane;
-    const float* xr = s_x + lane * FP;
+    const float* xr = R ? s_x + lane * (F + 1) : X + r;
+    const int64_t xs = R ? 1 : N;
     const uint32_t lab = TASK == 0 ? label[r] : 0u;
     const double yr = TASK == 1 ? (double)y[r] : 0.0;
-    for (int t = t0 + group; t < t1; t += kBlock / R) {
+    for (int t = t0 + group; t < t1; t += kWalkThreads / RB) {
       if ((bits[(int64_t)t * words + (r >> 5)] >> (r & 31)) & 1u) continue;  // in the bag
       const uint32_t tg = (uint32_t)(tree0 + t);
-      PNode nd = load_node(nodes, tree_start[t]);
-      uint32_t depth = 0;
-      while (nd.feature >= 0) {
-        float v;
-        if (nd.feature == perm)
-          v = X[(int64_t)perm * N + rand_u32(seed, kStreamImp, tg, (uint32_t)r, depth) % (uint32_t)N];
-        else
-          v = xr[nd.feature];
-        nd = load_node(nodes, nd.left + side_of(v, nd.thr));
-        ++depth;
-      }
+      const uint32_t leaf = walk<PACKED>(tr, t, xr, xs, [&](int f, uint32_t depth, float& x) {
+        if (f == perm)
+          x = X[(int64_t)perm * N + rand_u32(seed, kStreamImp, tg, (uint32_t)r, depth) % (uint32_t)N];
+      });
       ++n_pairs;
       if (TASK == 0) {
-        n_ok += (uint32_t)nd.left == lab ? 1ull : 0ull;
+        n_ok += leaf == lab ? 1ull : 0ull;
       } else {
-        const double e = (double)nd.thr - yr;
+        const double e = (double)__uint_as_float(leaf) - yr;
         e2 += e * e;
       }
     }
@@ -409,19 +548,45 @@ __global__ void __launch_bounds__(kBlock) k_export(int64_t e0, int64_t e1, int T
 
 unsigned elementwise_grid(int64_t n) { return (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 4096); }
 
-// Rows per block of the LDS-staged kernels: 64 while the block's rows (and
-// vote counters, C) fit 48 KB, else 32, else 0 (rows read from HBM).
-int staged_rows(int F, int C) {
-  if (4 * 64 * (F + 1 + C) <= 48 * 1024) return 64;
-  if (4 * 32 * (F + 1 + C) <= 48 * 1024) return 32;
-  return 0;
+// Rows per block of the walk kernels: 64 (32, 16) while the block's rows and
+// `per_row` more words each fit 48 KB of LDS, else 0 (rows read from HBM).
+// Few rows take fewer per block, so that a wave's lanes spread over trees.
+int staged_rows(int F, int per_row, int64_t n_rows) {
+  auto fits = [&](int r) { return (int64_t)4 * r * ((int64_t)F + 1 + per_row) <= 48 * 1024; };
+  if (n_rows <= 2 && fits(1)) return 1;
+  if (n_rows <= 16 && fits(4)) return 4;
+  if (n_rows <= 128 && fits(16)) return 16;
+  return fits(64) ? 64 : fits(32) ? 32 : 0;
 }
 
-// Tree chunks so that row blocks x chunks fill the chip even for few rows.
-int tree_chunks(int64_t row_blocks, int n_trees) {
+// Tree chunks so that row blocks x chunks fill the chip even for few rows: a
+// chunk keeps at least two trees per tree lane.
+int tree_chunks(int64_t row_blocks, int n_trees, int lanes) {
   int chunks = 1;
-  while (row_blocks * chunks < 2048 && chunks * 32 < n_trees) chunks *= 2;
+  while (row_blocks * chunks < 1024 && (int64_t)chunks * 4 * lanes <= n_trees) chunks *= 2;
   return chunks;
+}
+
+Trees trees_of(const Forest& f) {
+  return Trees{reinterpret_cast<const uint4*>(f.pairs.p), f.pair_base.p, f.pair_fbits, f.pnodes.p, f.tree_start.p,
+               f.n_trees};
+}
+
+// fn(integral_constant R, integral_constant PACKED) for the rows per block r.
+template <class Fn>
+void with_rows(int r, bool packed, Fn&& fn) {
+  auto go = [&](auto R) {
+    if (packed) fn(R, std::true_type());
+    else fn(R, std::false_type());
+  };
+  switch (r) {
+    case 64: go(std::integral_constant<int, 64>()); break;
+    case 32: go(std::integral_constant<int, 32>()); break;
+    case 16: go(std::integral_constant<int, 16>()); break;
+    case 4: go(std::integral_constant<int, 4>()); break;
+    case 1: go(std::integral_constant<int, 1>()); break;
+    default: go(std::integral_constant<int, 0>()); break;
+  }
 }
 
 }  // namespace
@@ -432,7 +597,6 @@ void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t
   if (T > 65535) fail(DTE_ERR_INVALID_ARGUMENT, "the out-of-bag pass handles at most 65535 trees");
   const int64_t words = (N + 31) / 32;
   DevBuf<uint32_t> bits((size_t)words * T);  // every word is written by k_inbag_bits_lds
-  const int gx = (int)std::min<int64_t>((N + kBlock - 1) / kBlock, 1024);
   hipLaunchKernelGGL(k_inbag_bits_lds, dim3((unsigned)T, (unsigned)((N + kBagRange - 1) / kBagRange)),
                      dim3(kBagThreads), 0, s, bits.p, N, words, f.tree_offset, f.seed);
   DevBuf<uint32_t> label;
@@ -456,34 +620,24 @@ void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t
   DevBuf<double> sse(1);
   DTE_HIP(hipMemsetAsync(counts.p, 0, counts.bytes(), s));
   DTE_HIP(hipMemsetAsync(sse.p, 0, sse.bytes(), s));
-  const int R = staged_rows(f.n_features, 0);
-  if (R) {
-    const int64_t row_blocks = (N + R - 1) / R;
-    const int tpb = (T + tree_chunks(row_blocks, T) - 1) / tree_chunks(row_blocks, T);
-    const dim3 grid((unsigned)row_blocks, (unsigned)((T + tpb - 1) / tpb));
-    const size_t lds = sizeof(float) * (size_t)R * (f.n_features + 1);
-    const uint32_t* lab = label.p;
-    const float* yp = yv.p;
-    const int Fn = f.n_features;
-    if (f.task == 0 && R == 64)
-      hipLaunchKernelGGL((k_oob_lds<0, 64>), grid, dim3(kBlock), lds, s, f.pnodes.p, f.tree_start.p, T, X, N, Fn,
-                         bits.p, words, lab, yp, f.tree_offset, f.seed, perm, tpb, counts.p, sse.p);
-    else if (f.task == 0)
-      hipLaunchKernelGGL((k_oob_lds<0, 32>), grid, dim3(kBlock), lds, s, f.pnodes.p, f.tree_start.p, T, X, N, Fn,
-                         bits.p, words, lab, yp, f.tree_offset, f.seed, perm, tpb, counts.p, sse.p);
-    else if (R == 64)
-      hipLaunchKernelGGL((k_oob_lds<1, 64>), grid, dim3(kBlock), lds, s, f.pnodes.p, f.tree_start.p, T, X, N, Fn,
-                         bits.p, words, lab, yp, f.tree_offset, f.seed, perm, tpb, counts.p, sse.p);
+  const int R = staged_rows(f.n_features, 0, N), RB = R ? R : 64;
+  const int64_t row_blocks = (N + RB - 1) / RB;
+  const int chunks = tree_chunks(row_blocks, T, kWalkThreads / RB);
+  const int tpb = (T + chunks - 1) / chunks;
+  const dim3 grid((unsigned)row_blocks, (unsigned)((T + tpb - 1) / tpb));
+  const size_t lds = R ? sizeof(float) * (size_t)R * (f.n_features + 1) : 0;
+  with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
+    constexpr int kR = decltype(r)::value;
+    constexpr bool kP = decltype(packed)::value;
+    if (f.task == 0)
+      hipLaunchKernelGGL((k_oob<0, kR, kP>), grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
+                         (const uint32_t*)bits.p, words, (const uint32_t*)label.p, (const float*)nullptr,
+                         f.tree_offset, f.seed, perm, tpb, counts.p, sse.p);
     else
-      hipLaunchKernelGGL((k_oob_lds<1, 32>), grid, dim3(kBlock), lds, s, f.pnodes.p, f.tree_start.p, T, X, N, Fn,
-                         bits.p, words, lab, yp, f.tree_offset, f.seed, perm, tpb, counts.p, sse.p);
-  } else if (f.task == 0) {
-    hipLaunchKernelGGL(k_oob<0>, dim3((unsigned)gx, (unsigned)T), dim3(kBlock), 0, s, f.pnodes.p, f.tree_start.p, X,
-                       N, bits.p, words, label.p, (const float*)nullptr, f.tree_offset, f.seed, perm, counts.p, sse.p);
-  } else {
-    hipLaunchKernelGGL(k_oob<1>, dim3((unsigned)gx, (unsigned)T), dim3(kBlock), 0, s, f.pnodes.p, f.tree_start.p, X,
-                       N, bits.p, words, (const uint32_t*)nullptr, yv.p, f.tree_offset, f.seed, perm, counts.p, sse.p);
-  }
+      hipLaunchKernelGGL((k_oob<1, kR, kP>), grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
+                         (const uint32_t*)bits.p, words, (const uint32_t*)nullptr, (const float*)yv.p, f.tree_offset,
+                         f.seed, perm, tpb, counts.p, sse.p);
+  });
   DTE_HIP(hipGetLastError());
   unsigned long long c[2];
   double e = 0.0;
@@ -539,67 +693,83 @@ void export_forest(const Forest& f, dte_node* nodes, int64_t nodes_cap, float* p
   DTE_HIP(hipStreamSynchronize(s));
 }
 
-void votes_to_float(int32_t* votes, int64_t n, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_votes_to_float, dim3(elementwise_grid(n)), dim3(kBlock), 0, s, votes, n);
+void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld, int row_major,
+                    int32_t* votes, float* sums, hipStream_t s, bool float_votes) {
+  if (n_rows <= 0) return;
+  const int F = f.n_features, C = f.n_classes;
+  Timer tm("predict", 0.0, s);
+  if (f.task == 0) {
+    const int R = staged_rows(F, C, n_rows), RB = R ? R : 64;
+    const int64_t row_blocks = (n_rows + RB - 1) / RB;
+    const int chunks = tree_chunks(row_blocks, f.n_trees, kWalkThreads / RB);
+    const int tpb = (f.n_trees + chunks - 1) / chunks;
+    const dim3 grid((unsigned)row_blocks, (unsigned)((f.n_trees + tpb - 1) / tpb));
+    const size_t lds = sizeof(uint32_t) * (size_t)RB * (C + (R ? F + 1 : 0));
+    const int64_t nv = n_rows * C;
+    const int mode = grid.y > 1 ? kVoteAdd : float_votes ? kVoteFloat : kVoteInt;
+    // votes cleared by a kernel (no memset node if the caller captures)
+    if (mode == kVoteAdd)
+      hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(nv)), dim3(kBlock), 0, s, reinterpret_cast<uint32_t*>(votes),
+                         nv);
+    with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
+      hipLaunchKernelGGL((k_predict_cls<decltype(r)::value, decltype(packed)::value>), grid, dim3(kWalkThreads), lds,
+                         s, trees_of(f), X, n_rows, ld, row_major, C, F, tpb, mode, (void*)votes);
+    });
+    if (mode == kVoteAdd && float_votes)
+      hipLaunchKernelGGL(k_votes_to_float, dim3(elementwise_grid(nv)), dim3(kBlock), 0, s, votes, nv);
+  } else {
+    // the chunk's leaf values are staged beside the rows
+    const int want = staged_rows(F, reg_chunk(64) + 1, n_rows);
+    const int R = want && staged_rows(F, reg_chunk(want) + 1, n_rows) == want ? want : 0;
+    const int RB = R ? R : 64;
+    const size_t lds = sizeof(float) * (size_t)RB * (reg_chunk(R) + 1 + (R ? F + 1 : 0));
+    with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
+      hipLaunchKernelGGL((k_predict_reg<decltype(r)::value, decltype(packed)::value>),
+                         dim3((unsigned)((n_rows + RB - 1) / RB)), dim3(kWalkThreads), lds, s, trees_of(f), X, n_rows,
+                         ld, row_major, F, sums);
+    });
+  }
   DTE_HIP(hipGetLastError());
 }
 
-void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld, int row_major,
-                    int32_t* votes, float* sums, hipStream_t s) {
-  if (n_rows <= 0) return;
-  if (f.task == 0) {
-    // votes cleared by a kernel (no memset node if the caller captures)
-    const int64_t nv = n_rows * f.n_classes;
-    hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(nv)), dim3(kBlock), 0, s, reinterpret_cast<uint32_t*>(votes), nv);
-    // Rows staged in LDS when a block's rows and votes fit 48 KB: 64 rows
-    // while F + C <= 191, 32 rows while F + C <= 383.
-    const int F = f.n_features, C = f.n_classes;
-    const int R = staged_rows(F, C);
-    if (R) {
-      const int64_t row_blocks = (n_rows + R - 1) / R;
-      const int chunks = tree_chunks(row_blocks, f.n_trees);
-      const int tpb = (f.n_trees + chunks - 1) / chunks;
-      const dim3 grid((unsigned)row_blocks, (unsigned)((f.n_trees + tpb - 1) / tpb));
-      const size_t lds = sizeof(uint32_t) * (size_t)R * (C + F + 1);
-      Timer tm("predict", 0.0, s);
-      if (R == 64)
-        hipLaunchKernelGGL(k_predict_cls_lds<64>, grid, dim3(kBlock), lds, s, f.pnodes.p, f.tree_start.p, f.n_trees,
-                           X, n_rows, ld, row_major, C, F, tpb, votes);
-      else
-        hipLaunchKernelGGL(k_predict_cls_lds<32>, grid, dim3(kBlock), lds, s, f.pnodes.p, f.tree_start.p, f.n_trees,
-                           X, n_rows, ld, row_major, C, F, tpb, votes);
-      DTE_HIP(hipGetLastError());
-      return;
-    }
-    const int64_t row_blocks = (n_rows + kRowsPerBlock - 1) / kRowsPerBlock;
-    const int chunks = tree_chunks(row_blocks, f.n_trees);
-    const int tpb = (f.n_trees + chunks - 1) / chunks;
-    const dim3 grid((unsigned)row_blocks, (unsigned)((f.n_trees + tpb - 1) / tpb));
-    Timer tm("predict", 0.0, s);
-    hipLaunchKernelGGL(k_predict_cls, grid, dim3(kBlock), sizeof(uint32_t) * kRowsPerBlock * f.n_classes, s,
-                       f.pnodes.p, f.tree_start.p, f.n_trees, X, n_rows, ld, row_major, f.n_classes, tpb, votes);
-  } else {
-    // Rows staged in LDS (with the chunk's leaf values) when they fit 48 KB.
-    const int F = f.n_features;
-    const int R = staged_rows(F, kRegChunk);
-    if (R) {
-      const int64_t row_blocks = (n_rows + R - 1) / R;
-      const size_t lds = sizeof(float) * (size_t)R * (kRegChunk + F + 1);
-      Timer tm("predict", 0.0, s);
-      if (R == 64)
-        hipLaunchKernelGGL(k_predict_reg_lds<64>, dim3((unsigned)row_blocks), dim3(kBlock), lds, s, f.pnodes.p,
-                           f.tree_start.p, f.n_trees, X, n_rows, ld, row_major, F, sums);
-      else
-        hipLaunchKernelGGL(k_predict_reg_lds<32>, dim3((unsigned)row_blocks), dim3(kBlock), lds, s, f.pnodes.p,
-                           f.tree_start.p, f.n_trees, X, n_rows, ld, row_major, F, sums);
-    } else {
-      const int grid = (int)std::min<int64_t>((n_rows + kBlock - 1) / kBlock, 65535);
-      Timer tm("predict", 0.0, s);
-      hipLaunchKernelGGL(k_predict_reg, dim3(grid), dim3(kBlock), 0, s, f.pnodes.p, f.tree_start.p, f.n_trees, X,
-                         n_rows, ld, row_major, sums);
-    }
+// Predict records of a forest (its canonical arrays are complete on stream
+// s).  max_tree: nodes of its largest tree.
+void build_predict_nodes(Forest& f, int64_t max_tree, hipStream_t s) {
+  const int64_t n = f.n_nodes;
+  const int T = f.n_trees;
+  const uint32_t* cls = f.task == 0 ? f.class_counts.p : nullptr;
+  const unsigned grid = (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 16384);
+  int fbits = 1;
+  while (((int64_t)1 << fbits) <= (int64_t)f.n_features) ++fbits;  // feature + 1, 0 for a leaf
+  // slots of a tree: a cluster of s pairs takes at most 1.6 s of them
+  auto slots = [](int64_t nodes) { return 8 + (nodes / 2) * 8 / 5 + 8; };
+  int pbits = 1;
+  while (((int64_t)1 << pbits) <= slots(max_tree)) ++pbits;
+  if (fbits + pbits > 32) {
+    PoolSuspend own;
+    f.pnodes.alloc(n);
+    hipLaunchKernelGGL(k_wide_nodes, dim3(grid), dim3(kBlock), 0, s, n, f.n_classes, f.task, f.feature.p,
+                       f.threshold.p, f.left.p, cls, f.value.p, f.pnodes.p);
+    DTE_HIP(hipGetLastError());
+    return;
   }
+  {
+    PoolSuspend own;  // kept with the forest
+    f.pairs.alloc((size_t)16 * T + (size_t)((n + 1) / 2) * 8 / 5);
+    f.pair_base.alloc(T);
+  }
+  f.pair_fbits = fbits;
+  PoolScope pool(s);
+  DevBuf<uint32_t> code(n), cbase(4 * (size_t)T);
+  DevBuf<unsigned int> cnt(4 * (size_t)T);
+  hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(4 * (int64_t)T)), dim3(kBlock), 0, s, cnt.p, 4 * (int64_t)T);
+  hipLaunchKernelGGL(k_cluster_count, dim3(grid), dim3(kBlock), 0, s, n, T, f.tree_start.p, f.feature.p, f.left.p,
+                     f.depth.p, code.p, cnt.p);
+  hipLaunchKernelGGL(k_cluster_bases, dim3(1), dim3(kBlock), 0, s, T, (const unsigned int*)cnt.p, f.pair_base.p,
+                     cbase.p);
+  hipLaunchKernelGGL(k_cluster_write, dim3(grid), dim3(kBlock), 0, s, n, T, f.tree_start.p, f.feature.p, f.left.p,
+                     f.depth.p, f.threshold.p, cls, f.value.p, f.n_classes, f.task, fbits, (const uint32_t*)code.p,
+                     (const int64_t*)f.pair_base.p, (const uint32_t*)cbase.p, reinterpret_cast<uint4*>(f.pairs.p));
   DTE_HIP(hipGetLastError());
 }
 

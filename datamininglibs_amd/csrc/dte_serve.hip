@@ -126,7 +126,7 @@ struct PinnedRows {
 };
 
 struct Resident {
-  Forest f;  // pnodes + tree_start only
+  Forest f;  // predict records only
   int64_t bytes = 0;
 };
 
@@ -209,7 +209,7 @@ double ms_since(Clock::time_point t0) {
   return std::chrono::duration<double, std::milli>(Clock::now() - t0).count();
 }
 
-int64_t forest_bytes(const Forest& f) { return (int64_t)(f.pnodes.bytes() + f.tree_start.bytes()); }
+int64_t forest_bytes(const Forest& f) { return (int64_t)(f.pairs.bytes() + f.pair_base.bytes() + f.pnodes.bytes() + f.tree_start.bytes()); }
 
 void free_slot_buffers(dte_server& s) {
   for (auto& sl : s.slots) {
@@ -519,11 +519,17 @@ int dte_server_load_forest(dte_server* s, const dte_forest* forest, int32_t* slo
     f.n_trees = src.n_trees;
     f.fixed_shift = src.fixed_shift;
     f.n_nodes = src.n_nodes;
-    f.tree_start.alloc(src.n_trees + 1);
-    f.pnodes.alloc(src.n_nodes);
+    f.pair_fbits = src.pair_fbits;
     hipStream_t ls = library_stream(s->device);
-    DTE_HIP(hipMemcpyAsync(f.tree_start.p, src.tree_start.p, src.tree_start.bytes(), hipMemcpyDeviceToDevice, ls));
-    DTE_HIP(hipMemcpyAsync(f.pnodes.p, src.pnodes.p, sizeof(PNode) * src.n_nodes, hipMemcpyDeviceToDevice, ls));
+    auto copy = [&](auto& dst, const auto& from) {
+      if (!from.p) return;
+      dst.alloc(from.n);
+      DTE_HIP(hipMemcpyAsync(dst.p, from.p, from.bytes(), hipMemcpyDeviceToDevice, ls));
+    };
+    copy(f.tree_start, src.tree_start);
+    copy(f.pairs, src.pairs);
+    copy(f.pair_base, src.pair_base);
+    copy(f.pnodes, src.pnodes);
     DTE_HIP(hipStreamSynchronize(ls));
     r->bytes = forest_bytes(f);
     s->st.hbm_in_use += r->bytes;
