@@ -137,14 +137,35 @@ struct ItemArgs {
   float* res_score;
   float* res_thr;
   int32_t* res_feat;
-  unsigned long long* bytes;  // algorithmic bytes counter (may be NULL)
+  unsigned long long* bytes;  // algorithmic bytes counter (NULL unless the profile is on)
   int node_major;        // 1: a grid of n_groups teams, each team walks its own group's draws in order
   uint32_t* scr_key;     // big-item scratch, one slab per block
   uint32_t* scr_aux;
   int64_t* scr_y;
   int64_t scr_stride;
   const unsigned int* n_dev;  // device-described level: n_groups = *n_dev
+  int spread;            // waves to keep busy (node_split)
 };
+
+// Parts that a node's draws are dealt to, so that `units` teams have work: a
+// level of few nodes is bound by the latency of one node's draws in a row
+// (about 8 us a draw), and its chip is idle.  With enough nodes a team takes
+// all draws of its node: later draws then profit from what earlier ones found.
+__device__ __forceinline__ int node_split(const ItemArgs& it, int64_t units, int64_t nodes) {
+  const int64_t s = nodes > 0 ? units / nodes : 1;
+  return (int)(s < 1 ? 1 : (s < it.per_group ? s : it.per_group));
+}
+
+// Counts a wave's algorithmic bytes for the profile.  Atomics on one address
+// pass at one in about 15 ns: a grid's 16 k waves on one counter took 250 us
+// of every tier, so a counter is kByteSlots words, one line each, and there
+// is none outside a profile.
+constexpr int kByteSlots = 64;
+constexpr int kByteStride = 16;
+constexpr int kByteWords = kByteSlots * kByteStride;  // of one counter
+__device__ __forceinline__ void add_bytes(unsigned long long* counter, unsigned long long v) {
+  atomicAdd(counter + (blockIdx.x & (kByteSlots - 1)) * kByteStride, v);
+}
 
 // Level slice and item count of a device-described level (a no-op for
 // launches whose arguments carry them).
@@ -1023,7 +1044,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
     if (t == 0) rf_write_result<MAXC, TASK, TEAM, IPT>(d, it, ridx, f, L.cr);
     team_sync<TEAM>();
   }
-  if (t == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (t == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
 
 // ------------------------------------- chunk-parallel big-node search ---
@@ -2267,7 +2288,7 @@ __device__ __forceinline__ void ert_block_body(DataArgs d, LevelArgs lv, ItemArg
     }
     __syncthreads();
   }
-  if (t == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (t == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_search_ert(DataArgs d, LevelArgs lv, ItemArgs it) {
@@ -2411,7 +2432,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_wave(DataArgs d, LevelArgs
       it.res_feat[ridx] = f;
     }
   }
-  if (lane == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (lane == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
 
 // Segment-per-node RF search for tiny nodes: a wave holds 64/SEG nodes, one
@@ -2460,27 +2481,36 @@ __device__ __forceinline__ BestCand seg_best(BestCand b) {
   return b;
 }
 
+template <int TASK>
+struct SegLds {
+  static constexpr int kTL = 2048;  // LDS copy of T's head
+  double inv[128], logc[128];
+  int64_t T[TASK == 0 ? kTL : 1];
+};
+
 template <int MAXC, int TASK, int SEG>
-__global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs lv, ItemArgs it) {
-  constexpr int NPW = kWave / SEG;  // nodes per wave
+__device__ __forceinline__ void rf_seg_body(DataArgs d, LevelArgs lv, ItemArgs it, int64_t bid, int64_t nblk,
+                                            SegLds<TASK>& S) {
+  constexpr int NPW = kWave / SEG;  // segments per wave
   resolve_level(lv, d.C);
   resolve_items(it);
-  if ((int64_t)blockIdx.x * kWaves * NPW >= it.n_groups) return;
-  constexpr int kTL = 2048;         // LDS copy of T's head
-  __shared__ double s_inv[128], s_logc[128];
-  __shared__ int64_t s_T[TASK == 0 ? kTL : 1];
-  load_tables(s_inv, s_logc);
-  const int64_t nTL = TASK == 0 ? load_t_prefix<kTL>(s_T, d.T, d.Tmax) : 0;
+  const int split = node_split(it, (int64_t)it.spread * NPW, it.n_groups);
+  const int64_t n_units = it.n_groups * split;
+  if (bid * kWaves * NPW >= n_units) return;
+  load_tables(S.inv, S.logc);
+  const int64_t nTL = TASK == 0 ? load_t_prefix<SegLds<TASK>::kTL>(S.T, d.T, d.Tmax) : 0;
   __syncthreads();
-  const LnCtxL lx{s_inv, s_logc, d.T, d.Tmax, d.igF, s_T, nTL};
+  const LnCtxL lx{S.inv, S.logc, d.T, d.Tmax, d.igF, S.T, nTL};
   const int sl = threadIdx.x & (SEG - 1);
   const int seg = (threadIdx.x & (kWave - 1)) / SEG;
   unsigned long long my_bytes = 0;
-  const int64_t wave_id = (int64_t)blockIdx.x * kWaves + threadIdx.x / kWave;
-  const int64_t n_waves = (int64_t)gridDim.x * kWaves;
-  for (int64_t g0 = wave_id * NPW; g0 < it.n_groups; g0 += n_waves * NPW) {
-    const int64_t g = g0 + seg;
-    const bool node_ok = g < it.n_groups;
+  const int64_t wave_id = bid * kWaves + threadIdx.x / kWave;
+  const int64_t n_waves = nblk * kWaves;
+  for (int64_t u0 = wave_id * NPW; u0 < n_units; u0 += n_waves * NPW) {
+    const int64_t u = u0 + seg;
+    const bool node_ok = u < n_units;
+    const int64_t g = split > 1 ? (int64_t)((uint32_t)u / (uint32_t)split) : u;
+    const int j1 = split > 1 ? (int)((uint32_t)u % (uint32_t)split) : 0;  // the unit's first draw
     uint32_t o = 0, i = 0, tg = 0, nid = 0;
     int m = 0;
     int64_t st = 0, n = 0, ssum = 0;
@@ -2514,7 +2544,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs 
       pay0 = lv.aux[st + sl];
       if (TASK == 1) y0 = lv.ey[st + sl];
     }
-    if (sl == 0 && node_ok && !pure) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
+    if (sl == 0 && node_ok && !pure && j1 == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
     // Draw pipeline: the key gather (and value offset) of draw jj + 1 and the
     // threshold values of draw jj - 1 are in flight while draw jj is ranked
     // and scored.
@@ -2522,7 +2552,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs 
     uint32_t key_nx = kNone;
     int64_t svo_nx = 0;
     if (!pure && it.per_group > 0) {
-      f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)it.j0) % (uint32_t)d.F);
+      f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + j1)) % (uint32_t)d.F);
       key_nx = valid ? d.K[(int64_t)f_nx * d.N + row] : kNone;
       svo_nx = d.SVoff[f_nx];
     }
@@ -2530,7 +2560,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs 
     int64_t p_ridx = 0;
     int p_f = 0;
     float p_score = 0.0f, p_lo = 0.0f, p_hi = 0.0f;
-    for (int jj = 0; jj < it.per_group; ++jj) {
+    for (int jj = j1; jj < it.per_group; jj += split) {
       const int j = it.j0 + jj;
       const int64_t ridx = (int64_t)o * it.D + j;
       if (pure) {
@@ -2544,8 +2574,8 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs 
       const int f = f_nx;
       const int64_t svo = svo_nx;
       uint32_t key = key_nx;
-      if (jj + 1 < it.per_group) {
-        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + 1)) % (uint32_t)d.F);
+      if (jj + split < it.per_group) {
+        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + split)) % (uint32_t)d.F);
         key_nx = valid ? d.K[(int64_t)f_nx * d.N + row] : kNone;
         svo_nx = d.SVoff[f_nx];
       }
@@ -2624,7 +2654,12 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs 
       it.res_feat[p_ridx] = p_f;
     }
   }
-  if (sl == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (sl == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
+}
+template <int MAXC, int TASK, int SEG>
+__global__ void __launch_bounds__(kBlock) k_search_rf_seg(DataArgs d, LevelArgs lv, ItemArgs it) {
+  __shared__ SegLds<TASK> S;
+  rf_seg_body<MAXC, TASK, SEG>(d, lv, it, blockIdx.x, gridDim.x, S);
 }
 
 // ------------------------------------ RF split search by bucket bounds ---
@@ -3179,30 +3214,43 @@ __device__ __forceinline__ void bound_pure(const DataArgs& d, const ItemArgs& it
 
 // Nodes of up to 64 IPT entries, one wave per node: the draws in order, the
 // next draw's key gather in flight.
+constexpr int kBoundLogB = 6;
+
 template <int MAXC, int TASK, int IPT>
-__global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_bound(DataArgs d, LevelArgs lv, ItemArgs it) {
-  constexpr int LOGB = 6;
+struct BoundWgLds {
+  using Wave = BoundLds<MAXC, TASK, kBoundLogB, IPT>;
+  float tf[TASK == 0 ? Wave::TAB : 1];
+  Wave l[kWaves];
+};
+
+template <int MAXC, int TASK, int IPT>
+__device__ __forceinline__ void rf_bound_body(DataArgs d, LevelArgs lv, ItemArgs it, int64_t bid, int64_t nblk,
+                                              BoundWgLds<MAXC, TASK, IPT>& S) {
+  constexpr int LOGB = kBoundLogB;
   using LdsT = BoundLds<MAXC, TASK, LOGB, IPT>;
   resolve_level(lv, d.C);
   resolve_items(it);
-  if ((int64_t)blockIdx.x * kWaves >= it.n_groups) return;  // no node for this workgroup
-  __shared__ float s_tf[TASK == 0 ? LdsT::TAB : 1];
-  __shared__ LdsT s_l[kWaves];
+  const int split = node_split(it, it.spread, it.n_groups);
+  const int64_t n_units = it.n_groups * split;
+  if (bid * kWaves >= n_units) return;  // no node for this workgroup
+  float* s_tf = S.tf;
   if (TASK == 0)
     for (int i = threadIdx.x; i < LdsT::TAB; i += kBlock) s_tf[i] = d.Tf[i];
   __syncthreads();
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  LdsT& L = s_l[wv];
+  LdsT& L = S.l[wv];
   const int lane = threadIdx.x & (kWave - 1);
   unsigned long long my_bytes = 0;
-  for (int64_t grp = (int64_t)blockIdx.x * kWaves + wv; grp < it.n_groups; grp += (int64_t)gridDim.x * kWaves) {
+  for (int64_t u = bid * kWaves + wv; u < n_units; u += nblk * kWaves) {
+    const int64_t grp = split > 1 ? (int64_t)((uint32_t)u / (uint32_t)split) : u;
+    const int j1 = split > 1 ? (int)((uint32_t)u % (uint32_t)split) : 0;  // the unit's first draw
     const uint32_t o = __builtin_amdgcn_readfirstlane(it.list ? it.list[grp] : (uint32_t)grp);
     const uint32_t i = __builtin_amdgcn_readfirstlane(lv.open_idx[o]);
     const uint32_t tg = (uint32_t)__builtin_amdgcn_readfirstlane(lv.tree_global[lv.tree[i]]);
     const uint32_t nid = __builtin_amdgcn_readfirstlane(lv.id[i]);
     BoundNode nd;
     if (bound_node<MAXC, TASK>(d, lv, i, L.ncls, nd)) {
-      if (lane == 0) bound_pure(d, it, o, tg, nid);
+      if (lane == 0 && j1 == 0) bound_pure(d, it, o, tg, nid);
       continue;
     }
     const int m = nd.m;
@@ -3225,11 +3273,11 @@ __global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_b
     float best_score = 0.0f;
     for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
     double thr = bound_units<TASK>(d, nd, best_score);
-    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)it.j0) % (uint32_t)d.F);
+    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + j1)) % (uint32_t)d.F);
     {
       gather_keys<IPT, kWave>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
     }
-    for (int jj = 0; jj < it.per_group; ++jj) {
+    for (int jj = j1; jj < it.per_group; jj += split) {
       const int j = it.j0 + jj;
       // once a retry draw passed 1e-3 the later ones are not looked at (k_decide2)
       if (it.j0 > 0 && (double)best_score > 1e-3) break;
@@ -3238,8 +3286,8 @@ __global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_b
 #pragma unroll
       for (int q = 0; q < IPT; ++q) key[q] = kn[q];
       mask_keys<IPT, kWave>(m, key);
-      if (jj + 1 < it.per_group) {
-        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + 1)) % (uint32_t)d.F);
+      if (jj + split < it.per_group) {
+        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + split)) % (uint32_t)d.F);
         gather_keys<IPT, kWave>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
       }
       DrawBest best;
@@ -3249,9 +3297,14 @@ __global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_b
       best_score = fmaxf(best_score, score);
       if (lane == 0) bound_write<TASK>(d, it, (int64_t)o * it.D + j, f, best, score);
     }
-    if (lane == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
+    if (lane == 0 && j1 == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
   }
-  if (lane == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (lane == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
+}
+template <int MAXC, int TASK, int IPT>
+__global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_bound(DataArgs d, LevelArgs lv, ItemArgs it) {
+  __shared__ BoundWgLds<MAXC, TASK, IPT> S;
+  rf_bound_body<MAXC, TASK, IPT>(d, lv, it, blockIdx.x, gridDim.x, S);
 }
 
 // Nodes of up to 2048 entries, one workgroup per node and draw at a time: 256
@@ -3287,24 +3340,37 @@ struct BoundTeamLds {
   int sp;
 };
 
-template <int MAXC, int TASK, int LOGB>
-__global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataArgs d, LevelArgs lv, ItemArgs it) {
+template <int MAXC, int TASK>
+struct BoundTeamWgLds {
+  static constexpr int LOGB = MAXC <= 16 ? 8 : 7;
+  float tf[TASK == 0 ? kTfMax : 1];
+  BoundTeamLds<MAXC, TASK, LOGB> l;
+};
+
+template <int MAXC, int TASK>
+__device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, ItemArgs it, int64_t bid, int64_t nblk,
+                                                   BoundTeamWgLds<MAXC, TASK>& S) {
+  constexpr int LOGB = BoundTeamWgLds<MAXC, TASK>::LOGB;
   using LdsT = BoundTeamLds<MAXC, TASK, LOGB>;
   constexpr int IPT = kTeamIpt2;
   constexpr int NB = LdsT::NB, PAIRS = LdsT::PAIRS;
   constexpr int NW = NB / kWave;  // waves with buckets
   resolve_level(lv, d.C);
   resolve_items(it);
-  if ((int64_t)blockIdx.x >= it.n_groups) return;  // no node for this workgroup
-  __shared__ float s_tf[TASK == 0 ? kTfMax : 1];
-  __shared__ LdsT L;
+  const int split = node_split(it, it.spread / kWaves, it.n_groups);
+  const int64_t n_units = it.n_groups * split;
+  if (bid >= n_units) return;  // no node for this workgroup
+  float* s_tf = S.tf;
+  LdsT& L = S.l;
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(t / kWave);
   if (TASK == 0)
     for (int i = t; i < kTfMax; i += kBlock) s_tf[i] = d.Tf[i];
   unsigned long long my_bytes = 0;
-  for (int64_t grp = blockIdx.x; grp < it.n_groups; grp += gridDim.x) {
+  for (int64_t u = bid; u < n_units; u += nblk) {
+    const int64_t grp = split > 1 ? (int64_t)((uint32_t)u / (uint32_t)split) : u;
+    const int j1 = split > 1 ? (int)((uint32_t)u % (uint32_t)split) : 0;  // the unit's first draw
     const uint32_t o = __builtin_amdgcn_readfirstlane(it.list ? it.list[grp] : (uint32_t)grp);
     const uint32_t i = __builtin_amdgcn_readfirstlane(lv.open_idx[o]);
     const uint32_t tg = (uint32_t)__builtin_amdgcn_readfirstlane(lv.tree_global[lv.tree[i]]);
@@ -3312,7 +3378,7 @@ __global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataA
     BoundNode nd;
     __syncthreads();  // the previous node's class totals are read no more
     if (bound_node<MAXC, TASK>(d, lv, i, L.ncls, nd)) {  // workgroup-uniform
-      if (t == 0) bound_pure(d, it, o, tg, nid);
+      if (t == 0 && j1 == 0) bound_pure(d, it, o, tg, nid);
       continue;
     }
     const int m = nd.m;
@@ -3338,11 +3404,11 @@ __global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataA
     float best_score = 0.0f;
     for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
     double thr = bound_units<TASK>(d, nd, best_score);
-    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)it.j0) % (uint32_t)d.F);
+    int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + j1)) % (uint32_t)d.F);
     {
       gather_keys<IPT, kBlock>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
     }
-    for (int jj = 0; jj < it.per_group; ++jj) {
+    for (int jj = j1; jj < it.per_group; jj += split) {
       const int j = it.j0 + jj;
       if (it.j0 > 0 && (double)best_score > 1e-3) break;
       const int f = f_nx;
@@ -3350,8 +3416,8 @@ __global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataA
 #pragma unroll
       for (int q = 0; q < IPT; ++q) key[q] = kn[q];
       mask_keys<IPT, kBlock>(m, key);
-      if (jj + 1 < it.per_group) {
-        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + 1)) % (uint32_t)d.F);
+      if (jj + split < it.per_group) {
+        f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + split)) % (uint32_t)d.F);
         gather_keys<IPT, kBlock>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
       }
       uint32_t kmin = kNone, kmax = 0;
@@ -3679,9 +3745,88 @@ __global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataA
       if (t == 0) bound_write<TASK>(d, it, (int64_t)o * it.D + j, f, best, score);
       __syncthreads();  // L.best, L.w are rewritten by the next draw
     }
-    if (t == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
+    if (t == 0 && j1 == 0) my_bytes += (unsigned long long)m * it.per_group * (TASK == 0 ? 12ull : 20ull);
   }
-  if (t == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (t == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
+}
+template <int MAXC, int TASK>
+__global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_bound_team(DataArgs d, LevelArgs lv, ItemArgs it) {
+  __shared__ BoundTeamWgLds<MAXC, TASK> S;
+  rf_bound_team_body<MAXC, TASK>(d, lv, it, blockIdx.x, gridDim.x, S);
+}
+
+// Random-forest tiers 0..4 of a phase in one launch.  A small level is bound
+// by the latency of its tiers, one launch after the other (35 to 100 us each
+// at 4,601 x 57, 100 trees); side by side the level takes as long as its
+// slowest tier.  Workgroups go to the tiers by their device counts, the
+// largest nodes first, at most cap[k] to a tier (they loop over its nodes);
+// the rest of the grid returns at once, which costs 1.5 ns a workgroup: with
+// the single tiers' caps, 17 k of them, a level without nodes took 26 us.
+struct RfTiers {
+  const uint32_t* list[5];
+  const unsigned int* n_dev[5];  // counts on the device, or NULL:
+  int64_t n[5];
+  unsigned long long* bytes[5];
+  int cap[5];                    // most blocks of a tier
+};
+
+// Blocks that a random-forest tier's units fill: 4 / 2 / 1 / 1 nodes per wave,
+// then a node per workgroup.
+__host__ __device__ __forceinline__ int64_t rf_tier_blocks(int tier, int64_t nodes, int per_group, int spread) {
+  const int per_wg = tier == 0 ? 4 * kWaves : (tier == 1 ? 2 * kWaves : (tier <= 3 ? kWaves : 1));
+  const int64_t target = (int64_t)spread / kWaves * per_wg;  // units of node_split
+  const int64_t all = nodes * per_group;
+  const int64_t units = nodes >= target ? nodes : (all < target ? all : target);
+  return (units + per_wg - 1) / per_wg;
+}
+
+template <size_t A, size_t B>
+constexpr size_t max_size() { return A > B ? A : B; }
+
+template <int MAXC, int TASK>
+__global__ void __launch_bounds__(kBlock, 3 - TASK) k_search_rf_all(DataArgs d, LevelArgs lv, ItemArgs it, RfTiers ts) {
+  using Seg = SegLds<TASK>;
+  using B1 = BoundWgLds<MAXC, TASK, 1>;
+  using B8 = BoundWgLds<MAXC, TASK, 8>;
+  using Tm = BoundTeamWgLds<MAXC, TASK>;
+  __shared__ __align__(16) unsigned char
+      s_raw[max_size<max_size<sizeof(Seg), sizeof(B1)>(), max_size<sizeof(B8), sizeof(Tm)>()>()];
+  int64_t bid = blockIdx.x, nblk = 0;
+  int tier = 4;
+  for (;; --tier) {
+    const int64_t n = ts.n_dev[tier] ? (int64_t)*ts.n_dev[tier] : ts.n[tier];
+    nblk = rf_tier_blocks(tier, n, it.per_group, it.spread);
+    nblk = nblk < ts.cap[tier] ? nblk : ts.cap[tier];
+    if (bid < nblk) break;
+    bid -= nblk;
+    if (tier == 0) return;
+  }
+  it.list = ts.list[tier];
+  it.n_groups = ts.n[tier];
+  it.n_dev = ts.n_dev[tier];
+  it.bytes = ts.bytes[tier];
+  switch (tier) {
+    case 0: rf_seg_body<MAXC, TASK, 16>(d, lv, it, bid, nblk, *reinterpret_cast<Seg*>(s_raw)); break;
+    case 1: rf_seg_body<MAXC, TASK, 32>(d, lv, it, bid, nblk, *reinterpret_cast<Seg*>(s_raw)); break;
+    case 2: rf_bound_body<MAXC, TASK, 1>(d, lv, it, bid, nblk, *reinterpret_cast<B1*>(s_raw)); break;
+    case 3: rf_bound_body<MAXC, TASK, 8>(d, lv, it, bid, nblk, *reinterpret_cast<B8*>(s_raw)); break;
+    default: rf_bound_team_body<MAXC, TASK>(d, lv, it, bid, nblk, *reinterpret_cast<Tm*>(s_raw)); break;
+  }
+}
+
+template <int MAXC, int TASK>
+void launch_search_rf_all(int64_t grid, hipStream_t s, const DataArgs& d, const LevelArgs& lv, const ItemArgs& it,
+                          const RfTiers& ts) {
+  hipLaunchKernelGGL((k_search_rf_all<MAXC, TASK>), dim3((unsigned)grid), dim3(kBlock), 0, s, d, lv, it, ts);
+}
+using RfAllFn = void (*)(int64_t, hipStream_t, const DataArgs&, const LevelArgs&, const ItemArgs&, const RfTiers&);
+RfAllFn pick_rf_all(int task, int C) {
+  if (task == 1) return launch_search_rf_all<1, 1>;
+  if (C <= 2) return launch_search_rf_all<2, 0>;
+  if (C <= 4) return launch_search_rf_all<4, 0>;
+  if (C <= 8) return launch_search_rf_all<8, 0>;
+  if (C <= 16) return launch_search_rf_all<16, 0>;
+  return launch_search_rf_all<32, 0>;
 }
 
 // ERT, one wave per item (any node size; lanes stride over the entries).
@@ -3803,7 +3948,7 @@ __device__ __forceinline__ void ert_wave_body(DataArgs d, LevelArgs lv, ItemArgs
       it.res_feat[ridx] = f;
     }
   }
-  if (lane == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (lane == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_search_ert_wave(DataArgs d, LevelArgs lv, ItemArgs it) {
@@ -3954,7 +4099,7 @@ __device__ __forceinline__ void ert_seg_body(DataArgs d, LevelArgs lv, ItemArgs 
       xe_c = xe_n;
     }
   }
-  if (my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
 // Four waves per SIMD (128 VGPRs, no spills; three at the unbounded 131).
 template <int MAXC, int TASK, int SEG>
@@ -4118,7 +4263,7 @@ __device__ __forceinline__ void ert_team_body(DataArgs d, LevelArgs lv, ItemArgs
       for (int q = 0; q < IPT; ++q) xe_c[q] = xe_n[q];
     }
   }
-  if (lane == 0 && my_bytes && it.bytes) atomicAdd(it.bytes, my_bytes);
+  if (lane == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_search_ert_team(DataArgs d, LevelArgs lv, ItemArgs it) {
@@ -4126,15 +4271,12 @@ __global__ void __launch_bounds__(kBlock) k_search_ert_team(DataArgs d, LevelArg
   ert_team_body<MAXC, TASK>(d, lv, it, blockIdx.x, gridDim.x, s_inv, s_logc);
 }
 
-// All extra-trees tiers of a phase in one launch: workgroups [first[k],
-// first[k + 1]) run tier k's code over tier k's list (each tier exactly as
-// its own kernel would, with its share of the grid).  Small level steps
-// are latency-bound, tier after tier; in one launch the tiers run side by
-// side without a join between them.
-constexpr int64_t kErtMergeEntries = (int64_t)8 << 20;
+// All extra-trees tiers of a phase in one launch (each tier exactly as its own
+// kernel would run, with its share of the grid; see RfTiers).
+constexpr int64_t kMergeEntries = (int64_t)8 << 20;
 
 struct ErtTiers {
-  int64_t first[7];
+  int cap[6];  // most blocks of a tier
   const uint32_t* list[6];
   const unsigned int* n_dev[6];
   unsigned long long* bytes[6];
@@ -4144,15 +4286,23 @@ struct ErtTiers {
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock, 3) k_search_ert_all(DataArgs d, LevelArgs lv, ItemArgs it, ErtTiers ts) {
   __shared__ double s_inv[128], s_logc[128];
-  const int64_t b = blockIdx.x;
-  int k = 0;
-  while (k < 5 && b >= ts.first[k + 1]) ++k;
+  int64_t bid = blockIdx.x, nblk = 0;
+  int k = 5;
+  for (;; --k) {
+    // nodes per block: 16 / 8 / 4 / 4; items per block: 4, 1
+    const int64_t n = (int64_t)*ts.n_dev[k] * (k >= 4 ? it.per_group : 1);
+    const int per_wg = k == 0 ? 4 * kWaves : (k == 1 ? 2 * kWaves : (k <= 4 ? kWaves : 1));
+    nblk = (n + per_wg - 1) / per_wg;
+    nblk = nblk < ts.cap[k] ? nblk : ts.cap[k];
+    if (bid < nblk) break;
+    bid -= nblk;
+    if (k == 0) return;
+  }
   ItemArgs a = it;
   a.list = ts.list[k];
   a.n_groups = 0;
   a.n_dev = ts.n_dev[k];
   a.bytes = ts.bytes[k];
-  const int64_t bid = b - ts.first[k], nblk = ts.first[k + 1] - ts.first[k];
   switch (k) {
     case 0: ert_seg_body<MAXC, TASK, 16>(d, lv, a, bid, nblk, s_inv, s_logc); break;
     case 1: ert_seg_body<MAXC, TASK, 32>(d, lv, a, bid, nblk, s_inv, s_logc); break;
@@ -4181,8 +4331,7 @@ ErtAllFn pick_ert_all(int task, int C) {
 // Split a list of open positions (or all of them) by node size into the
 // wave tier and the block tier.  Order inside a tier is irrelevant: every
 // item writes its own result slot.
-// Wave-aggregated: one global atomic per wave and tier.  Tier k holds the
-// groups with cuts[k-1] < m <= cuts[k].
+// Tier k holds the groups with cuts[k-1] < m <= cuts[k].
 struct Cuts {
   int c[kMaxTiers];  // ascending; the last tier takes everything above
   int n;             // number of tiers
@@ -4202,21 +4351,29 @@ __device__ __forceinline__ int tier_of(int m, const Cuts& cuts) {
   return tier;
 }
 
-// Each wave owns a contiguous range of the list: it counts its tiers, takes
-// one slot range per tier with a single atomic, then writes its entries.
-// Workgroups of a tier split: every wave adds its tier counts with one
-// global atomic per tier, so the grid bounds the atomics on those few words.
-constexpr int kTierGrid = 256;
-__global__ void k_tier_split(const uint32_t* list, int64_t n, const uint32_t* open_idx, const int32_t* node_m, Cuts cuts,
-                             TierLists out, unsigned int* counts, const unsigned int* n_dev, const int64_t* off_dev) {
+// Each wave owns a contiguous range of the list: it counts its tiers, the
+// workgroup takes one slot range per tier with a single atomic instruction
+// (all tiers' counters lie in one line), then the waves write their entries.
+// Bound by those atomics, which pass one at a time per line: 1,024 waves with
+// an atomic per tier took 85 us for 150 k nodes, 64 workgroups of 16 waves take
+// about 10 us.
+constexpr int kTierGrid = 64;
+constexpr int kTierBlock = 1024;
+__global__ void __launch_bounds__(kTierBlock) k_tier_split(const uint32_t* list, int64_t n, const uint32_t* open_idx,
+                                                           const int32_t* node_m, Cuts cuts, TierLists out,
+                                                           unsigned int* counts, const unsigned int* n_dev,
+                                                           const int64_t* off_dev) {
+  constexpr int NW = kTierBlock / kWave;
+  __shared__ unsigned int s_cnt[NW][kMaxTiers], s_base[NW][kMaxTiers];
   if (n_dev) n = *n_dev;            // device-described level
   if (off_dev) node_m += *off_dev;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = (int64_t)blockIdx.x * kWaves + threadIdx.x / kWave;
-  const int64_t n_waves = (int64_t)gridDim.x * kWaves;
+  const int wv = threadIdx.x / kWave;
+  const int64_t wave = (int64_t)blockIdx.x * NW + wv;
+  const int64_t n_waves = (int64_t)gridDim.x * NW;
   const int64_t per = (((n + n_waves - 1) / n_waves) + kWave - 1) & ~(int64_t)(kWave - 1);
   const int64_t lo = wave * per, hi = min(lo + per, n);
-  if (lo >= hi) return;  // wave-uniform
+  if ((int64_t)blockIdx.x * NW * per >= n) return;  // workgroup-uniform
   unsigned int cnt[kMaxTiers];
 #pragma unroll
   for (int k = 0; k < kMaxTiers; ++k) cnt[k] = 0;
@@ -4227,13 +4384,24 @@ __global__ void k_tier_split(const uint32_t* list, int64_t n, const uint32_t* op
     for (int k = 0; k < kMaxTiers; ++k)
       if (k < cuts.n) cnt[k] += (unsigned int)__popcll(__ballot(tier == k));
   }
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < kMaxTiers; ++k) s_cnt[wv][k] = cnt[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < kMaxTiers) {
+    unsigned int sum = 0;
+    for (int x = 0; x < NW; ++x) sum += s_cnt[x][threadIdx.x];
+    unsigned int base = sum ? atomicAdd(&counts[threadIdx.x], sum) : 0u;
+    for (int x = 0; x < NW; ++x) {
+      s_base[x][threadIdx.x] = base;
+      base += s_cnt[x][threadIdx.x];
+    }
+  }
+  __syncthreads();
   unsigned int base[kMaxTiers];
 #pragma unroll
-  for (int k = 0; k < kMaxTiers; ++k) {
-    unsigned int b0 = 0;
-    if (lane == 0 && k < cuts.n && cnt[k]) b0 = atomicAdd(&counts[k], cnt[k]);
-    base[k] = __shfl(b0, 0, kWave);
-  }
+  for (int k = 0; k < kMaxTiers; ++k) base[k] = s_base[wv][k];
   const uint64_t below = (1ull << lane) - 1ull;
   for (int64_t b = lo; b < hi; b += kWave) {
     const int64_t g = b + lane;
@@ -4510,7 +4678,7 @@ __device__ __forceinline__ void part_block_body(DataArgs d, LevelArgs lv, PartAr
     }
     __syncthreads();
   }
-  if (t == 0 && my_bytes && pa.bytes) atomicAdd(pa.bytes, my_bytes);
+  if (t == 0 && my_bytes && pa.bytes) add_bytes(pa.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_partition(DataArgs d, LevelArgs lv, PartArgs pa) {
@@ -4675,7 +4843,7 @@ __global__ void __launch_bounds__(kBlock) k_part_chunk_finish(DataArgs d, LevelA
     base += tot;
     __syncthreads();
   }
-  if (t == 0 && pa.bytes) atomicAdd(pa.bytes, (unsigned long long)m * (TASK == 0 ? 12ull : 20ull));
+  if (t == 0 && pa.bytes) add_bytes(pa.bytes, (unsigned long long)m * (TASK == 0 ? 12ull : 20ull));
 }
 
 template <int TASK>
@@ -4815,7 +4983,7 @@ __device__ __forceinline__ void part_wave_body(DataArgs d, LevelArgs lv, PartArg
       }
     }
   }
-  if (lane == 0 && my_bytes && pa.bytes) atomicAdd(pa.bytes, my_bytes);
+  if (lane == 0 && my_bytes && pa.bytes) add_bytes(pa.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_partition_wave(DataArgs d, LevelArgs lv, PartArgs pa,
@@ -4907,7 +5075,7 @@ __device__ __forceinline__ void part_seg_body(DataArgs d, LevelArgs lv, PartArgs
       if (TASK == 1) pa.ney[st + pos] = ey;
     }
   }
-  if (sl == 0 && my_bytes && pa.bytes) atomicAdd(pa.bytes, my_bytes);
+  if (sl == 0 && my_bytes && pa.bytes) add_bytes(pa.bytes, my_bytes);
 }
 template <int MAXC, int TASK, int SEG>
 __global__ void __launch_bounds__(kBlock) k_partition_seg(DataArgs d, LevelArgs lv, PartArgs pa,
@@ -4916,10 +5084,9 @@ __global__ void __launch_bounds__(kBlock) k_partition_seg(DataArgs d, LevelArgs 
 }
 
 // All partition tiers of a level step in one launch (small data, see
-// k_search_ert_all): workgroups [first[k], first[k + 1]) run tier k
-// (16-lane segments, 32-lane segments, a wave, a workgroup per node).
+// RfTiers): 16-lane segments, 32-lane segments, a wave, a workgroup per node.
 struct PartTiers {
-  int64_t first[5];
+  int cap[4];  // most blocks of a tier
   const uint32_t* list[4];
   const unsigned int* n_dev[4];
   int64_t n_bound;  // list capacity (the device counts hold the sizes)
@@ -4927,11 +5094,17 @@ struct PartTiers {
 
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_partition_all(DataArgs d, LevelArgs lv, PartArgs pa, PartTiers pt) {
-  const int64_t b = blockIdx.x;
-  int k = 0;
-  while (k < 3 && b >= pt.first[k + 1]) ++k;
+  int64_t bid = blockIdx.x, nblk = 0;
+  int k = 3;
+  for (;; --k) {
+    const int per_wg = k == 0 ? 4 * kWaves : (k == 1 ? 2 * kWaves : (k == 2 ? kWaves : 1));
+    nblk = ((int64_t)*pt.n_dev[k] + per_wg - 1) / per_wg;
+    nblk = nblk < pt.cap[k] ? nblk : pt.cap[k];
+    if (bid < nblk) break;
+    bid -= nblk;
+    if (k == 0) return;
+  }
   pa.n_dev = pt.n_dev[k];
-  const int64_t bid = b - pt.first[k], nblk = pt.first[k + 1] - pt.first[k];
   switch (k) {
     case 0: part_seg_body<MAXC, TASK, 16>(d, lv, pa, pt.list[0], pt.n_bound, bid, nblk); break;
     case 1: part_seg_body<MAXC, TASK, 32>(d, lv, pa, pt.list[1], pt.n_bound, bid, nblk); break;
@@ -5528,7 +5701,7 @@ void launch_search(int algorithm, int tier, int grid, hipStream_t s, const DataA
       case 1: hipLaunchKernelGGL((k_search_rf_seg<MAXC, TASK, 32>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       case 2: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       case 3: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 8>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      case 4: hipLaunchKernelGGL((k_search_rf_bound_team<MAXC, TASK, MAXC <= 16 ? 8 : 7>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      case 4: hipLaunchKernelGGL((k_search_rf_bound_team<MAXC, TASK>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       default: hipLaunchKernelGGL((k_search_rf<MAXC, TASK, 256, true>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
     }
   } else {
@@ -6050,9 +6223,12 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   DevBuf<int32_t> tree_global(T);
   DTE_HIP(hipMemcpyAsync(tree_global.p, tg_h.data(), 4 * T, hipMemcpyHostToDevice, s));
 
-  DevBuf<unsigned long long> search_bytes(kMaxTiers), part_bytes(1);  // search: one counter per tier
-  DTE_HIP(hipMemsetAsync(search_bytes.p, 0, 8 * kMaxTiers, s));
-  DTE_HIP(hipMemsetAsync(part_bytes.p, 0, 8, s));
+  // profile: algorithmic bytes, search (one counter per tier) and partition
+  const bool count_bytes = profiling_enabled();
+  DevBuf<unsigned long long> byte_counts(count_bytes ? (kMaxTiers + 1) * kByteWords : 1);
+  auto tier_bytes = [&](int tier) { return count_bytes ? byte_counts.p + (size_t)tier * kByteWords : nullptr; };
+  unsigned long long* const part_bytes = tier_bytes(kMaxTiers);
+  if (count_bytes) DTE_HIP(hipMemsetAsync(byte_counts.p, 0, byte_counts.bytes(), s));
 
   // ---- root entries.
   int64_t E = 0;
@@ -6314,12 +6490,18 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   }
   DevBuf<uint32_t> tier_list[kMaxTiers];
   DevBuf<unsigned int> tier_cnt(kMaxTiers);
+  auto tier_grid = [](int64_t n) { return (unsigned)std::min<int64_t>((n + kTierBlock - 1) / kTierBlock, kTierGrid); };
   auto tier_lists = [&]() {
     TierLists tl{};
     for (int k = 0; k < kMaxTiers; ++k) tl.l[k] = tier_list[k].p;
     return tl;
   };
   const int wave_grid_cap = num_cu * 16;
+  const int spread_waves = num_cu * 12;  // three waves per SIMD, the least the bounded tiers run at
+  // two rounds of workgroups at the merged kernel's three a CU
+  auto merged_cap = [num_cu](int tier) { return tier <= 3 ? num_cu * 6 : num_cu * 3; };
+  const bool small_data = E <= kMergeEntries;
+  const RfAllFn rf_all = pick_rf_all(task, C);
   LevelArgs lv{};
   int64_t trace_tier[3] = {0, 0, 0};
   // Side stream of the split search's tiers beside the chunk pipeline
@@ -6347,7 +6529,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   auto run_phase = [&](ItemArgs it) {
     for (auto& tl : tier_list) tl.reserve(it.n_groups);
     DTE_HIP(hipMemsetAsync(tier_cnt.p, 0, 4 * kMaxTiers, s));
-    hipLaunchKernelGGL(k_tier_split, dim3(std::min(grid_for(it.n_groups), kTierGrid)), dim3(kBlock), 0, s, it.list, it.n_groups,
+    hipLaunchKernelGGL(k_tier_split, dim3(tier_grid(it.n_groups)), dim3(kTierBlock), 0, s, it.list, it.n_groups,
                        lv.open_idx, lv.m, cuts, tier_lists(), tier_cnt.p, nullptr, nullptr);
     unsigned int cnt[kMaxTiers];
     DTE_HIP(hipMemcpyAsync(cnt, tier_cnt.p, 4 * kMaxTiers, hipMemcpyDeviceToHost, s));
@@ -6366,24 +6548,40 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       DTE_HIP(hipEventRecord(side.fork, s));
       DTE_HIP(hipStreamWaitEvent(ts, side.fork, 0));
     }
-    for (int tier = 0; tier < cuts.n; ++tier) {
+    const bool merged = rf && small_data && others;
+    if (merged) {
+      RfTiers rt{};
+      int64_t blocks = 0;
+      for (int tier = 0; tier < 5; ++tier) {
+        rt.cap[tier] = merged_cap(tier);
+        blocks += std::min<int64_t>(rf_tier_blocks(tier, cnt[tier], it.per_group, it.spread), rt.cap[tier]);
+        rt.list[tier] = tier_list[tier].p;
+        rt.n[tier] = cnt[tier];
+        rt.bytes[tier] = it.bytes ? it.bytes + (size_t)tier * kByteWords : nullptr;
+        trace_tier[tier <= 2 ? 0 : (tier == 3 ? 1 : 2)] += cnt[tier];
+      }
+      Timer tk("search_merged", 0.0, ts);
+      rf_all(blocks, ts, d, lv, it, rt);
+    }
+    for (int tier = merged ? 5 : 0; tier < cuts.n; ++tier) {
       if (!cnt[tier]) continue;
       ItemArgs a = it;
       a.list = tier_list[tier].p;
       a.n_groups = cnt[tier];
-      a.bytes = it.bytes ? it.bytes + tier : nullptr;
+      a.bytes = it.bytes ? it.bytes + (size_t)tier * kByteWords : nullptr;
       trace_tier[rf ? (tier <= 2 ? 0 : (tier == 3 ? 1 : 2)) : (tier <= 2 ? 0 : (tier <= 4 ? 1 : 2))] += cnt[tier];
       if (rf && tier == 5) continue;  // below, after the side launches
       int grid;
-      if (tier <= 3) {
+      if (rf) {
+        grid = (int)std::min<int64_t>(rf_tier_blocks(tier, cnt[tier], it.per_group, it.spread),
+                                      tier <= 3 ? wave_grid_cap : search_grid_cap);
+      } else if (tier <= 3) {
         // node-major tiers: 4 / 2 / 1 / 1 nodes per wave
         const int npw = tier == 0 ? 4 : (tier == 1 ? 2 : 1);
         grid = (int)std::min<int64_t>((cnt[tier] + npw * kWaves - 1) / (npw * kWaves), wave_grid_cap);
-      } else if (rf && tier == 4) {
-        grid = (int)std::min<int64_t>(cnt[tier], search_grid_cap);  // one node per workgroup
       } else {
         const int64_t items = (int64_t)cnt[tier] * it.per_group;
-        const bool whole = tier == (rf ? 4 : 5);
+        const bool whole = tier == 5;
         const int per_block = whole ? 1 : kWaves;
         const int cap = whole ? search_grid_cap : wave_grid_cap;
         grid = (int)std::min<int64_t>((items + per_block - 1) / per_block, cap);
@@ -6395,7 +6593,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       ItemArgs a = it;
       a.list = tier_list[5].p;
       a.n_groups = cnt[5];
-      a.bytes = it.bytes ? it.bytes + 5 : nullptr;
+      a.bytes = it.bytes ? it.bytes + (size_t)5 * kByteWords : nullptr;
       Timer tk(search_family(algorithm, 5), 0.0, s);
       big(bigst, d, lv, a, tier_list[5].p, cnt[5], s, num_cu);
     }
@@ -6421,7 +6619,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       a.list = lst + c0;
       a.n_groups = std::min<int64_t>(kPlainChunk, it.n_groups - c0);
       a.node_major = 1;
-      a.bytes = it.bytes ? it.bytes + tier : nullptr;
+      a.bytes = it.bytes ? it.bytes + (size_t)tier * kByteWords : nullptr;
       Timer tk(search_family(algorithm, tier), 0.0, s);
       search(algorithm, tier, (int)a.n_groups, s, d, lv, a);
       DTE_HIP(hipStreamSynchronize(s));
@@ -6449,7 +6647,8 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   // memory and run on capped grids; counters are cleared by a kernel.  The
   // buffers are sized once for the largest level possible: a level has at
   // most one node per entry, and at most T * N / (min_node + 1) open nodes.
-  DevBuf<unsigned long long> graph_bytes(kMaxTiers + 1);  // search tiers, partition
+  DevBuf<unsigned long long> graph_bytes(count_bytes ? (kMaxTiers + 1) * kByteWords : 1);  // search tiers, partition
+  auto graph_counter = [&](int tier) { return count_bytes ? graph_bytes.p + (size_t)tier * kByteWords : nullptr; };
   int64_t graph_replays = 0;
   auto device_levels = [&](int depth0) {
     int64_t min1 = (int64_t)std::max(p.min_node_size, 0) + 1, W = 0;
@@ -6508,17 +6707,16 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     h.n = n_level;
     h.depth = depth0;
     DTE_HIP(hipMemcpyAsync(dlv.p, &h, sizeof(h), hipMemcpyHostToDevice, s));
-    DTE_HIP(hipMemsetAsync(graph_bytes.p, 0, graph_bytes.bytes(), s));
+    if (count_bytes) DTE_HIP(hipMemsetAsync(graph_bytes.p, 0, graph_bytes.bytes(), s));
     DevLevel* L = dlv.p;
     const bool rf = algorithm == DTE_RANDOM_FOREST;
     constexpr int kElemGrid = 1024;
-    // Extra trees on small data (at most kErtMergeEntries entries over all
+    // Extra trees on small data (at most kMergeEntries entries over all
     // trees): one launch for all search tiers of a phase.  Its levels are
     // small and latency-bound, and side by side the tiers finish sooner
     // (4,601 x 57, 100 trees: 12.3k -> 15.9k trees/s); on large data the
     // merged kernel's register budget (the largest tier's) costs more
     // occupancy than the overlap gains (64 forests: 8.2k -> 6.9k).
-    const bool small_data = E <= kErtMergeEntries;
     const bool ert_merged = !rf && small_data;
     const ErtAllFn ert_all = pick_ert_all(task, C);
     // likewise the partition tiers of a step (both algorithms)
@@ -6574,30 +6772,45 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       it.scr_aux = scr_aux.p;
       it.scr_y = scr_y.p;
       it.scr_stride = scr_stride;
+      it.spread = spread_waves;
       // split search of one phase over the tiers; nodes above cut_block
       // (tier 5) take one workgroup per item through its scratch slab
       auto phase = [&](const uint32_t* list, const unsigned int* n_dev, unsigned int* cnt, int per_group, int j0) {
-        hipLaunchKernelGGL(k_tier_split, dim3(kTierGrid), dim3(kBlock), 0, s, list, (int64_t)0,
+        hipLaunchKernelGGL(k_tier_split, dim3(kTierGrid), dim3(kTierBlock), 0, s, list, (int64_t)0,
                            (const uint32_t*)open_idx.p, (const int32_t*)o_m.p, cuts, tier_lists(), cnt, n_dev,
                            (const int64_t*)&L->off);
         if (ert_merged) {
           ErtTiers ts{};
           int64_t acc = 0;
           for (int k = 0; k < 6; ++k) {
-            ts.first[k] = acc;
-            acc += k <= 4 ? wave_grid_cap : search_grid_cap;
+            ts.cap[k] = k <= 4 ? num_cu * 6 : search_grid_cap;
+            acc += ts.cap[k];
             ts.list[k] = tier_list[k].p;
             ts.n_dev[k] = cnt + k;
-            ts.bytes[k] = graph_bytes.p + k;
+            ts.bytes[k] = graph_counter(k);
           }
-          ts.first[6] = acc;
           ItemArgs a = it;
           a.per_group = per_group;
           a.j0 = j0;
           ert_all(acc, s, d, lvd, a, ts);
           return;
         }
-        for (int tier = 0; tier < cuts.n; ++tier) {
+        if (rf && small_data) {
+          RfTiers ts{};
+          for (int tier = 0; tier < 5; ++tier) {
+            ts.cap[tier] = merged_cap(tier);
+            ts.list[tier] = tier_list[tier].p;
+            ts.n_dev[tier] = cnt + tier;
+            ts.bytes[tier] = graph_counter(tier);
+          }
+          ItemArgs a = it;
+          a.per_group = per_group;
+          a.j0 = j0;
+          int64_t blocks = 0;
+          for (int c : ts.cap) blocks += c;
+          rf_all(blocks, s, d, lvd, a, ts);
+        }
+        for (int tier = rf && small_data ? 5 : 0; tier < cuts.n; ++tier) {
           if (rf && tier == 5 && !big_tier) continue;  // no node above cut_block in these levels
           ItemArgs a = it;
           a.list = tier_list[tier].p;
@@ -6605,7 +6818,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
           a.n_dev = cnt + tier;
           a.per_group = per_group;
           a.j0 = j0;
-          a.bytes = graph_bytes.p + tier;
+          a.bytes = graph_counter(tier);
           const int grid = tier <= (rf ? 3 : 4) ? wave_grid_cap : search_grid_cap;
           search(algorithm, rf && tier == 5 ? 6 : tier, grid, s, d, lvd, a);
         }
@@ -6646,8 +6859,8 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       pa.l_sum = l_sum.p;
       pa.l_hash = l_hash.p;
       pa.split_ok = split_ok.p;
-      pa.bytes = graph_bytes.p + kMaxTiers;
-      hipLaunchKernelGGL(k_tier_split, dim3(kTierGrid), dim3(kBlock), 0, s, (const uint32_t*)nullptr, (int64_t)0,
+      pa.bytes = graph_counter(kMaxTiers);
+      hipLaunchKernelGGL(k_tier_split, dim3(kTierGrid), dim3(kTierBlock), 0, s, (const uint32_t*)nullptr, (int64_t)0,
                          (const uint32_t*)open_idx.p, (const int32_t*)o_m.p, kPartCuts, tier_lists(), L->ptier,
                          (const unsigned int*)&L->n_open, (const int64_t*)&L->off);
       PartArgs p0 = pa, p1 = pa, p2 = pa, p3 = pa;
@@ -6658,15 +6871,13 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       p3.list = tier_list[3].p;
       if (small_data) {
         PartTiers pt{};
-        const int64_t g[4] = {wave_grid_cap, wave_grid_cap, wave_grid_cap, search_grid_cap};
         int64_t acc = 0;
         for (int k = 0; k < 4; ++k) {
-          pt.first[k] = acc;
-          acc += g[k];
+          pt.cap[k] = k <= 2 ? num_cu * 8 : search_grid_cap;
+          acc += pt.cap[k];
           pt.list[k] = tier_list[k].p;
           pt.n_dev[k] = L->ptier + k;
         }
-        pt.first[4] = acc;
         pt.n_bound = NO;
         partition_all(acc, s, d, lvd, pa, pt);
       } else {
@@ -6883,11 +7094,12 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       it.res_score = res_score.p;
       it.res_thr = res_thr.p;
       it.res_feat = res_feat.p;
-      it.bytes = search_bytes.p;
+      it.bytes = tier_bytes(0);
       it.scr_key = scr_key.p;
       it.scr_aux = scr_aux.p;
       it.scr_y = scr_y.p;
       it.scr_stride = scr_stride;
+      it.spread = spread_waves;
       if (plain) plain_phase(it); else run_phase(it);
       DecideArgs da{};
       da.n_open = n_open;
@@ -6938,7 +7150,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       pa.l_sum = l_sum.p;
       pa.l_hash = l_hash.p;
       pa.split_ok = split_ok.p;
-      pa.bytes = part_bytes.p;
+      pa.bytes = part_bytes;
       if (plain) {
         const uint32_t* lst = identity_list(n_open);
         Timer tm("partition", 0.0, s);
@@ -6951,7 +7163,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       } else {
         for (auto& tl : tier_list) tl.reserve(n_open);
         DTE_HIP(hipMemsetAsync(tier_cnt.p, 0, 4 * kMaxTiers, s));
-        hipLaunchKernelGGL(k_tier_split, dim3(std::min(grid_for(n_open), kTierGrid)), dim3(kBlock), 0, s, (const uint32_t*)nullptr,
+        hipLaunchKernelGGL(k_tier_split, dim3(tier_grid(n_open)), dim3(kTierBlock), 0, s, (const uint32_t*)nullptr,
                            n_open, lv.open_idx, lv.m, kPartCutsHost, tier_lists(), tier_cnt.p, nullptr, nullptr);
         unsigned int pc[kMaxTiers];
         DTE_HIP(hipMemcpyAsync(pc, tier_cnt.p, 4 * kMaxTiers, hipMemcpyDeviceToHost, s));
@@ -7075,10 +7287,16 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     }
   }
   const int64_t n_nodes = off_level;
-  if (profiling_enabled()) {
-    unsigned long long sb[kMaxTiers];
-    DTE_HIP(hipMemcpyAsync(sb, search_bytes.p, 8 * kMaxTiers, hipMemcpyDeviceToHost, s));
-    DTE_HIP(hipStreamSynchronize(s));
+  if (count_bytes) {
+    auto totals = [&](const DevBuf<unsigned long long>& counters) {
+      std::vector<unsigned long long> w((kMaxTiers + 1) * kByteWords);
+      DTE_HIP(hipMemcpyAsync(w.data(), counters.p, w.size() * 8, hipMemcpyDeviceToHost, s));
+      DTE_HIP(hipStreamSynchronize(s));
+      std::vector<unsigned long long> t(kMaxTiers + 1, 0);
+      for (size_t x = 0; x < w.size(); x += kByteStride) t[x / kByteWords] += w[x];
+      return t;
+    };
+    const std::vector<unsigned long long> sb = totals(byte_counts);
     double total = 0;
     for (int tier = 0; tier < kMaxTiers; ++tier) {
       if (!sb[tier]) continue;
@@ -7086,11 +7304,9 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       total += (double)sb[tier];
     }
     profile_add_bytes("split_search", total);
-    profile_add_bytes("partition", (double)read_one(part_bytes.p, s));
+    profile_add_bytes("partition", (double)sb[kMaxTiers]);
     if (graph_replays) {
-      unsigned long long gb[kMaxTiers + 1];
-      DTE_HIP(hipMemcpyAsync(gb, graph_bytes.p, sizeof(gb), hipMemcpyDeviceToHost, s));
-      DTE_HIP(hipStreamSynchronize(s));
+      const std::vector<unsigned long long> gb = totals(graph_bytes);
       double g_search = 0;
       for (int tier = 0; tier < kMaxTiers; ++tier) g_search += (double)gb[tier];
       // level steps of the graphs: their split-search bytes (partition bytes
