@@ -2166,6 +2166,47 @@ __global__ void k_v2_items(DataArgs d, LevelArgs lv, const uint32_t* groups, int
   }
 }
 
+// Loads in flight for a walk over a node's entries by a team of TEAM threads:
+// f(e, in, row, aux, value, target) for e = t, t + TEAM, ... < m, in order, kWalk
+// steps' loads issued together.  One step at a time was bound by the latency
+// of its chain (row, then the value it points at, then the payload of a left
+// entry): about 1.8 us a step of a workgroup, 1.4 ms for the roots of 20
+// forests of up to 200,000 rows; 0.39 ms with eight.
+// Steps of a team that ends past m read the last entry again and come with
+// `in` false, so that f may use ballots over the whole wave.
+constexpr int kWalk = 8;
+template <int TASK, int TEAM, class F>
+__device__ __forceinline__ void walk_entries(const LevelArgs& lv, int64_t st, int m, const float* Xf, F&& f) {
+  const int t = TEAM == kWave ? (int)(threadIdx.x & (kWave - 1)) : (int)threadIdx.x;
+  const uint32_t* row = lv.row + st;
+  const uint32_t* aux = lv.aux + st;
+  const int64_t* ey = TASK == 1 ? lv.ey + st : nullptr;
+  for (int e0 = 0; e0 < m; e0 += TEAM * kWalk) {
+    uint32_t r[kWalk], a[kWalk];
+    float x[kWalk];
+    int64_t y[TASK == 1 ? kWalk : 1];
+#pragma unroll
+    for (int q = 0; q < kWalk; ++q)
+      if (e0 + q * TEAM < m) {
+        const uint32_t e = (uint32_t)min(e0 + q * TEAM + t, m - 1);
+        r[q] = row[e];
+        a[q] = aux[e];
+        if constexpr (TASK == 1) y[q] = ey[e];
+      }
+#pragma unroll
+    for (int q = 0; q < kWalk; ++q)
+      if (e0 + q * TEAM < m) x[q] = Xf[r[q]];
+#pragma unroll
+    for (int q = 0; q < kWalk; ++q)
+      if (e0 + q * TEAM < m) {
+        const int e = e0 + q * TEAM + t;
+        int64_t yq = 0;
+        if constexpr (TASK == 1) yq = y[q];
+        f(e, e < m, r[q], a[q], x[q], yq);
+      }
+  }
+}
+
 // ------------------------------------------------ ERT split search ------
 // One block per item: threshold = fp32 mean of 10 node values drawn with
 // replacement (gpuert.cu:167-183, summed in draw order), then a 2 x C
@@ -2219,21 +2260,17 @@ __device__ __forceinline__ void ert_block_body(DataArgs d, LevelArgs lv, ItemArg
     for (int c = 0; c < MAXC; ++c) loc[c] = 0;
     uint64_t nl = 0;
     int64_t sl = 0;
-    for (int e = t; e < m; e += kBlock) {
-      const uint32_t row = lv.row[st + e];
-      if (side_of(Xf[row], thr) == 0) {
-        const uint32_t a = lv.aux[st + e];
-        const uint32_t w = a & 0xFFFFu;
-        nl += w;
-        if (TASK == 0) {
-          const int lab = (int)(a >> 16);
+    walk_entries<TASK, kBlock>(lv, st, m, Xf, [&](int, bool in, uint32_t, uint32_t a, float x, int64_t y) {
+      const uint32_t w = in && side_of(x, thr) == 0 ? a & 0xFFFFu : 0u;
+      nl += w;
+      if (TASK == 0) {
+        const int lab = (int)(a >> 16);
 #pragma unroll
-          for (int c = 0; c < MAXC; ++c) loc[c] += (c == lab) ? w : 0u;
-        } else {
-          sl += (int64_t)w * lv.ey[st + e];
-        }
+        for (int c = 0; c < MAXC; ++c) loc[c] += (c == lab) ? w : 0u;
+      } else {
+        sl += (int64_t)w * y;
       }
-    }
+    });
     if (TASK == 0) {
 #pragma unroll
       for (int c = 0; c < MAXC; ++c) {
@@ -3875,15 +3912,8 @@ __device__ __forceinline__ void ert_wave_body(DataArgs d, LevelArgs lv, ItemArgs
     uint32_t lc = 0;
     int64_t nl_u = 0, nl_l = 0, sl = 0;
     bool any_loc = false;  // wave-uniform
-    for (int e0 = 0; e0 < m; e0 += kWave) {
-      const int e = e0 + lane;
-      bool left = false;
-      uint32_t a = 0;
-      if (e < m) {
-        const uint32_t row = lv.row[st + e];
-        left = side_of(Xf[row], thr) == 0;
-        if (left) a = lv.aux[st + e];
-      }
+    walk_entries<TASK, kWave>(lv, st, m, Xf, [&](int, bool in, uint32_t, uint32_t a, float x, int64_t y) {
+      const bool left = in && side_of(x, thr) == 0;
       const uint32_t w = a & 0xFFFFu;
       if (TASK == 0) {
         const int lab = (int)(a >> 16);
@@ -3905,9 +3935,9 @@ __device__ __forceinline__ void ert_wave_body(DataArgs d, LevelArgs lv, ItemArgs
         }
       } else if (left) {
         nl_l += w;
-        sl += (int64_t)w * lv.ey[st + e];
+        sl += (int64_t)w * y;
       }
-    }
+    });
     const int64_t nl = nl_u + ((TASK == 1 || any_loc) ? wave_sum_i64(nl_l) : 0);
     if (lane == 0) my_bytes += (unsigned long long)m * (TASK == 0 ? 12ull : 20ull);
     float score;
@@ -4558,8 +4588,11 @@ struct PartArgs {
 };
 
 // Side bits of the first pass kept for the scatter pass (nodes of up to
-// 64 Ki entries), which then reads no X.
+// 64 Ki entries), which then reads no X; with the left entries before each
+// word of 64 the scatter needs no scan, no barrier and no order of its own.
+// Larger nodes are scattered 64 Ki entries at a time, their sides taken again.
 constexpr int kSideWords = 1024;
+constexpr int kSideEntries = kSideWords * kWave;
 
 template <int MAXC, int TASK>
 __device__ __forceinline__ void part_block_body(DataArgs d, LevelArgs lv, PartArgs pa, int64_t bid, int64_t nblk) {
@@ -4567,6 +4600,7 @@ __device__ __forceinline__ void part_block_body(DataArgs d, LevelArgs lv, PartAr
   if (pa.n_dev) pa.n_open = *pa.n_dev;
   if ((int64_t)bid >= pa.n_open) return;
   __shared__ unsigned long long s_side[kSideWords];
+  __shared__ uint32_t s_pre[kSideWords];
   __shared__ uint32_t s_w[kWaves];
   __shared__ uint32_t s_cls[MAXC];
   __shared__ unsigned long long s_cnt, s_sum, s_hash;
@@ -4596,29 +4630,25 @@ __device__ __forceinline__ void part_block_body(DataArgs d, LevelArgs lv, PartAr
     uint64_t cnt = 0, hsh = 0;
     int64_t sm = 0;
     uint32_t ml = 0;
-    const bool keep = m <= kSideWords * kWave;
-    for (int e = t; e < m; e += kBlock) {
-      const uint32_t row = lv.row[st + e];
-      const bool isl = side_of(Xf[row], thr) == 0;
+    const bool keep = m <= kSideEntries;
+    walk_entries<TASK, kBlock>(lv, st, m, Xf, [&](int e, bool in, uint32_t row, uint32_t a, float x, int64_t y) {
+      const bool isl = in && side_of(x, thr) == 0;
       if (keep) {
         const unsigned long long bits = __ballot(isl);
-        if ((t & (kWave - 1)) == 0) s_side[e / kWave] = bits;
+        if ((t & (kWave - 1)) == 0 && in) s_side[e / kWave] = bits;
       }
-      if (isl) {
-        const uint32_t a = lv.aux[st + e];
-        const uint32_t w = a & 0xFFFFu;
-        ++ml;
-        cnt += w;
-        hsh += (uint64_t)w * mix64(row);
-        if (TASK == 0) {
-          const int lab = (int)(a >> 16);
+      const uint32_t w = isl ? a & 0xFFFFu : 0u;
+      ml += isl ? 1u : 0u;
+      cnt += w;
+      hsh += (uint64_t)w * mix64(row);
+      if (TASK == 0) {
+        const int lab = (int)(a >> 16);
 #pragma unroll
-          for (int c = 0; c < MAXC; ++c) loc[c] += (c == lab) ? w : 0u;
-        } else {
-          sm += (int64_t)w * lv.ey[st + e];
-        }
+        for (int c = 0; c < MAXC; ++c) loc[c] += (c == lab) ? w : 0u;
+      } else {
+        sm += (int64_t)w * y;
       }
-    }
+    });
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) {
       cnt += __shfl_xor(cnt, off, kWave);
@@ -4654,26 +4684,61 @@ __device__ __forceinline__ void part_block_body(DataArgs d, LevelArgs lv, PartAr
     }
     if (TASK == 0 && t < d.C) pa.l_cls[o * d.C + t] = s_cls[t];
     if (ok) {
-      // Stable scatter, tile by tile.
-      uint32_t lbase = 0, rbase = (uint32_t)mL;
-      for (int e0 = 0; e0 < m; e0 += kBlock) {
-        const int e = e0 + t;
-        uint32_t row = 0, isl = 0;
-        if (e < m) {
-          row = lv.row[st + e];
-          isl = keep ? (uint32_t)(s_side[e / kWave] >> (e & (kWave - 1))) & 1u
-                     : (side_of(Xf[row], thr) == 0 ? 1u : 0u);
+      uint32_t lbase = 0;  // left entries before the segment
+      for (int s0 = 0; s0 < m; s0 += kSideEntries) {
+        const int sm_ = min(m - s0, kSideEntries);
+        if (!keep) {
+          walk_entries<0, kBlock>(lv, st + s0, sm_, Xf, [&](int e, bool in, uint32_t, uint32_t, float x, int64_t) {
+            const unsigned long long bits = __ballot(in && side_of(x, thr) == 0);
+            if ((t & (kWave - 1)) == 0 && in) s_side[e / kWave] = bits;
+          });
+          __syncthreads();
+        }
+        const int words = (sm_ + kWave - 1) / kWave;
+        constexpr int WPT = kSideWords / kBlock;
+        uint32_t pc[WPT], mine = 0;
+#pragma unroll
+        for (int q = 0; q < WPT; ++q) {
+          const int x = t * WPT + q;
+          pc[q] = x < words ? (uint32_t)__popcll(s_side[x]) : 0u;
+          mine += pc[q];
         }
         uint32_t tot;
-        const uint32_t pl = block_excl_scan(isl, s_w, &tot);
-        if (e < m) {
-          const uint32_t pos = isl ? lbase + pl : rbase + (uint32_t)(e - e0) - pl;
-          pa.nrow[st + pos] = row;
-          pa.naux[st + pos] = lv.aux[st + e];
-          if (TASK == 1) pa.ney[st + pos] = lv.ey[st + e];
+        uint32_t before = block_excl_scan(mine, s_w, &tot);
+#pragma unroll
+        for (int q = 0; q < WPT; ++q) {
+          s_pre[t * WPT + q] = before;
+          before += pc[q];
+        }
+        __syncthreads();
+        const uint32_t rbase = (uint32_t)mL + (uint32_t)s0 - lbase;  // rights before the segment follow every left
+        for (int e0 = 0; e0 < sm_; e0 += kBlock * kWalk) {
+          uint32_t row[kWalk], aux[kWalk];
+          int64_t y[TASK == 1 ? kWalk : 1];
+#pragma unroll
+          for (int q = 0; q < kWalk; ++q)
+            if (e0 + q * kBlock < sm_) {
+              const int64_t g = st + s0 + min(e0 + q * kBlock + t, sm_ - 1);
+              row[q] = lv.row[g];
+              aux[q] = lv.aux[g];
+              if constexpr (TASK == 1) y[q] = lv.ey[g];
+            }
+#pragma unroll
+          for (int q = 0; q < kWalk; ++q) {
+            const int e = e0 + q * kBlock + t;
+            if (e < sm_) {
+              const unsigned long long bits = s_side[e / kWave];
+              const uint32_t pl = s_pre[e / kWave] + (uint32_t)__popcll(bits & ((1ull << (e & (kWave - 1))) - 1ull));
+              const bool isl = (bits >> (e & (kWave - 1))) & 1ull;
+              const uint32_t pos = isl ? lbase + pl : rbase + (uint32_t)e - pl;
+              pa.nrow[st + pos] = row[q];
+              pa.naux[st + pos] = aux[q];
+              if constexpr (TASK == 1) pa.ney[st + pos] = y[q];
+            }
+          }
         }
         lbase += tot;
-        rbase += (uint32_t)min(kBlock, m - e0) - tot;
+        __syncthreads();  // s_side, s_pre and s_w are rewritten
       }
     }
     __syncthreads();
@@ -4681,7 +4746,7 @@ __device__ __forceinline__ void part_block_body(DataArgs d, LevelArgs lv, PartAr
   if (t == 0 && my_bytes && pa.bytes) add_bytes(pa.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock) k_partition(DataArgs d, LevelArgs lv, PartArgs pa) {
+__global__ void __launch_bounds__(kBlock, 4 - TASK) k_partition(DataArgs d, LevelArgs lv, PartArgs pa) {
   part_block_body<MAXC, TASK>(d, lv, pa, blockIdx.x, gridDim.x);
 }
 
@@ -4912,29 +4977,21 @@ __device__ __forceinline__ void part_wave_body(DataArgs d, LevelArgs lv, PartArg
     uint32_t ml = 0;
     uint32_t side = 0;  // bit k: entry k * 64 + lane goes left (nodes of up to 2048 entries)
     const bool keep = m <= 32 * kWave;
-    for (int e0 = 0; e0 < m; e0 += kWave) {
-      const int e = e0 + lane;
-      bool isl = false;
-      if (e < m) {
-        const uint32_t row = lv.row[st + e];
-        isl = side_of(Xf[row], thr) == 0;
-        if (isl && keep) side |= 1u << (e0 / kWave);
-        if (isl) {
-          const uint32_t a = lv.aux[st + e];
-          const uint32_t w = a & 0xFFFFu;
-          cnt += w;
-          hsh += (uint64_t)w * mix64(row);
-          if (TASK == 0) {
-            const int lab = (int)(a >> 16);
+    walk_entries<TASK, kWave>(lv, st, m, Xf, [&](int e, bool in, uint32_t row, uint32_t a, float x, int64_t y) {
+      const bool isl = in && side_of(x, thr) == 0;
+      if (isl && keep) side |= 1u << (e / kWave);
+      const uint32_t w = isl ? a & 0xFFFFu : 0u;
+      cnt += w;
+      hsh += (uint64_t)w * mix64(row);
+      if (TASK == 0) {
+        const int lab = (int)(a >> 16);
 #pragma unroll
-            for (int c = 0; c < MAXC; ++c) loc[c] += (c == lab) ? w : 0u;
-          } else {
-            sm += (int64_t)w * lv.ey[st + e];
-          }
-        }
+        for (int c = 0; c < MAXC; ++c) loc[c] += (c == lab) ? w : 0u;
+      } else {
+        sm += (int64_t)w * y;
       }
       ml += (uint32_t)__popcll(__ballot(isl));
-    }
+    });
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) {
       cnt += __shfl_xor(cnt, off, kWave);
@@ -4962,31 +5019,42 @@ __device__ __forceinline__ void part_wave_body(DataArgs d, LevelArgs lv, PartArg
     }
     if (ok) {
       uint32_t lbase = 0, rbase = (uint32_t)mL;
-      for (int e0 = 0; e0 < m; e0 += kWave) {
-        const int e = e0 + lane;
-        uint32_t row = 0;
-        bool isl = false;
-        if (e < m) {
-          row = lv.row[st + e];
-          isl = keep ? ((side >> (e0 / kWave)) & 1u) != 0 : side_of(Xf[row], thr) == 0;
-        }
-        const uint64_t bl = __ballot(isl);
-        const uint64_t br = __ballot(e < m && !isl);
-        if (e < m) {
-          const uint32_t pos = isl ? lbase + (uint32_t)__popcll(bl & lt_mask) : rbase + (uint32_t)__popcll(br & lt_mask);
-          pa.nrow[st + pos] = row;
-          pa.naux[st + pos] = lv.aux[st + e];
-          if (TASK == 1) pa.ney[st + pos] = lv.ey[st + e];
-        }
-        lbase += (uint32_t)__popcll(bl);
-        rbase += (uint32_t)__popcll(br);
+      for (int e0 = 0; e0 < m; e0 += kWave * kWalk) {
+        uint32_t row[kWalk], aux[kWalk];
+        int64_t y[TASK == 1 ? kWalk : 1];
+#pragma unroll
+        for (int q = 0; q < kWalk; ++q)
+          if (e0 + q * kWave < m) {
+            const int64_t g = st + min(e0 + q * kWave + lane, m - 1);
+            row[q] = lv.row[g];
+            aux[q] = lv.aux[g];
+            if constexpr (TASK == 1) y[q] = lv.ey[g];
+          }
+#pragma unroll
+        for (int q = 0; q < kWalk; ++q)
+          if (e0 + q * kWave < m) {
+            const int e = e0 + q * kWave + lane;
+            bool isl = false;
+            if (e < m) isl = keep ? ((side >> (e / kWave)) & 1u) != 0 : side_of(Xf[row[q]], thr) == 0;
+            const uint64_t bl = __ballot(isl);
+            const uint64_t br = __ballot(e < m && !isl);
+            if (e < m) {
+              const uint32_t pos =
+                  isl ? lbase + (uint32_t)__popcll(bl & lt_mask) : rbase + (uint32_t)__popcll(br & lt_mask);
+              pa.nrow[st + pos] = row[q];
+              pa.naux[st + pos] = aux[q];
+              if constexpr (TASK == 1) pa.ney[st + pos] = y[q];
+            }
+            lbase += (uint32_t)__popcll(bl);
+            rbase += (uint32_t)__popcll(br);
+          }
       }
     }
   }
   if (lane == 0 && my_bytes && pa.bytes) add_bytes(pa.bytes, my_bytes);
 }
 template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock) k_partition_wave(DataArgs d, LevelArgs lv, PartArgs pa,
+__global__ void __launch_bounds__(kBlock, 5 - TASK) k_partition_wave(DataArgs d, LevelArgs lv, PartArgs pa,
                                                            const uint32_t* list, int64_t n_list) {
   part_wave_body<MAXC, TASK>(d, lv, pa, list, n_list, blockIdx.x, gridDim.x);
 }
@@ -5093,7 +5161,7 @@ struct PartTiers {
 };
 
 template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock) k_partition_all(DataArgs d, LevelArgs lv, PartArgs pa, PartTiers pt) {
+__global__ void __launch_bounds__(kBlock, 4 - TASK) k_partition_all(DataArgs d, LevelArgs lv, PartArgs pa, PartTiers pt) {
   int64_t bid = blockIdx.x, nblk = 0;
   int k = 3;
   for (;; --k) {
