@@ -97,16 +97,15 @@ __device__ __forceinline__ DataArgs forest_data(const DataArgs& d, int tree) {
 // level steps that run without a host round trip (captured in a hipGraph and
 // replayed level after level): the kernels read them at entry instead of
 // taking them as launch arguments.
-struct DevLevel {
+struct alignas(128) DevLevel {
   int64_t off;                    // level-major offset of the level
   int64_t n;                      // nodes of the level
   int64_t depth;
   unsigned int n_open;            // open nodes (total of the open-flag scan)
-  unsigned int n_retry;           // open nodes that draw retries
   unsigned int n_next;            // nodes of the next level
   unsigned int tier[kMaxTiers];   // split-search tier sizes, first phase
-  unsigned int rtier[kMaxTiers];  // the same, retry phase
   unsigned int ptier[kMaxTiers];  // partition tier sizes
+  unsigned int rtier[kMaxTiers];  // split-search tier sizes, retry phase
 };
 
 struct LevelArgs {
@@ -4391,12 +4390,9 @@ constexpr int kTierGrid = 64;
 constexpr int kTierBlock = 1024;
 __global__ void __launch_bounds__(kTierBlock) k_tier_split(const uint32_t* list, int64_t n, const uint32_t* open_idx,
                                                            const int32_t* node_m, Cuts cuts, TierLists out,
-                                                           unsigned int* counts, const unsigned int* n_dev,
-                                                           const int64_t* off_dev) {
+                                                           unsigned int* counts) {
   constexpr int NW = kTierBlock / kWave;
   __shared__ unsigned int s_cnt[NW][kMaxTiers], s_base[NW][kMaxTiers];
-  if (n_dev) n = *n_dev;            // device-described level
-  if (off_dev) node_m += *off_dev;
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = threadIdx.x / kWave;
   const int64_t wave = (int64_t)blockIdx.x * NW + wv;
@@ -4475,92 +4471,101 @@ struct DecideArgs {
   const uint32_t* retry_list;
   int64_t n_retry;
   const unsigned int* n_open_dev;   // device-described level
-  const unsigned int* n_retry_dev;
 };
 
-__global__ void k_decide1(DataArgs d, LevelArgs lv, DecideArgs a, int algorithm) {
-  resolve_level(lv, d.C);
-  if (a.n_open_dev) a.n_open = *a.n_open_dev;
-  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < a.n_open;
-       o += (int64_t)gridDim.x * blockDim.x) {
-    const float* rs = a.res_score + o * a.D;
-    const float* rt = a.res_thr + o * a.D;
-    const int32_t* rf = a.res_feat + o * a.D;
-    int D0 = a.D0, R = a.R;
-    if (d.forests) {  // joint build: the node's own forest's draws
-      const DataArgs dd = forest_data(d, lv.tree[lv.open_idx[o]]);
-      D0 = dd.D0;
-      R = dd.R;
-    }
-    float bs = rs[0], bt = rt[0];
-    int bf = rf[0];
-    for (int j = 1; j < D0; ++j)
-      if (split_better(rs[j], rf[j], rt[j], bs, bf, bt)) {
-        bs = rs[j];
-        bf = rf[j];
-        bt = rt[j];
-      }
-    uint32_t need = 0;
-    if (R > 0 && (double)bs <= 1e-3) {
-      const uint32_t i = lv.open_idx[o];
-      bool pure = false;
-      if (algorithm == 0 && d.C > 0 && lv.cls) {
-        uint32_t mx = 0;
-        for (int c = 0; c < d.C; ++c) mx = max(mx, lv.cls[(int64_t)i * d.C + c]);
-        pure = (int64_t)mx == (int64_t)lv.count[i];
-      }
-      if (pure) {
-        const uint32_t tg = (uint32_t)lv.tree_global[lv.tree[i]];
-        for (int r = 0; r < R; ++r) {
-          const int f = (int)(rand_u32(d.seed, kStreamFeat, tg, lv.id[i], (uint64_t)(D0 + r)) % (uint32_t)d.F);
-          if (split_better(0.0f, f, 0.0f, bs, bf, bt)) {
-            bs = 0.0f;
-            bf = f;
-            bt = 0.0f;
-          }
-        }
-      } else {
-        need = 1;
-      }
-    }
-    a.ch_score[o] = bs;
-    a.ch_thr[o] = bt;
-    a.ch_feat[o] = bf;
-    a.retry_flag[o] = need;
+// The best of a node's first draws into ch_*; returns whether it draws retries.
+__device__ __forceinline__ bool decide_first(const DataArgs& d, const LevelArgs& lv, const DecideArgs& a, int64_t o,
+                                             int algorithm) {
+  const float* rs = a.res_score + o * a.D;
+  const float* rt = a.res_thr + o * a.D;
+  const int32_t* rf = a.res_feat + o * a.D;
+  int D0 = a.D0, R = a.R;
+  if (d.forests) {  // joint build: the node's own forest's draws
+    const DataArgs dd = forest_data(d, lv.tree[lv.open_idx[o]]);
+    D0 = dd.D0;
+    R = dd.R;
   }
+  float bs = rs[0], bt = rt[0];
+  int bf = rf[0];
+  for (int j = 1; j < D0; ++j)
+    if (split_better(rs[j], rf[j], rt[j], bs, bf, bt)) {
+      bs = rs[j];
+      bf = rf[j];
+      bt = rt[j];
+    }
+  uint32_t need = 0;
+  if (R > 0 && (double)bs <= 1e-3) {
+    const uint32_t i = lv.open_idx[o];
+    bool pure = false;
+    if (algorithm == 0 && d.C > 0 && lv.cls) {
+      uint32_t mx = 0;
+      for (int c = 0; c < d.C; ++c) mx = max(mx, lv.cls[(int64_t)i * d.C + c]);
+      pure = (int64_t)mx == (int64_t)lv.count[i];
+    }
+    if (pure) {
+      const uint32_t tg = (uint32_t)lv.tree_global[lv.tree[i]];
+      for (int r = 0; r < R; ++r) {
+        const int f = (int)(rand_u32(d.seed, kStreamFeat, tg, lv.id[i], (uint64_t)(D0 + r)) % (uint32_t)d.F);
+        if (split_better(0.0f, f, 0.0f, bs, bf, bt)) {
+          bs = 0.0f;
+          bf = f;
+          bt = 0.0f;
+        }
+      }
+    } else {
+      need = 1;
+    }
+  }
+  a.ch_score[o] = bs;
+  a.ch_thr[o] = bt;
+  a.ch_feat[o] = bf;
+  return need != 0;
+}
+
+__global__ void k_decide1(DataArgs d, LevelArgs lv, DecideArgs a, int algorithm) {
+  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < a.n_open;
+       o += (int64_t)gridDim.x * blockDim.x)
+    a.retry_flag[o] = decide_first(d, lv, a, o, algorithm) ? 1u : 0u;
 }
 
 // Phase 2: continue the sequential retry rule on the nodes that needed it.
-__global__ void k_decide2(DataArgs d, LevelArgs lv, DecideArgs a) {
-  resolve_level(lv, d.C);
-  if (a.n_retry_dev) a.n_retry = *a.n_retry_dev;
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < a.n_retry;
-       q += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t o = a.retry_list[q];
-    float bs = a.ch_score[o], bt = a.ch_thr[o];
-    int bf = a.ch_feat[o];
-    const float* rs = a.res_score + (int64_t)o * a.D;
-    const float* rt = a.res_thr + (int64_t)o * a.D;
-    const int32_t* rf = a.res_feat + (int64_t)o * a.D;
-    int D0 = a.D0, R = a.R;
-    if (d.forests) {  // joint build: the node's own forest's draws
-      const DataArgs dd = forest_data(d, lv.tree[lv.open_idx[o]]);
-      D0 = dd.D0;
-      R = dd.R;
-    }
-    for (int r = 0; r < R; ++r) {
-      if ((double)bs > 1e-3) break;
-      const int j = D0 + r;
-      if (split_better(rs[j], rf[j], rt[j], bs, bf, bt)) {
-        bs = rs[j];
-        bf = rf[j];
-        bt = rt[j];
-      }
-    }
-    a.ch_score[o] = bs;
-    a.ch_thr[o] = bt;
-    a.ch_feat[o] = bf;
+__device__ __forceinline__ void decide_retry(const DataArgs& d, const LevelArgs& lv, const DecideArgs& a, int64_t o) {
+  float bs = a.ch_score[o], bt = a.ch_thr[o];
+  int bf = a.ch_feat[o];
+  const float* rs = a.res_score + (int64_t)o * a.D;
+  const float* rt = a.res_thr + (int64_t)o * a.D;
+  const int32_t* rf = a.res_feat + (int64_t)o * a.D;
+  int D0 = a.D0, R = a.R;
+  if (d.forests) {  // joint build: the node's own forest's draws
+    const DataArgs dd = forest_data(d, lv.tree[lv.open_idx[o]]);
+    D0 = dd.D0;
+    R = dd.R;
   }
+  for (int r = 0; r < R; ++r) {
+    if ((double)bs > 1e-3) break;
+    const int j = D0 + r;
+    if (split_better(rs[j], rf[j], rt[j], bs, bf, bt)) {
+      bs = rs[j];
+      bf = rf[j];
+      bt = rt[j];
+    }
+  }
+  a.ch_score[o] = bs;
+  a.ch_thr[o] = bt;
+  a.ch_feat[o] = bf;
+}
+
+__global__ void k_decide2(DataArgs d, LevelArgs lv, DecideArgs a) {
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < a.n_retry; q += (int64_t)gridDim.x * blockDim.x)
+    decide_retry(d, lv, a, a.retry_list[q]);
+}
+
+// The same of a device-described level, over the retry flags.
+__global__ void k_decide2_dev(DataArgs d, LevelArgs lv, DecideArgs a) {
+  resolve_level(lv, d.C);
+  const int64_t n = *a.n_open_dev;
+  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < n; o += (int64_t)gridDim.x * blockDim.x)
+    if (a.retry_flag[o]) decide_retry(d, lv, a, o);
 }
 
 // ------------------------------------------------------ partition -------
@@ -5250,72 +5255,71 @@ __device__ __forceinline__ void resolve_children(ChildArgs& a) {
   }
 }
 
+__device__ __forceinline__ uint32_t child_count(const ChildArgs& a, int64_t i) {
+  return a.open[i] && a.split_ok[a.open_pos[i]] ? 2u : 0u;
+}
+
 __global__ void k_children_count(ChildArgs a) {
-  resolve_children(a);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n_level;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    uint32_t nc = 0;
-    if (a.open[i]) {
-      const uint32_t o = a.open_pos[i];
-      nc = a.split_ok[o] ? 2u : 0u;
+       i += (int64_t)gridDim.x * blockDim.x)
+    a.nchild[i] = child_count(a, i);
+}
+
+__device__ __forceinline__ void child_write(const DataArgs& d, const ChildArgs& a, int64_t i) {
+  const int64_t gi = a.off_level + i;
+  if (a.nchild[i] == 0) {
+    a.o_feature[gi] = -1;
+    a.o_thr[gi] = -1.0f;
+    a.o_score[gi] = 0.0f;
+    a.o_left[gi] = -1;
+    return;
+  }
+  const uint32_t o = a.open_pos[i];
+  const int tr = a.o_tree[gi];
+  const DataArgs dd = forest_data(d, tr);
+  a.o_feature[gi] = a.ch_feat[o];
+  a.o_thr[gi] = a.ch_thr[o];
+  a.o_score[gi] = a.ch_score[o];
+  const uint32_t p = a.cpos[i];
+  const int64_t gl = a.off_next + p;
+  a.o_left[gi] = gl;
+  const uint32_t first = a.cpos[a.lf[tr]];
+  const uint32_t idl = a.base[tr] + (a.lf[tr + 1] - a.lf[tr]) + (p - first);
+  const int m = a.o_m[gi];
+  const int mL = a.l_m[o];
+  const int cnt = a.o_count[gi];
+  const int cL = a.l_count[o];
+  const int64_t st = a.start[i];
+  for (int s = 0; s < 2; ++s) {
+    const int64_t g = gl + s;
+    a.o_tree[g] = tr;
+    a.o_id[g] = idl + s;
+    a.o_depth[g] = a.depth + 1;
+    const int cm = s == 0 ? mL : m - mL;
+    const int cc = s == 0 ? cL : cnt - cL;
+    a.o_m[g] = cm;
+    a.o_count[g] = cc;
+    a.o_hash[g] = s == 0 ? a.l_hash[o] : a.o_hash[gi] - a.l_hash[o];
+    if (d.C > 0 && a.o_cls) {
+      for (int c = 0; c < d.C; ++c) {
+        const uint32_t lc = a.l_cls[(int64_t)o * d.C + c];
+        a.o_cls[g * d.C + c] = s == 0 ? lc : a.o_cls[gi * d.C + c] - lc;
+      }
+      a.o_value[g] = 0.0f;
+    } else {
+      const int64_t sm = s == 0 ? a.l_sum[o] : a.o_sum[gi] - a.l_sum[o];
+      a.o_sum[g] = sm;
+      a.o_value[g] = (float)ldexp_d((double)sm / (double)cc, -dd.shift);
     }
-    a.nchild[i] = nc;
+    a.n_start[p + s] = s == 0 ? st : st + mL;
+    a.n_open[p + s] = (cc > dd.min_node && a.depth + 1 < dd.max_depth) ? 1 : 0;
   }
 }
 
 __global__ void k_children_write(DataArgs d, ChildArgs a) {
-  resolve_children(a);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n_level;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t gi = a.off_level + i;
-    if (a.nchild[i] == 0) {
-      a.o_feature[gi] = -1;
-      a.o_thr[gi] = -1.0f;
-      a.o_score[gi] = 0.0f;
-      a.o_left[gi] = -1;
-      continue;
-    }
-    const uint32_t o = a.open_pos[i];
-    const int tr = a.o_tree[gi];
-    const DataArgs dd = forest_data(d, tr);
-    a.o_feature[gi] = a.ch_feat[o];
-    a.o_thr[gi] = a.ch_thr[o];
-    a.o_score[gi] = a.ch_score[o];
-    const uint32_t p = a.cpos[i];
-    const int64_t gl = a.off_next + p;
-    a.o_left[gi] = gl;
-    const uint32_t first = a.cpos[a.lf[tr]];
-    const uint32_t idl = a.base[tr] + (a.lf[tr + 1] - a.lf[tr]) + (p - first);
-    const int m = a.o_m[gi];
-    const int mL = a.l_m[o];
-    const int cnt = a.o_count[gi];
-    const int cL = a.l_count[o];
-    const int64_t st = a.start[i];
-    for (int s = 0; s < 2; ++s) {
-      const int64_t g = gl + s;
-      a.o_tree[g] = tr;
-      a.o_id[g] = idl + s;
-      a.o_depth[g] = a.depth + 1;
-      const int cm = s == 0 ? mL : m - mL;
-      const int cc = s == 0 ? cL : cnt - cL;
-      a.o_m[g] = cm;
-      a.o_count[g] = cc;
-      a.o_hash[g] = s == 0 ? a.l_hash[o] : a.o_hash[gi] - a.l_hash[o];
-      if (d.C > 0 && a.o_cls) {
-        for (int c = 0; c < d.C; ++c) {
-          const uint32_t lc = a.l_cls[(int64_t)o * d.C + c];
-          a.o_cls[g * d.C + c] = s == 0 ? lc : a.o_cls[gi * d.C + c] - lc;
-        }
-        a.o_value[g] = 0.0f;
-      } else {
-        const int64_t sm = s == 0 ? a.l_sum[o] : a.o_sum[gi] - a.l_sum[o];
-        a.o_sum[g] = sm;
-        a.o_value[g] = (float)ldexp_d((double)sm / (double)cc, -dd.shift);
-      }
-      a.n_start[p + s] = s == 0 ? st : st + mL;
-      a.n_open[p + s] = (cc > dd.min_node && a.depth + 1 < dd.max_depth) ? 1 : 0;
-    }
-  }
+       i += (int64_t)gridDim.x * blockDim.x)
+    child_write(d, a, i);
 }
 
 // Per-tree bookkeeping for the next level: first index and base id.
@@ -5538,37 +5542,17 @@ __global__ void k_finalize(FinalArgs a) {
 // Partition tiers: 16- and 32-lane segments, a wave, a workgroup per node.
 constexpr Cuts kPartCuts{{16, 32, 512, 0x7FFFFFFF, 0, 0}, 4};
 
-__global__ void k_open_list_dev(const uint8_t* open, const uint32_t* pos, const DevLevel* L, uint32_t* list) {
-  const int64_t n = L->n;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    if (open[i]) list[pos[i]] = (uint32_t)i;
-}
-
-__global__ void k_compact_list_dev(const uint32_t* flag, const uint32_t* pos, const unsigned int* n_dev,
-                                   uint32_t* list) {
-  const int64_t n = *n_dev;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    if (flag[i]) list[pos[i]] = (uint32_t)i;
-}
-
 // Exclusive scan of n u32 (n read from the device) into out[0..n], out[n] =
 // total, also stored to *total: kDScanBlocks workgroups each own a
 // contiguous range (per-range sums; then every range sums the sums before
 // it for its offset and is rescanned in tiles of kScanTile).  Two kernels:
 // a level step is a chain of short launches, each a fixed latency.
-constexpr int kDScanBlocks = 512;
+constexpr int kDScanBlocks = 256;
 
-__device__ __forceinline__ int64_t dscan_n(const int64_t* n64, const unsigned int* n32) {
-  return n64 ? *n64 : (int64_t)*n32;
-}
-
-// In: uint32_t counts, or uint8_t flags (a level's open flags, scanned as
-// they are).
-template <class In>
-__global__ void __launch_bounds__(kBlock) k_dscan_sums(const In* in, const int64_t* n64,
-                                                       const unsigned int* n32, uint32_t* sums) {
+// Sums of a level's open flags.
+__global__ void __launch_bounds__(kBlock) k_open_sums(const uint8_t* in, const DevLevel* L, uint32_t* sums) {
   __shared__ uint32_t s_w[kWaves];
-  const int64_t n = dscan_n(n64, n32);
+  const int64_t n = L->n;
   const int64_t per = (n + kDScanBlocks - 1) / kDScanBlocks;
   const int64_t lo = blockIdx.x * per, hi = min(lo + per, n);
   uint32_t acc = 0;
@@ -5578,23 +5562,41 @@ __global__ void __launch_bounds__(kBlock) k_dscan_sums(const In* in, const int64
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-template <class In>
-__global__ void __launch_bounds__(kBlock) k_dscan_apply(const In* in, const int64_t* n64,
-                                                        const unsigned int* n32, const uint32_t* sums, uint32_t* out,
-                                                        unsigned int* total) {
+// Children of the level's nodes (2 or 0, kept for the scan) and their sums.
+__global__ void __launch_bounds__(kBlock) k_child_sums(ChildArgs a, uint32_t* sums) {
   __shared__ uint32_t s_w[kWaves];
-  const int64_t n = dscan_n(n64, n32);
+  resolve_children(a);
+  const int64_t n = a.n_level;
   const int64_t per = (n + kDScanBlocks - 1) / kDScanBlocks;
   const int64_t lo = blockIdx.x * per, hi = min(lo + per, n);
+  uint32_t acc = 0;
+  for (int64_t i = lo + threadIdx.x; i < hi; i += kBlock) {
+    const uint32_t nc = child_count(a, i);
+    a.nchild[i] = nc;
+    acc += nc;
+  }
+  uint32_t tot;
+  block_excl_scan(acc, s_w, &tot);
+  if (threadIdx.x == 0) sums[blockIdx.x] = tot;
+}
+
+// Sum of the ranges before the workgroup's; the last one stores the total.
+__device__ __forceinline__ uint32_t dscan_carry(const uint32_t* sums, uint32_t* s_w, uint32_t* total, uint32_t* out_n) {
   uint32_t part = 0;
   for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) part += sums[i];
   uint32_t carry;
-  (void)block_excl_scan(part, s_w, &carry);  // sum of the ranges before this one
+  (void)block_excl_scan(part, s_w, &carry);
   if (blockIdx.x == kDScanBlocks - 1 && threadIdx.x == 0) {
     const uint32_t tot = carry + sums[blockIdx.x];
-    out[n] = tot;
-    if (total) *total = tot;
+    if (out_n) *out_n = tot;
+    *total = tot;
   }
+  return carry;
+}
+
+// Exclusive scan of in[lo, hi) from carry, handed over as f(i, in[i], prefix).
+template <class In, class F>
+__device__ __forceinline__ void dscan_range(const In* in, int64_t lo, int64_t hi, uint32_t carry, uint32_t* s_w, F&& f) {
   for (int64_t t0 = lo; t0 < hi; t0 += kScanTile) {
     uint32_t v[16];
     uint32_t sum = 0;
@@ -5609,7 +5611,7 @@ __global__ void __launch_bounds__(kBlock) k_dscan_apply(const In* in, const int6
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       const int64_t idx = t0 + (int64_t)threadIdx.x * 16 + k;
-      if (idx < hi) out[idx] = base;
+      if (idx < hi) f(idx, v[k], base);
       base += v[k];
     }
     carry += tile_tot;
@@ -5617,28 +5619,111 @@ __global__ void __launch_bounds__(kBlock) k_dscan_apply(const In* in, const int6
   }
 }
 
-// End of a level step: the next level becomes current; its counters start
-// at zero (a kernel, so that a captured step holds no memset node).
-__device__ __forceinline__ void level_advance(DevLevel* L) {
-  L->off += L->n;
-  L->n = L->n_next;
-  L->depth += 1;
-  L->n_open = 0;
-  L->n_retry = 0;
-  L->n_next = 0;
-  for (int k = 0; k < kMaxTiers; ++k) L->tier[k] = L->rtier[k] = L->ptier[k] = 0;
+__global__ void __launch_bounds__(kBlock) k_child_scan(const uint32_t* in, DevLevel* L, const uint32_t* sums,
+                                                       uint32_t* out) {
+  __shared__ uint32_t s_w[kWaves];
+  const int64_t n = L->n;
+  const int64_t per = (n + kDScanBlocks - 1) / kDScanBlocks;
+  const int64_t lo = blockIdx.x * per, hi = min(lo + per, n);
+  const uint32_t carry = dscan_carry(sums, s_w, &L->n_next, out + n);
+  __syncthreads();
+  dscan_range(in, lo, hi, carry, s_w, [&](int64_t i, uint32_t, uint32_t at) { out[i] = at; });
 }
 
-// Last kernel of a device level step: the per-tree cursors of the next level
-// (k_tree_update's work) and, by one thread, the level advance.  Nothing in
-// the kernel reads L, so the advance cannot race with the tree update.
-__global__ void k_tree_update_advance(int n_trees, const uint32_t* cpos, const uint32_t* lf, const uint32_t* base,
-                                      uint32_t* lf_next, uint32_t* base_next, DevLevel* L) {
-  const int tr = blockIdx.x * blockDim.x + threadIdx.x;
-  if (tr == 0) level_advance(L);
-  if (tr > n_trees) return;
-  lf_next[tr] = cpos[lf[tr]];
-  if (tr < n_trees) base_next[tr] = base[tr] + (lf[tr + 1] - lf[tr]);
+// A level's open nodes: their positions, their list, and the lists of the
+// search's and the partition's tiers, in one pass (four launches before, each
+// 3 to 12 us however small the level).  A workgroup takes its tiers' slots
+// with one atomic instruction (k_tier_split has the reason).
+__global__ void __launch_bounds__(kBlock) k_level_lists(const uint8_t* open, DevLevel* L, const uint32_t* sums,
+                                                        const int32_t* node_m, uint32_t* open_pos, uint32_t* open_idx,
+                                                        Cuts cuts, TierLists out, Cuts pcuts, TierLists pout) {
+  __shared__ uint32_t s_w[kWaves];
+  __shared__ unsigned int s_tier[2 * kMaxTiers];
+  const int t = threadIdx.x;
+  const int64_t n = L->n;
+  const int64_t per = (n + kDScanBlocks - 1) / kDScanBlocks;
+  const int64_t lo = blockIdx.x * per, hi = min(lo + per, n);
+  node_m += L->off;
+  if (t < 2 * kMaxTiers) s_tier[t] = 0;
+  const uint32_t carry = dscan_carry(sums, s_w, &L->n_open, nullptr);
+  __syncthreads();
+  for (int64_t i = lo + t; i < hi; i += kBlock)
+    if (open[i]) {
+      const int m = node_m[i];
+      atomicAdd(&s_tier[tier_of(m, cuts)], 1u);
+      atomicAdd(&s_tier[kMaxTiers + tier_of(m, pcuts)], 1u);
+    }
+  __syncthreads();
+  if (t < 2 * kMaxTiers) {
+    const unsigned int c = s_tier[t];
+    if (c) s_tier[t] = atomicAdd(t < kMaxTiers ? &L->tier[t] : &L->ptier[t - kMaxTiers], c);
+  }
+  __syncthreads();
+  dscan_range(open, lo, hi, carry, s_w, [&](int64_t i, uint32_t v, uint32_t at) {
+    open_pos[i] = at;
+    if (v) {
+      open_idx[at] = (uint32_t)i;
+      const int m = node_m[i];
+      const int k = tier_of(m, cuts), pk = tier_of(m, pcuts);
+      const unsigned int o = atomicAdd(&s_tier[k], 1u), po = atomicAdd(&s_tier[kMaxTiers + pk], 1u);
+      out.l[k][o] = at;
+      pout.l[pk][po] = at;
+    }
+  });
+}
+
+// k_decide1 of a device-described level, which also lists the nodes that
+// draw retries by search tier.
+constexpr int kDecideGrid = 256;
+__global__ void __launch_bounds__(kTierBlock) k_decide1_dev(DataArgs d, LevelArgs lv, DecideArgs a, int algorithm,
+                                                            Cuts cuts, TierLists out, unsigned int* counts) {
+  __shared__ unsigned int s_tier[kMaxTiers];
+  resolve_level(lv, d.C);
+  const int t = threadIdx.x;
+  const int64_t n = *a.n_open_dev;
+  const int64_t first = blockIdx.x * (int64_t)kTierBlock + t, step = (int64_t)gridDim.x * kTierBlock;
+  if (blockIdx.x * (int64_t)kTierBlock >= n) return;  // workgroup-uniform
+  if (t < kMaxTiers) s_tier[t] = 0;
+  __syncthreads();
+  for (int64_t o = first; o < n; o += step) {
+    const bool need = decide_first(d, lv, a, o, algorithm);
+    a.retry_flag[o] = need ? 1u : 0u;
+    if (need) atomicAdd(&s_tier[tier_of(lv.m[lv.open_idx[o]], cuts)], 1u);
+  }
+  __syncthreads();
+  if (t < kMaxTiers) {
+    const unsigned int c = s_tier[t];
+    if (c) s_tier[t] = atomicAdd(&counts[t], c);
+  }
+  __syncthreads();
+  for (int64_t o = first; o < n; o += step)
+    if (a.retry_flag[o]) {  // this thread's own store
+      const int k = tier_of(lv.m[lv.open_idx[o]], cuts);
+      out.l[k][atomicAdd(&s_tier[k], 1u)] = (uint32_t)o;
+    }
+}
+
+
+// Last kernel of a device level step: the children, the per-tree cursors of
+// the next level (k_tree_update's work), and by one thread the next level's
+// description with its counters at zero -- a second DevLevel, since every
+// workgroup reads the current one.
+__global__ void k_children_write_dev(DataArgs d, ChildArgs a, int n_trees, uint32_t* lf_next, uint32_t* base_next,
+                                     DevLevel* next) {
+  resolve_children(a);
+  const int64_t first = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  if (first == 0) {
+    DevLevel n{};
+    n.off = a.off_next;
+    n.n = a.lvl->n_next;
+    n.depth = a.depth + 1;
+    *next = n;
+  }
+  for (int64_t tr = first; tr <= n_trees; tr += step) {
+    lf_next[tr] = a.cpos[a.lf[tr]];
+    if (tr < n_trees) base_next[tr] = a.base[tr] + (a.lf[tr + 1] - a.lf[tr]);
+  }
+  for (int64_t i = first; i < a.n_level; i += step) child_write(d, a, i);
 }
 
 // ------------------------------------------------------ small helpers ---
@@ -6566,8 +6651,8 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   };
   const int wave_grid_cap = num_cu * 16;
   const int spread_waves = num_cu * 12;  // three waves per SIMD, the least the bounded tiers run at
-  // two rounds of workgroups at the merged kernel's three a CU
-  auto merged_cap = [num_cu](int tier) { return tier <= 3 ? num_cu * 6 : num_cu * 3; };
+  // a little over the merged kernel's three workgroups a CU
+  auto merged_cap = [num_cu](int tier) { return tier <= 3 ? num_cu * 4 : num_cu * 3; };
   const bool small_data = E <= kMergeEntries;
   const RfAllFn rf_all = pick_rf_all(task, C);
   LevelArgs lv{};
@@ -6598,7 +6683,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     for (auto& tl : tier_list) tl.reserve(it.n_groups);
     DTE_HIP(hipMemsetAsync(tier_cnt.p, 0, 4 * kMaxTiers, s));
     hipLaunchKernelGGL(k_tier_split, dim3(tier_grid(it.n_groups)), dim3(kTierBlock), 0, s, it.list, it.n_groups,
-                       lv.open_idx, lv.m, cuts, tier_lists(), tier_cnt.p, nullptr, nullptr);
+                       lv.open_idx, lv.m, cuts, tier_lists(), tier_cnt.p);
     unsigned int cnt[kMaxTiers];
     DTE_HIP(hipMemcpyAsync(cnt, tier_cnt.p, 4 * kMaxTiers, hipMemcpyDeviceToHost, s));
     DTE_HIP(hipStreamSynchronize(s));
@@ -6748,8 +6833,6 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     fit_to(ch_thr, NO);
     fit_to(ch_feat, NO);
     fit_to(retry_flag, NO);
-    fit_to(retry_pos, NO + 1);
-    fit_to(retry_list, NO + 1);
     fit_to(l_m, NO);
     fit_to(l_count, NO);
     fit_to(l_cls, task == 0 ? NO * C : 1);
@@ -6769,14 +6852,20 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       scr_stride = max_m;
     }
     DevBuf<uint32_t> dsums(kDScanBlocks);
-    DevBuf<DevLevel> dlv(1);
+    DevBuf<DevLevel> dlv(2);  // even and odd levels
+    constexpr int kPartLists = 4;
+    DevBuf<uint32_t> part_list[kPartLists];
+    TierLists part_lists{};
+    for (int k = 0; k < kPartLists; ++k) {
+      part_list[k].alloc(NO);
+      part_lists.l[k] = part_list[k].p;
+    }
     DevLevel h{};
     h.off = off_level;
     h.n = n_level;
     h.depth = depth0;
     DTE_HIP(hipMemcpyAsync(dlv.p, &h, sizeof(h), hipMemcpyHostToDevice, s));
     if (count_bytes) DTE_HIP(hipMemsetAsync(graph_bytes.p, 0, graph_bytes.bytes(), s));
-    DevLevel* L = dlv.p;
     const bool rf = algorithm == DTE_RANDOM_FOREST;
     constexpr int kElemGrid = 1024;
     // Extra trees on small data (at most kMergeEntries entries over all
@@ -6790,15 +6879,10 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     // likewise the partition tiers of a step (both algorithms)
     const PartAllFn partition_all = pick_part_all(task, C);
 
-    auto dscan = [&](const auto* in, const int64_t* n64, const unsigned int* n32, uint32_t* out,
-                     unsigned int* total) {
-      using In = std::remove_cv_t<std::remove_pointer_t<decltype(in)>>;
-      hipLaunchKernelGGL(k_dscan_sums<In>, dim3(kDScanBlocks), dim3(kBlock), 0, s, in, n64, n32, dsums.p);
-      hipLaunchKernelGGL(k_dscan_apply<In>, dim3(kDScanBlocks), dim3(kBlock), 0, s, in, n64, n32, dsums.p, out,
-                         total);
-    };
     // One level step; par = 1 swaps the ping-pong buffers.
     auto enqueue = [&](int par) {
+      DevLevel* const L = dlv.p + par;
+      DevLevel* const L_next = dlv.p + (par ^ 1);
       int64_t* cs = par ? w_start_next.p : w_start.p;
       int64_t* ns = par ? w_start.p : w_start_next.p;
       uint8_t* co = par ? w_open_next.p : w_open.p;
@@ -6813,10 +6897,12 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       uint32_t* nax = par ? cur_aux : nxt_aux;
       int64_t* cey = par ? nxt_ey : cur_ey;
       int64_t* ney = par ? cur_ey : nxt_ey;
-      // open list
-      dscan((const uint8_t*)co, &L->n, nullptr, open_pos.p, &L->n_open);
-      hipLaunchKernelGGL(k_open_list_dev, dim3(kElemGrid), dim3(kBlock), 0, s, co, open_pos.p, (const DevLevel*)L,
-                         open_idx.p);
+      // open nodes, by search and partition tier
+      hipLaunchKernelGGL(k_open_sums, dim3(kDScanBlocks), dim3(kBlock), 0, s, (const uint8_t*)co, (const DevLevel*)L,
+                         dsums.p);
+      hipLaunchKernelGGL(k_level_lists, dim3(kDScanBlocks), dim3(kBlock), 0, s, (const uint8_t*)co, L,
+                         (const uint32_t*)dsums.p, (const int32_t*)o_m.p, open_pos.p, open_idx.p, cuts, tier_lists(),
+                         kPartCuts, part_lists);
       LevelArgs lvd{};
       lvd.tree = o_tree.p;
       lvd.id = o_id.p;
@@ -6843,10 +6929,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       it.spread = spread_waves;
       // split search of one phase over the tiers; nodes above cut_block
       // (tier 5) take one workgroup per item through its scratch slab
-      auto phase = [&](const uint32_t* list, const unsigned int* n_dev, unsigned int* cnt, int per_group, int j0) {
-        hipLaunchKernelGGL(k_tier_split, dim3(kTierGrid), dim3(kTierBlock), 0, s, list, (int64_t)0,
-                           (const uint32_t*)open_idx.p, (const int32_t*)o_m.p, cuts, tier_lists(), cnt, n_dev,
-                           (const int64_t*)&L->off);
+      auto phase = [&](unsigned int* cnt, int per_group, int j0) {
         if (ert_merged) {
           ErtTiers ts{};
           int64_t acc = 0;
@@ -6891,7 +6974,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
           search(algorithm, rf && tier == 5 ? 6 : tier, grid, s, d, lvd, a);
         }
       };
-      phase(nullptr, &L->n_open, L->tier, D0, 0);
+      phase(L->tier, D0, 0);
       DecideArgs da{};
       da.D0 = D0;
       da.R = R;
@@ -6904,15 +6987,12 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       da.ch_feat = ch_feat.p;
       da.retry_flag = retry_flag.p;
       da.n_open_dev = &L->n_open;
-      hipLaunchKernelGGL(k_decide1, dim3(kElemGrid), dim3(kBlock), 0, s, d, lvd, da, algorithm);
+      // the retry phase's tier lists take the place of the first phase's
+      hipLaunchKernelGGL(k_decide1_dev, dim3(kDecideGrid), dim3(kTierBlock), 0, s, d, lvd, da, algorithm, cuts,
+                         tier_lists(), L->rtier);
       if (R > 0) {
-        dscan(retry_flag.p, nullptr, &L->n_open, retry_pos.p, &L->n_retry);
-        hipLaunchKernelGGL(k_compact_list_dev, dim3(kElemGrid), dim3(kBlock), 0, s, (const uint32_t*)retry_flag.p,
-                           (const uint32_t*)retry_pos.p, (const unsigned int*)&L->n_open, retry_list.p);
-        phase(retry_list.p, &L->n_retry, L->rtier, R, D0);
-        da.retry_list = retry_list.p;
-        da.n_retry_dev = &L->n_retry;
-        hipLaunchKernelGGL(k_decide2, dim3(kElemGrid), dim3(kBlock), 0, s, d, lvd, da);
+        phase(L->rtier, R, D0);
+        hipLaunchKernelGGL(k_decide2_dev, dim3(kElemGrid), dim3(kBlock), 0, s, d, lvd, da);
       }
       // partition
       PartArgs pa{};
@@ -6928,30 +7008,27 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       pa.l_hash = l_hash.p;
       pa.split_ok = split_ok.p;
       pa.bytes = graph_counter(kMaxTiers);
-      hipLaunchKernelGGL(k_tier_split, dim3(kTierGrid), dim3(kTierBlock), 0, s, (const uint32_t*)nullptr, (int64_t)0,
-                         (const uint32_t*)open_idx.p, (const int32_t*)o_m.p, kPartCuts, tier_lists(), L->ptier,
-                         (const unsigned int*)&L->n_open, (const int64_t*)&L->off);
       PartArgs p0 = pa, p1 = pa, p2 = pa, p3 = pa;
       p0.n_dev = L->ptier + 0;
       p1.n_dev = L->ptier + 1;
       p2.n_dev = L->ptier + 2;
       p3.n_dev = L->ptier + 3;
-      p3.list = tier_list[3].p;
+      p3.list = part_list[3].p;
       if (small_data) {
         PartTiers pt{};
         int64_t acc = 0;
         for (int k = 0; k < 4; ++k) {
           pt.cap[k] = k <= 2 ? num_cu * 8 : search_grid_cap;
           acc += pt.cap[k];
-          pt.list[k] = tier_list[k].p;
+          pt.list[k] = part_list[k].p;
           pt.n_dev[k] = L->ptier + k;
         }
         pt.n_bound = NO;
         partition_all(acc, s, d, lvd, pa, pt);
       } else {
-        partition_seg16(wave_grid_cap, s, d, lvd, p0, tier_list[0].p, NO);  // grid from the bound; count from p0.n_dev
-        partition_seg32(wave_grid_cap, s, d, lvd, p1, tier_list[1].p, NO);
-        partition_wave(wave_grid_cap, s, d, lvd, p2, tier_list[2].p, NO);
+        partition_seg16(wave_grid_cap, s, d, lvd, p0, part_list[0].p, NO);  // grid from the bound; count from p0.n_dev
+        partition_seg32(wave_grid_cap, s, d, lvd, p1, part_list[1].p, NO);
+        partition_wave(wave_grid_cap, s, d, lvd, p2, part_list[2].p, NO);
         partition(search_grid_cap, s, d, lvd, p3);
       }
       // children
@@ -6988,11 +7065,10 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       ca.start = cs;
       ca.n_start = ns;
       ca.n_open = no;
-      hipLaunchKernelGGL(k_children_count, dim3(kElemGrid), dim3(kBlock), 0, s, ca);
-      dscan(nchild.p, &L->n, nullptr, cpos.p, &L->n_next);
-      hipLaunchKernelGGL(k_children_write, dim3(kElemGrid), dim3(kBlock), 0, s, d, ca);
-      hipLaunchKernelGGL(k_tree_update_advance, dim3(grid_for(T + 1)), dim3(kBlock), 0, s, T,
-                         (const uint32_t*)cpos.p, (const uint32_t*)clf, (const uint32_t*)cbase, nlf, nbase, L);
+      hipLaunchKernelGGL(k_child_sums, dim3(kDScanBlocks), dim3(kBlock), 0, s, ca, dsums.p);
+      hipLaunchKernelGGL(k_child_scan, dim3(kDScanBlocks), dim3(kBlock), 0, s, (const uint32_t*)nchild.p, L,
+                         (const uint32_t*)dsums.p, cpos.p);
+      hipLaunchKernelGGL(k_children_write_dev, dim3(kElemGrid), dim3(kBlock), 0, s, d, ca, T, nlf, nbase, L_next);
       DTE_HIP(hipGetLastError());
     };
 
@@ -7049,7 +7125,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
           DTE_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
           for (int64_t b = 0;; ++b) {
             replay(kStepBatch);
-            DTE_HIP(hipMemcpyAsync(pin + (b & 1), &L->n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+            DTE_HIP(hipMemcpyAsync(pin + (b & 1), &dlv.p[par].n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
             DTE_HIP(hipEventRecord(ev[b & 1], s));
             if (b > 0) {
               DTE_HIP(hipEventSynchronize(ev[(b - 1) & 1]));
@@ -7069,7 +7145,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       }
     }
     int64_t fin[2];  // DevLevel.off, DevLevel.n
-    DTE_HIP(hipMemcpyAsync(fin, dlv.p, sizeof(fin), hipMemcpyDeviceToHost, s));
+    DTE_HIP(hipMemcpyAsync(fin, dlv.p + par, sizeof(fin), hipMemcpyDeviceToHost, s));
     DTE_HIP(hipStreamSynchronize(s));
     if (fin[1] != 0) fail(DTE_ERR_INTERNAL, "level graph: nodes left after the last level step");
     off_level = fin[0];
@@ -7232,7 +7308,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
         for (auto& tl : tier_list) tl.reserve(n_open);
         DTE_HIP(hipMemsetAsync(tier_cnt.p, 0, 4 * kMaxTiers, s));
         hipLaunchKernelGGL(k_tier_split, dim3(tier_grid(n_open)), dim3(kTierBlock), 0, s, (const uint32_t*)nullptr,
-                           n_open, lv.open_idx, lv.m, kPartCutsHost, tier_lists(), tier_cnt.p, nullptr, nullptr);
+                           n_open, lv.open_idx, lv.m, kPartCutsHost, tier_lists(), tier_cnt.p);
         unsigned int pc[kMaxTiers];
         DTE_HIP(hipMemcpyAsync(pc, tier_cnt.p, 4 * kMaxTiers, hipMemcpyDeviceToHost, s));
         DTE_HIP(hipStreamSynchronize(s));
