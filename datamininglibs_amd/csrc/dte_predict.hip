@@ -81,32 +81,63 @@ __global__ void __launch_bounds__(kBlock) k_cluster_count(int64_t n, int T, cons
                                                           const int32_t* __restrict__ left,
                                                           const int32_t* __restrict__ depth, uint32_t* code,
                                                           unsigned int* cnt) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t n_up = (n + kBlock - 1) / kBlock * kBlock;
-  for (int64_t g = blockIdx.x * (int64_t)kBlock + threadIdx.x; g < n_up; g += (int64_t)gridDim.x * kBlock) {
-    int key = -1;  // 4 * tree + class
-    int32_t first = 0;
-    if (g < n && feature[g] >= 0 && depth[g] % kClusterLevels == 0) {
-      first = left[g];
-      // the root's cluster has a line of its own, behind the root pair
-      if (depth[g] > 0) key = 4 * tree_of(g, T, ts) + slot_class(cluster_at(first, feature, left).n);
+  // Slots are taken kCountPer nodes a thread at a time, with one atomic
+  // instruction for the workgroup's first tree: an atomic per wave and class
+  // took 0.2 ms for 50 trees of 2.6 M nodes, whose counters share seven lines
+  // before).
+  constexpr int kCountPer = 8;
+  __shared__ unsigned int s_cnt[4], s_base[4];
+  const int t = threadIdx.x;
+  const int lane = t & (kWave - 1);
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (int64_t c0 = blockIdx.x * (int64_t)(kBlock * kCountPer); c0 < n; c0 += (int64_t)gridDim.x * (kBlock * kCountPer)) {
+    const int tree0 = tree_of(c0, T, ts);
+    const int64_t end0 = ts[tree0 + 1];
+    if (t < 4) s_cnt[t] = 0;
+    __syncthreads();
+    int cls[kCountPer];
+    int32_t first[kCountPer];
+    unsigned int at[kCountPer], run[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < kCountPer; ++q) {
+      const int64_t g = c0 + q * kBlock + t;
+      cls[q] = -1;
+      first[q] = 0;
+      if (g < n && feature[g] >= 0 && depth[g] % kClusterLevels == 0) {
+        first[q] = left[g];
+        // the root's cluster has a line of its own, behind the root pair
+        if (depth[g] > 0) cls[q] = slot_class(cluster_at(first[q], feature, left).n);
+        if (cls[q] >= 0 && g >= end0) {  // a later tree's
+          code[first[q]] = atomicAdd(&cnt[4 * (int64_t)tree_of(g, T, ts) + cls[q]], 1u) * 4u + (unsigned)cls[q];
+          cls[q] = -1;
+        }
+      }
+      at[q] = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint64_t same = __ballot(cls[q] == k);
+        if (cls[q] == k) at[q] = run[k] + (unsigned int)__popcll(same & below);
+        run[k] += (unsigned int)__popcll(same);
+      }
     }
-    uint64_t todo = __ballot(key >= 0);
-    while (todo) {
-      const int l = (int)__ffsll((unsigned long long)todo) - 1;
-      const int k = __shfl(key, l, kWave);
-      const uint64_t same = __ballot(key == k);
-      unsigned int at = 0;
-      if (lane == l) at = atomicAdd(&cnt[k], (unsigned int)__popcll(same));
-      at = __shfl(at, l, kWave);
-      if (key == k) code[first] = (at + (unsigned int)__popcll(same & ((1ull << lane) - 1ull))) * 4u + (unsigned)(k & 3);
-      todo &= ~same;
+    unsigned int wave0[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      unsigned int b = 0;
+      if (lane == 0 && run[k]) b = atomicAdd(&s_cnt[k], run[k]);
+      wave0[k] = (unsigned int)__shfl((int)b, 0, kWave);
     }
+    __syncthreads();
+    if (t < 4) s_base[t] = s_cnt[t] ? atomicAdd(&cnt[4 * (int64_t)tree0 + t], s_cnt[t]) : 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kCountPer; ++q)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (cls[q] == k) code[first[q]] = (s_base[k] + wave0[k] + at[q]) * 4u + (unsigned)k;
+    __syncthreads();  // s_cnt is cleared, s_base rewritten
   }
 }
-
-// Bases (in pairs) of the trees and of their slot classes: 8 pairs for the
-// root and its cluster, then the slots of 8, 4, 2 and 1 pairs.
 __global__ void __launch_bounds__(kBlock) k_cluster_bases(int T, const unsigned int* __restrict__ cnt,
                                                           int64_t* __restrict__ tbase,
                                                           uint32_t* __restrict__ cbase) {
@@ -388,23 +419,32 @@ constexpr uint32_t kStreamImp = 0x00706d69u;
 // (tree, range of kBagRange rows): every draw of the tree is generated, the
 // range's bits are set in LDS and written out once.
 constexpr int kBagThreads = 1024;
-constexpr int64_t kBagRange = (int64_t)1 << 20;  // rows per workgroup: 128 KB of bits
+constexpr int64_t kBagRange = (int64_t)1 << 19;  // rows per workgroup: at most 64 KB of bits
+// Workgroups beside each other on a tree's draws, so that few trees fill the
+// chip (100 trees of 200,003 rows: 0.115 ms at one workgroup a tree, 0.05 ms at five);
+// with several, each adds its bits to words that start at zero.
 __global__ void __launch_bounds__(kBagThreads) k_inbag_bits_lds(uint32_t* bits, int64_t N, int64_t words,
                                                                 int32_t tree0, uint64_t seed) {
-  __shared__ uint32_t s_bits[kBagRange / 32];
+  extern __shared__ uint32_t s_bits[];
   const int t = blockIdx.x;
   const int64_t r0 = (int64_t)blockIdx.y * kBagRange;
   const int64_t nw = (min(kBagRange, N - r0) + 31) / 32;  // words of this range
+  const int64_t per = (N + gridDim.z - 1) / gridDim.z;
+  const int64_t i0 = blockIdx.z * per, i1 = min(N, i0 + per);
   for (int64_t w = threadIdx.x; w < nw; w += kBagThreads) s_bits[w] = 0;
   __syncthreads();
   const uint32_t tg = (uint32_t)(tree0 + t);
-  for (int64_t i = threadIdx.x; i < N; i += kBagThreads) {
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += kBagThreads) {
     const int64_t r = (int64_t)(rand_u32(seed, kStreamBoot, tg, 0, (uint64_t)i) % (uint32_t)N) - r0;
     if (r >= 0 && r < kBagRange) atomicOr(&s_bits[r >> 5], 1u << (r & 31));
   }
   __syncthreads();
   uint32_t* bt = bits + (int64_t)t * words + r0 / 32;
-  for (int64_t w = threadIdx.x; w < nw; w += kBagThreads) bt[w] = s_bits[w];
+  for (int64_t w = threadIdx.x; w < nw; w += kBagThreads) {
+    const uint32_t v = s_bits[w];
+    if (gridDim.z == 1) bt[w] = v;
+    else if (v) atomicOr(&bt[w], v);
+  }
 }
 
 // Every (tree, row) pair whose row is out of the tree's bag is routed
@@ -414,59 +454,106 @@ __global__ void __launch_bounds__(kBagThreads) k_inbag_bits_lds(uint32_t* bits, 
 // Classification counts the pairs whose tree vote equals the label;
 // regression sums the squared errors of the leaf values.
 //
-// R rows staged in LDS x 512 / R tree lanes, trees [t0, t1) of the block's
-// chunk (R = 0: rows read from X, 64 x 8); the permuted feature always reads
-// its drawn row from X.
+// A block's R rows are staged in LDS (R = 0: 64 rows read from X); the
+// permuted feature always reads its drawn row from X.  The block lists the
+// pairs of its rows and kOobChunk trees that are out of the bag and deals them
+// to its threads: with a row and a share of the trees to each lane, 63 % of the
+// lanes stood idle.  Every block adds its counts once, to one of kOobSlots
+// lines: a wave's atomics on one line pass at one in about 15 ns, and 50,000 of
+// them were most of the 0.88 ms that 200,003 rows x 96 and 100 trees took
+// before; 0.51 ms now).
+constexpr int kOobChunk = 64;
+constexpr int kOobSlots = 64;
+struct alignas(128) OobSlot {
+  unsigned long long pairs, right, bad;  // bad: labels that are no class
+  double sse;
+};
+
 template <int TASK, int R, bool PACKED>
 __global__ void __launch_bounds__(kWalkThreads) k_oob(Trees tr, const float* __restrict__ X, int64_t N, int F,
                                                       const uint32_t* __restrict__ bits, int64_t words,
-                                                      const uint32_t* __restrict__ label, const float* __restrict__ y,
-                                                      int32_t tree0, uint64_t seed, int perm, int trees_per_block,
-                                                      unsigned long long* counts, double* sse) {
+                                                      const float* __restrict__ y, int n_classes, int32_t tree0,
+                                                      uint64_t seed, int perm, int trees_per_block, OobSlot* slots) {
   extern __shared__ float s_x[];  // R rows of F + 1 floats
   constexpr int RB = R ? R : 64;
-  const int lane = threadIdx.x % RB;
-  const int group = threadIdx.x / RB;
+  constexpr int NW = kWalkThreads / kWave;
+  __shared__ uint16_t s_pair[RB * kOobChunk];  // row | tree of the chunk << 6
+  __shared__ float s_y[RB];
+  __shared__ unsigned int s_n;
+  __shared__ unsigned long long s_right[NW], s_bad;
+  __shared__ double s_sse[NW];
+  const int t = threadIdx.x;
+  const int lane = t & (kWave - 1);
   const int64_t row0 = (int64_t)blockIdx.x * RB;
   const int nr = (int)min<int64_t>(RB, N - row0);
   const int t0 = blockIdx.y * trees_per_block;
   const int t1 = min(tr.T, t0 + trees_per_block);
   if (R) stage_rows<RB>(X, row0, nr, N, 0, F, s_x);
-  __syncthreads();
+  if (t < kWave) {
+    const float yr = t < nr ? y[row0 + t] : 0.0f;
+    if (t < RB) s_y[t] = yr;
+    const bool bad = TASK == 0 && t < nr && !(yr >= 0.0f && yr < (float)n_classes && truncf(yr) == yr);
+    const uint64_t b = __ballot(bad);
+    if (t == 0) s_bad = blockIdx.y == 0 ? __popcll(b) : 0;
+  }
   unsigned long long n_pairs = 0, n_ok = 0;
   double e2 = 0.0;
-  if (lane < nr) {
-    const int64_t r = row0 + lane;
-    const float* xr = R ? s_x + lane * (F + 1) : X + r;
-    const int64_t xs = R ? 1 : N;
-    const uint32_t lab = TASK == 0 ? label[r] : 0u;
-    const double yr = TASK == 1 ? (double)y[r] : 0.0;
-    for (int t = t0 + group; t < t1; t += kWalkThreads / RB) {
-      if ((bits[(int64_t)t * words + (r >> 5)] >> (r & 31)) & 1u) continue;  // in the bag
-      const uint32_t tg = (uint32_t)(tree0 + t);
-      const uint32_t leaf = walk<PACKED>(tr, t, xr, xs, [&](int f, uint32_t depth, float& x) {
+  for (int c0 = t0; c0 < t1; c0 += kOobChunk) {
+    __syncthreads();  // the last chunk's list is read no more
+    if (t == 0) s_n = 0;
+    __syncthreads();
+    const int want = min(kOobChunk, t1 - c0) * RB;
+    for (int x0 = 0; x0 < want; x0 += kWalkThreads) {
+      const int x = x0 + t, row = x % RB, tc = x / RB;
+      const int64_t r = row0 + row;
+      const bool out = x < want && row < nr &&
+                       !((bits[(int64_t)(c0 + tc) * words + (r >> 5)] >> (r & 31)) & 1u);
+      const uint64_t b = __ballot(out);
+      unsigned int at = 0;
+      if (lane == 0 && b) at = atomicAdd(&s_n, (unsigned int)__popcll(b));
+      at = (unsigned int)__shfl((int)at, 0, kWave);
+      if (out) s_pair[at + (unsigned int)__popcll(b & ((1ull << lane) - 1ull))] = (uint16_t)(row | tc << 6);
+    }
+    __syncthreads();
+    const int n = (int)s_n;
+    n_pairs += (unsigned long long)n;
+    for (int p = t; p < n; p += kWalkThreads) {
+      const int row = s_pair[p] & 63, tree = c0 + (s_pair[p] >> 6);
+      const int64_t r = row0 + row;
+      const float* xr = R ? s_x + row * (F + 1) : X + r;
+      const uint32_t tg = (uint32_t)(tree0 + tree);
+      const uint32_t leaf = walk<PACKED>(tr, tree, xr, R ? 1 : N, [&](int f, uint32_t depth, float& x) {
         if (f == perm)
           x = X[(int64_t)perm * N + rand_u32(seed, kStreamImp, tg, (uint32_t)r, depth) % (uint32_t)N];
       });
-      ++n_pairs;
       if (TASK == 0) {
-        n_ok += leaf == lab ? 1ull : 0ull;
+        n_ok += (float)leaf == s_y[row] ? 1ull : 0ull;
       } else {
-        const double e = (double)__uint_as_float(leaf) - yr;
+        const double e = (double)__uint_as_float(leaf) - (double)s_y[row];
         e2 += e * e;
       }
     }
   }
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) {
-    n_pairs += __shfl_xor(n_pairs, off, kWave);
     n_ok += __shfl_xor(n_ok, off, kWave);
     if (TASK == 1) e2 += __shfl_xor(e2, off, kWave);
   }
-  if ((threadIdx.x & (kWave - 1)) == 0 && n_pairs) {
-    atomicAdd(&counts[0], n_pairs);
-    if (TASK == 0) atomicAdd(&counts[1], n_ok);
-    else atomicAdd(sse, e2);
+  if (lane == 0) {
+    s_right[t / kWave] = n_ok;
+    s_sse[t / kWave] = e2;
+  }
+  __syncthreads();
+  if (t == 0) {
+    for (int w = 1; w < NW; ++w) {
+      n_ok += s_right[w];
+      e2 += s_sse[w];
+    }
+    OobSlot& o = slots[blockIdx.x % kOobSlots];
+    if (n_pairs) atomicAdd(&o.pairs, n_pairs);
+    if (n_ok) atomicAdd(&o.right, n_ok);
+    if (s_bad) atomicAdd(&o.bad, s_bad);
+    if (TASK == 1 && n_pairs) atomicAdd(&o.sse, e2);
   }
 }
 
@@ -595,31 +682,19 @@ void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t
                   hipStream_t s) {
   const int T = f.n_trees;
   if (T > 65535) fail(DTE_ERR_INVALID_ARGUMENT, "the out-of-bag pass handles at most 65535 trees");
+  PoolScope pool(s);
   const int64_t words = (N + 31) / 32;
-  DevBuf<uint32_t> bits((size_t)words * T);  // every word is written by k_inbag_bits_lds
-  hipLaunchKernelGGL(k_inbag_bits_lds, dim3((unsigned)T, (unsigned)((N + kBagRange - 1) / kBagRange)),
-                     dim3(kBagThreads), 0, s, bits.p, N, words, f.tree_offset, f.seed);
-  DevBuf<uint32_t> label;
-  DevBuf<float> yv;
-  if (f.task == 0) {
-    std::vector<uint32_t> lab(N);
-    for (int64_t i = 0; i < N; ++i) {
-      const int c = (int)targets[i];
-      if (c < 0 || c >= f.n_classes || (float)c != targets[i]) fail(DTE_ERR_INVALID_ARGUMENT, "class label out of range");
-      lab[i] = (uint32_t)c;
-    }
-    label.alloc(N);
-    DTE_HIP(hipMemcpyAsync(label.p, lab.data(), 4 * N, hipMemcpyHostToDevice, s));
-    DTE_HIP(hipStreamSynchronize(s));
-  } else {
-    yv.alloc(N);
-    DTE_HIP(hipMemcpyAsync(yv.p, targets, 4 * N, hipMemcpyHostToDevice, s));
-    DTE_HIP(hipStreamSynchronize(s));
-  }
-  DevBuf<unsigned long long> counts(2);
-  DevBuf<double> sse(1);
-  DTE_HIP(hipMemsetAsync(counts.p, 0, counts.bytes(), s));
-  DTE_HIP(hipMemsetAsync(sse.p, 0, sse.bytes(), s));
+  const int64_t ranges = (N + kBagRange - 1) / kBagRange;
+  DevBuf<uint32_t> bits((size_t)words * T);
+  const unsigned parts = (unsigned)std::max<int64_t>(1, std::min<int64_t>(8, 512 / (T * ranges)));
+  if (parts > 1)
+    hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(words * T)), dim3(kBlock), 0, s, bits.p, words * T);
+  hipLaunchKernelGGL(k_inbag_bits_lds, dim3((unsigned)T, (unsigned)ranges, parts), dim3(kBagThreads),
+                     4 * (std::min(N, kBagRange) + 31) / 32, s, bits.p, N, words, f.tree_offset, f.seed);
+  DevBuf<float> yv(N);
+  DTE_HIP(hipMemcpyAsync(yv.p, targets, 4 * N, hipMemcpyHostToDevice, s));
+  DevBuf<OobSlot> slots(kOobSlots);
+  DTE_HIP(hipMemsetAsync(slots.p, 0, slots.bytes(), s));
   const int R = staged_rows(f.n_features, 0, N), RB = R ? R : 64;
   const int64_t row_blocks = (N + RB - 1) / RB;
   const int chunks = tree_chunks(row_blocks, T, kWalkThreads / RB);
@@ -629,23 +704,25 @@ void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t
   with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
     constexpr int kR = decltype(r)::value;
     constexpr bool kP = decltype(packed)::value;
-    if (f.task == 0)
-      hipLaunchKernelGGL((k_oob<0, kR, kP>), grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
-                         (const uint32_t*)bits.p, words, (const uint32_t*)label.p, (const float*)nullptr,
-                         f.tree_offset, f.seed, perm, tpb, counts.p, sse.p);
-    else
-      hipLaunchKernelGGL((k_oob<1, kR, kP>), grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
-                         (const uint32_t*)bits.p, words, (const uint32_t*)nullptr, (const float*)yv.p, f.tree_offset,
-                         f.seed, perm, tpb, counts.p, sse.p);
+    auto kernel = f.task == 0 ? k_oob<0, kR, kP> : k_oob<1, kR, kP>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
+                       (const uint32_t*)bits.p, words, (const float*)yv.p, f.n_classes, f.tree_offset, f.seed, perm,
+                       tpb, slots.p);
   });
   DTE_HIP(hipGetLastError());
-  unsigned long long c[2];
-  double e = 0.0;
-  DTE_HIP(hipMemcpyAsync(c, counts.p, sizeof(c), hipMemcpyDeviceToHost, s));
-  DTE_HIP(hipMemcpyAsync(&e, sse.p, sizeof(e), hipMemcpyDeviceToHost, s));
+  std::vector<OobSlot> h(kOobSlots);
+  DTE_HIP(hipMemcpyAsync(h.data(), slots.p, sizeof(OobSlot) * kOobSlots, hipMemcpyDeviceToHost, s));
   DTE_HIP(hipStreamSynchronize(s));
-  out[0] = (double)c[0];
-  out[1] = f.task == 0 ? (double)c[1] : e;
+  unsigned long long pairs = 0, right = 0;
+  double sse = 0.0;
+  for (const OobSlot& o : h) {
+    if (o.bad) fail(DTE_ERR_INVALID_ARGUMENT, "class label out of range");
+    pairs += o.pairs;
+    right += o.right;
+    sse += o.sse;
+  }
+  out[0] = (double)pairs;
+  out[1] = f.task == 0 ? (double)right : sse;
 }
 
 // The records are made on the GPU, in the order the caller gets them, and
