@@ -144,6 +144,8 @@ struct ItemArgs {
   int64_t scr_stride;
   const unsigned int* n_dev;  // device-described level: n_groups = *n_dev
   int spread;            // waves to keep busy (node_split)
+  const uint32_t* gk;    // keys of the phase's draws by entry: draw q of entry e at gk[q * gk_stride + e]
+  int64_t gk_stride;     // (NULL: gathered from K; see k_gather_draws)
 };
 
 // Parts that a node's draws are dealt to, so that `units` teams have work: a
@@ -1074,7 +1076,14 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
 // in fp32 included, is walked.  Entry order inside a bucket does not matter:
 // the walk sorts by key and scores only boundaries between distinct keys from
 // integer prefix sums.
-constexpr int kV2Tile = 16384;   // entries per tile
+// Entries per tile: a tile of a larger node adds its whole bucket table to the
+// item's, so its size is what the merging of tables costs against the number
+// of workgroups (big_pipeline: at least kV2TileRounds a slot of the chip).
+// 8 trees of 4M rows, 21 draws, a level of few nodes: 1.62 ms at 16,384
+// entries, 1.35 at 65,536.
+constexpr int kV2Tile = 16384;
+constexpr int kV2TileMax = 65536;  // entry numbers of a tile in 16 bits (k_v2_collect)
+constexpr int kV2TileRounds = 6;
 constexpr int kXcds = 8;          // XCDs of an MI355X, one L2 each
 constexpr int kV2MaxB = 4096;    // buckets per item
 constexpr int kV2Ipt = kIpt;     // entries per lane of the bucket evaluator
@@ -1129,6 +1138,7 @@ struct V2Task {
 
 struct V2Args {
   const V2Item* items;
+  int tile;         // entries per tile
   int64_t n_items;
   const V2Tile* tiles;
   // per bucket: k_v2_hist's counts, overwritten by k_v2_bound with the totals
@@ -1149,7 +1159,7 @@ struct V2Args {
   double* res_g;
   uint32_t* res_key;
   uint32_t* res_prev;
-  uint32_t* gkey;   // keys in entry order, item-major
+  uint32_t* gkey;   // keys in entry order, item-major, or (gathered) the phase's keys by draw
   // scratch slots of the selected buckets
   uint32_t* skey;
   uint32_t* saux;
@@ -1166,7 +1176,7 @@ struct V2Args {
 // Tiles are issued feature-major and split in eighths across the XCDs (see
 // big_pipeline).  The bucket table lives in dynamic LDS: [c * nb + b] class
 // counts, or nb sums above, nb sums below, nb weights.
-template <int TASK>
+template <int TASK, bool GATHERED>  // GATHERED: gkey holds the keys already (k_gather_draws)
 __global__ void __launch_bounds__(kBlock) k_v2_hist(DataArgs d, LevelArgs lv, V2Args a) {
   extern __shared__ uint64_t s_tab[];
   const V2Tile tl = a.tiles[blockIdx.x];
@@ -1182,44 +1192,67 @@ __global__ void __launch_bounds__(kBlock) k_v2_hist(DataArgs d, LevelArgs lv, V2
   const int64_t mu = TASK == 1 ? v2_centre(it) : 0;
   __syncthreads();
   const uint32_t* Kf = d.K + (int64_t)it.f * d.N;
-  const int n = min(kV2Tile, it.m - (int)tl.e0);
+  const int n = min(a.tile, it.m - (int)tl.e0);
   const int64_t e0 = it.start + tl.e0;
   uint32_t* gkey = a.gkey + it.soff + tl.e0;
+  // Two stages ahead of the counting: the next step's payloads (and rows) are
+  // in flight, and its keys once their rows are there.  The table leaves a CU
+  // three workgroups, too few to cover a step's loads from outside the wave.
   constexpr int U = 8;
-  for (int base = 0; base < n; base += kBlock * U) {
-    uint32_t rows[U], aux[U], keys[U];
+  struct Step {
+    uint32_t rows[GATHERED ? 1 : U], aux[U], keys[U];
     int64_t y[TASK == 1 ? U : 1];
+  };
+  auto fetch = [&](int base, Step& st) {
+    if (base >= n) return;  // workgroup-uniform
 #pragma unroll
     for (int q = 0; q < U; ++q) {
-      const int e = base + t + q * kBlock;
-      if (e < n) {
-        rows[q] = lv.row[e0 + e];
-        aux[q] = lv.aux[e0 + e];
-        if (TASK == 1) y[q] = lv.ey[e0 + e];
-      }
+      const int e = min(base + t + q * kBlock, n - 1);
+      if (GATHERED) st.keys[q] = gkey[e];
+      else st.rows[q] = lv.row[e0 + e];
+      st.aux[q] = lv.aux[e0 + e];
+      if (TASK == 1) st.y[q] = lv.ey[e0 + e];
     }
+  };
+  auto gather = [&](int base, Step& st) {
+    if (GATHERED || base >= n) return;
 #pragma unroll
-    for (int q = 0; q < U; ++q)
-      if (base + t + q * kBlock < n) keys[q] = Kf[rows[q]];
+    for (int q = 0; q < U; ++q) st.keys[q] = Kf[st.rows[GATHERED ? 0 : q]];
+  };
+  auto count = [&](int base, const Step& st) {
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       const int e = base + t + q * kBlock;
       if (e < n) {
-        gkey[e] = keys[q];
-        const uint32_t b = v2_bucket(keys[q], it);
-        const uint32_t w = aux[q] & 0xFFFFu;
+        if (!GATHERED) gkey[e] = st.keys[q];
+        const uint32_t b = v2_bucket(st.keys[q], it);
+        const uint32_t w = st.aux[q] & 0xFFFFu;
         if (TASK == 0) {
-          atomicAdd(&s_cls[(aux[q] >> 16) * (uint32_t)nb + b], w);
+          atomicAdd(&s_cls[(st.aux[q] >> 16) * (uint32_t)nb + b], w);
         } else {
-          const int64_t dy = y[q] - mu;
+          const int64_t dy = st.y[q] - mu;
           atomicAdd(&s_n[b], w);
           atomicAdd(dy < 0 ? &s_neg[b] : &s_pos[b], (unsigned long long)((int64_t)w * dy));
         }
       }
     }
+  };
+  constexpr int kStep = kBlock * U;
+  Step s0, s1;
+  fetch(0, s0);
+  gather(0, s0);
+  fetch(kStep, s1);
+  for (int base = 0; base < n; base += 2 * kStep) {
+    gather(base + kStep, s1);
+    count(base, s0);
+    fetch(base + 2 * kStep, s0);
+    if (base + kStep >= n) break;
+    gather(base + 2 * kStep, s0);
+    count(base + kStep, s1);
+    fetch(base + 3 * kStep, s1);
   }
   __syncthreads();
-  const bool only = it.m <= kV2Tile;  // the item's only tile: plain stores
+  const bool only = it.m <= a.tile;  // the item's only tile: plain stores
   if (TASK == 0) {
     uint32_t* g = a.bcls + (int64_t)it.boff * d.C;
     for (int i = t; i < words; i += kBlock) {
@@ -1582,7 +1615,7 @@ __global__ void __launch_bounds__(kBlock) k_v2_collect(DataArgs d, LevelArgs lv,
   }
   if (t == 0) s_n = 0;
   __syncthreads();
-  const int n = min(kV2Tile, it.m - (int)tl.e0);
+  const int n = min(a.tile, it.m - (int)tl.e0);
   const int64_t e0 = it.start + tl.e0;
   const uint32_t* gkey = a.gkey + it.soff + tl.e0;
   const int lane = t & (kWave - 1);
@@ -2767,6 +2800,7 @@ __device__ __forceinline__ float chord_gap_f32(float a, float s) {
 struct BoundNode {
   int m;
   int64_t n;
+  int64_t start;  // first entry
   const uint32_t* row;  // the node's entries (wave-uniform bases: the loads
   const uint32_t* aux;  // take a scalar base and a 32-bit lane offset)
   const int64_t* ey;
@@ -2791,7 +2825,9 @@ __device__ __forceinline__ void for_entries(int m, F&& f) {
     if (q * TEAM < m) f(q, min(t + (uint32_t)(q * TEAM), (uint32_t)(m - 1)));
 }
 
-// Keys of a draw; kNone past the node's entries.
+// Keys of a draw; kNone past the node's entries.  Kf: the feature's keys by
+// row, or the draw's keys of the node by entry with rows = the entry numbers
+// (draw_base).
 template <int IPT, int TEAM>
 __device__ __forceinline__ void gather_keys(const uint32_t* Kf, int m, const uint32_t (&rows)[IPT],
                                             uint32_t (&key)[IPT]) {
@@ -2800,6 +2836,10 @@ __device__ __forceinline__ void gather_keys(const uint32_t* Kf, int m, const uin
     asm volatile("" : "+v"(r));  // 32-bit here: else every row is kept as a 64-bit pair
     key[q] = Kf[r];
   });
+}
+__device__ __forceinline__ const uint32_t* draw_base(const DataArgs& d, const ItemArgs& it, int f, int q,
+                                                     int64_t start) {
+  return it.gk ? it.gk + q * it.gk_stride + start : d.K + (int64_t)f * d.N;
 }
 template <int IPT, int TEAM>
 __device__ __forceinline__ void mask_keys(int m, uint32_t (&key)[IPT]) {
@@ -3194,6 +3234,7 @@ __device__ __forceinline__ bool bound_node(const DataArgs& d, const LevelArgs& l
   nd.m = __builtin_amdgcn_readfirstlane(lv.m[i]);
   nd.n = __builtin_amdgcn_readfirstlane(lv.count[i]);
   const int64_t st = lv.start[i];
+  nd.start = st;
   nd.row = lv.row + st;
   nd.aux = lv.aux + st;
   nd.ey = TASK == 1 ? lv.ey + st : nullptr;
@@ -3248,6 +3289,124 @@ __device__ __forceinline__ void bound_pure(const DataArgs& d, const ItemArgs& it
   }
 }
 
+// ------------------------------------------- all draws' keys of a level ---
+// A draw's key costs the fabric a 64-byte piece of a line per entry (rows of a
+// node lie anywhere), so a level with many draws moves 64 D bytes an entry.
+// With the keys of a row side by side (KR, rows of FS words), the entry's row
+// comes over once, whole, and its D keys are written in entry order, where
+// every search kernel reads them back streaming: 4 FS + 8 D bytes.  Taken
+// where that is at most a third, with more keys than the caches hold
+// (key_rows_pay).  Fits of 64 features in ms, without and with: 4M rows, 21
+// draws, 8 trees 175 and 141; 1M, 21, 16 trees 75 and 69; 250 k, 21 26.9 and
+// 27.5; 1M, 11 draws 51 and 50 (regression), 43 and 44 (8 classes).
+// A wave takes 64 entries of a node at a time through LDS: rows in, 16 bytes a
+// lane, and a column out per draw (an odd row stride: no bank conflicts).
+// 20 M entries, 64 features, 21 draws: 1.7 ms a level, 7 GB at 4.1 TB/s (a copy
+// runs at 4.7); the searches it feeds fell from 7.3 to 3.4 ms a level.
+constexpr int kGatherWaves = 2;
+constexpr int kGatherRun = 8;        // tiles a wave takes in a row
+constexpr int kGatherMaxFS = 112;    // 2 waves' rows in 64 KB of LDS
+constexpr int64_t kGatherMinKeys = (int64_t)32 << 20;
+
+inline bool key_rows_pay(int64_t N, int F, int draws) {
+  const int FS = (F + 15) / 16 * 16;
+  return FS <= kGatherMaxFS && draws <= kWave && N * F >= kGatherMinKeys && 64 * draws >= 3 * (4 * FS + 8 * draws);
+}
+
+// KR[row * FS + f] = K[f][row], zero above F; 64 rows a workgroup.
+__global__ void __launch_bounds__(kBlock) k_key_rows(const uint32_t* __restrict__ K, int64_t N, int F, int FS,
+                                                     uint32_t* __restrict__ KR) {
+  extern __shared__ uint32_t s_rows[];
+  const int64_t row0 = blockIdx.x * (int64_t)kWave;
+  const int nr = (int)min<int64_t>(kWave, N - row0);
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int f = threadIdx.x / kWave; f < FS; f += kWaves)
+    s_rows[lane * (FS + 1) + f] = f < F && lane < nr ? K[(int64_t)f * N + row0 + lane] : 0u;
+  __syncthreads();
+  for (int x = threadIdx.x; x < nr * FS; x += kBlock) KR[row0 * FS + x] = s_rows[x / FS * (FS + 1) + x % FS];
+}
+
+// Nodes whose draws are gathered: the lists of search tiers 2 .. 5, one after
+// the other.
+struct DrawNodes {
+  const uint32_t* list[4];
+  int64_t first[5];
+};
+__device__ __forceinline__ uint32_t draw_node(const DrawNodes& dn, int64_t q) {
+  int k = 0;
+  while (k < 3 && q >= dn.first[k + 1]) ++k;
+  return dn.list[k][q - dn.first[k]];
+}
+
+__global__ void k_draw_tiles(LevelArgs lv, DrawNodes dn, uint32_t* tiles) {
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < dn.first[4]; q += (int64_t)gridDim.x * blockDim.x)
+    tiles[q] = (uint32_t)((lv.m[lv.open_idx[draw_node(dn, q)]] + kWave - 1) / kWave);
+}
+
+__global__ void __launch_bounds__(kGatherWaves * kWave)
+    k_gather_draws(DataArgs d, LevelArgs lv, const uint32_t* __restrict__ KR, int FS, DrawNodes dn,
+                   const uint32_t* __restrict__ toff, int draws, uint32_t* __restrict__ gk, int64_t stride) {
+  extern __shared__ uint32_t s_rows[];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  uint32_t* S = s_rows + wv * kWave * (FS + 1);
+  const int64_t n = dn.first[4];
+  const int64_t total = toff[n];
+  const int lpr = FS / 4;  // 16-byte pieces of a row
+  const int sub = lane >> 4, c = lane & 15;
+  for (int64_t run = (int64_t)blockIdx.x * kGatherWaves + wv; run * kGatherRun < total;
+       run += (int64_t)gridDim.x * kGatherWaves) {
+    int64_t tile = run * kGatherRun;
+    const int64_t t1 = min(tile + kGatherRun, total);
+    int64_t q = 0, hi = n - 1;  // the last node whose first tile is at most `tile`
+    while (q < hi) {
+      const int64_t mid = (q + hi + 1) >> 1;
+      if ((int64_t)toff[mid] <= tile) q = mid;
+      else hi = mid - 1;
+    }
+    for (; tile < t1; ++q) {
+      const uint32_t o = __builtin_amdgcn_readfirstlane(draw_node(dn, q));
+      const uint32_t i = __builtin_amdgcn_readfirstlane(lv.open_idx[o]);
+      const int m = __builtin_amdgcn_readfirstlane(lv.m[i]);
+      const int64_t st = lv.start[i];
+      const uint32_t tg = (uint32_t)lv.tree_global[lv.tree[i]], nid = lv.id[i];
+      const int fl = lane < draws ? (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)lane) % (uint32_t)d.F) : 0;
+      const int64_t first = toff[q], last = min(t1, (int64_t)toff[q + 1]);
+      for (; tile < last; ++tile) {
+        const int e0 = (int)(tile - first) * kWave;
+        const int cnt = min(kWave, m - e0);
+        const int64_t at = st + e0 + min(lane, cnt - 1);
+        const uint32_t row = lv.row[at];
+        for (int c0 = 0; c0 < lpr; c0 += 16)
+          for (int i0 = 0; i0 < cnt; i0 += 32) {
+            uint4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              const uint32_t r = (uint32_t)__shfl((int)row, i0 + u * 4 + sub, kWave);
+              if (c0 + c < lpr) v[u] = *reinterpret_cast<const uint4*>(KR + (int64_t)r * FS + 4 * (c0 + c));
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+              if (c0 + c < lpr) {
+                uint32_t* w = S + (i0 + u * 4 + sub) * (FS + 1) + 4 * (c0 + c);
+                w[0] = v[u].x;
+                w[1] = v[u].y;
+                w[2] = v[u].z;
+                w[3] = v[u].w;
+              }
+          }
+        team_sync<kWave>();
+        uint32_t* out = gk + at;
+        for (int j = 0; j < draws; ++j) {
+          const uint32_t key = S[lane * (FS + 1) + __builtin_amdgcn_readlane(fl, j)];
+          if (lane < cnt) out[j * stride] = key;
+        }
+        team_sync<kWave>();
+      }
+    }
+  }
+}
+
 // Nodes of up to 64 IPT entries, one wave per node: the draws in order, the
 // next draw's key gather in flight.
 constexpr int kBoundLogB = 6;
@@ -3292,8 +3451,9 @@ __device__ __forceinline__ void rf_bound_body(DataArgs d, LevelArgs lv, ItemArgs
     const int m = nd.m;
     uint32_t rows[IPT], kn[IPT];
     BoundPay<TASK, IPT> pay;
+    const bool by_row = !it.gk;
     for_entries<IPT, kWave>(m, [&](int q, uint32_t e) {
-      rows[q] = nd.row[e];
+      rows[q] = by_row ? nd.row[e] : e;
       pay.a[q] = nd.aux[e];
       if constexpr (TASK == 1) pay.t[q] = nd.ey[e];
     });
@@ -3310,9 +3470,7 @@ __device__ __forceinline__ void rf_bound_body(DataArgs d, LevelArgs lv, ItemArgs
     for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
     double thr = bound_units<TASK>(d, nd, best_score);
     int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + j1)) % (uint32_t)d.F);
-    {
-      gather_keys<IPT, kWave>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
-    }
+    gather_keys<IPT, kWave>(draw_base(d, it, f_nx, j1, nd.start), m, rows, kn);
     for (int jj = j1; jj < it.per_group; jj += split) {
       const int j = it.j0 + jj;
       // once a retry draw passed 1e-3 the later ones are not looked at (k_decide2)
@@ -3324,7 +3482,7 @@ __device__ __forceinline__ void rf_bound_body(DataArgs d, LevelArgs lv, ItemArgs
       mask_keys<IPT, kWave>(m, key);
       if (jj + split < it.per_group) {
         f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + split)) % (uint32_t)d.F);
-        gather_keys<IPT, kWave>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
+        gather_keys<IPT, kWave>(draw_base(d, it, f_nx, jj + split, nd.start), m, rows, kn);
       }
       DrawBest best;
       bound_draw<MAXC, TASK, LOGB, IPT>(d, nd, s_tf, L, key, pay, thr, best);
@@ -3420,9 +3578,10 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
     const int m = nd.m;
     uint32_t rows[IPT], kn[IPT];
     BoundPay<TASK, IPT> pay;
+    const bool by_row = !it.gk;
     auto entries = [&](auto&& f) { for_entries<IPT, kBlock>(m, f); };
     entries([&](int q, uint32_t e) {
-      rows[q] = nd.row[e];
+      rows[q] = by_row ? nd.row[e] : e;
       pay.a[q] = nd.aux[e];
       if constexpr (TASK == 1) pay.t[q] = nd.ey[e];
     });
@@ -3441,9 +3600,7 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
     for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
     double thr = bound_units<TASK>(d, nd, best_score);
     int f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(it.j0 + j1)) % (uint32_t)d.F);
-    {
-      gather_keys<IPT, kBlock>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
-    }
+    gather_keys<IPT, kBlock>(draw_base(d, it, f_nx, j1, nd.start), m, rows, kn);
     for (int jj = j1; jj < it.per_group; jj += split) {
       const int j = it.j0 + jj;
       if (it.j0 > 0 && (double)best_score > 1e-3) break;
@@ -3454,7 +3611,7 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
       mask_keys<IPT, kBlock>(m, key);
       if (jj + split < it.per_group) {
         f_nx = (int)(rand_u32(d.seed, kStreamFeat, tg, nid, (uint64_t)(j + split)) % (uint32_t)d.F);
-        gather_keys<IPT, kBlock>(d.K + (int64_t)f_nx * d.N, m, rows, kn);
+        gather_keys<IPT, kBlock>(draw_base(d, it, f_nx, jj + split, nd.start), m, rows, kn);
       }
       uint32_t kmin = kNone, kmax = 0;
       entries([&](int q, uint32_t) {
@@ -5954,7 +6111,7 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
     while (k1 < n_all && (k1 == k0 || slots + B.host_items[k1].n_w <= kV2Batch)) {
       V2Item& bi = B.host_items[k1];
       bi.boff = (int32_t)nb;
-      bi.soff = el;
+      bi.soff = it.gk ? (k1 % it.per_group) * it.gk_stride + bi.start : el;
       el += bi.m;
       slots += bi.n_w;
       nb += bi.nb;
@@ -5962,6 +6119,8 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
       ++k1;
     }
     const int64_t n_items = k1 - k0;
+    const int tile = (int)std::min<int64_t>(
+        kV2TileMax, std::max<int64_t>(kV2Tile, el / ((int64_t)num_cu * 3 * kV2TileRounds) / kBlock * kBlock));
     // Tiles feature-major: the tiles in flight gather from a few feature
     // columns of K at a time instead of from all of them, so the columns stay
     // in the caches.  The results do not depend on the tile order (counts,
@@ -5971,9 +6130,19 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
     for (int f = 0; f < d.F; ++f) B.host_fcount[(size_t)f + 1] += B.host_fcount[(size_t)f];
     B.host_forder.resize((size_t)n_items);
     for (int64_t k = k0; k < k1; ++k) B.host_forder[B.host_fcount[(size_t)B.host_items[k].f]++] = (uint32_t)(k - k0);
-    for (const uint32_t li : B.host_forder)
-      for (int e0 = 0; e0 < B.host_items[k0 + li].m; e0 += kV2Tile)
-        B.host_forder_tiles.push_back(V2Tile{li, (uint32_t)e0});
+    if (it.gk) {
+      // keys gathered already: a node's draws side by side, which read the
+      // same payloads
+      for (int64_t g0 = k0, g1; g0 < k1; g0 = g1) {
+        for (g1 = g0 + 1; g1 < k1 && B.host_items[g1].grp == B.host_items[g0].grp;) ++g1;
+        for (int e0 = 0; e0 < B.host_items[g0].m; e0 += tile)
+          for (int64_t k = g0; k < g1; ++k) B.host_forder_tiles.push_back(V2Tile{(uint32_t)(k - k0), (uint32_t)e0});
+      }
+    } else {
+      for (const uint32_t li : B.host_forder)
+        for (int e0 = 0; e0 < B.host_items[k0 + li].m; e0 += tile)
+          B.host_forder_tiles.push_back(V2Tile{li, (uint32_t)e0});
+    }
     {
       // Workgroups go to the 8 XCDs round robin (workgroup w to XCD w % 8),
       // each XCD with its own L2: XCD x takes the x-th eighth of the
@@ -6030,6 +6199,7 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
     V2Args a{};
     a.items = B.items.p;
     a.n_items = n_items;
+    a.tile = tile;
     a.tiles = B.htiles.p;
     a.bcls = B.bcls.p;
     a.bn = B.bn.p;
@@ -6049,7 +6219,7 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
     a.res_g = B.res_g.p;
     a.res_key = B.res_key.p;
     a.res_prev = B.res_prev.p;
-    a.gkey = B.skey2.p;
+    a.gkey = it.gk ? const_cast<uint32_t*>(it.gk) : B.skey2.p;
     a.skey = B.skey.p;
     a.saux = B.saux.p;
     a.sy = B.sy.p;
@@ -6065,7 +6235,7 @@ void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const Ite
       // Algorithmic bytes of the batch's items (12 B per entry, 20 B for
       // regression) belong to the kernel that reads every entry.
       Timer tm("chunk_hist", profiling_enabled() ? (double)el * (TASK == 0 ? 12.0 : 20.0) : 0.0, s);
-      hipLaunchKernelGGL(k_v2_hist<TASK>, tiles, dim3(kBlock), (unsigned)(4 * bucket_words * nb_max), s, d, lv, a);
+      hipLaunchKernelGGL((it.gk ? k_v2_hist<TASK, true> : k_v2_hist<TASK, false>), tiles, dim3(kBlock), (unsigned)(4 * bucket_words * nb_max), s, d, lv, a);
     }
     {
       Timer tm("chunk_bound", 0.0, s);
@@ -6679,6 +6849,22 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       }
     }
   } side;
+  // Keys of a level's first draws by entry (k_gather_draws), if they pay and
+  // leave half of the free memory.
+  const int FS = (d.F + 15) / 16 * 16;
+  DevBuf<uint32_t> key_rows, draw_keys, draw_tiles, draw_toff;
+  bool use_rows = algorithm == DTE_RANDOM_FOREST && !plain && key_rows_pay(d.N, d.F, D0);
+  if (use_rows) {
+    size_t free_b = 0, total_b = 0;
+    DTE_HIP(hipMemGetInfo(&free_b, &total_b));
+    use_rows = 4 * ((size_t)d.N * FS + (size_t)E * D0) <= free_b / 2;
+  }
+  if (use_rows) {
+    key_rows.alloc((size_t)d.N * FS);
+    draw_keys.alloc((size_t)E * D0);
+    hipLaunchKernelGGL(k_key_rows, dim3((unsigned)((d.N + kWave - 1) / kWave)), dim3(kBlock),
+                       (unsigned)(4 * kWave * (FS + 1)), s, d.K, d.N, d.F, FS, key_rows.p);
+  }
   auto run_phase = [&](ItemArgs it) {
     for (auto& tl : tier_list) tl.reserve(it.n_groups);
     DTE_HIP(hipMemsetAsync(tier_cnt.p, 0, 4 * kMaxTiers, s));
@@ -6694,6 +6880,24 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     // tiers touch other nodes and run beside it on a side stream.
     bool others = false;
     for (int tier = 0; tier < 5; ++tier) others = others || cnt[tier] > 0;
+    if (use_rows && it.j0 == 0 && cnt[2] + cnt[3] + cnt[4] + cnt[5] > 0) {
+      Timer tk("gather_draws", 0.0, s);
+      DrawNodes dn{};
+      for (int k = 0; k < 4; ++k) {
+        dn.list[k] = tier_list[2 + k].p;
+        dn.first[k + 1] = dn.first[k] + cnt[2 + k];
+      }
+      const int64_t n = dn.first[4];
+      draw_tiles.reserve(n + 1);
+      draw_toff.reserve(n + 1);
+      hipLaunchKernelGGL(k_draw_tiles, dim3(grid_for(n)), dim3(kBlock), 0, s, lv, dn, draw_tiles.p);
+      scan_u32(draw_tiles.p, n, draw_toff.p, s, scan_tmp);
+      hipLaunchKernelGGL(k_gather_draws, dim3((unsigned)num_cu * 16), dim3(kGatherWaves * kWave),
+                         (unsigned)(4 * kGatherWaves * kWave * (FS + 1)), s, d, lv, (const uint32_t*)key_rows.p, FS, dn,
+                         (const uint32_t*)draw_toff.p, it.per_group, draw_keys.p, E);
+      it.gk = draw_keys.p;
+      it.gk_stride = E;
+    }
     const bool overlap = rf && cnt[5] > 0 && others;
     hipStream_t ts = s;
     if (overlap) {
