@@ -6485,6 +6485,27 @@ void prepare_data(FitData& fd, const float* X_dev_in, const float* y_host, int64
   }
 }
 
+// The arrays of a forest of n_nodes nodes in one allocation, with room for its
+// predict records if max_tree, the nodes of its largest tree, is given.
+void take_forest(Forest& f, int64_t max_tree) {
+  const size_t n = (size_t)f.n_nodes, trees = (size_t)f.n_trees + 1;
+  const size_t cls = f.task == 0 ? n * f.n_classes : 1;
+  f.slab.alloc(Forest::slab_bytes(8 * trees) + 8 * Forest::slab_bytes(4 * n) + 2 * Forest::slab_bytes(8 * n) +
+               Forest::slab_bytes(4 * cls) + (max_tree ? predict_slab_bytes(f, max_tree) : 0));
+  f.take(f.tree_start, trees);
+  f.take(f.feature, n);
+  f.take(f.left, n);
+  f.take(f.depth, n);
+  f.take(f.count, n);
+  f.take(f.n_entries, n);
+  f.take(f.threshold, n);
+  f.take(f.score, n);
+  f.take(f.value, n);
+  f.take(f.rowhash, n);
+  f.take(f.sum_fixed, n);
+  f.take(f.class_counts, cls);
+}
+
 // A joint build of several extra-trees forests (dte_fit_many): the trees of
 // forest f are batch trees [t0, t0 + T) of one build whose level steps serve
 // every forest at once.
@@ -7689,20 +7710,10 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   fo->n_nodes = n_nodes;
   fo->n_leaves = (n_nodes + T) / 2;  // per tree: nodes = 2 splits + 1, leaves = splits + 1
   fo->has_stats = true;
-  PoolSuspend own;  // the forest outlives the fit
-  fo->tree_start.alloc(T + 1);
+  std::unique_ptr<PoolSuspend> own;  // the forest outlives the fit, unless it is merged or sliced
+  if (whole) own = std::make_unique<PoolSuspend>();
+  take_forest(*fo, whole ? *std::max_element(per_tree.begin(), per_tree.end()) : 0);
   DTE_HIP(hipMemcpyAsync(fo->tree_start.p, ts.data(), 8 * (T + 1), hipMemcpyHostToDevice, s));
-  fo->feature.alloc(n_nodes);
-  fo->left.alloc(n_nodes);
-  fo->depth.alloc(n_nodes);
-  fo->count.alloc(n_nodes);
-  fo->n_entries.alloc(n_nodes);
-  fo->threshold.alloc(n_nodes);
-  fo->score.alloc(n_nodes);
-  fo->value.alloc(n_nodes);
-  fo->rowhash.alloc(n_nodes);
-  fo->class_counts.alloc(task == 0 ? (size_t)n_nodes * C : 1);
-  fo->sum_fixed.alloc(n_nodes);
   FinalArgs fa{};
   fa.n_nodes = n_nodes;
   fa.C = C;
@@ -7767,18 +7778,9 @@ Forest* merge_forests(std::vector<std::unique_ptr<Forest>>& parts, hipStream_t s
   const int C = fo->n_classes;
   const size_t W = fo->task == 0 ? (size_t)C : 1;
   PoolSuspend own;  // the forest outlives the fit
-  fo->tree_start.alloc(T + 1);
-  fo->feature.alloc(n);
-  fo->left.alloc(n);
-  fo->depth.alloc(n);
-  fo->count.alloc(n);
-  fo->n_entries.alloc(n);
-  fo->threshold.alloc(n);
-  fo->score.alloc(n);
-  fo->value.alloc(n);
-  fo->rowhash.alloc(n);
-  fo->class_counts.alloc(fo->task == 0 ? (size_t)n * C : 1);
-  fo->sum_fixed.alloc(n);
+  int64_t largest = 1;  // a bound of its largest tree
+  for (auto& q : parts) largest = std::max(largest, q->n_nodes);
+  take_forest(*fo, largest);
   int64_t off = 0;
   int t_off = 0;
   for (auto& q : parts) {
@@ -7947,19 +7949,8 @@ std::vector<Forest*> fit_joint(const float* const* X, const float* const* y, con
       tsf[q] = ts[jf.t0 + q] - off;
       if (q) max_tree = std::max(max_tree, tsf[q] - tsf[q - 1]);
     }
-    fo->tree_start.alloc(jf.T + 1);
+    take_forest(*fo, max_tree);
     DTE_HIP(hipMemcpyAsync(fo->tree_start.p, tsf.data(), 8 * (size_t)(jf.T + 1), hipMemcpyHostToDevice, s));
-    fo->feature.alloc(nn);
-    fo->left.alloc(nn);
-    fo->depth.alloc(nn);
-    fo->count.alloc(nn);
-    fo->n_entries.alloc(nn);
-    fo->threshold.alloc(nn);
-    fo->score.alloc(nn);
-    fo->value.alloc(nn);
-    fo->rowhash.alloc(nn);
-    fo->class_counts.alloc(task == 0 ? (size_t)nn * Cf : 1);
-    fo->sum_fixed.alloc(nn);
     SliceArgs sa{off, nn, all->n_classes, task == 0 ? Cf : 0,
                  all->feature.p, all->left.p, all->depth.p, all->count.p, all->n_entries.p,
                  all->threshold.p, all->score.p, all->value.p, all->rowhash.p,

@@ -811,20 +811,36 @@ void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld,
 
 // Predict records of a forest (its canonical arrays are complete on stream
 // s).  max_tree: nodes of its largest tree.
+namespace {
+// Feature bits of the packed records' links, or 0: wide records.
+int packed_feature_bits(const Forest& f, int64_t max_tree) {
+  int fbits = 1;
+  while (((int64_t)1 << fbits) <= (int64_t)f.n_features) ++fbits;  // feature + 1, 0 for a leaf
+  // slots of a tree: a cluster of s pairs takes at most 1.6 s of them
+  const int64_t slots = 8 + (max_tree / 2) * 8 / 5 + 8;
+  int pbits = 1;
+  while (((int64_t)1 << pbits) <= slots) ++pbits;
+  return fbits + pbits > 32 ? 0 : fbits;
+}
+size_t packed_pairs(const Forest& f) { return (size_t)16 * f.n_trees + (size_t)((f.n_nodes + 1) / 2) * 8 / 5; }
+}  // namespace
+
+size_t predict_slab_bytes(const Forest& f, int64_t max_tree) {
+  if (!packed_feature_bits(f, max_tree)) return Forest::slab_bytes(sizeof(PNode) * (size_t)f.n_nodes);
+  return Forest::slab_bytes(sizeof(PPair) * packed_pairs(f)) + Forest::slab_bytes(sizeof(int64_t) * (size_t)f.n_trees);
+}
+
 void build_predict_nodes(Forest& f, int64_t max_tree, hipStream_t s) {
   const int64_t n = f.n_nodes;
   const int T = f.n_trees;
   const uint32_t* cls = f.task == 0 ? f.class_counts.p : nullptr;
   const unsigned grid = (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 16384);
-  int fbits = 1;
-  while (((int64_t)1 << fbits) <= (int64_t)f.n_features) ++fbits;  // feature + 1, 0 for a leaf
-  // slots of a tree: a cluster of s pairs takes at most 1.6 s of them
-  auto slots = [](int64_t nodes) { return 8 + (nodes / 2) * 8 / 5 + 8; };
-  int pbits = 1;
-  while (((int64_t)1 << pbits) <= slots(max_tree)) ++pbits;
-  if (fbits + pbits > 32) {
-    PoolSuspend own;
-    f.pnodes.alloc(n);
+  const int fbits = packed_feature_bits(f, max_tree);
+  if (!fbits) {
+    {
+      PoolSuspend own;  // kept with the forest
+      f.take(f.pnodes, n);
+    }
     hipLaunchKernelGGL(k_wide_nodes, dim3(grid), dim3(kBlock), 0, s, n, f.n_classes, f.task, f.feature.p,
                        f.threshold.p, f.left.p, cls, f.value.p, f.pnodes.p);
     DTE_HIP(hipGetLastError());
@@ -832,8 +848,8 @@ void build_predict_nodes(Forest& f, int64_t max_tree, hipStream_t s) {
   }
   {
     PoolSuspend own;  // kept with the forest
-    f.pairs.alloc((size_t)16 * T + (size_t)((n + 1) / 2) * 8 / 5);
-    f.pair_base.alloc(T);
+    f.take(f.pairs, packed_pairs(f));
+    f.take(f.pair_base, T);
   }
   f.pair_fbits = fbits;
   PoolScope pool(s);
