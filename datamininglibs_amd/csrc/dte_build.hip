@@ -2508,23 +2508,66 @@ __global__ void __launch_bounds__(kBlock) k_search_rf_wave(DataArgs d, LevelArgs
 // per SEG-lane segment (one entry per lane, m <= SEG, C <= SEG), and loops
 // over the node's draws, so node statistics and entry loads are shared by
 // all draws.  Shuffles, scans and reductions stay inside the segment.
+// Scans and sums of a 16- or 32-lane segment in DPP moves (a shuffle goes
+// through the LDS pipe).  All lanes of a segment are active together.
 template <int SEG>
-__device__ __forceinline__ int64_t seg_excl_i64(int64_t v) {
-  const int sl = threadIdx.x & (SEG - 1);
-  int64_t x = v;
-#pragma unroll
-  for (int off = 1; off < SEG; off <<= 1) {
-    const int64_t y = __shfl_up(x, off, SEG);
-    if (sl >= off) x += y;
-  }
-  return x - v;
+__device__ __forceinline__ uint32_t seg_incl_u32(uint32_t x) {
+  static_assert(SEG == 16 || SEG == 32, "");
+  x += dpp_u32<0x111>(x, 0u);
+  x += dpp_u32<0x112>(x, 0u);
+  x += dpp_u32<0x114>(x, 0u);
+  x += dpp_u32<0x118>(x, 0u);
+  if constexpr (SEG == 32) x += dpp_u32<0x142, 0xa>(x, 0u);
+  return x;
+}
+template <int SEG>
+__device__ __forceinline__ int64_t seg_incl_i64(int64_t x) {
+  static_assert(SEG == 16 || SEG == 32, "");
+  x += dpp_i64<0x111>(x);
+  x += dpp_i64<0x112>(x);
+  x += dpp_i64<0x114>(x);
+  x += dpp_i64<0x118>(x);
+  if constexpr (SEG == 32) x += dpp_i64<0x142, 0xa>(x);
+  return x;
 }
 
 template <int SEG>
 __device__ __forceinline__ int64_t seg_sum_i64(int64_t v) {
-#pragma unroll
-  for (int off = SEG / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, SEG);
-  return v;
+  if constexpr (SEG == kWave) {
+    return wave_sum_i64(v);
+  } else {
+    v += dpp_i64<0x128>(v);  // row_ror: every lane gets the row's sum
+    v += dpp_i64<0x124>(v);
+    v += dpp_i64<0x122>(v);
+    v += dpp_i64<0x121>(v);
+    if constexpr (SEG == 32) v += __shfl_xor(v, 16, 32);
+    return v;
+  }
+}
+
+// f(r, value of lane r of this lane's row of 16), r = 0 .. 15.
+template <class F, int... R>
+__device__ __forceinline__ void row_lanes_impl(uint32_t v, F&& f, std::integer_sequence<int, R...>) {
+  (f(R, dpp_u32<0x150 + R>(v, 0u)), ...);
+}
+template <class F>
+__device__ __forceinline__ void row_lanes(uint32_t v, F&& f) {
+  row_lanes_impl(v, f, std::make_integer_sequence<int, 16>{});
+}
+
+// Rank of a lane's key among its segment's, ties by lane.
+template <int SEG>
+__device__ __forceinline__ uint32_t seg_rank(uint32_t key) {
+  const int rl = threadIdx.x & 15;
+  uint32_t cnt = 0;
+  const uint32_t next = key + 1u;
+  row_lanes(key, [&](int r, uint32_t k) { cnt += k < (r < rl ? next : key) ? 1u : 0u; });
+  if constexpr (SEG == 32) {  // the other row's lanes all come before or after
+    const uint32_t other = (uint32_t)__shfl_xor((int)key, 16, 32);
+    const uint32_t lim = (threadIdx.x & 16) ? next : key;
+    row_lanes(other, [&](int, uint32_t k) { cnt += k < lim ? 1u : 0u; });
+  }
+  return cnt;
 }
 
 template <int SEG>
@@ -2534,20 +2577,23 @@ __device__ __forceinline__ uint32_t seg_max_u32(uint32_t v) {
   return v;
 }
 
+// Largest positive gain of a segment whose lanes are in key order, the lowest
+// key among equals (positive doubles order as their bits).
 template <int SEG>
-__device__ __forceinline__ BestCand seg_best(BestCand b) {
-#pragma unroll
-  for (int off = SEG / 2; off > 0; off >>= 1) {
-    const double g = __shfl_xor(b.g, off, SEG);
-    const uint32_t k = __shfl_xor(b.key, off, SEG);
-    const uint32_t p = __shfl_xor(b.prev, off, SEG);
-    if (cand_better(g, k, b.g, b.key)) {
-      b.g = g;
-      b.key = k;
-      b.prev = p;
-    }
-  }
-  return b;
+__device__ __forceinline__ BestCand seg_best(double gain, uint32_t key, uint32_t prev) {
+  const int64_t g = __builtin_bit_cast(int64_t, gain > 0.0 ? gain : 0.0);
+  int64_t b = g;
+  auto take = [&](int64_t o) { b = o > b ? o : b; };
+  take(dpp_i64<0x128>(b));
+  take(dpp_i64<0x124>(b));
+  take(dpp_i64<0x122>(b));
+  take(dpp_i64<0x121>(b));
+  if constexpr (SEG == 32) take(__shfl_xor(b, 16, 32));
+  const int base = threadIdx.x & (kWave - 1) & ~(SEG - 1);
+  const uint64_t win = (__ballot(b > 0 && g == b) >> base) & ((1ull << SEG) - 1ull);
+  const int w = win ? (int)__ffsll((unsigned long long)win) - 1 : 0;
+  const uint32_t k = (uint32_t)__shfl((int)key, w, SEG), p = (uint32_t)__shfl((int)prev, w, SEG);
+  return win ? BestCand{__builtin_bit_cast(double, b), k, p} : BestCand{0.0, kNone, kNone};
 }
 
 template <int TASK>
@@ -2648,13 +2694,9 @@ __device__ __forceinline__ void rf_seg_body(DataArgs d, LevelArgs lv, ItemArgs i
         key_nx = valid ? d.K[(int64_t)f_nx * d.N + row] : kNone;
         svo_nx = d.SVoff[f_nx];
       }
-      // rank inside the segment (ties by lane), then move entries into key order
-      uint32_t cnt = 0;
-#pragma unroll
-      for (int r = 0; r < SEG; ++r) {
-        const uint32_t kr = __shfl(key, r, SEG);
-        cnt += (r < m && (kr < key || (kr == key && r < sl))) ? 1u : 0u;
-      }
+      // rank inside the segment (ties by lane; lanes past m hold kNone), then
+      // move entries into key order
+      const uint32_t cnt = seg_rank<SEG>(key);
       const uint32_t rank = valid ? cnt : (uint32_t)sl;
       const uint32_t dst = (uint32_t)(threadIdx.x & (kWave - 1) & ~(SEG - 1)) + rank;
       key = ds_permute_u32(dst, key);
@@ -2666,37 +2708,36 @@ __device__ __forceinline__ void rf_seg_body(DataArgs d, LevelArgs lv, ItemArgs i
         yv = (int64_t)(((uint64_t)hi << 32) | lo);
       }
       const uint32_t w = valid ? (pay & 0xFFFFu) : 0u;
-      const uint32_t prevk = __shfl_up(key, 1, SEG);
+      const uint32_t prevk = (uint32_t)__shfl_up((int)key, 1, SEG);
       const bool cand = valid && sl >= 1 && prevk < key;
       double gval = 0.0;
+      const uint32_t nl = seg_incl_u32<SEG>(w) - w;
       if (TASK == 0) {
+        // class weights before the entry: two classes to a word, each word
+        // scanned, and the entry's half picked
         const uint32_t lab = pay >> 16;
-        uint32_t pre = 0;
+        const uint32_t wv2 = (lab & 1u) ? w << 16 : w;
+        uint32_t mine = 0;
+        constexpr int PAIRS = (MAXC + 1) / 2;
 #pragma unroll
-        for (int r = 0; r < SEG; ++r) {
-          const uint32_t pr = __shfl(pay, r, SEG);
-          pre += (r < sl && (pr >> 16) == lab) ? (pr & 0xFFFFu) : 0u;
-        }
-        const uint32_t ncl = __shfl(ncls_lane, (int)lab, SEG);
-        int64_t dl = 0, dr = 0;
-        if (valid) {
-          dl = lx.t(pre + w) - lx.t(pre);
-          dr = lx.t(ncl - pre - w) - lx.t(ncl - pre);
-        }
-        const int64_t slv = seg_excl_i64<SEG>(dl);
-        const int64_t srv = SR0 + seg_excl_i64<SEG>(dr);
-        const int64_t nl = seg_excl_i64<SEG>((int64_t)w);
-        if (cand) {
-          const int64_t q = (slv - lx.t((uint64_t)nl)) + (srv - lx.t((uint64_t)(n - nl)));
-          gval = ig_from_fixed(P + q, lx.F, inv);
-        }
+        for (int p = 0; p < PAIRS; ++p)
+          if (2 * p < d.C) {
+            const bool own = (lab >> 1) == (uint32_t)p;
+            const uint32_t x = seg_incl_u32<SEG>(own ? wv2 : 0u);
+            if (own) mine = x;
+          }
+        const uint32_t pre = ((lab & 1u) ? mine >> 16 : mine & 0xFFFFu) - w;
+        const uint32_t ncl = (uint32_t)__shfl((int)ncls_lane, (int)lab, SEG);
+        int64_t dt = 0;  // left and right terms move together
+        if (valid) dt = (S.T[pre + w] - S.T[pre]) + (S.T[ncl - pre - w] - S.T[ncl - pre]);
+        const int64_t q = SR0 + (seg_incl_i64<SEG>(dt) - dt);
+        if (cand) gval = ig_from_fixed(P + (q - S.T[nl] - S.T[(uint32_t)n - nl]), lx.F, inv);
       } else {
-        const int64_t pn = seg_excl_i64<SEG>((int64_t)w);
-        const int64_t ps = seg_excl_i64<SEG>((int64_t)w * yv);
-        if (cand) gval = variance_gain(pn, ps, n - pn, ssum - ps, 0);
+        const int64_t wy = (int64_t)w * yv;
+        const int64_t ps = seg_incl_i64<SEG>(wy) - wy;
+        if (cand) gval = variance_gain((int64_t)nl, ps, n - (int64_t)nl, ssum - ps, 0);
       }
-      BestCand b = (cand && gval > 0.0) ? BestCand{gval, key, prevk} : BestCand{0.0, kNone, kNone};
-      b = seg_best<SEG>(b);
+      const BestCand b = seg_best<SEG>(cand ? gval : 0.0, key, prevk);
       if (pend) {
         it.res_score[p_ridx] = p_score;
         it.res_thr[p_ridx] = p_has ? midpoint(p_lo, p_hi) : 0.0f;
@@ -6824,8 +6865,12 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   bigst.max_dev = fd.max_fixed;
   Cuts cuts{};
   if (algorithm == DTE_RANDOM_FOREST) {
-    const int c16 = (task == 1 || C <= 16) ? 16 : 0;
-    const int c32 = (task == 1 || C <= 32) ? 32 : 0;
+    // the segment tiers take x ln x terms from the table's head in LDS: a node
+    // of 32 entries must weigh less than it (a multiplicity of 64 hardly ever
+    // occurs in a bootstrap; such a fit starts at the wave tier)
+    const bool light = task == 1 || 32 * (int64_t)w_max < SegLds<0>::kTL;
+    const int c16 = light && (task == 1 || C <= 16) ? 16 : 0;
+    const int c32 = light ? 32 : 0;
     cuts = Cuts{{c16, std::max(c16, c32), std::min(64, cut_team), cut_team, cut_block, 0x7FFFFFFF}, 6};
   } else {
     // segment tiers need a lane per class
