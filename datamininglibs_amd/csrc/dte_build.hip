@@ -2377,16 +2377,17 @@ __device__ __forceinline__ uint32_t ds_permute_u32(uint32_t dst_lane, uint32_t v
 
 __device__ __forceinline__ int64_t wave_excl_i64(int64_t v) { return wave_incl_scan_i64(v) - v; }
 
-__device__ __forceinline__ int64_t wave_sum_i64(int64_t v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
-}
+// All lanes active.
+__device__ __forceinline__ int64_t wave_sum_i64(int64_t v) { return wave_last_i64(wave_incl_scan_i64(v)); }
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor(v, off, kWave));
-  return v;
+  v = max(v, dpp_u32<0x111>(v, 0u));
+  v = max(v, dpp_u32<0x112>(v, 0u));
+  v = max(v, dpp_u32<0x114>(v, 0u));
+  v = max(v, dpp_u32<0x118>(v, 0u));
+  v = max(v, dpp_u32<0x142, 0xa>(v, 0u));
+  v = max(v, dpp_u32<0x143, 0xc>(v, 0u));
+  return wave_last(v);
 }
 
 
@@ -4097,7 +4098,7 @@ __device__ __forceinline__ void ert_wave_body(DataArgs d, LevelArgs lv, ItemArgs
       xs = Xf[lv.row[st + pos]];
     }
     float acc = 0.0f;
-    for (int s = 0; s < 10; ++s) acc = acc + __shfl(xs, s, kWave);
+    for (int s = 0; s < 10; ++s) acc = acc + __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(xs), s));
     const float thr = acc / 10.0f;
     // Left-side counts.  Extra-trees entries weigh 1 (every row once), so a
     // chunk's class counts are popcounts of ballots: lane c accumulates
@@ -4161,8 +4162,8 @@ __device__ __forceinline__ void ert_wave_body(DataArgs d, LevelArgs lv, ItemArgs
         tr = xlnx_fixed(nc - lc, F, s_inv, s_logc);
       }
       const int64_t P = xlnx_fixed((uint64_t)n, F, s_inv, s_logc) - wave_sum_i64(tn);
-      const int64_t Q = (wave_sum_i64(tl) - xlnx_fixed((uint64_t)nl, F, s_inv, s_logc)) +
-                        (wave_sum_i64(tr) - xlnx_fixed((uint64_t)(n - nl), F, s_inv, s_logc));
+      const int64_t Q = wave_sum_i64(tl + tr) - xlnx_fixed((uint64_t)nl, F, s_inv, s_logc) -
+                        xlnx_fixed((uint64_t)(n - nl), F, s_inv, s_logc);
       score = (float)ig_from_fixed(P + Q, F, inv);
     } else {
       sl = wave_sum_i64(sl);
@@ -4254,15 +4255,17 @@ __device__ __forceinline__ void ert_seg_body(DataArgs d, LevelArgs lv, ItemArgs 
     }
     const uint32_t mm = m > 0 ? (uint32_t)m : 1u;
     // The gathers of draw j (< 0: none): the drawn feature, this lane's
-    // threshold sample (lanes sl < 10) and its entry's value.
+    // threshold sample (the first 10 lanes of every row of 16, so that the rows
+    // of a segment each sum them) and its entry's value.
+    const int rl = lane & 15;
     auto gather = [&](int j, int& f, float& xs, float& xe) {
       const uint32_t jj = j >= 0 ? (uint32_t)j : 0u;
       f = (int)(rand_u32(dd.seed, kStreamFeat, tg, nid, (uint64_t)jj) % (uint32_t)dd.F);
       const uint32_t pos =
-          rand_u32(dd.seed, kStreamThr, tg, nid, (uint64_t)jj * 10 + (uint32_t)(sl < 10 ? sl : 0)) % mm;
+          rand_u32(dd.seed, kStreamThr, tg, nid, (uint64_t)jj * 10 + (uint32_t)(rl < 10 ? rl : 0)) % mm;
       const uint32_t rp = (uint32_t)__shfl((int)row, base + (int)pos, kWave);
       const float* Xf = dd.X + (int64_t)f * dd.N;
-      xs = (j >= 0 && node_ok && sl < 10) ? Xf[rp] : 0.0f;
+      xs = (j >= 0 && node_ok && rl < 10) ? Xf[rp] : 0.0f;
       xe = (j >= 0 && valid) ? Xf[row] : 0.0f;
     };
     auto draw_of = [&](int q) { return (node_ok && q < it.per_group) ? item_draw(d, dd, it, q) : -1; };
@@ -4275,7 +4278,9 @@ __device__ __forceinline__ void ert_seg_body(DataArgs d, LevelArgs lv, ItemArgs 
       float xs_n = 0.0f, xe_n = 0.0f;
       if (q + 1 < it.per_group) gather(j_n, f_n, xs_n, xe_n);
       float acc = 0.0f;
-      for (int s = 0; s < 10; ++s) acc = acc + __shfl(xs_c, base + s, kWave);
+      row_lanes(__float_as_uint(xs_c), [&](int s, uint32_t x) {
+        if (s < 10) acc = acc + __uint_as_float(x);
+      });
       const float thr = acc / 10.0f;
       const bool left = valid && j_c >= 0 && side_of(xe_c, thr) == 0;
       int64_t nl, sls = 0;
@@ -4306,8 +4311,8 @@ __device__ __forceinline__ void ert_seg_body(DataArgs d, LevelArgs lv, ItemArgs 
           tl = xlnx_fixed(lc, F, s_inv, s_logc);
           tr = xlnx_fixed(nc - lc, F, s_inv, s_logc);
         }
-        const int64_t Q = (seg_sum_i64<SEG>(tl) - xlnx_fixed((uint64_t)nl, F, s_inv, s_logc)) +
-                          (seg_sum_i64<SEG>(tr) - xlnx_fixed((uint64_t)(n - nl), F, s_inv, s_logc));
+        const int64_t Q = seg_sum_i64<SEG>(tl + tr) - xlnx_fixed((uint64_t)nl, F, s_inv, s_logc) -
+                          xlnx_fixed((uint64_t)(n - nl), F, s_inv, s_logc);
         score = (float)ig_from_fixed(P + Q, F, inv);
       } else {
         score = (float)variance_gain(nl, sls, n - nl, ssum - sls, dd.shift);
@@ -4421,7 +4426,7 @@ __device__ __forceinline__ void ert_team_body(DataArgs d, LevelArgs lv, ItemArgs
       if (qd + 1 < it.per_group) gather(j_n, f_n, xs_n, xe_n);
       if (j_c >= 0) {  // wave-uniform
         float acc = 0.0f;
-        for (int s2 = 0; s2 < 10; ++s2) acc = acc + __shfl(xs_c, s2, kWave);
+        for (int s2 = 0; s2 < 10; ++s2) acc = acc + __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(xs_c), s2));
         const float thr = acc / 10.0f;
         bool left[IPT];
 #pragma unroll
@@ -4469,8 +4474,8 @@ __device__ __forceinline__ void ert_team_body(DataArgs d, LevelArgs lv, ItemArgs
             tl = xlnx_fixed(lc, F, s_inv, s_logc);
             tr = xlnx_fixed(nc - lc, F, s_inv, s_logc);
           }
-          const int64_t Q = (wave_sum_i64(tl) - xlnx_fixed((uint64_t)nl, F, s_inv, s_logc)) +
-                            (wave_sum_i64(tr) - xlnx_fixed((uint64_t)(n - nl), F, s_inv, s_logc));
+          const int64_t Q = wave_sum_i64(tl + tr) - xlnx_fixed((uint64_t)nl, F, s_inv, s_logc) -
+                            xlnx_fixed((uint64_t)(n - nl), F, s_inv, s_logc);
           score = (float)ig_from_fixed(P + Q, F, inv);
         } else {
           score = (float)variance_gain(nl, sls, n - nl, ssum - sls, dd.shift);
@@ -5636,7 +5641,9 @@ __global__ void __launch_bounds__(kBlock) k_boot_compact(const uint32_t* mult, c
   }
   wm = wave_max_u32(wm);
   if ((threadIdx.x & (kWave - 1)) == 0) {
-    atomicMax(w_max, wm);
+    // one word for all waves: an atomic each, one after the other, was most of
+    // 87 us for 100 trees of 4,601 rows; few raise the maximum
+    if (wm > __hip_atomic_load(w_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(w_max, wm);
     atomicAdd((unsigned long long*)&root_hash[tr], (unsigned long long)hsh);
     if (yfix) atomicAdd((unsigned long long*)&root_sum[tr], (unsigned long long)sm);
   }

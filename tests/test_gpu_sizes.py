@@ -1,0 +1,213 @@
+"""HIP kernels at the sizes where their tiers, tiles and staging change, bit
+for bit against the CPU oracle (or a plain walk of the model)."""
+import numpy as np
+import pytest
+
+from datamininglibs_amd import capi, synth
+import pyoracle
+from parity import assert_same_forest, fit_both
+
+pytestmark = pytest.mark.gpu
+
+RF, ERT = capi.RANDOM_FOREST, capi.EXTRA_TREES
+
+
+def _targets(kind, X, rng):
+    n = X.shape[1]
+    if kind == "reg":
+        return dict(task=capi.REGRESSION), (np.sin(4 * X[0]) + X[1] * X[2] + 0.1 * rng.standard_normal(n))
+    c = int(kind)
+    s = X[:3].sum(0) + 0.4 * rng.standard_normal(n)
+    return dict(n_classes=c), np.clip(np.argsort(np.argsort(s)) * c // n, 0, c - 1)
+
+
+@pytest.mark.parametrize("kind", ["2", "9", "16", "32", "reg"])
+@pytest.mark.parametrize("n", [26, 51, 101, 811, 3241])
+def test_rf_tiers_around_their_limits(kind, n):
+    """Bootstraps of these row counts hold about 16, 32, 64, 512 and 2048
+    distinct rows, on both sides of each tier's limit over 12 trees; the last
+    one has nodes above the workgroup tier inside the level graphs."""
+    rng = np.random.default_rng(n)
+    X = rng.random((9, n)).astype(np.float32)
+    X[6:] = np.floor(X[6:] * [[3], [8], [40]])  # ties
+    kw, y = _targets(kind, X, rng)
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, n_trees=12, k=4, min_node_size=1, seed=n, **kw)
+    assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("kind", ["3", "reg"])
+def test_rf_keys_in_clusters(kind):
+    """Features that follow one another: below the first splits a node's keys
+    fill a sliver of the feature's range, or two ends of it."""
+    rng = np.random.default_rng(5)
+    n = 2600
+    X = np.empty((6, n), np.float32)
+    X[0] = rng.random(n)
+    X[1] = X[0] + 1e-4 * rng.random(n)
+    X[2] = X[0] ** 9
+    X[3] = np.where(rng.random(n) < 0.5, X[0], 100 - X[0])
+    X[4] = np.floor(X[0] * 30)
+    X[5] = np.where(rng.random(n) < 0.97, 0, rng.random(n))
+    kw, y = _targets(kind, X, rng)
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, n_trees=10, k=3, min_node_size=1, **kw)
+    assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("target", ["constant", "zero_one", "offset", "spike"])
+def test_rf_regression_targets_of_little_variance(target):
+    """Gains of exactly or nearly nothing: rounding decides, and retries run."""
+    rng = np.random.default_rng(8)
+    n = 5000
+    X = rng.random((6, n)).astype(np.float32)
+    X[3:] = X[3:] < 0.1
+    y = {"constant": np.full(n, 5.25), "zero_one": rng.integers(0, 2, n),
+         "offset": 1e6 + 1e-2 * rng.standard_normal(n), "spike": (np.arange(n) == 7) * 1e3}[target]
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, task=capi.REGRESSION, n_trees=4, k=2)
+    assert_same_forest(g, o)
+
+
+def test_rf_retries_on_sparse_features():
+    rng = np.random.default_rng(9)
+    X = (rng.random((40, 3000)) < 0.004).astype(np.float32)
+    X[0] = rng.random(3000)
+    y = (rng.random(3000) < 0.02).astype(np.float32)
+    g, o = fit_both(X, y, algorithm=RF, n_trees=6, k=2, min_node_size=1)
+    assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("kind", ["4", "24", "reg"])
+def test_rf_chunk_pipeline_tiles_and_single_key_buckets(kind):
+    """Roots of two tiles; features of fewer values than buckets (a bucket a
+    key) beside continuous ones."""
+    rng = np.random.default_rng(13)
+    n = 45_000
+    X = rng.random((6, n)).astype(np.float32)
+    X[3] = np.floor(X[3] * 2)
+    X[4] = np.floor(X[4] * 300)
+    X[5] = np.floor(X[5] ** 4 * 3000)
+    kw, y = _targets(kind, X, rng)
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, n_trees=2, k=3, max_depth=9, **kw)
+    assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("kind,n,f,k", [("5", 2_100_011, 16, 6), ("reg", 1_770_001, 19, 10)])
+def test_rf_keys_gathered_by_row(kind, n, f, k):
+    """Large enough for the row-major keys; deep enough for every tier that
+    reads the gathered keys."""
+    rng = np.random.default_rng(17)
+    X = rng.random((f, n), dtype=np.float32)
+    X[3] = np.floor(X[3] * 7)
+    kw, y = _targets(kind, X, rng)
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, n_trees=1, k=k, max_depth=15, **kw)
+    assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("task", [capi.CLASSIFICATION, capi.REGRESSION])
+@pytest.mark.parametrize("n", [255, 2049, 65_536, 65_537, 140_001])
+def test_ert_nodes_around_the_walk_and_side_words(task, n):
+    """Extra trees' roots hold every row: one step of a wave's or workgroup's
+    walk more or less, and one or several spans of the partition's side words."""
+    if task == capi.REGRESSION:
+        X, y = synth.sine_regression(seed=n, n=n, f=6)
+    else:
+        X, y = synth.gaussian_classes(seed=n, n=n, f=6, n_informative=4, n_classes=3)
+    g, o = fit_both(X, y, algorithm=ERT, task=task, n_trees=2, k=3, max_depth=6, n_classes=3)
+    assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("task", [capi.CLASSIFICATION, capi.REGRESSION])
+@pytest.mark.parametrize("depth", [1, 2, 12])
+def test_export_equals_the_canonical_arrays(task, depth):
+    """Roots first, then each tree's other nodes in order; leaves' payloads in
+    node order.  Depth 1: trees of a single node."""
+    if task == capi.REGRESSION:
+        X, y = synth.sine_regression(seed=3, n=900, f=5)
+    else:
+        X, y = synth.gaussian_classes(seed=3, n=900, f=5, n_informative=4, n_classes=3)
+    p = capi.default_params(RF, task=task, n_trees=7, n_features_per_node=2, max_depth=depth,
+                            n_classes=0 if task else 3, seed=2)
+    g = capi.fit(X, y, p)
+    c = g.canonical()
+    nodes, probs = g.export()
+    ts = c["tree_start"]
+    order = np.concatenate([ts[:-1]] + [np.arange(a + 1, b) for a, b in zip(ts[:-1], ts[1:])])
+    where = np.empty(g.n_nodes, np.int64)
+    where[order] = np.arange(g.n_nodes)
+    inner = c["feature"][order] >= 0
+    assert np.array_equal(nodes["attribute"][inner], c["feature"][order][inner])
+    assert np.array_equal(nodes["split_point"][inner], c["threshold"][order][inner])
+    assert np.array_equal(nodes["child_start"][inner], where[c["left"][order][inner]])
+    assert np.array_equal(nodes["child_count"], np.where(inner, 2, 0))
+    leaf = order[~inner]
+    width = 1 if task else 3
+    assert np.array_equal(nodes["probability_start"][~inner], width * np.arange(leaf.size))
+    if task:
+        assert np.array_equal(probs, c["value"][leaf])
+    else:
+        counts = c["class_counts"].reshape(-1, 3)[leaf].astype(np.float64)
+        want = counts / counts.sum(1, keepdims=True)
+        # one division in fp32: half a unit in the last place of a value <= 1
+        assert np.abs(probs.reshape(-1, 3) - want).max() <= 2.0 ** -24
+
+
+@pytest.mark.parametrize("task", [capi.CLASSIFICATION, capi.REGRESSION])
+@pytest.mark.parametrize("rows", [1, 2, 3, 16, 17, 64, 128, 129, 1001])
+def test_predict_row_counts(task, rows):
+    """Both sides of every change of rows per block, and a ragged last block;
+    the call without allocations takes the same kernels."""
+    if task == capi.REGRESSION:
+        X, y = synth.sine_regression(seed=4, n=1500, f=7)
+        Xp, _ = synth.sine_regression(seed=5, n=rows, f=7)
+    else:
+        X, y = synth.gaussian_classes(seed=4, n=1500, f=7, n_informative=4, n_classes=5)
+        Xp, _ = synth.gaussian_classes(seed=5, n=rows, f=7, n_informative=4, n_classes=5)
+    g, o = fit_both(X, y, algorithm=RF, task=task, n_trees=70, k=2, max_depth=14, min_node_size=1, n_classes=5)
+    want = o.predict(Xp)
+    got = g.predict(Xp), g.predict_noalloc(Xp)
+    for v in got:
+        assert np.array_equal(np.asarray(v, np.float64), np.asarray(want, np.float64))
+
+
+def test_predict_with_wide_records():
+    """A feature number and a pair number that do not fit 32 bits together."""
+    rng = np.random.default_rng(6)
+    f, depth, rows = 1 << 22, 9, 5
+    n = 2 ** (depth + 1) - 1
+    nodes = np.zeros(n, capi.NODE_DTYPE)
+    inner = np.arange(n) < n // 2
+    nodes["child_start"] = np.where(inner, 2 * np.arange(n) + 1, -1)
+    nodes["child_count"] = np.where(inner, 2, 0)
+    nodes["attribute"] = np.where(inner, rng.integers(0, f, n), -1)
+    nodes["attribute"][0] = f - 1
+    nodes["split_point"] = np.where(inner, 0.5, -1).astype(np.float32)
+    nodes["probability_start"] = np.where(inner, -1, np.arange(n) - n // 2)
+    value = rng.standard_normal(n - n // 2).astype(np.float32)
+    g = capi.import_forest(nodes, value, 1, 1, f, capi.REGRESSION)
+    X = rng.random((f, rows), dtype=np.float32)
+    got = g.predict(X)
+    for r in range(rows):
+        i = 0
+        while inner[i]:
+            i = 2 * i + 1 + int(X[nodes["attribute"][i], r] >= 0.5)
+        assert got[r] == value[i - n // 2]
+
+
+@pytest.mark.parametrize("n,trees", [(40, 3), (1000, 64), (1000, 130)])
+def test_out_of_bag_lists_over_tree_chunks(n, trees):
+    """Fewer rows than a block, one chunk of trees and several."""
+    X, y = synth.gaussian_classes(seed=n, n=n, f=6, n_informative=4, n_classes=3)
+    p = capi.default_params(RF, n_trees=trees, n_features_per_node=2, max_depth=8, n_classes=3, seed=4)
+    Xd = capi.DeviceArray.from_numpy(X)
+    g = capi.fit_device(Xd.ptr, n, 6, y, p)
+    o = pyoracle.fit(X, y, algorithm=RF, n_trees=trees, k=2, max_depth=8, n_classes=3, seed=4)
+    for perm in (-1, 1):
+        assert capi.oob_evaluate(g, Xd.ptr, y, n, perm) == pyoracle.oob_evaluate(o, X, y, seed=4, permuted_feature=perm)
+    bad = y.copy()
+    bad[n // 2] = 3
+    with pytest.raises(Exception):
+        capi.oob_evaluate(g, Xd.ptr, bad, n)
+    bad[n // 2] = 0.5
+    with pytest.raises(Exception):
+        capi.oob_evaluate(g, Xd.ptr, bad, n)
+    g.close()
+    Xd.free()
