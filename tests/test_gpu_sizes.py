@@ -144,10 +144,7 @@ def test_export_equals_the_canonical_arrays(task, depth):
     if task:
         assert np.array_equal(probs, c["value"][leaf])
     else:
-        counts = c["class_counts"].reshape(-1, 3)[leaf].astype(np.float64)
-        want = counts / counts.sum(1, keepdims=True)
-        # one division in fp32: half a unit in the last place of a value <= 1
-        assert np.abs(probs.reshape(-1, 3) - want).max() <= 2.0 ** -24
+        assert np.array_equal(probs, c["class_counts"].reshape(-1, 3)[leaf].ravel().astype(np.float32))
 
 
 @pytest.mark.parametrize("task", [capi.CLASSIFICATION, capi.REGRESSION])
