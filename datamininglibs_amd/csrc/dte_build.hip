@@ -34,6 +34,7 @@
 #include <cstdlib>
 #include <chrono>
 #include <memory>
+#include <utility>
 
 #include "dte_block.h"
 #include "dte_internal.h"

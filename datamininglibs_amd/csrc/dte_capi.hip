@@ -858,8 +858,10 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
     r.get(depth.data(), 4 * n);
     // structure: trees tile [0, n); children adjacent inside their tree
     if (ts[0] != 0 || ts[T] != n) fail(DTE_ERR_INVALID_ARGUMENT, "forest file tree table out of range");
+    bool level_order = true;
     for (int t = 0; t < T; ++t) {
       if (ts[t + 1] <= ts[t]) fail(DTE_ERR_INVALID_ARGUMENT, "forest file tree table out of range");
+      int64_t next = ts[t] + 1;
       if (depth[ts[t]] != 0) fail(DTE_ERR_INVALID_ARGUMENT, "forest file root depth");
       for (int64_t g = ts[t]; g < ts[t + 1]; ++g) {
         if (feature[g] < 0) {
@@ -871,7 +873,10 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
           fail(DTE_ERR_INVALID_ARGUMENT, "forest file child link out of range");
         if (depth[left[g]] != depth[g] + 1 || depth[left[g] + 1] != depth[g] + 1)
           fail(DTE_ERR_INVALID_ARGUMENT, "forest file depths inconsistent");
+        level_order = level_order && left[g] == next;
+        next += 2;
       }
+      level_order = level_order && next == ts[t + 1];
     }
     set_device(device_id);
     hipStream_t s = library_stream(device_id);
@@ -887,6 +892,7 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
     f.algorithm = h.algorithm;
     f.n_nodes = n;
     f.n_leaves = count_leaves(feature);
+    f.level_order = level_order;
     f.has_stats = h.has_stats != 0;
     f.seed = h.seed;
     f.tree_offset = h.tree_offset;

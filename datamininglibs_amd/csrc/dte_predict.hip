@@ -2,9 +2,9 @@
 // source/gpudte.cu:311-359) and the host launch loop of
 // GpuDteAlgorithm<T>::Predict (gpudte_algorithm.cc:292-311):
 //
-//  * nodes are 8-byte records, sibling pairs side by side, three levels of a
-//    subtree in one cache line (build_predict_nodes); a visit loads the pair
-//    of children while the node's feature value is read and compared;
+//  * nodes are 8-byte records, siblings side by side, a tree's top levels in
+//    level order and below them three levels of a subtree in one cache line
+//    (build_predict_nodes);
 //  * classification: every (row, tree) pair is walked exactly once (FIX of
 //    the truncated grid, gpudte_algorithm.cc:297-305) and votes are integer
 //    sums, so the result is order-free;
@@ -27,13 +27,24 @@ constexpr int kWalkThreads = 512;  // a block's rows in LDS serve eight waves
 // ------------------------------------------------------ node layout ----
 // Bound by the rate of cache lines that come over the fabric for the deep
 // levels (16-byte records in level order: a line per visited level, 79 GB for
-// 200 M walks of 60 M nodes, 16.0 ms).  Here a tree's pairs are grouped by
-// clusters of three levels -- the pair at depth 1, 4, 7, .. and up to six
-// pairs below it, 16 B each -- in slots of 1, 2, 4 or 8 pairs aligned to
-// their size, so that a cluster never straddles a 128-byte line and a walk
-// touches one line per three levels.  The root shares a line with the cluster
-// below it.
+// 200 M walks of 60 M nodes, 16.0 ms).  Below kTopLevels a tree's pairs are
+// grouped by clusters of three levels -- the pair below a node at depth 9, 12,
+// .. and up to six pairs below it, 16 B each -- in slots of 1, 2, 4 or 8 pairs
+// aligned to their size, so that a cluster never straddles a 128-byte line and
+// a walk touches one line per three levels.  The top levels stay in the caches
+// whatever their order; there the lines that the 64 rows of a wave touch in one
+// step count, fewest in level order.  600,000 rows x 6, 64 trees of 8,000 nodes:
+// 0.69 ms with 16-byte records, 0.81 clustered from the root, 0.64 like this;
+// 1M x 128, 64 trees of 300,000 nodes: 5.2, 4.1, 4.1 ms.
 constexpr int kClusterLevels = 3;
+constexpr int kTopLevels = 9;  // a multiple of kClusterLevels
+
+// Pair of the children of a node above kTopLevels: the tree's pairs in level
+// order behind the root's (canonical order is level order, so the children of
+// the tree's k-th internal node are its nodes 2k - 1 and 2k).
+__device__ __forceinline__ uint32_t top_pair(int64_t first, int64_t tree_start) {
+  return 1u + (uint32_t)((first - tree_start - 1) >> 1);
+}
 
 // Slot class of a cluster of s pairs: 2^class slots of a pair.
 __device__ __forceinline__ int slot_class(int s) { return s <= 1 ? 0 : s <= 2 ? 1 : s <= 4 ? 2 : 3; }
@@ -73,9 +84,9 @@ __device__ __forceinline__ Cluster cluster_at(int32_t head, const int32_t* __res
   return c;
 }
 
-// Every internal node at a depth divisible by three heads the cluster of its
-// children: its slot class and number among the tree's clusters of that class.
-// One atomic per wave, tree and class.
+// From kTopLevels on, every internal node at a depth divisible by three heads
+// the cluster of its children: its slot class and number among the tree's
+// clusters of that class.
 __global__ void __launch_bounds__(kBlock) k_cluster_count(int64_t n, int T, const int64_t* __restrict__ ts,
                                                           const int32_t* __restrict__ feature,
                                                           const int32_t* __restrict__ left,
@@ -103,10 +114,9 @@ __global__ void __launch_bounds__(kBlock) k_cluster_count(int64_t n, int T, cons
       const int64_t g = c0 + q * kBlock + t;
       cls[q] = -1;
       first[q] = 0;
-      if (g < n && feature[g] >= 0 && depth[g] % kClusterLevels == 0) {
+      if (g < n && feature[g] >= 0 && depth[g] >= kTopLevels && depth[g] % kClusterLevels == 0) {
         first[q] = left[g];
-        // the root's cluster has a line of its own, behind the root pair
-        if (depth[g] > 0) cls[q] = slot_class(cluster_at(first[q], feature, left).n);
+        cls[q] = slot_class(cluster_at(first[q], feature, left).n);
         if (cls[q] >= 0 && g >= end0) {  // a later tree's
           code[first[q]] = atomicAdd(&cnt[4 * (int64_t)tree_of(g, T, ts) + cls[q]], 1u) * 4u + (unsigned)cls[q];
           cls[q] = -1;
@@ -138,7 +148,9 @@ __global__ void __launch_bounds__(kBlock) k_cluster_count(int64_t n, int T, cons
     __syncthreads();  // s_cnt is cleared, s_base rewritten
   }
 }
-__global__ void __launch_bounds__(kBlock) k_cluster_bases(int T, const unsigned int* __restrict__ cnt,
+__global__ void __launch_bounds__(kBlock) k_cluster_bases(int T, const int64_t* __restrict__ ts,
+                                                          const int32_t* __restrict__ depth,
+                                                          const unsigned int* __restrict__ cnt,
                                                           int64_t* __restrict__ tbase,
                                                           uint32_t* __restrict__ cbase) {
   __shared__ int64_t s_sum[kBlock];
@@ -149,7 +161,14 @@ __global__ void __launch_bounds__(kBlock) k_cluster_bases(int T, const unsigned 
     int64_t size = 0;
     if (i < T) {
       const unsigned int* c = cnt + 4 * (int64_t)i;
-      uint32_t at = 8;
+      // nodes of the top levels: a prefix of the tree
+      int64_t lo = ts[i], hi = ts[i + 1];
+      while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (depth[mid] <= kTopLevels) lo = mid + 1;
+        else hi = mid;
+      }
+      uint32_t at = (1u + (uint32_t)((lo - ts[i]) >> 1) + 7u) & ~7u;
       cbase[4 * (int64_t)i + 3] = at;
       at += 8u * c[3];
       cbase[4 * (int64_t)i + 2] = at;
@@ -204,9 +223,10 @@ __global__ void __launch_bounds__(kBlock) k_cluster_write(int64_t n, int T, cons
                                                           const int64_t* __restrict__ tbase,
                                                           const uint32_t* __restrict__ cbase, uint4* __restrict__ out) {
   for (int64_t g = blockIdx.x * (int64_t)kBlock + threadIdx.x; g < n; g += (int64_t)gridDim.x * kBlock) {
-    if (depth[g] % kClusterLevels != 0) continue;
+    const int32_t dg = depth[g];
+    if (dg >= kTopLevels && dg % kClusterLevels != 0) continue;
     const int32_t f = feature[g];
-    const bool root = depth[g] == 0;
+    const bool root = dg == 0;
     if (f < 0 && !root) continue;
     const int t = tree_of(g, T, ts);
     const uint32_t* cb = cbase + 4 * (int64_t)t;
@@ -217,9 +237,24 @@ __global__ void __launch_bounds__(kBlock) k_cluster_write(int64_t n, int T, cons
       tree[0] = make_uint4(r.x, r.y, 0u, 0u);
       if (f < 0) continue;
     }
-    const Cluster c = cluster_at(left[g], feature, left);
     auto slot = [&](int32_t first) { return cb[code[first] & 3u] + ((code[first] >> 2) << (code[first] & 3u)); };
-    const uint32_t at = root ? 1u : slot(c.head);
+    auto record = [&](int32_t i, uint32_t child) {
+      const int32_t cf = feature[i];
+      return cf < 0 ? leaf_record(i, C, task, cls, value)
+                    : make_uint2(__float_as_uint(thr[i]), child << fbits | (uint32_t)(cf + 1));
+    };
+    auto put = [&](uint32_t where, uint2 l, uint2 r) { tree[where] = make_uint4(l.x, l.y, r.x, r.y); };
+    if (dg < kTopLevels) {
+      const int32_t h = left[g];
+      auto below = [&](int32_t i) -> uint32_t {  // pair of a child's children
+        if (feature[i] < 0) return 0u;
+        return dg + 1 < kTopLevels ? top_pair(left[i], ts[t]) : slot(left[i]);
+      };
+      put(top_pair(h, ts[t]), record(h, below(h)), record(h + 1, below(h + 1)));
+      continue;
+    }
+    const Cluster c = cluster_at(left[g], feature, left);
+    const uint32_t at = slot(c.head);
     // breadth-first places of the pairs in the cluster's slots
     uint32_t next = at + 1u, mid[2], low[4];
 #pragma unroll
@@ -232,12 +267,6 @@ __global__ void __launch_bounds__(kBlock) k_cluster_write(int64_t n, int T, cons
       low[k] = next;
       next += c.low[k] >= 0;
     }
-    auto record = [&](int32_t i, uint32_t child) {
-      const int32_t cf = feature[i];
-      return cf < 0 ? leaf_record(i, C, task, cls, value)
-                    : make_uint2(__float_as_uint(thr[i]), child << fbits | (uint32_t)(cf + 1));
-    };
-    auto put = [&](uint32_t where, uint2 l, uint2 r) { tree[where] = make_uint4(l.x, l.y, r.x, r.y); };
     put(at, record(c.head, mid[0]), record(c.head + 1, mid[1]));
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -291,12 +320,14 @@ __device__ __forceinline__ uint32_t walk(const Trees& tr, int t, const float* xr
     const uint32_t fmask = (1u << tr.fbits) - 1u;
     uint2 nd = *reinterpret_cast<const uint2*>(tree);
     while (nd.y & fmask) {
-      const uint4 kids = tree[nd.y >> tr.fbits];  // in flight beside the feature value
       const int f = (int)(nd.y & fmask) - 1;
       float x = xr[f * xs];
       visit(f, depth, x);
-      const bool right = side_of(x, __uint_as_float(nd.x)) != 0;
-      nd = right ? make_uint2(kids.z, kids.w) : make_uint2(kids.x, kids.y);
+      // the child alone: the pair in flight beside the feature value takes
+      // twice the lanes' share of the L1 (regression 600,000 x 6, 64 trees:
+      // 0.36 ms with the pair, 0.33 with the child)
+      const uint2* kids = reinterpret_cast<const uint2*>(tree + (nd.y >> tr.fbits));
+      nd = kids[side_of(x, __uint_as_float(nd.x))];
       ++depth;
     }
     return nd.x;
@@ -814,6 +845,7 @@ void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld,
 namespace {
 // Feature bits of the packed records' links, or 0: wide records.
 int packed_feature_bits(const Forest& f, int64_t max_tree) {
+  if (!f.level_order) return 0;
   int fbits = 1;
   while (((int64_t)1 << fbits) <= (int64_t)f.n_features) ++fbits;  // feature + 1, 0 for a leaf
   // slots of a tree: a cluster of s pairs takes at most 1.6 s of them
@@ -858,7 +890,8 @@ void build_predict_nodes(Forest& f, int64_t max_tree, hipStream_t s) {
   hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(4 * (int64_t)T)), dim3(kBlock), 0, s, cnt.p, 4 * (int64_t)T);
   hipLaunchKernelGGL(k_cluster_count, dim3(grid), dim3(kBlock), 0, s, n, T, f.tree_start.p, f.feature.p, f.left.p,
                      f.depth.p, code.p, cnt.p);
-  hipLaunchKernelGGL(k_cluster_bases, dim3(1), dim3(kBlock), 0, s, T, (const unsigned int*)cnt.p, f.pair_base.p,
+  hipLaunchKernelGGL(k_cluster_bases, dim3(1), dim3(kBlock), 0, s, T, f.tree_start.p, f.depth.p,
+                     (const unsigned int*)cnt.p, f.pair_base.p,
                      cbase.p);
   hipLaunchKernelGGL(k_cluster_write, dim3(grid), dim3(kBlock), 0, s, n, T, f.tree_start.p, f.feature.p, f.left.p,
                      f.depth.p, f.threshold.p, cls, f.value.p, f.n_classes, f.task, fbits, (const uint32_t*)code.p,

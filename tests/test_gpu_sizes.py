@@ -165,6 +165,52 @@ def test_predict_row_counts(task, rows):
         assert np.array_equal(np.asarray(v, np.float64), np.asarray(want, np.float64))
 
 
+@pytest.mark.parametrize("shape", ["full", "chain", "mixed"])
+@pytest.mark.parametrize("depth", [0, 1, 8, 9, 10, 12, 13, 17])
+def test_predict_over_the_top_levels_and_clusters(shape, depth):
+    """Trees that end above, at and below the level where clusters begin, with
+    full, one-sided and random subtrees."""
+    if shape == "full" and depth > 13:
+        depth = 14
+    rng = np.random.default_rng(depth)
+    trees, f, rows = 3, 5, 200
+    nodes, front, base = [], trees, 0
+    for level in range(depth + 1):
+        if level == depth:
+            split = np.zeros(front, bool)
+        elif shape == "full":
+            split = np.ones(front, bool)
+        elif shape == "chain":
+            split = np.arange(front) % 2 == level % 2 if level else np.ones(front, bool)
+        else:
+            split = rng.random(front) < (0.95 if level < 5 else 0.6)
+        lv = np.zeros(front, capi.NODE_DTYPE)
+        lv["child_start"] = np.where(split, base + front + 2 * (np.cumsum(split) - 1), -1)
+        lv["child_count"] = np.where(split, 2, 0)
+        lv["attribute"] = np.where(split, rng.integers(0, f, front), -1)
+        lv["split_point"] = np.where(split, rng.uniform(0.2, 0.8, front), -1).astype(np.float32)
+        nodes.append(lv)
+        base += front
+        front = 2 * int(split.sum())
+        if not front:
+            break
+    nodes = np.concatenate(nodes)
+    leaf = nodes["child_count"] == 0
+    nodes["probability_start"] = np.where(leaf, np.cumsum(leaf) - 1, -1)
+    value = rng.integers(-9, 10, int(leaf.sum())).astype(np.float32)  # sums are exact
+    g = capi.import_forest(nodes, value, trees, 1, f, capi.REGRESSION)
+    X = rng.random((f, rows), dtype=np.float32)
+    want = np.zeros(rows)
+    for t in range(trees):
+        at = np.full(rows, t)
+        while not leaf[at].all():
+            n = nodes[at]
+            right = X[np.maximum(n["attribute"], 0), np.arange(rows)] >= n["split_point"]
+            at = np.where(leaf[at], at, n["child_start"] + right)
+        want += value[nodes["probability_start"][at]]
+    assert np.array_equal(g.predict(X), want.astype(np.float32))
+
+
 def test_predict_with_wide_records():
     """A feature number and a pair number that do not fit 32 bits together."""
     rng = np.random.default_rng(6)
