@@ -41,10 +41,10 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_rf_1m128.json")
 KERNEL_SYMBOL = {
     "search_seg16": "dte::(anonymous namespace)::k_search_rf_seg<16, 0, 16>",
     "search_seg32": "dte::(anonymous namespace)::k_search_rf_seg<16, 0, 32>",
-    "search_seg64": "dte::(anonymous namespace)::k_search_rf_seg<16, 0, 64>",
-    "search_team64": "dte::(anonymous namespace)::k_search_rf<16, 0, 64, false>",
-    "search_block": "dte::(anonymous namespace)::k_search_rf<16, 0, 256, false>",
-    "chunk_eval": "dte::(anonymous namespace)::k_v2_eval<16, 0>",
+    "search_seg64": "dte::(anonymous namespace)::k_search_rf_bound<16, 0, 1>",
+    "search_team64": "dte::(anonymous namespace)::k_search_rf_bound<16, 0, 8>",
+    "search_block": "dte::(anonymous namespace)::k_search_rf_bound_team<16, 0>",
+    "chunk_hist": "dte::(anonymous namespace)::k_v2_hist<0, false>",
 }
 
 
@@ -462,9 +462,10 @@ def main():
 
     # Roofline of the dominant split-search kernel.
     # single-kernel families that carry algorithmic bytes (the chunk
-    # pipeline's evaluation kernel carries its items' bytes)
+    # pipeline's histogram kernel, which reads every entry, carries its items'
+    # bytes)
     fam = {k: v_ for k, v_ in stats.items()
-           if (k.startswith("search_") and k != "search_chunked") or k == "chunk_eval"}
+           if (k.startswith("search_") and k not in ("search_chunked", "search_merged")) or k == "chunk_hist"}
     dom = max(fam, key=lambda k: fam[k]["total_ms"])
     ds = fam[dom]
     avg_ms = ds["total_ms"] / max(1, ds["launches"])

@@ -86,11 +86,12 @@ typedef struct dte_params {
                                   17-31; the reference restarts its RNG per batch instead, D7) */
   /* Split-search tuning; 0 keeps the default, dte_autotune picks them for a
    * data set.  Results do not depend on them, only the time does. */
-  int32_t cut_team;            /* RF: largest node (distinct rows) searched by one wave per draw,
-                                  64..512 (default 512); smaller nodes use 16/32/64-lane segments */
-  int32_t cut_block;           /* RF: largest node searched by one workgroup per draw, cut_team..2048
+  int32_t cut_team;            /* RF: largest node (distinct rows) searched by one wave, 64..512
+                                  (default 512); up to 32 rows by 16/32-lane segments */
+  int32_t cut_block;           /* RF: largest node searched by one workgroup, cut_team..2048
                                   (default 2048); larger nodes take the bucketed chunk pipeline */
-  int32_t bucket_target;       /* RF: rows per key bucket aimed at in that pipeline, 64..512 (384) */
+  int32_t bucket_target;       /* RF: sets the key buckets of that pipeline, which aim at a sixth of
+                                  it in rows, 64..512 (384) */
   int32_t cut_ert;             /* ERT: largest node searched by one wave per draw, 64..2^20 (4096) */
   int32_t reserved[2];         /* must be zero */
 } dte_params;
