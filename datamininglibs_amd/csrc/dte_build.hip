@@ -6044,12 +6044,12 @@ const char* search_family(int algorithm, int tier) {
   return algorithm == DTE_RANDOM_FOREST ? rf[tier] : ert[tier];
 }
 
-// RF tiers: 0/1/2 = one 16/32/64-lane segment per node (one entry per lane,
-// draws looped in the kernel); 3 = wave teams (four items per workgroup);
-// 4 = whole workgroup per item within the LDS capacity; 5 = the chunk
-// pipeline (big_pipeline); 6 = whole workgroup per item of any size (the
-// plain driver).  ERT tiers: 0/1/2 = one 16/32/64-lane segment per node
-// (draws looped in the kernel), 3 = one wave per node (entries in
+// RF tiers: 0/1 = one 16/32-lane segment per node (one entry per lane, draws
+// looped in the kernel); 2/3 = a wave per node, bounded search (1 / 8 entries
+// per lane); 4 = a workgroup per node, bounded search; 5 = the chunk pipeline
+// (big_pipeline); 6 = a workgroup per item of any size (the plain driver, few
+// nodes above cut_block).  ERT tiers: 0/1/2 = one 16/32/64-lane segment per
+// node (draws looped in the kernel), 3 = one wave per node (entries in
 // registers), 4 = one wave per item, 5 = workgroup per item.
 template <int MAXC, int TASK>
 void launch_search(int algorithm, int tier, int grid, hipStream_t s, const DataArgs& d, const LevelArgs& lv,
@@ -6925,19 +6925,31 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       }
     }
   } side;
-  // Keys of a level's first draws by entry (k_gather_draws), if they pay and
-  // leave half of the free memory.
+  // Keys of a level's first draws by entry (k_gather_draws), if they pay and,
+  // with the scratch of the chunk pipeline's largest batch, leave half of the
+  // free memory; without them the searches gather from K.
   const int FS = (d.F + 15) / 16 * 16;
   DevBuf<uint32_t> key_rows, draw_keys, draw_tiles, draw_toff;
   bool use_rows = algorithm == DTE_RANDOM_FOREST && !plain && key_rows_pay(d.N, d.F, D0);
   if (use_rows) {
     size_t free_b = 0, total_b = 0;
     DTE_HIP(hipMemGetInfo(&free_b, &total_b));
-    use_rows = 4 * ((size_t)d.N * FS + (size_t)E * D0) <= free_b / 2;
+    const int64_t slots = std::min<int64_t>(kV2Batch, (int64_t)T * N * D0) + N;
+    const size_t batch = (size_t)slots * (task == 0 ? 16 : 32);
+    use_rows = 4 * ((size_t)d.N * FS + (size_t)E * D0) + batch <= free_b / 2;
   }
   if (use_rows) {
-    key_rows.alloc((size_t)d.N * FS);
-    draw_keys.alloc((size_t)E * D0);
+    try {
+      key_rows.alloc((size_t)d.N * FS);
+      draw_keys.alloc((size_t)E * D0);
+    } catch (const std::exception&) {  // another thread's fit took the memory
+      (void)hipGetLastError();
+      key_rows.release();
+      draw_keys.release();
+      use_rows = false;
+    }
+  }
+  if (use_rows) {
     hipLaunchKernelGGL(k_key_rows, dim3((unsigned)((d.N + kWave - 1) / kWave)), dim3(kBlock),
                        (unsigned)(4 * kWave * (FS + 1)), s, d.K, d.N, d.F, FS, key_rows.p);
   }
@@ -7148,12 +7160,13 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     if (count_bytes) DTE_HIP(hipMemsetAsync(graph_bytes.p, 0, graph_bytes.bytes(), s));
     const bool rf = algorithm == DTE_RANDOM_FOREST;
     constexpr int kElemGrid = 1024;
-    // Extra trees on small data (at most kMergeEntries entries over all
-    // trees): one launch for all search tiers of a phase.  Its levels are
-    // small and latency-bound, and side by side the tiers finish sooner
-    // (4,601 x 57, 100 trees: 12.3k -> 15.9k trees/s); on large data the
-    // merged kernel's register budget (the largest tier's) costs more
-    // occupancy than the overlap gains (64 forests: 8.2k -> 6.9k).
+    // Small data (at most kMergeEntries entries over all trees): one launch
+    // for all search tiers of a phase.  Its levels are small and
+    // latency-bound, and side by side the tiers finish sooner (4,601 x 57, 100
+    // extra trees: 12.3k -> 15.9k trees/s; random forest of 3.2 M entries, a
+    // level of its deepest: 0.92 -> 0.77 ms); on large data the merged
+    // kernel's register budget (the largest tier's) costs more occupancy than
+    // the overlap gains (64 extra-trees forests: 8.2k -> 6.9k).
     const bool ert_merged = !rf && small_data;
     const ErtAllFn ert_all = pick_ert_all(task, C);
     // likewise the partition tiers of a step (both algorithms)
