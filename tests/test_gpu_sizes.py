@@ -254,3 +254,36 @@ def test_out_of_bag_lists_over_tree_chunks(n, trees):
         capi.oob_evaluate(g, Xd.ptr, bad, n)
     g.close()
     Xd.free()
+
+
+def test_predict_of_a_file_out_of_level_order(tmp_path):
+    """A forest file may hold a level's sibling pairs in another order than
+    their parents': it loads, and predicts the same."""
+    rng = np.random.default_rng(3)
+    n = 31
+    nodes = np.zeros(n, capi.NODE_DTYPE)
+    inner = np.arange(n) < 15
+    nodes["child_start"] = np.where(inner, 2 * np.arange(n) + 1, -1)
+    nodes["child_count"] = np.where(inner, 2, 0)
+    nodes["attribute"] = np.where(inner, rng.integers(0, 4, n), -1)
+    nodes["split_point"] = np.where(inner, rng.uniform(0.2, 0.8, n), -1).astype(np.float32)
+    nodes["probability_start"] = np.where(inner, -1, np.arange(n) - 15)
+    value = np.arange(16, dtype=np.float32)
+    g = capi.import_forest(nodes, value, 1, 1, 4, capi.REGRESSION)
+    path = tmp_path / "forest"
+    g.save(path)
+    raw = bytearray(path.read_bytes())
+    head = 8 + 4 + 8 * 4 + 3 * 8 + 16  # header, tree table of one tree
+    order = np.arange(n)
+    order[3:7] = [5, 6, 3, 4]
+    cols = np.frombuffer(bytes(raw[head:head + 20 * n]), np.int32).reshape(5, n).copy()
+    left = cols[2]  # feature, threshold, left, depth, value
+    left[1], left[2] = left[2], left[1]
+    raw[head:head + 20 * n] = cols[:, order].tobytes()
+    h = 0xCBF29CE484222325
+    for b in raw[:-8]:
+        h = (h ^ b) * 0x100000001B3 & (2 ** 64 - 1)
+    raw[-8:] = h.to_bytes(8, "little")
+    path.write_bytes(bytes(raw))
+    X = rng.random((4, 300), dtype=np.float32)
+    assert np.array_equal(capi.load_forest(path).predict(X), g.predict(X))
