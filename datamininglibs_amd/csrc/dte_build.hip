@@ -38,6 +38,7 @@
 
 #include "dte_block.h"
 #include "dte_internal.h"
+#include "dte_limits.h"
 
 namespace dte {
 
@@ -2823,8 +2824,9 @@ struct BoundLds {
   int64_t below_s[1];
   uint32_t ncls[TASK == 0 ? MAXC : 1];
   BoundList list;
-  uint32_t stk_k[IPT + 1];
+  uint32_t stk_k[IPT + 1];  // from 1 on
   uint32_t stk_b[IPT + 1];
+  static_assert(wave_stack(kWave * IPT) <= IPT, "ranges of the wave tier");
 };
 
 // Value of the lane below (lane 0: `first`) through DPP wave_shr:1.
@@ -3550,7 +3552,7 @@ __global__ void __launch_bounds__(kBlock, IPT == 1 ? 5 : 4 - TASK) k_search_rf_b
 // all waves through a list per wave, in rounds of at most kTeamList of them.
 constexpr int kTeamIpt2 = kCap / kBlock;  // entries per thread
 constexpr int kTeamList = 128;
-constexpr int kTeamStack = kCap / kWave + 1;  // disjoint ranges of more than 64 entries
+static_assert(kBoundRun == kWave, "a run is an entry per lane");
 
 template <int MAXC, int TASK, int LOGB>
 struct BoundTeamLds {
@@ -3573,7 +3575,8 @@ struct BoundTeamLds {
   uint16_t lidx[kWaves][kTeamList];
   BoundList list[kWaves];
   DrawBest best[kWaves];
-  uint32_t stk_k[kTeamStack], stk_b[kTeamStack];
+  uint32_t stk_k[kTeamStack];  // first keys and widths (log2) of ranges to split again
+  uint8_t stk_b[kTeamStack];
   int sp;
 };
 
@@ -3854,16 +3857,16 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
             const int x = (int)__ffsll((unsigned long long)mk) - 1;
             const int bx = wv * kWave + x;
             const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)L.wgt[bx]);
-            if (w > (uint32_t)kWave) {
+            if (w > (uint32_t)kBoundRun) {
               // more than a list: a single key has only its edge, a wider
               // bucket is split again
               const uint32_t klo = k0 + ((uint32_t)bx << shift);
-              if (!shift) {
+              if (!team_splits_again(w, shift)) {
                 bound_edge<TASK, LOGB>(d, nd, L, klo, bx, best);
               } else if (lane == 0) {
-                const int at = atomicAdd(&L.sp, 1);
+                const int at = atomicAdd(&L.sp, 1);  // below kTeamStack
                 L.stk_k[at] = klo;
-                L.stk_b[at] = (uint32_t)shift;
+                L.stk_b[at] = (uint8_t)shift;
               }
             } else {
               if (wsel + w > (uint32_t)kTeamList) break;
@@ -3949,7 +3952,7 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
         more = sp > 0;
         if (more) {
           k0 = __builtin_amdgcn_readfirstlane(L.stk_k[sp - 1]);
-          sb = (int)__builtin_amdgcn_readfirstlane(L.stk_b[sp - 1]);
+          sb = (int)__builtin_amdgcn_readfirstlane((uint32_t)L.stk_b[sp - 1]);
         }
         __syncthreads();
         if (more && t == 0) L.sp = sp - 1;
@@ -6865,7 +6868,7 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   // k_search_rf_bound counts two classes in a word: its nodes weigh at most
   // 65535 (a bootstrap's multiplicities hardly ever pass 15, so this bites at
   // no node size; the pipeline takes any weight).
-  const int m_packed = (int)std::max<int64_t>(1, 65535 / (int64_t)std::max<uint32_t>(w_max, 1));
+  const int m_packed = (int)std::max<int64_t>(1, kBoundWeight / (int64_t)std::max<uint32_t>(w_max, 1));
   const int cut_team = std::min(m_packed, p.cut_team ? p.cut_team : kDefCutTeam);
   const int cut_block =
       std::min(m_packed, std::max(cut_team, std::min(kCap, p.cut_block ? p.cut_block : kDefCutBlock)));

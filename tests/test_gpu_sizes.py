@@ -287,3 +287,21 @@ def test_predict_of_a_file_out_of_level_order(tmp_path):
     path.write_bytes(bytes(raw))
     X = rng.random((4, 300), dtype=np.float32)
     assert np.array_equal(capi.load_forest(path).predict(X), g.predict(X))
+
+
+@pytest.mark.parametrize("kind", ["2", "10", "reg"])
+def test_rf_many_heavy_buckets(kind):
+    """Roots of about 2,000 rows whose features have 35 or 36 common values
+    among some 300 rare ones, and labels of noise: most common values weigh
+    more than a wave's list, share their bucket with rare keys, and survive
+    the bound, so many ranges wait to be split again (test_search_limits.py)."""
+    rng = np.random.default_rng(21)
+    n, f = 3150, 8
+    X = np.empty((f, n), np.float32)
+    for j in range(f):
+        c = 35 + j % 2
+        X[j] = np.where(rng.random(n) < 0.92, rng.integers(0, c, n) + 0.5, c * rng.random(n))
+    kw = dict(task=capi.REGRESSION) if kind == "reg" else dict(n_classes=int(kind))
+    y = rng.standard_normal(n) if kind == "reg" else rng.integers(0, int(kind), n)
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, n_trees=60, k=6, max_depth=4, **kw)
+    assert_same_forest(g, o)

@@ -1,0 +1,17 @@
+"""Sizes of the split search's LDS arrays against a host model of what they
+must hold (tests/cpp/search_limits.cc over csrc/dte_limits.h)."""
+import os
+import subprocess
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def test_ranges_of_the_workgroup_tier_fit_their_stack(tmp_path):
+    exe = str(tmp_path / "search_limits")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", exe, os.path.join(HERE, "cpp", "search_limits.cc")], check=True)
+    p = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout
+    # a bootstrapped node alone holds more ranges than its entries suggest
+    # (2048 entries: 33 ranges of more than 64)
+    bootstrap = max(int(line.split()[1]) for line in p.stdout.splitlines() if line.startswith("bootstrap"))
+    assert bootstrap > 2048 // 64 + 1
