@@ -1312,6 +1312,12 @@ __device__ __forceinline__ double reg_gain_error(double N, double y_max) {
   return 0.25 * N * e * e * 1.1e6;
 }
 
+// fp32 score of a variance gain that must not pass for none: a positive gain's
+// score may round to 0, and its threshold still decides among draws of score 0.
+__device__ __forceinline__ float reg_score_bound(double gain, int shift) {
+  return gain > 0.0 ? fmaxf((float)ldexp_d(gain, -2 * shift), FLT_TRUE_MIN) : 0.0f;
+}
+
 // Upper bound of the variance criterion over left weights [n0, n1] and left
 // target sums [lo, hi], for a node of weight N, target sum S and largest
 // deviation M: f(n, s) = s^2 / n + (S - s)^2 / (N - n) is convex, so its
@@ -1448,13 +1454,13 @@ __global__ void __launch_bounds__(kBlock) k_v2_bound(DataArgs d, LevelArgs lv, V
       float ub = -1.0f;
       if (w) {
         const double u = reg_box_bound((double)la, (double)(la + w), (double)(sa + sn), (double)(sa + sp), N, S, M);
-        ub = (float)ldexp_d(u * (1.0 + 2e-6) + E, -2 * d.shift);
+        ub = reg_score_bound(u * (1.0 + 2e-6) + E, d.shift);
         if (la > 0) {
           const double g = variance_gain(la, su, it.n_w - la, it.ssum - su, 0);
           best = fmaxf(best, (float)ldexp_d(g, -2 * d.shift));
           if (it.width == 1) {
             a.res_g[gb] = g;
-            ub = (float)ldexp_d(g, -2 * d.shift);
+            ub = reg_score_bound(g, d.shift);
           }
         } else if (it.width == 1) {
           ub = 0.0f;
@@ -3019,6 +3025,15 @@ __device__ __forceinline__ void bound_edge(const DataArgs& d, const BoundNode& n
   if (g > 0.0 && cand_better(g, key, best.g, best.key)) best = DrawBest{g, key, kEdge};
 }
 
+// Least gain whose fp32 score can equal the score of gain thr.  Variances have
+// no scale: above the largest fp32 number all scores are infinity, below the
+// normal ones they are 2^-149 apart.
+template <int TASK>
+__device__ __forceinline__ double bound_cut(const DataArgs& d, double thr) {
+  if (TASK == 0) return thr * (1.0 - 1e-6);
+  return fmin(thr, ldexp_d((double)FLT_MAX, 2 * d.shift)) * (1.0 - 1e-6) - ldexp_d(1.0, 2 * d.shift - 148);
+}
+
 // One draw of a node.  thr: lower bound of the node's best gain that matters
 // here (nats, or fixed-point units squared); returns the draw's best in
 // `best` (none when no candidate of it can be the node's best) and raises thr
@@ -3156,7 +3171,7 @@ __device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& n
       }
       eb = __uint_as_float(wave_max_u32(__float_as_uint(eb)));
       thr = fmax(thr, (double)eb);
-      const float thr_f = (float)(thr * (1.0 - 1e-6));
+      const float thr_f = (float)bound_cut<TASK>(d, thr);
 #pragma unroll
       for (int r = 0; r < NR; ++r) mask[r] = __ballot(ub[r] >= thr_f && ub[r] > 0.0f);
     } else {
@@ -3196,7 +3211,7 @@ __device__ __forceinline__ void bound_draw(const DataArgs& d, const BoundNode& n
 #pragma unroll
       for (int off = kWave / 2; off > 0; off >>= 1) eb = fmax(eb, __shfl_xor(eb, off, kWave));
       thr = fmax(thr, eb);
-      const double thr_d = thr * (1.0 - 1e-6);
+      const double thr_d = bound_cut<TASK>(d, thr);
 #pragma unroll
       for (int r = 0; r < NR; ++r) mask[r] = __ballot(ub[r] >= thr_d && ub[r] > 0.0);
     }
@@ -3847,7 +3862,7 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
         __syncthreads();
 #pragma unroll
         for (int x = 0; x < kWaves; ++x) thr = fmax(thr, L.eb[x]);
-        const double thr_d = thr * (1.0 - 1e-6);
+        const double thr_d = bound_cut<TASK>(d, thr);
         uint64_t mk = __ballot(ub >= thr_d && ub > 0.0);
         // ---- surviving buckets, in rounds of at most kTeamList entries a wave
         for (;;) {

@@ -305,3 +305,21 @@ def test_rf_many_heavy_buckets(kind):
     y = rng.standard_normal(n) if kind == "reg" else rng.integers(0, int(kind), n)
     g, o = fit_both(X, y.astype(np.float32), algorithm=RF, n_trees=60, k=6, max_depth=4, **kw)
     assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("n,trees,depth", [(1500, 800, 4), (40_000, 4, 5)])
+@pytest.mark.parametrize("target", ["1e17", "3e18", "1e19", "1e25", "constant 1e-5", "constant 3e-7"])
+def test_rf_regression_scores_at_the_ends_of_fp32(target, n, trees, depth):
+    """Variances around and above the largest fp32 number: draws of different
+    gains have the score infinity there, and the lowest feature wins.
+    Variances of rounding alone, near the smallest.  Enough nodes for a
+    node's draws to be searched one after the other."""
+    rng = np.random.default_rng(n)
+    X = rng.random((6, n)).astype(np.float32)
+    X[4:] = np.floor(X[4:] * 5)
+    if target.startswith("constant"):
+        y = np.full(n, float(target.split()[1]))
+    else:
+        y = float(target) * (rng.standard_normal(n) + X[1])
+    g, o = fit_both(X, y.astype(np.float32), algorithm=RF, task=capi.REGRESSION, n_trees=trees, k=3, max_depth=depth)
+    assert_same_forest(g, o)
