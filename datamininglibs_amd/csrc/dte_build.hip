@@ -81,6 +81,7 @@ struct DataArgs {
   const int64_t* T;  // T[x] = xlnx_fixed(x, igF) for x <= Tmax (classification)
   int64_t Tmax;
   const float* Tf;   // x ln x in fp32 for x < kTfMax (bounds of the random-forest search)
+  int no_bound;      // regression: a target is not finite, so sums wrap and only exact scores count
   // Joint build of several extra-trees forests in one set of level steps:
   // the data of batch tree t is forests[forest_of_tree[t]], whose D0 / R
   // are its mandatory and retry draws; C is the joint class width in every
@@ -1454,7 +1455,7 @@ __global__ void __launch_bounds__(kBlock) k_v2_bound(DataArgs d, LevelArgs lv, V
       float ub = -1.0f;
       if (w) {
         const double u = reg_box_bound((double)la, (double)(la + w), (double)(sa + sn), (double)(sa + sp), N, S, M);
-        ub = reg_score_bound(u * (1.0 + 2e-6) + E, d.shift);
+        ub = d.no_bound ? __builtin_inff() : reg_score_bound(u * (1.0 + 2e-6) + E, d.shift);
         if (la > 0) {
           const double g = variance_gain(la, su, it.n_w - la, it.ssum - su, 0);
           best = fmaxf(best, (float)ldexp_d(g, -2 * d.shift));
@@ -3523,7 +3524,7 @@ __device__ __forceinline__ void rf_bound_body(DataArgs d, LevelArgs lv, ItemArgs
 #pragma unroll
       for (int off = kWave / 2; off > 0; off >>= 1) M = fmax(M, __shfl_xor(M, off, kWave));
       nd.M = M * (1.0 + 1e-12);
-      nd.E = reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
+      nd.E = d.no_bound ? __builtin_inf() : reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
     }
     // the node's best score so far: the draws before this phase
     float best_score = 0.0f;
@@ -3655,7 +3656,7 @@ __device__ __forceinline__ void rf_bound_team_body(DataArgs d, LevelArgs lv, Ite
       __syncthreads();
       for (int x = 0; x < kWaves; ++x) M = fmax(M, L.eb[x]);
       nd.M = M * (1.0 + 1e-12);
-      nd.E = reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
+      nd.E = d.no_bound ? __builtin_inf() : reg_gain_error((double)nd.n, fabs((double)nd.mu) + nd.M);
     }
     float best_score = 0.0f;
     for (int q = 0; q < it.j0; ++q) best_score = fmaxf(best_score, it.res_score[(int64_t)o * it.D + q]);
@@ -6478,6 +6479,7 @@ void prepare_data(FitData& fd, const float* X_dev_in, const float* y_host, int64
   DevBuf<uint32_t>& label = fd.label;
   DevBuf<int64_t>& yfix = fd.yfix;
   int& shift = fd.shift;
+  int no_bound = 0;
   DevBuf<uint32_t>& K = fd.K;
   DevBuf<float>& SV = fd.SV;
   DevBuf<int64_t>& SVoff = fd.SVoff;
@@ -6500,7 +6502,12 @@ void prepare_data(FitData& fd, const float* X_dev_in, const float* y_host, int64
     DTE_HIP(hipStreamSynchronize(s));
   } else {
     double mx = 0;
-    for (int64_t i = 0; i < N; ++i) mx = std::max(mx, std::fabs((double)y_host[i]));
+    bool finite = true;
+    for (int64_t i = 0; i < N; ++i) {
+      mx = std::max(mx, std::fabs((double)y_host[i]));
+      finite = finite && std::isfinite(y_host[i]);
+    }
+    no_bound = finite ? 0 : 1;
     shift = fixed_shift(mx, N);
     fd.max_fixed = std::ldexp(mx, shift) + 1.0;
     std::vector<int64_t> yf(N);
@@ -6537,6 +6544,7 @@ void prepare_data(FitData& fd, const float* X_dev_in, const float* y_host, int64
   d.F = F;
   d.C = task == 0 ? C : 0;
   d.shift = shift;
+  d.no_bound = no_bound;
   d.seed = p.seed;
   d.min_node = p.min_node_size;
   d.max_depth = p.max_depth;

@@ -323,3 +323,16 @@ def test_rf_regression_scores_at_the_ends_of_fp32(target, n, trees, depth):
         y = float(target) * (rng.standard_normal(n) + X[1])
     g, o = fit_both(X, y.astype(np.float32), algorithm=RF, task=capi.REGRESSION, n_trees=trees, k=3, max_depth=depth)
     assert_same_forest(g, o)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("n,trees,depth", [(1500, 800, 4), (40_000, 4, 6)])
+def test_rf_regression_with_a_target_that_is_not_finite(bad, n, trees, depth):
+    """Such a target's fixed-point value is the least integer and sums wrap:
+    no bound of a gain holds, the scores are those of the oracle's sums."""
+    rng = np.random.default_rng(n)
+    X = rng.random((6, n)).astype(np.float32)
+    y = (rng.standard_normal(n) + X[1]).astype(np.float32)
+    y[n // 3] = bad
+    g, o = fit_both(X, y, algorithm=RF, task=capi.REGRESSION, n_trees=trees, k=3, max_depth=depth)
+    assert_same_forest(g, o)
