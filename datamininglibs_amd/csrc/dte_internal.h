@@ -236,8 +236,9 @@ struct Forest {
   DevBuf<PNode> pnodes;        // wide predict records (n_nodes), or empty
   // Build diagnostics (absent for imported forests).
   bool has_stats = false;
-  // Every tree's nodes in level order, children in their parents' order (a file
-  // from elsewhere may hold another order; it takes the wide predict records).
+  // Every tree's nodes in level order, children in their parents' order and
+  // tree (a file from elsewhere may hold another order, an imported model's
+  // root be another tree's child; they take the wide predict records).
   bool level_order = true;
   DevBuf<int32_t> feature, left, depth, count, n_entries;
   DevBuf<float> threshold, score, value;

@@ -628,11 +628,13 @@ __global__ void __launch_bounds__(kBlock) k_export_leaves(int64_t n, int T, cons
 }
 
 // Records and leaf payloads of export nodes [e0, e1); pos[e] = leaves before e.
+// level_order: children lie in their parents' trees (else a tree's root may be
+// another tree's child).
 __global__ void __launch_bounds__(kBlock) k_export(int64_t e0, int64_t e1, int T, const int64_t* __restrict__ ts,
                                                    const int32_t* __restrict__ feature,
                                                    const int32_t* __restrict__ left, const float* __restrict__ thr,
                                                    const float* __restrict__ value,
-                                                   const uint32_t* __restrict__ cls, int P,
+                                                   const uint32_t* __restrict__ cls, int P, bool level_order,
                                                    const uint32_t* __restrict__ pos, dte_node* __restrict__ nodes,
                                                    float* __restrict__ probs) {
   const uint32_t p0 = pos[e0];
@@ -642,7 +644,9 @@ __global__ void __launch_bounds__(kBlock) k_export(int64_t e0, int64_t e1, int T
     dte_node d;
     const int32_t f = feature[g];
     if (f >= 0) {
-      d.child_start = (int32_t)(T + (int64_t)left[g] - t - 1);
+      const int64_t l = left[g];
+      const int lt = level_order ? t : tree_of(l, T, ts);
+      d.child_start = !level_order && l == ts[lt] ? lt : (int32_t)(T + l - lt - 1);
       d.child_count = 2;
       d.probability_start = -1;
       d.attribute = f;
@@ -791,7 +795,7 @@ void export_forest(const Forest& f, dte_node* nodes, int64_t nodes_cap, float* p
     const int64_t e0 = c * kExportChunk, e1 = std::min(n, e0 + kExportChunk);
     hipLaunchKernelGGL(k_export, dim3(elementwise_grid(e1 - e0)), dim3(kBlock), 0, s, e0, e1, T, f.tree_start.p,
                        f.feature.p, f.left.p, f.threshold.p, f.value.p,
-                       f.task == 0 ? f.class_counts.p : (const uint32_t*)nullptr, P, pos.p, d_nodes.p, d_probs.p);
+                       f.task == 0 ? f.class_counts.p : (const uint32_t*)nullptr, P, f.level_order, pos.p, d_nodes.p, d_probs.p);
     DTE_HIP(hipGetLastError());
     DTE_HIP(hipMemcpyAsync(nodes + e0, d_nodes.p, sizeof(dte_node) * (e1 - e0), hipMemcpyDeviceToHost, s));
     if (first[c + 1] > first[c])

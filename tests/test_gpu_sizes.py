@@ -336,3 +336,25 @@ def test_rf_regression_with_a_target_that_is_not_finite(bad, n, trees, depth):
     y[n // 3] = bad
     g, o = fit_both(X, y, algorithm=RF, task=capi.REGRESSION, n_trees=trees, k=3, max_depth=depth)
     assert_same_forest(g, o)
+
+
+def test_import_of_a_root_that_is_another_trees_child():
+    """Roots 1 and 2, leaves, are the children of root 0: they lie side by
+    side, so the model stands, and exports as it came.  A root and another
+    node as children cannot lie side by side: refused."""
+    nodes = np.zeros(3, capi.NODE_DTYPE)
+    nodes["attribute"] = [0, -1, -1]
+    nodes["child_count"] = [2, 0, 0]
+    nodes["child_start"] = [1, -1, -1]
+    nodes["split_point"] = np.array([0.5, -1, -1], np.float32)
+    nodes["probability_start"] = [-1, 0, 1]
+    value = np.array([1, 10], np.float32)
+    g = capi.import_forest(nodes, value, 3, 1, 2, capi.REGRESSION)
+    X = np.random.default_rng(1).random((2, 500), dtype=np.float32)
+    assert np.array_equal(g.predict(X), np.where(X[0] < 0.5, 12, 21).astype(np.float32))
+    out, probs = g.export()
+    assert out["child_start"][0] == 1 and out["child_count"][:3].tolist() == [2, 0, 0]
+    assert probs[out["probability_start"][1]] == 1 and probs[out["probability_start"][2]] == 10
+    g.close()
+    with pytest.raises(Exception):  # roots 0 and 1, child 2 of root 0
+        capi.import_forest(nodes, value, 2, 1, 2, capi.REGRESSION)
