@@ -23,6 +23,9 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kWalkThreads = 512;  // a block's rows in LDS serve eight waves
+// Row blocks of a launch: it holds fewer than 2^32 threads in a direction.
+// More rows (537 M at 64 a block) take several launches.
+constexpr int64_t kMaxRowBlocks = 0xFFFFFFFFll / kWalkThreads;
 
 // ------------------------------------------------------ node layout ----
 // Bound by the rate of cache lines that come over the fabric for the deep
@@ -504,7 +507,8 @@ template <int TASK, int R, bool PACKED>
 __global__ void __launch_bounds__(kWalkThreads) k_oob(Trees tr, const float* __restrict__ X, int64_t N, int F,
                                                       const uint32_t* __restrict__ bits, int64_t words,
                                                       const float* __restrict__ y, int n_classes, int32_t tree0,
-                                                      uint64_t seed, int perm, int trees_per_block, OobSlot* slots) {
+                                                      uint64_t seed, int perm, int trees_per_block,
+                                                      int64_t block0, OobSlot* slots) {
   extern __shared__ float s_x[];  // R rows of F + 1 floats
   constexpr int RB = R ? R : 64;
   constexpr int NW = kWalkThreads / kWave;
@@ -515,7 +519,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_oob(Trees tr, const float* __r
   __shared__ double s_sse[NW];
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
-  const int64_t row0 = (int64_t)blockIdx.x * RB;
+  const int64_t row0 = (block0 + blockIdx.x) * RB;
   const int nr = (int)min<int64_t>(RB, N - row0);
   const int t0 = blockIdx.y * trees_per_block;
   const int t1 = min(tr.T, t0 + trees_per_block);
@@ -734,15 +738,17 @@ void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t
   const int64_t row_blocks = (N + RB - 1) / RB;
   const int chunks = tree_chunks(row_blocks, T, kWalkThreads / RB);
   const int tpb = (T + chunks - 1) / chunks;
-  const dim3 grid((unsigned)row_blocks, (unsigned)((T + tpb - 1) / tpb));
   const size_t lds = R ? sizeof(float) * (size_t)R * (f.n_features + 1) : 0;
   with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
     constexpr int kR = decltype(r)::value;
     constexpr bool kP = decltype(packed)::value;
     auto kernel = f.task == 0 ? k_oob<0, kR, kP> : k_oob<1, kR, kP>;
-    hipLaunchKernelGGL(kernel, grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
-                       (const uint32_t*)bits.p, words, (const float*)yv.p, f.n_classes, f.tree_offset, f.seed, perm,
-                       tpb, slots.p);
+    for (int64_t b0 = 0; b0 < row_blocks; b0 += kMaxRowBlocks) {
+      const dim3 grid((unsigned)std::min(row_blocks - b0, kMaxRowBlocks), (unsigned)((T + tpb - 1) / tpb));
+      hipLaunchKernelGGL(kernel, grid, dim3(kWalkThreads), lds, s, trees_of(f), X, N, f.n_features,
+                         (const uint32_t*)bits.p, words, (const float*)yv.p, f.n_classes, f.tree_offset, f.seed, perm,
+                         tpb, b0, slots.p);
+    }
   });
   DTE_HIP(hipGetLastError());
   std::vector<OobSlot> h(kOobSlots);
@@ -815,17 +821,22 @@ void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld,
     const int64_t row_blocks = (n_rows + RB - 1) / RB;
     const int chunks = tree_chunks(row_blocks, f.n_trees, kWalkThreads / RB);
     const int tpb = (f.n_trees + chunks - 1) / chunks;
-    const dim3 grid((unsigned)row_blocks, (unsigned)((f.n_trees + tpb - 1) / tpb));
+    const unsigned tree_blocks = (unsigned)((f.n_trees + tpb - 1) / tpb);
     const size_t lds = sizeof(uint32_t) * (size_t)RB * (C + (R ? F + 1 : 0));
     const int64_t nv = n_rows * C;
-    const int mode = grid.y > 1 ? kVoteAdd : float_votes ? kVoteFloat : kVoteInt;
+    const int mode = tree_blocks > 1 ? kVoteAdd : float_votes ? kVoteFloat : kVoteInt;
     // votes cleared by a kernel (no memset node if the caller captures)
     if (mode == kVoteAdd)
       hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(nv)), dim3(kBlock), 0, s, reinterpret_cast<uint32_t*>(votes),
                          nv);
     with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
-      hipLaunchKernelGGL((k_predict_cls<decltype(r)::value, decltype(packed)::value>), grid, dim3(kWalkThreads), lds,
-                         s, trees_of(f), X, n_rows, ld, row_major, C, F, tpb, mode, (void*)votes);
+      for (int64_t r0 = 0; r0 < n_rows; r0 += kMaxRowBlocks * RB) {
+        const int64_t rows = std::min(n_rows - r0, kMaxRowBlocks * RB);
+        hipLaunchKernelGGL((k_predict_cls<decltype(r)::value, decltype(packed)::value>),
+                           dim3((unsigned)((rows + RB - 1) / RB), tree_blocks), dim3(kWalkThreads), lds, s,
+                           trees_of(f), row_major ? X + r0 * ld : X + r0, rows, ld, row_major, C, F, tpb, mode,
+                           (void*)(votes + r0 * C));
+      }
     });
     if (mode == kVoteAdd && float_votes)
       hipLaunchKernelGGL(k_votes_to_float, dim3(elementwise_grid(nv)), dim3(kBlock), 0, s, votes, nv);
@@ -836,9 +847,12 @@ void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld,
     const int RB = R ? R : 64;
     const size_t lds = sizeof(float) * (size_t)RB * (reg_chunk(R) + 1 + (R ? F + 1 : 0));
     with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
-      hipLaunchKernelGGL((k_predict_reg<decltype(r)::value, decltype(packed)::value>),
-                         dim3((unsigned)((n_rows + RB - 1) / RB)), dim3(kWalkThreads), lds, s, trees_of(f), X, n_rows,
-                         ld, row_major, F, sums);
+      for (int64_t r0 = 0; r0 < n_rows; r0 += kMaxRowBlocks * RB) {
+        const int64_t rows = std::min(n_rows - r0, kMaxRowBlocks * RB);
+        hipLaunchKernelGGL((k_predict_reg<decltype(r)::value, decltype(packed)::value>),
+                           dim3((unsigned)((rows + RB - 1) / RB)), dim3(kWalkThreads), lds, s, trees_of(f),
+                           row_major ? X + r0 * ld : X + r0, rows, ld, row_major, F, sums + r0);
+      }
     });
   }
   DTE_HIP(hipGetLastError());

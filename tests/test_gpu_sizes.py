@@ -1,5 +1,7 @@
 """HIP kernels at the sizes where their tiers, tiles and staging change, bit
 for bit against the CPU oracle (or a plain walk of the model)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -358,3 +360,82 @@ def test_import_of_a_root_that_is_another_trees_child():
     g.close()
     with pytest.raises(Exception):  # roots 0 and 1, child 2 of root 0
         capi.import_forest(nodes, value, 2, 1, 2, capi.REGRESSION)
+
+
+def _stumps(task):
+    """Three trees of one split each, at 0.25, 0.5 and 0.75 of the only feature."""
+    nodes = np.zeros(9, capi.NODE_DTYPE)
+    inner = np.arange(9) < 3
+    nodes["attribute"] = np.where(inner, 0, -1)
+    nodes["child_count"] = np.where(inner, 2, 0)
+    nodes["child_start"] = np.where(inner, 3 + 2 * np.arange(9), -1)
+    nodes["split_point"] = np.where(inner, 0.25 * (1 + np.arange(9)), -1).astype(np.float32)
+    width = 1 if task else 2
+    nodes["probability_start"] = np.where(inner, -1, width * (np.arange(9) - 3))
+    probs = np.array([1, 10] * 3 if task else [1, 0, 0, 1] * 3, np.float32)
+    return capi.import_forest(nodes, probs, 3, width, 1, task)
+
+
+def _repeated(values, n):
+    """values, a prime number of them, over and over: no two blocks alike."""
+    return np.resize(values, n)
+
+
+@pytest.mark.parametrize("task,row_major", [(capi.CLASSIFICATION, 0), (capi.REGRESSION, 1)])
+def test_predict_of_more_rows_than_a_launch_holds(task, row_major):
+    """2^32 threads are 537 M rows at 64 a block of 512."""
+    n = (1 << 29) + 777
+    x = np.random.default_rng(1).random(1_000_003, dtype=np.float32)
+    right = (x >= 0.25).astype(np.int32) + (x >= 0.5) + (x >= 0.75)
+    g = _stumps(task)
+    X = capi.DeviceArray.from_numpy(_repeated(x, n))
+    width = 1 if task else 2
+    out = np.full((n, width), -1, np.float32 if task else np.int32)
+    D = capi.DeviceArray.from_numpy(out)
+    p = ctypes.c_void_p
+    capi._check(capi.lib().dte_predict_device(g.handle, p(X.ptr), n, 1 if row_major else n, row_major,
+                                              None if task else p(D.ptr), p(D.ptr) if task else None, None))
+    capi._check(capi.lib().dte_memcpy_to_host(0, p(out.ctypes.data), p(D.ptr), out.nbytes))
+    if task:
+        assert np.array_equal(out[:, 0], _repeated((3 + 9 * right).astype(np.float32), n))
+    else:
+        want = np.stack([3 - right, right], 1)
+        assert np.array_equal(out.reshape(-1), _repeated(want, 2 * n))
+    g.close()
+    X.free()
+    D.free()
+
+
+def test_out_of_bag_of_more_rows_than_a_launch_holds(tmp_path):
+    """Every row's label is what its tree says, so all pairs are right; a
+    bootstrap leaves a row out with probability 1 / e."""
+    n = (1 << 29) + 777
+    Xf = np.linspace(0, 1, 64, dtype=np.float32).reshape(1, -1)
+    g = capi.fit(Xf, (Xf[0] >= 0.5).astype(np.float32), capi.default_params(RF, n_trees=1, n_classes=2, max_depth=2))
+    thr = float(g.canonical()["threshold"][0])
+    path = tmp_path / "forest"
+    g.save(path)
+    g.close()
+    raw = bytearray(path.read_bytes())
+    at = 8 + 4 + 8 * 4 + 8  # fit_rows
+    assert int.from_bytes(raw[at:at + 8], "little") == 64
+    raw[at:at + 8] = n.to_bytes(8, "little")
+    h = 0xCBF29CE484222325
+    for b in raw[:-8]:
+        h = (h ^ b) * 0x100000001B3 & (2 ** 64 - 1)
+    raw[-8:] = h.to_bytes(8, "little")
+    path.write_bytes(bytes(raw))
+    g = capi.load_forest(path)
+    x = np.random.default_rng(1).random(1_000_003, dtype=np.float32)
+    y = _repeated((x >= thr).astype(np.float32), n)
+    X = capi.DeviceArray.from_numpy(_repeated(x, n))
+    pairs, good = capi.oob_evaluate(g, X.ptr, y, n)
+    assert good == pairs
+    # the count of rows left out has variance N (1 / e - 2 / e^2)
+    assert abs(pairs - n / np.e) < 6 * np.sqrt(0.0973 * n)
+    y[-1] = 1 - y[-1]
+    y[0] = 1 - y[0]
+    pairs2, good2 = capi.oob_evaluate(g, X.ptr, y, n)
+    assert pairs2 == pairs and pairs - 2 <= good2 <= pairs
+    g.close()
+    X.free()
