@@ -6150,10 +6150,11 @@ constexpr int kV2TargetDiv = 6;
 
 // Chunk-parallel search of the big items of one phase (see k_v2_*): items in
 // batches of at most kV2Batch scratch slots (a slot per unit of bootstrap
-// weight, the bound of a bucket's entries).  A batch's scratch is 16 B
-// (classification) to 40 B (regression) per slot, so 1.5 Gi slots hold most
+// weight, the bound of a bucket's entries).  A batch's scratch is four words a
+// slot, and two targets for regression, so 1.5 Gi slots (24 or 48 GB) hold most
 // of a level of a 200-tree 1M-row fit in one batch.
 constexpr int64_t kV2Batch = (int64_t)1536 << 20;
+constexpr size_t v2_slot_bytes(int task) { return 4 * sizeof(uint32_t) + (task == 1 ? 2 * sizeof(int64_t) : 0); }
 
 template <int MAXC, int TASK>
 void big_pipeline(BigState& B, const DataArgs& d, const LevelArgs& lv, const ItemArgs& it, const uint32_t* groups,
@@ -6959,9 +6960,12 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   bool use_rows = algorithm == DTE_RANDOM_FOREST && !plain && key_rows_pay(d.N, d.F, D0);
   if (use_rows) {
     size_t free_b = 0, total_b = 0;
+    int dev;
+    DTE_HIP(hipGetDevice(&dev));
     DTE_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += pool_cached(dev);  // what an earlier fit left counts as free
     const int64_t slots = std::min<int64_t>(kV2Batch, (int64_t)T * N * D0) + N;
-    const size_t batch = (size_t)slots * (task == 0 ? 16 : 32);
+    const size_t batch = (size_t)(slots + slots / 4) * v2_slot_bytes(task);  // reserve() adds a quarter
     use_rows = 4 * ((size_t)d.N * FS + (size_t)E * D0) + batch <= free_b / 2;
   }
   if (use_rows) {

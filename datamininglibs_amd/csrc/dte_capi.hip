@@ -195,6 +195,15 @@ void pool_free(void* p, size_t bytes, int dev, hipStream_t owner) {
   g_pool[{dev, owner}].emplace(bytes, p);
 }
 
+size_t pool_cached(int dev) {
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  size_t bytes = 0;
+  for (const auto& kv : g_pool)
+    if (kv.first.first == dev)
+      for (const auto& b : kv.second) bytes += b.first;
+  return bytes;
+}
+
 size_t pool_trim() {
   std::lock_guard<std::mutex> lk(g_pool_mu);
   size_t freed = 0;

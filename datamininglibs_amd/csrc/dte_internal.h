@@ -52,6 +52,9 @@ void* pool_alloc(size_t bytes, size_t* got, int* dev, hipStream_t* owner);
 void pool_free(void* p, size_t bytes, int dev, hipStream_t owner);
 // Frees every cached block (all devices); returns the bytes released.
 size_t pool_trim();
+// Bytes of the cached blocks of a device: free to a fit as hipMemGetInfo's are,
+// since an allocation that finds no memory trims the pool.
+size_t pool_cached(int dev);
 bool pool_on();  // inside a PoolScope (and not suspended) on this thread
 
 struct PoolScope {

@@ -439,3 +439,41 @@ def test_out_of_bag_of_more_rows_than_a_launch_holds(tmp_path):
     assert pairs2 == pairs and pairs - 2 <= good2 <= pairs
     g.close()
     X.free()
+
+
+def test_a_second_fit_takes_the_row_major_keys_like_the_first():
+    """The scratch that a fit leaves cached is free to the next one: with
+    little other memory it must not turn the row-major keys away."""
+    n, f, k = 2_100_011, 16, 6
+    rng = np.random.default_rng(17)
+    X = capi.DeviceArray.from_numpy(rng.random((f, n), dtype=np.float32))
+    y = rng.integers(0, 5, n).astype(np.float32)
+    p = capi.default_params(RF, n_trees=1, n_features_per_node=k, max_depth=6, n_classes=5)
+
+    def gathers():
+        capi.profile_reset()
+        capi.profiling(True)
+        g = capi.fit_device(X.ptr, n, f, y, p)
+        capi.profiling(False)
+        g.close()
+        return capi.profile_stats().get("gather_draws", {"launches": 0})["launches"]
+
+    capi.release_cached_memory()
+    first = gathers()
+    assert first > 0
+    scratch = capi.release_cached_memory()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    fill = []
+    try:
+        for _ in range(2):  # what is left after a large allocation may be more than was free beside it
+            assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            if free.value > scratch + (620 << 20):
+                fill.append(capi.DeviceArray(free.value - scratch - (600 << 20)))
+        assert gathers() == first
+        assert gathers() == first
+    finally:
+        for b in fill:
+            b.free()
+        X.free()
+        capi.release_cached_memory()
