@@ -1,6 +1,8 @@
-// Limits of the bounded split search that its LDS arrays are sized by.  Plain
-// C++: host code can check them without the kernels.
+// Limits that LDS arrays are sized by: the bounded split search and the
+// out-of-bag pass.  Plain C++: host code can check them without the kernels.
 #pragma once
+
+#include <cstdint>
 
 namespace dte {
 
@@ -17,5 +19,11 @@ constexpr int kTeamStack = kBoundWeight / (kBoundRun + 1);
 
 // The wave tier decides by entries, and a node's entries bound its ranges.
 constexpr int wave_stack(int entries) { return entries / (kBoundRun + 1); }
+
+// Rows whose in-bag bits a workgroup of the out-of-bag pass holds, and their
+// words: at most 64 KB, what any launch may have.
+constexpr int64_t kBagRange = (int64_t)1 << 19;
+constexpr int64_t bag_lds_bytes(int64_t rows) { return ((rows < kBagRange ? rows : kBagRange) + 31) / 32 * 4; }
+static_assert(bag_lds_bytes(kBagRange) == 65536, "");
 
 }  // namespace dte

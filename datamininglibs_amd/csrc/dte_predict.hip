@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "dte_internal.h"
+#include "dte_limits.h"
 
 namespace dte {
 namespace {
@@ -453,7 +454,6 @@ constexpr uint32_t kStreamImp = 0x00706d69u;
 // (tree, range of kBagRange rows): every draw of the tree is generated, the
 // range's bits are set in LDS and written out once.
 constexpr int kBagThreads = 1024;
-constexpr int64_t kBagRange = (int64_t)1 << 19;  // rows per workgroup: at most 64 KB of bits
 // Workgroups beside each other on a tree's draws, so that few trees fill the
 // chip (100 trees of 200,003 rows: 0.115 ms at one workgroup a tree, 0.05 ms at five);
 // with several, each adds its bits to words that start at zero.
@@ -729,7 +729,7 @@ void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t
   if (parts > 1)
     hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(words * T)), dim3(kBlock), 0, s, bits.p, words * T);
   hipLaunchKernelGGL(k_inbag_bits_lds, dim3((unsigned)T, (unsigned)ranges, parts), dim3(kBagThreads),
-                     4 * (std::min(N, kBagRange) + 31) / 32, s, bits.p, N, words, f.tree_offset, f.seed);
+                     (unsigned)bag_lds_bytes(N), s, bits.p, N, words, f.tree_offset, f.seed);
   DevBuf<float> yv(N);
   DTE_HIP(hipMemcpyAsync(yv.p, targets, 4 * N, hipMemcpyHostToDevice, s));
   DevBuf<OobSlot> slots(kOobSlots);

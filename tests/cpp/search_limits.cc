@@ -1,6 +1,7 @@
 // Host model of the workgroup tier's ranges (dte_build.hip:
 // rf_bound_team_body): every bucket that may be split again is pushed before
 // the last one pushed is taken.  Prints the most ranges that wait at a time.
+// With an argument: the words of the out-of-bag pass instead.
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
@@ -50,7 +51,17 @@ int most_waiting(const std::vector<Entry>& node, int log_buckets) {
   return (int)most;
 }
 
-int main() {
+// In-bag bits of the out-of-bag pass: whole words, no more than needed.
+bool bag_words_fit() {
+  for (int64_t rows : {1, 31, 32, 33, 40, 64, 1000, (1 << 19) - 1, 1 << 19, (1 << 19) + 1, 1 << 30}) {
+    const int64_t held = std::min(rows, kBagRange), bytes = bag_lds_bytes(rows);
+    if (bytes % 4 || bytes > 65536 || bytes * 8 < held || bytes * 8 >= held + 32) return false;
+  }
+  return true;
+}
+
+int main(int argc, char**) {
+  if (argc > 1) return bag_words_fit() ? 0 : 1;
   std::mt19937 rng(1);
   int most = 0;
   for (int log_buckets : {7, 8}) {

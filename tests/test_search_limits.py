@@ -6,9 +6,19 @@ import subprocess
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def test_ranges_of_the_workgroup_tier_fit_their_stack(tmp_path):
+def _build(tmp_path):
     exe = str(tmp_path / "search_limits")
     subprocess.run(["g++", "-O2", "-std=c++17", "-o", exe, os.path.join(HERE, "cpp", "search_limits.cc")], check=True)
+    return exe
+
+
+def test_in_bag_bits_of_a_workgroup_take_whole_words(tmp_path):
+    """Every row count's bits fit, in no more words than they need."""
+    assert subprocess.run([_build(tmp_path), "bag"], timeout=60).returncode == 0
+
+
+def test_ranges_of_the_workgroup_tier_fit_their_stack(tmp_path):
+    exe = _build(tmp_path)
     p = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, p.stdout
     # a bootstrapped node alone holds more ranges than its entries suggest
