@@ -6930,6 +6930,10 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
   const RfAllFn rf_all = pick_rf_all(task, C);
   LevelArgs lv{};
   int64_t trace_tier[3] = {0, 0, 0};
+  // Keys of a level's first draws by entry (k_gather_draws), read on the side
+  // stream: declared before it, so that a fit that fails gives them up after
+  // the stream's last wait.
+  DevBuf<uint32_t> key_rows, draw_keys, draw_tiles, draw_toff;
   // Side stream of the split search's tiers beside the chunk pipeline
   // (created on first use; default priority).
   struct SideStream {
@@ -6952,11 +6956,10 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
       }
     }
   } side;
-  // Keys of a level's first draws by entry (k_gather_draws), if they pay and,
-  // with the scratch of the chunk pipeline's largest batch, leave half of the
-  // free memory; without them the searches gather from K.
+  // The draws' keys are gathered if they pay and, with the scratch of the chunk
+  // pipeline's largest batch, leave half of the free memory; without them the
+  // searches gather from K.
   const int FS = (d.F + 15) / 16 * 16;
-  DevBuf<uint32_t> key_rows, draw_keys, draw_tiles, draw_toff;
   bool use_rows = algorithm == DTE_RANDOM_FOREST && !plain && key_rows_pay(d.N, d.F, D0);
   if (use_rows) {
     size_t free_b = 0, total_b = 0;

@@ -25,3 +25,13 @@ def test_ranges_of_the_workgroup_tier_fit_their_stack(tmp_path):
     # (2048 entries: 33 ranges of more than 64)
     bootstrap = max(int(line.split()[1]) for line in p.stdout.splitlines() if line.startswith("bootstrap"))
     assert bootstrap > 2048 // 64 + 1
+
+
+def test_buffers_of_the_side_stream_outlive_it():
+    """A fit's buffers go back to the pool in the reverse order of their
+    declarations: those that kernels of the side stream read come before it."""
+    src = open(os.path.join(HERE, "..", "datamininglibs_amd", "csrc", "dte_build.hip")).read()
+    side = src.index("struct SideStream {")
+    for buffer in ("key_rows, draw_keys", "rowA, auxA", "res_score, res_thr", "BigState bigst", "tier_list[kMaxTiers]"):
+        at = src.index(buffer)
+        assert src.rindex("Forest* fit_batch(", 0, side) < at < side, buffer
