@@ -176,17 +176,24 @@ void* pool_alloc(size_t bytes, size_t* got, int* dev, hipStream_t* owner) {
       return p;
     }
   }
+  void* p = device_malloc(want);
+  *got = want;
+  return p;
+}
+
+void* device_malloc(size_t bytes) {
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, want);
+  hipError_t e = hipMalloc(&p, bytes);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     pool_trim();
-    e = hipMalloc(&p, want);
+    e = hipMalloc(&p, bytes);
   }
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
     fail(e == hipErrorOutOfMemory ? DTE_ERR_OUT_OF_MEMORY : DTE_ERR_HIP,
          std::string("hipMalloc: ") + hipGetErrorString(e));
-  *got = want;
+  }
   return p;
 }
 
@@ -1091,9 +1098,7 @@ int dte_device_alloc(int32_t device_id, int64_t bytes, void** out) {
   return guarded([&] {
     if (!out || bytes < 0) fail(DTE_ERR_INVALID_ARGUMENT, "bad arguments");
     set_device(device_id);
-    void* p = nullptr;
-    DTE_HIP(hipMalloc(&p, bytes > 0 ? (size_t)bytes : 1));
-    *out = p;
+    *out = device_malloc(bytes > 0 ? (size_t)bytes : 1);
   });
 }
 

@@ -35,7 +35,8 @@ void select_device(int device);
   } while (0)
 
 // ------------------------------------------------------- scratch pool --
-// Device blocks of a fit's temporaries are cached per (device, stream) when
+// Device blocks of the temporaries of a fit, an export, an out-of-bag pass and
+// a forest's predict records are cached per (device, stream) when
 // released and handed back to later requests on the same stream, so that the
 // growing per-level buffers and repeated fits do not call hipMalloc / hipFree
 // (which synchronise the device) inside the level loop.  Reuse on the same
@@ -52,6 +53,8 @@ void* pool_alloc(size_t bytes, size_t* got, int* dev, hipStream_t* owner);
 void pool_free(void* p, size_t bytes, int dev, hipStream_t owner);
 // Frees every cached block (all devices); returns the bytes released.
 size_t pool_trim();
+// hipMalloc; without memory once more after pool_trim.
+void* device_malloc(size_t bytes);
 // Bytes of the cached blocks of a device: free to a fit as hipMemGetInfo's are,
 // since an allocation that finds no memory trims the pool.
 size_t pool_cached(int dev);
@@ -112,7 +115,7 @@ struct DevBuf {
       pooled = true;
       n = count;
     } else {
-      DTE_HIP(hipMalloc((void**)&p, count * sizeof(T)));
+      p = (T*)device_malloc(count * sizeof(T));
       pooled = false;
       n = count;
     }

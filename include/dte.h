@@ -302,8 +302,11 @@ int dte_device_free(int32_t device_id, void* ptr);
 int dte_memcpy_to_device(int32_t device_id, void* dst, const void* src, int64_t bytes);
 int dte_memcpy_to_host(int32_t device_id, void* dst, const void* src, int64_t bytes);
 
-/* Frees the device memory a fit keeps cached for later fits on the same
- * stream (its per-level scratch; see dte_fit).  The reference allocates and
+/* Frees the device memory that fits keep cached for later fits on the same
+ * stream (their per-level scratch; see dte_fit), and that exports, out-of-bag
+ * passes, imports and loads keep likewise (an export of 8 Mi nodes and more
+ * about 160 MB, its leaf payloads and 8 bytes a node).  The library does so by
+ * itself when one of its own allocations finds no memory.  The reference allocates and
  * frees its buffers around every fit (gpudte_algorithm.cc:486-596,
  * gpudte_algorithm_shared.cc:30-52), so it has no counterpart; callers that
  * size other allocations from the free memory call this first.

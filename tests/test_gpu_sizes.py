@@ -441,6 +441,19 @@ def test_out_of_bag_of_more_rows_than_a_launch_holds(tmp_path):
     X.free()
 
 
+def _leave_free(left):
+    """Allocations that leave about `left` bytes of the device free.  (What is
+    left after a large one may be more than was free beside it: twice.)"""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    fill = []
+    for _ in range(2):
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        if free.value > left + (20 << 20):
+            fill.append(capi.DeviceArray(free.value - left))
+    return fill
+
+
 def test_a_second_fit_takes_the_row_major_keys_like_the_first():
     """The scratch that a fit leaves cached is free to the next one: with
     little other memory it must not turn the row-major keys away."""
@@ -462,18 +475,36 @@ def test_a_second_fit_takes_the_row_major_keys_like_the_first():
     first = gathers()
     assert first > 0
     scratch = capi.release_cached_memory()
-    hip = ctypes.CDLL("libamdhip64.so.7")
-    free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    fill = []
+    fill = _leave_free(scratch + (600 << 20))
     try:
-        for _ in range(2):  # what is left after a large allocation may be more than was free beside it
-            assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-            if free.value > scratch + (620 << 20):
-                fill.append(capi.DeviceArray(free.value - scratch - (600 << 20)))
         assert gathers() == first
         assert gathers() == first
     finally:
         for b in fill:
             b.free()
         X.free()
+        capi.release_cached_memory()
+
+
+def test_cached_scratch_gives_way_to_allocations_of_the_library():
+    """What an out-of-bag pass and a fit leave cached is no loss to a caller
+    of the library who needs the memory."""
+    n, f = 1_000_003, 32
+    rng = np.random.default_rng(2)
+    X = capi.DeviceArray.from_numpy(rng.random((f, n), dtype=np.float32))
+    y = rng.integers(0, 3, n).astype(np.float32)
+    g = capi.fit_device(X.ptr, n, f, y, capi.default_params(RF, n_trees=4, max_depth=4, n_classes=3))
+    capi.release_cached_memory()
+    fill = _leave_free(1 << 30)
+    try:
+        capi.oob_evaluate(g, X.ptr, y, n)
+        h = capi.fit_device(X.ptr, n, f, y, capi.default_params(RF, n_trees=1, max_depth=2, n_classes=3))
+        h.close()
+        held = capi.DeviceArray(900 << 20)  # more than is left beside the scratch
+        held.free()
+    finally:
+        for b in fill:
+            b.free()
+        X.free()
+        g.close()
         capi.release_cached_memory()
