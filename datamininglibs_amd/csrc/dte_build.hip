@@ -48,8 +48,6 @@ const LnTable& host_ln_table();
 namespace {
 
 constexpr int kIpt = 8;                 // elements per thread in the LDS sort
-constexpr int kTeamIpt = 8;             // entries per lane of the wave-per-item tier
-static_assert(kWave * kTeamIpt >= kMaxCutTeam, "wave tier capacity");
 constexpr int kCap = kBlock * kIpt;     // LDS chunk capacity (2048)
 constexpr int kHistWords = 8192;        // LDS histogram words (32 KB)
 constexpr int kMaxBuckets = 2048;       // bucket table of the big-item path
@@ -794,11 +792,11 @@ __device__ __forceinline__ void load_tables(double* s_inv, double* s_logc) {
   }
 }
 
-// Node statistics of one item, computed by every lane of the team.
-template <int MAXC, int TASK, int TEAM, int IPT, class LX>
+// Node statistics of one item, computed by the whole workgroup.
+template <int MAXC, int TASK>
 __device__ __forceinline__ bool node_context(const DataArgs& d, const LevelArgs& lv, uint32_t i, NodeCtx& nc,
-                                             TeamLds<MAXC, TASK, TEAM, IPT>& L, const LX& lx) {
-  const int t = team_tid<TEAM>();
+                                             TeamLds<MAXC, TASK, kBlock, kIpt>& L, const LnCtx& lx) {
+  const int t = threadIdx.x;
   nc.C = d.C;
   nc.n = lv.count[i];
   nc.ssum = 0;
@@ -807,10 +805,10 @@ __device__ __forceinline__ bool node_context(const DataArgs& d, const LevelArgs&
   if constexpr (TASK == 0) {
     const uint32_t my = t < d.C ? lv.cls[(int64_t)i * d.C + t] : 0u;
     if (t < d.C) L.ncls[t] = my;
-    const uint32_t mx = team_reduce_max<TEAM>(my, L.w);
+    const uint32_t mx = team_reduce_max<kBlock>(my, L.w);
     const int64_t tn = t < d.C ? lx.t(my) : 0;
     int64_t tsum = 0;  // sum of T(n_c) over the classes (lanes < C)
-    (void)team_excl_scan_i64<TEAM>(tn, L.w64, &tsum);
+    (void)team_excl_scan_i64<kBlock>(tn, L.w64, &tsum);
     nc.P = lx.t((uint64_t)nc.n) - tsum;
     nc.inv = 1.0 / ((double)nc.n * kLn2);
     return (int64_t)mx == nc.n;  // pure node
@@ -820,14 +818,14 @@ __device__ __forceinline__ bool node_context(const DataArgs& d, const LevelArgs&
   }
 }
 
-// Evaluate one RF item on a team; returns through L.cr.  BIG: the item may
-// exceed the team's LDS capacity (whole-workgroup teams of the plain driver):
-// bucket it through the workgroup's scratch slab.
-template <int MAXC, int TASK, int TEAM, int IPT, bool BIG>
+// Evaluate one RF item on a workgroup; returns through L.cr.  An item above
+// the LDS capacity is bucketed through the workgroup's scratch slab.
+template <int MAXC, int TASK>
 __device__ void rf_item(const DataArgs& d, const LevelArgs& lv, const ItemArgs& it, int f, uint32_t i, const NodeCtx& nc,
-                        TeamLds<MAXC, TASK, TEAM, IPT>& L, const LnCtx& lx, uint32_t* s_boff, int team_index) {
-  constexpr int CAP = TeamLds<MAXC, TASK, TEAM, IPT>::CAP;
-  const int t = team_tid<TEAM>();
+                        TeamLds<MAXC, TASK, kBlock, kIpt>& L, const LnCtx& lx, uint32_t* s_boff) {
+  constexpr int IPT = kIpt;
+  constexpr int CAP = kCap;
+  const int t = threadIdx.x;
   const int m = lv.m[i];
   const int64_t st = lv.start[i];
   const uint32_t* Kf = d.K + (int64_t)f * d.N;
@@ -846,7 +844,7 @@ __device__ void rf_item(const DataArgs& d, const LevelArgs& lv, const ItemArgs& 
     uint32_t rows[IPT];
 #pragma unroll
     for (int q = 0; q < IPT; ++q) {
-      const int e = t + q * TEAM;
+      const int e = t + q * kBlock;
       if (e < m) {
         rows[q] = lv.row[st + e];
         L.aux[e] = lv.aux[st + e];
@@ -855,7 +853,7 @@ __device__ void rf_item(const DataArgs& d, const LevelArgs& lv, const ItemArgs& 
     }
 #pragma unroll
     for (int q = 0; q < IPT; ++q) {
-      const int e = t + q * TEAM;
+      const int e = t + q * kBlock;
       if (e < m) {
         const uint32_t key = Kf[rows[q]];
         L.u.srt.k[0][e] = key;
@@ -864,126 +862,124 @@ __device__ void rf_item(const DataArgs& d, const LevelArgs& lv, const ItemArgs& 
         kmax = max(kmax, key);
       }
     }
-    kmin = team_reduce_min<TEAM>(kmin, L.w);
-    kmax = team_reduce_max<TEAM>(kmax, L.w);
-    for (int e = t; e < m; e += TEAM) L.u.srt.k[0][e] -= kmin;
-    team_sync<TEAM>();
-    sort_and_eval<MAXC, TASK, TEAM, IPT>(m, bit_length(kmax - kmin), kmin, nc, L, lx);
+    kmin = team_reduce_min<kBlock>(kmin, L.w);
+    kmax = team_reduce_max<kBlock>(kmax, L.w);
+    for (int e = t; e < m; e += kBlock) L.u.srt.k[0][e] -= kmin;
+    __syncthreads();
+    sort_and_eval<MAXC, TASK, kBlock, IPT>(m, bit_length(kmax - kmin), kmin, nc, L, lx);
     return;
   }
-  if constexpr (TEAM == 256 && BIG) {
-    // Big node: bucket by dense key into this block's scratch slab, then
-    // pack consecutive buckets into LDS-sized chunks.
-    const uint32_t S = d.S[f];
-    const int words = (TASK == 0) ? d.C : 3;
-    int wbits = 0;
-    while ((1 << (wbits + 1)) * words <= kHistWords) ++wbits;
-    while (((S + (1u << wbits) - 1) >> wbits) > (uint32_t)kMaxBuckets) ++wbits;
-    const int W = 1 << wbits;
-    const int NB = (int)((S + (uint32_t)W - 1) >> wbits);
-    uint32_t* skey = it.scr_key + (int64_t)team_index * it.scr_stride;
-    uint32_t* saux = it.scr_aux + (int64_t)team_index * it.scr_stride;
-    int64_t* sy = TASK == 1 ? it.scr_y + (int64_t)team_index * it.scr_stride : nullptr;
-    for (int b = t; b <= NB; b += 256) s_boff[b] = 0;
+  // Big node: bucket by dense key into this block's scratch slab, then
+  // pack consecutive buckets into LDS-sized chunks.
+  const uint32_t S = d.S[f];
+  const int words = (TASK == 0) ? d.C : 3;
+  int wbits = 0;
+  while ((1 << (wbits + 1)) * words <= kHistWords) ++wbits;
+  while (((S + (1u << wbits) - 1) >> wbits) > (uint32_t)kMaxBuckets) ++wbits;
+  const int W = 1 << wbits;
+  const int NB = (int)((S + (uint32_t)W - 1) >> wbits);
+  uint32_t* skey = it.scr_key + (int64_t)blockIdx.x * it.scr_stride;
+  uint32_t* saux = it.scr_aux + (int64_t)blockIdx.x * it.scr_stride;
+  int64_t* sy = TASK == 1 ? it.scr_y + (int64_t)blockIdx.x * it.scr_stride : nullptr;
+  for (int b = t; b <= NB; b += 256) s_boff[b] = 0;
+  __syncthreads();
+  constexpr int U = 8;
+  for (int e0 = 0; e0 < m; e0 += 256 * U) {
+    uint32_t rows[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int e = e0 + t + q * 256;
+      rows[q] = e < m ? lv.row[st + e] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int e = e0 + t + q * 256;
+      if (e < m) atomicAdd(&s_boff[Kf[rows[q]] >> wbits], 1u);
+    }
+  }
+  __syncthreads();
+  {
+    const int per = (NB + 255) / 256;
+    const int b0 = t * per, b1 = min(b0 + per, NB);
+    uint32_t loc = 0;
+    for (int b = b0; b < b1; ++b) loc += s_boff[b];
+    uint32_t base = team_excl_scan<256>(loc, L.w, nullptr);
+    for (int b = b0; b < b1; ++b) {
+      const uint32_t c = s_boff[b];
+      s_boff[b] = base;
+      base += c;
+    }
+    if (t == 0) s_boff[NB] = (uint32_t)m;
     __syncthreads();
-    constexpr int U = 8;
-    for (int e0 = 0; e0 < m; e0 += 256 * U) {
-      uint32_t rows[U];
+    for (int b = t; b < NB; b += 256) L.u.bpos[b] = s_boff[b];
+    __syncthreads();
+  }
+  for (int e0 = 0; e0 < m; e0 += 256 * U) {
+    uint32_t rows[U], auxv[U], keys[U];
+    int64_t yv[U];
 #pragma unroll
-      for (int q = 0; q < U; ++q) {
-        const int e = e0 + t + q * 256;
-        rows[q] = e < m ? lv.row[st + e] : 0u;
+    for (int q = 0; q < U; ++q) {
+      const int e = e0 + t + q * 256;
+      if (e < m) {
+        rows[q] = lv.row[st + e];
+        auxv[q] = lv.aux[st + e];
+        if (TASK == 1) yv[q] = lv.ey[st + e];
       }
+    }
 #pragma unroll
-      for (int q = 0; q < U; ++q) {
-        const int e = e0 + t + q * 256;
-        if (e < m) atomicAdd(&s_boff[Kf[rows[q]] >> wbits], 1u);
+    for (int q = 0; q < U; ++q) {
+      const int e = e0 + t + q * 256;
+      if (e < m) keys[q] = Kf[rows[q]];
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int e = e0 + t + q * 256;
+      if (e < m) {
+        const uint32_t pos = atomicAdd(&L.u.bpos[keys[q] >> wbits], 1u);
+        skey[pos] = keys[q];
+        saux[pos] = auxv[q];
+        if (TASK == 1) sy[pos] = yv[q];
       }
+    }
+  }
+  __syncthreads();
+  int b = 0;
+  while (b < NB) {
+    const uint32_t cb = s_boff[b + 1] - s_boff[b];
+    if (cb == 0) {
+      ++b;
+      continue;
+    }
+    if (cb > (uint32_t)CAP) {
+      eval_hist_bucket<MAXC, TASK, IPT>(skey + s_boff[b], saux + s_boff[b], TASK == 1 ? sy + s_boff[b] : nullptr,
+                                        cb, (uint32_t)b << wbits, W, nc, L, lx);
+      ++b;
+      continue;
+    }
+    int be = b;
+    uint32_t tot = 0;
+    while (be < NB) {
+      const uint32_t c = s_boff[be + 1] - s_boff[be];
+      if (c > (uint32_t)CAP || tot + c > (uint32_t)CAP) break;
+      tot += c;
+      ++be;
+    }
+    const uint32_t e0 = s_boff[b];
+    const uint32_t kbase = (uint32_t)b << wbits;
+    for (int e = t; e < (int)tot; e += 256) {
+      L.u.srt.k[0][e] = skey[e0 + e] - kbase;
+      L.u.srt.v[0][e] = (uint16_t)e;
+      L.aux[e] = saux[e0 + e];
+      if (TASK == 1) L.y[e] = sy[e0 + e];
     }
     __syncthreads();
-    {
-      const int per = (NB + 255) / 256;
-      const int b0 = t * per, b1 = min(b0 + per, NB);
-      uint32_t loc = 0;
-      for (int b = b0; b < b1; ++b) loc += s_boff[b];
-      uint32_t base = team_excl_scan<256>(loc, L.w, nullptr);
-      for (int b = b0; b < b1; ++b) {
-        const uint32_t c = s_boff[b];
-        s_boff[b] = base;
-        base += c;
-      }
-      if (t == 0) s_boff[NB] = (uint32_t)m;
-      __syncthreads();
-      for (int b = t; b < NB; b += 256) L.u.bpos[b] = s_boff[b];
-      __syncthreads();
-    }
-    for (int e0 = 0; e0 < m; e0 += 256 * U) {
-      uint32_t rows[U], auxv[U], keys[U];
-      int64_t yv[U];
-#pragma unroll
-      for (int q = 0; q < U; ++q) {
-        const int e = e0 + t + q * 256;
-        if (e < m) {
-          rows[q] = lv.row[st + e];
-          auxv[q] = lv.aux[st + e];
-          if (TASK == 1) yv[q] = lv.ey[st + e];
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < U; ++q) {
-        const int e = e0 + t + q * 256;
-        if (e < m) keys[q] = Kf[rows[q]];
-      }
-#pragma unroll
-      for (int q = 0; q < U; ++q) {
-        const int e = e0 + t + q * 256;
-        if (e < m) {
-          const uint32_t pos = atomicAdd(&L.u.bpos[keys[q] >> wbits], 1u);
-          skey[pos] = keys[q];
-          saux[pos] = auxv[q];
-          if (TASK == 1) sy[pos] = yv[q];
-        }
-      }
-    }
-    __syncthreads();
-    int b = 0;
-    while (b < NB) {
-      const uint32_t cb = s_boff[b + 1] - s_boff[b];
-      if (cb == 0) {
-        ++b;
-        continue;
-      }
-      if (cb > (uint32_t)CAP) {
-        eval_hist_bucket<MAXC, TASK, IPT>(skey + s_boff[b], saux + s_boff[b], TASK == 1 ? sy + s_boff[b] : nullptr,
-                                          cb, (uint32_t)b << wbits, W, nc, L, lx);
-        ++b;
-        continue;
-      }
-      int be = b;
-      uint32_t tot = 0;
-      while (be < NB) {
-        const uint32_t c = s_boff[be + 1] - s_boff[be];
-        if (c > (uint32_t)CAP || tot + c > (uint32_t)CAP) break;
-        tot += c;
-        ++be;
-      }
-      const uint32_t e0 = s_boff[b];
-      const uint32_t kbase = (uint32_t)b << wbits;
-      for (int e = t; e < (int)tot; e += 256) {
-        L.u.srt.k[0][e] = skey[e0 + e] - kbase;
-        L.u.srt.v[0][e] = (uint16_t)e;
-        L.aux[e] = saux[e0 + e];
-        if (TASK == 1) L.y[e] = sy[e0 + e];
-      }
-      __syncthreads();
-      sort_and_eval<MAXC, TASK, 256, IPT>((int)tot, bit_length((uint32_t)(be - b) * (uint32_t)W - 1u), kbase, nc,
-                                          L, lx);
-      b = be;
-    }
+    sort_and_eval<MAXC, TASK, 256, IPT>((int)tot, bit_length((uint32_t)(be - b) * (uint32_t)W - 1u), kbase, nc,
+                                        L, lx);
+    b = be;
   }
 }
 
-template <int MAXC, int TASK, int TEAM, int IPT>
+template <int MAXC, int TASK>
 __device__ __forceinline__ void rf_write_result(const DataArgs& d, const ItemArgs& it, int64_t ridx, int f,
                                                 const Carry<MAXC, TASK>& cr) {
   float score = 0.0f, thr = 0.0f;
@@ -998,31 +994,26 @@ __device__ __forceinline__ void rf_write_result(const DataArgs& d, const ItemArg
 }
 
 // ------------------------------------------------- RF split search ------
-// One team per (node, feature draw) item, grid-stride over items.  TEAM=64:
-// four independent wave teams per workgroup for medium nodes (up to 64*IPT
-// entries).  TEAM=256: whole workgroup; nodes up to 256*IPT entries are
-// sorted in LDS, larger ones are bucketed by dense key into a scratch slab
-// first.  Every boundary between distinct values is scored.
-template <int MAXC, int TASK, int TEAM, bool BIG>
+// One workgroup per (node, feature draw) item, grid-stride over items: the
+// plain driver's nodes of any size, and the few nodes above cut_block of the
+// level graphs.  Nodes of up to 2048 entries are sorted in LDS, larger ones
+// are bucketed by dense key into a scratch slab first.  Every boundary between
+// distinct values is scored.
+template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, ItemArgs it) {
-  constexpr int IPT = TEAM == kWave ? kTeamIpt : kIpt;
-  constexpr int NT = kBlock / TEAM;
   resolve_level(lv, d.C);
   resolve_items(it);
-  if ((int64_t)blockIdx.x * NT >= it.n_groups * it.per_group) return;
+  const int64_t n_items = it.n_groups * it.per_group;
+  if ((int64_t)blockIdx.x >= n_items) return;
   __shared__ double s_inv[128], s_logc[128];
-  __shared__ TeamLds<MAXC, TASK, TEAM, IPT> s_team[NT];
-  __shared__ uint32_t s_boff[BIG ? kMaxBuckets + 1 : 1];
+  __shared__ TeamLds<MAXC, TASK, kBlock, kIpt> L;
+  __shared__ uint32_t s_boff[kMaxBuckets + 1];
   load_tables(s_inv, s_logc);
   __syncthreads();
   const LnCtx lx{s_inv, s_logc, d.T, d.Tmax, d.igF};
-  const int team = TEAM == 256 ? 0 : (int)(threadIdx.x / kWave);
-  TeamLds<MAXC, TASK, TEAM, IPT>& L = s_team[team];
-  const int t = team_tid<TEAM>();
+  const int t = threadIdx.x;
   unsigned long long my_bytes = 0;
-  const int64_t n_items = it.n_groups * it.per_group;
-  const int team_global = (int)blockIdx.x * NT + team;
-  for (int64_t item = team_global; item < n_items; item += (int64_t)gridDim.x * NT) {
+  for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int64_t grp = it.node_major ? item % it.n_groups : item / it.per_group;
     const int j = it.j0 + (int)(it.node_major ? item / it.n_groups : item % it.per_group);
     const uint32_t o = it.list ? it.list[grp] : (uint32_t)grp;
@@ -1031,7 +1022,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
                         (uint32_t)d.F);
     const int64_t ridx = (int64_t)o * it.D + j;
     NodeCtx nc;
-    const bool pure = node_context<MAXC, TASK, TEAM, IPT>(d, lv, i, nc, L, lx);
+    const bool pure = node_context<MAXC, TASK>(d, lv, i, nc, L, lx);
     if (pure) {
       // Every boundary of a pure node has gain exactly 0: no positive split.
       if (t == 0) {
@@ -1039,14 +1030,14 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
         it.res_thr[ridx] = 0.0f;
         it.res_feat[ridx] = f;
       }
-      team_sync<TEAM>();
+      __syncthreads();
       continue;
     }
     if (t == 0) my_bytes += (unsigned long long)lv.m[i] * (TASK == 0 ? 12ull : 20ull);
-    rf_item<MAXC, TASK, TEAM, IPT, BIG>(d, lv, it, f, i, nc, L, lx, s_boff, (int)blockIdx.x);
-    team_sync<TEAM>();
-    if (t == 0) rf_write_result<MAXC, TASK, TEAM, IPT>(d, it, ridx, f, L.cr);
-    team_sync<TEAM>();
+    rf_item<MAXC, TASK>(d, lv, it, f, i, nc, L, lx, s_boff);
+    __syncthreads();
+    if (t == 0) rf_write_result<MAXC, TASK>(d, it, ridx, f, L.cr);
+    __syncthreads();
   }
   if (t == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
 }
@@ -2374,17 +2365,10 @@ __global__ void __launch_bounds__(kBlock) k_search_ert(DataArgs d, LevelArgs lv,
   ert_block_body<MAXC, TASK>(d, lv, it, blockIdx.x, gridDim.x, s_inv, s_logc);
 }
 
-// ------------------------------------------ wave-per-item split search --
-// Small nodes: one wave64 per (node, draw) item, several items per block, no
-// block barriers.  RF: each lane holds one entry (m <= 64); the rank of its
-// key is counted over the wave, ds_permute moves the entries into key order,
-// and the per-class running sums of the fixed-point x ln x terms become
-// wave exclusive scans of per-lane deltas.
+// ------------------------------------------------ wave and segment moves --
 __device__ __forceinline__ uint32_t ds_permute_u32(uint32_t dst_lane, uint32_t v) {
   return (uint32_t)__builtin_amdgcn_ds_permute((int)(dst_lane << 2), (int)v);
 }
-
-__device__ __forceinline__ int64_t wave_excl_i64(int64_t v) { return wave_incl_scan_i64(v) - v; }
 
 // All lanes active.
 __device__ __forceinline__ int64_t wave_sum_i64(int64_t v) { return wave_last_i64(wave_incl_scan_i64(v)); }
@@ -2399,125 +2383,6 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return wave_last(v);
 }
 
-
-template <int MAXC, int TASK>
-__global__ void __launch_bounds__(kBlock) k_search_rf_wave(DataArgs d, LevelArgs lv, ItemArgs it) {
-  resolve_level(lv, d.C);
-  resolve_items(it);
-  if ((int64_t)blockIdx.x * kWaves >= it.n_groups * it.per_group) return;
-  __shared__ double s_inv[128], s_logc[128];
-  load_tables(s_inv, s_logc);
-  __syncthreads();
-  const LnCtx lx{s_inv, s_logc, d.T, d.Tmax, d.igF};
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wv = threadIdx.x / kWave;
-  unsigned long long my_bytes = 0;
-  const int64_t n_items = it.n_groups * it.per_group;
-  for (int64_t item = (int64_t)blockIdx.x * kWaves + wv; item < n_items; item += (int64_t)gridDim.x * kWaves) {
-    const int64_t grp = item / it.per_group;
-    const int j = it.j0 + (int)(item % it.per_group);
-    const uint32_t o = it.list ? it.list[grp] : (uint32_t)grp;
-    const uint32_t i = lv.open_idx[o];
-    const uint32_t nid = lv.id[i];
-    const int f = (int)(rand_u32(d.seed, kStreamFeat, (uint32_t)lv.tree_global[lv.tree[i]], nid, (uint64_t)j) %
-                        (uint32_t)d.F);
-    const int m = lv.m[i];
-    const int64_t st = lv.start[i];
-    const int64_t n = lv.count[i];
-    const int64_t ridx = (int64_t)o * it.D + j;
-    // node statistics
-    uint32_t ncls_lane = 0;
-    int F = 0;
-    int64_t P = 0, SR0 = 0;
-    double inv = 0.0;
-    if (TASK == 0) {
-      ncls_lane = lane < d.C ? lv.cls[(int64_t)i * d.C + lane] : 0u;
-      if ((int64_t)wave_max_u32(ncls_lane) == n) {
-        if (lane == 0) {
-          it.res_score[ridx] = 0.0f;
-          it.res_thr[ridx] = 0.0f;
-          it.res_feat[ridx] = f;
-        }
-        continue;
-      }
-      F = d.igF;
-      inv = 1.0 / ((double)n * kLn2);
-      SR0 = wave_sum_i64(lane < d.C ? lx.t(ncls_lane) : 0);
-      P = lx.t((uint64_t)n) - SR0;
-    }
-    if (lane == 0) my_bytes += (unsigned long long)m * (TASK == 0 ? 12ull : 20ull);
-    const bool valid = lane < m;
-    uint32_t key = kNone, pay = 0;
-    int64_t yv = 0;
-    if (valid) {
-      const uint32_t row = lv.row[st + lane];
-      pay = lv.aux[st + lane];
-      key = d.K[(int64_t)f * d.N + row];
-      if (TASK == 1) yv = lv.ey[st + lane];
-    }
-    uint32_t cnt = 0;
-    for (int r = 0; r < m; ++r) {
-      const uint32_t kr = __shfl(key, r, kWave);
-      cnt += (kr < key || (kr == key && r < lane)) ? 1u : 0u;
-    }
-    const uint32_t rank = valid ? cnt : (uint32_t)lane;
-    key = ds_permute_u32(rank, key);
-    pay = ds_permute_u32(rank, pay);
-    if (TASK == 1) {
-      const uint32_t lo = ds_permute_u32(rank, (uint32_t)(uint64_t)yv);
-      const uint32_t hi = ds_permute_u32(rank, (uint32_t)((uint64_t)yv >> 32));
-      yv = (int64_t)(((uint64_t)hi << 32) | lo);
-    }
-    const uint32_t w = valid ? (pay & 0xFFFFu) : 0u;
-    const uint32_t prevk = __shfl_up(key, 1, kWave);
-    const bool cand = valid && lane >= 1 && prevk < key;
-    double g = 0.0;
-    if (TASK == 0) {
-      const uint32_t lab = pay >> 16;
-      uint32_t pre = 0;
-      for (int r = 0; r < m; ++r) {
-        const uint32_t pr = __shfl(pay, r, kWave);
-        pre += (r < lane && (pr >> 16) == lab) ? (pr & 0xFFFFu) : 0u;
-      }
-      const uint32_t nc = __shfl(ncls_lane, (int)lab, kWave);
-      int64_t dl = 0, dr = 0;
-      if (valid) {
-        dl = lx.t(pre + w) - lx.t(pre);
-        dr = lx.t(nc - pre - w) - lx.t(nc - pre);
-      }
-      const int64_t sl = wave_excl_i64(dl);
-      const int64_t sr = SR0 + wave_excl_i64(dr);
-      const int64_t nl = wave_excl_i64((int64_t)w);
-      if (cand) {
-        const int64_t q = (sl - lx.t((uint64_t)nl)) + (sr - lx.t((uint64_t)(n - nl)));
-        g = ig_from_fixed(P + q, F, inv);
-      }
-    } else {
-      const int64_t pn = wave_excl_i64((int64_t)w);
-      const int64_t ps = wave_excl_i64((int64_t)w * yv);
-      if (cand) g = variance_gain(pn, ps, n - pn, lv.sum[i] - ps, 0);
-    }
-    BestCand b = (cand && g > 0.0) ? BestCand{g, key, prevk} : BestCand{0.0, kNone, kNone};
-    b = wave_best(b);
-    if (lane == 0) {
-      float score = 0.0f, thr = 0.0f;
-      if (b.key != kNone) {
-        const float* sv = d.SV + d.SVoff[f];
-        score = (float)(TASK == 0 ? b.g : ldexp_d(b.g, -2 * d.shift));
-        thr = midpoint(sv[b.prev], sv[b.key]);
-      }
-      it.res_score[ridx] = score;
-      it.res_thr[ridx] = thr;
-      it.res_feat[ridx] = f;
-    }
-  }
-  if (lane == 0 && my_bytes && it.bytes) add_bytes(it.bytes, my_bytes);
-}
-
-// Segment-per-node RF search for tiny nodes: a wave holds 64/SEG nodes, one
-// per SEG-lane segment (one entry per lane, m <= SEG, C <= SEG), and loops
-// over the node's draws, so node statistics and entry loads are shared by
-// all draws.  Shuffles, scans and reductions stay inside the segment.
 // Scans and sums of a 16- or 32-lane segment in DPP moves (a shuffle goes
 // through the LDS pipe).  All lanes of a segment are active together.
 template <int SEG>
@@ -2613,6 +2478,10 @@ struct SegLds {
   int64_t T[TASK == 0 ? kTL : 1];
 };
 
+// Segment-per-node RF search for tiny nodes: a wave holds 64 / SEG nodes, one
+// per SEG-lane segment (one entry per lane, m <= SEG, C <= SEG), and loops
+// over the node's draws (its unit's, in a level of few nodes), so node
+// statistics and entry loads are shared by the draws.
 template <int MAXC, int TASK, int SEG>
 __device__ __forceinline__ void rf_seg_body(DataArgs d, LevelArgs lv, ItemArgs it, int64_t bid, int64_t nblk,
                                             SegLds<TASK>& S) {
@@ -2840,7 +2709,6 @@ struct BoundLds {
 __device__ __forceinline__ float lane_below_f32(float v, float first) {
   return __uint_as_float(dpp_u32<0x138>(__float_as_uint(v), __float_as_uint(first)));
 }
-__device__ __forceinline__ float wave_last_f32(float v) { return __uint_as_float(wave_last(__float_as_uint(v))); }
 
 // fp32 chord_gap.
 __device__ __forceinline__ float chord_gap_f32(float a, float s) {
@@ -6080,7 +5948,7 @@ void launch_search(int algorithm, int tier, int grid, hipStream_t s, const DataA
       case 2: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 1>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       case 3: hipLaunchKernelGGL((k_search_rf_bound<MAXC, TASK, 8>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
       case 4: hipLaunchKernelGGL((k_search_rf_bound_team<MAXC, TASK>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
-      default: hipLaunchKernelGGL((k_search_rf<MAXC, TASK, 256, true>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
+      default: hipLaunchKernelGGL((k_search_rf<MAXC, TASK>), dim3(grid), dim3(kBlock), 0, s, d, lv, it); break;
     }
   } else {
     switch (tier) {
