@@ -23,7 +23,19 @@ namespace dte {
 namespace {
 
 constexpr int kWave = 64;
-constexpr int kWalkThreads = 512;  // a block's rows in LDS serve eight waves
+// Threads of a walk block.  Eight waves a block's rows in LDS keep the CU full
+// where a block's LDS holds it to four; but a block walks as many trees at once
+// as a row has lanes, and what its CU's neighbours miss grows with them.  Models
+// past the caches (kBigModel) under many row blocks (kManyBlocks, where blocks
+// start at different times and drift over all trees) take four: 1M x 128, 64
+// trees of 300,000 nodes 4.65 ms at 512 threads, 3.8 at 256; 200 trees 17.1 and
+// 12.9; 400 trees 37.8 and 28.5.  The other side of the line: 300,000 x 128, 64
+// trees of 83,000 nodes 0.86 and 0.88; 100,000 x 128, 64 trees of 230,000 nodes
+// 0.39 and 0.40; 300,000 x 128, 200 trees of 1,700 nodes 0.82 and 1.27.
+constexpr int kWalkThreads = 512;
+constexpr int kBigWalkThreads = 256;
+constexpr int64_t kBigModel = (int64_t)6 << 20;  // nodes
+constexpr int64_t kManyBlocks = 4096;
 // Row blocks of a launch: it holds fewer than 2^32 threads in a direction.
 // More rows (537 M at 64 a block) take several launches.
 constexpr int64_t kMaxRowBlocks = 0xFFFFFFFFll / kWalkThreads;
@@ -348,17 +360,17 @@ __device__ __forceinline__ uint32_t walk(const Trees& tr, int t, const float* xr
 }
 
 // Stages a block's R rows of F features in LDS, F + 1 floats apart.
-template <int R>
+template <int R, int NT>
 __device__ __forceinline__ void stage_rows(const float* __restrict__ X, int64_t row0, int nr, int64_t ld,
                                            int row_major, int F, float* s_x) {
   const int FP = F + 1;
   if (row_major) {
-    for (int i = threadIdx.x; i < nr * F; i += kWalkThreads) {
+    for (int i = threadIdx.x; i < nr * F; i += NT) {
       const int r = i / F, f = i - r * F;
       s_x[r * FP + f] = X[(row0 + r) * ld + f];
     }
   } else {
-    for (int i = threadIdx.x; i < R * F; i += kWalkThreads) {
+    for (int i = threadIdx.x; i < R * F; i += NT) {
       const int f = i / R, r = i - f * R;
       if (r < nr) s_x[r * FP + f] = X[(int64_t)f * ld + row0 + r];
     }
@@ -369,10 +381,10 @@ __device__ __forceinline__ void stage_rows(const float* __restrict__ X, int64_t 
 // chunks), or it alone covers its rows' trees and stores them.
 enum VoteMode { kVoteAdd = 0, kVoteInt = 1, kVoteFloat = 2 };
 
-// A block's R rows x (512 / R) tree lanes; R = 0: rows read from X, 64 rows
-// x 8 tree lanes.
-template <int R, bool PACKED>
-__global__ void __launch_bounds__(kWalkThreads) k_predict_cls(Trees tr, const float* __restrict__ X, int64_t n_rows,
+// A block's R rows x (NT / R) tree lanes; R = 0: rows read from X, 64 rows
+// x NT / 64 tree lanes.
+template <int R, bool PACKED, int NT>
+__global__ void __launch_bounds__(NT) k_predict_cls(Trees tr, const float* __restrict__ X, int64_t n_rows,
                                                               int64_t ld, int row_major, int C, int F,
                                                               int trees_per_block, int mode, void* __restrict__ out) {
   extern __shared__ uint32_t s_mem[];
@@ -385,17 +397,17 @@ __global__ void __launch_bounds__(kWalkThreads) k_predict_cls(Trees tr, const fl
   const int nr = (int)min<int64_t>(RB, n_rows - row0);
   const int t0 = blockIdx.y * trees_per_block;
   const int t1 = min(tr.T, t0 + trees_per_block);
-  for (int i = threadIdx.x; i < RB * C; i += kWalkThreads) s_votes[i] = 0;
-  if (R) stage_rows<RB>(X, row0, nr, ld, row_major, F, s_x);
+  for (int i = threadIdx.x; i < RB * C; i += NT) s_votes[i] = 0;
+  if (R) stage_rows<RB, NT>(X, row0, nr, ld, row_major, F, s_x);
   __syncthreads();
   if (lane < nr) {
     const float* xr = R ? s_x + lane * (F + 1) : row_major ? X + (row0 + lane) * ld : X + row0 + lane;
     const int64_t xs = R || row_major ? 1 : ld;
-    for (int t = t0 + group; t < t1; t += kWalkThreads / RB)
+    for (int t = t0 + group; t < t1; t += NT / RB)
       atomicAdd(&s_votes[lane * C + walk<PACKED>(tr, t, xr, xs, [](int, uint32_t, float&) {})], 1u);
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < nr * C; i += kWalkThreads) {
+  for (int i = threadIdx.x; i < nr * C; i += NT) {
     const uint32_t v = s_votes[i];
     const int64_t o = row0 * C + i;
     if (mode == kVoteFloat) {
@@ -414,8 +426,8 @@ __global__ void __launch_bounds__(kWalkThreads) k_predict_cls(Trees tr, const fl
 // that order whatever R is.
 constexpr int reg_chunk(int R) { return kWalkThreads / (R ? R : 64) > 32 ? kWalkThreads / (R ? R : 64) : 32; }
 
-template <int R, bool PACKED>
-__global__ void __launch_bounds__(kWalkThreads) k_predict_reg(Trees tr, const float* __restrict__ X, int64_t n_rows,
+template <int R, bool PACKED, int NT>
+__global__ void __launch_bounds__(NT) k_predict_reg(Trees tr, const float* __restrict__ X, int64_t n_rows,
                                                               int64_t ld, int row_major, int F,
                                                               float* __restrict__ sums) {
   extern __shared__ float s_mem_f[];
@@ -427,7 +439,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_predict_reg(Trees tr, const fl
   const int group = threadIdx.x / RB;
   const int64_t row0 = (int64_t)blockIdx.x * RB;
   const int nr = (int)min<int64_t>(RB, n_rows - row0);
-  if (R) stage_rows<RB>(X, row0, nr, ld, row_major, F, s_x);
+  if (R) stage_rows<RB, NT>(X, row0, nr, ld, row_major, F, s_x);
   __syncthreads();
   const float* xr = R ? s_x + lane * (F + 1) : row_major ? X + (row0 + lane) * ld : X + row0 + lane;
   const int64_t xs = R || row_major ? 1 : ld;
@@ -435,7 +447,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_predict_reg(Trees tr, const fl
   for (int c0 = 0; c0 < tr.T; c0 += CH) {
     const int c1 = min(tr.T, c0 + CH);
     if (lane < nr)
-      for (int t = c0 + group; t < c1; t += kWalkThreads / RB)
+      for (int t = c0 + group; t < c1; t += NT / RB)
         s_val[lane * (CH + 1) + (t - c0)] = __uint_as_float(walk<PACKED>(tr, t, xr, xs, [](int, uint32_t, float&) {}));
     __syncthreads();
     if (group == 0 && lane < nr)
@@ -523,7 +535,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_oob(Trees tr, const float* __r
   const int nr = (int)min<int64_t>(RB, N - row0);
   const int t0 = blockIdx.y * trees_per_block;
   const int t1 = min(tr.T, t0 + trees_per_block);
-  if (R) stage_rows<RB>(X, row0, nr, N, 0, F, s_x);
+  if (R) stage_rows<RB, kWalkThreads>(X, row0, nr, N, 0, F, s_x);
   if (t < kWave) {
     const float yr = t < nr ? y[row0 + t] : 0.0f;
     if (t < RB) s_y[t] = yr;
@@ -715,6 +727,23 @@ void with_rows(int r, bool packed, Fn&& fn) {
   }
 }
 
+// The same with integral_constant NT for a prediction of row_blocks blocks of r
+// rows (fewer than 32: few blocks).
+template <class Fn>
+void with_walk(const Forest& f, int r, int64_t row_blocks, Fn&& fn) {
+  const bool big = f.n_nodes >= kBigModel && row_blocks >= kManyBlocks;
+  with_rows(r, f.pairs.p != nullptr, [&](auto R, auto packed) {
+    constexpr int kR = decltype(R)::value;
+    if constexpr (kR == 0 || kR >= 32) {
+      if (big) {
+        fn(R, packed, std::integral_constant<int, kBigWalkThreads>());
+        return;
+      }
+    }
+    fn(R, packed, std::integral_constant<int, kWalkThreads>());
+  });
+}
+
 }  // namespace
 
 void oob_evaluate(const Forest& f, const float* X, const float* targets, int64_t N, int perm, double out[2],
@@ -829,11 +858,12 @@ void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld,
     if (mode == kVoteAdd)
       hipLaunchKernelGGL(k_zero_u32, dim3(elementwise_grid(nv)), dim3(kBlock), 0, s, reinterpret_cast<uint32_t*>(votes),
                          nv);
-    with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
+    with_walk(f, R, row_blocks, [&](auto r, auto packed, auto nt) {
+      constexpr int kThreads = decltype(nt)::value;
       for (int64_t r0 = 0; r0 < n_rows; r0 += kMaxRowBlocks * RB) {
         const int64_t rows = std::min(n_rows - r0, kMaxRowBlocks * RB);
-        hipLaunchKernelGGL((k_predict_cls<decltype(r)::value, decltype(packed)::value>),
-                           dim3((unsigned)((rows + RB - 1) / RB), tree_blocks), dim3(kWalkThreads), lds, s,
+        hipLaunchKernelGGL((k_predict_cls<decltype(r)::value, decltype(packed)::value, kThreads>),
+                           dim3((unsigned)((rows + RB - 1) / RB), tree_blocks), dim3(kThreads), lds, s,
                            trees_of(f), row_major ? X + r0 * ld : X + r0, rows, ld, row_major, C, F, tpb, mode,
                            (void*)(votes + r0 * C));
       }
@@ -846,11 +876,12 @@ void predict_forest(const Forest& f, const float* X, int64_t n_rows, int64_t ld,
     const int R = want && staged_rows(F, reg_chunk(want) + 1, n_rows) == want ? want : 0;
     const int RB = R ? R : 64;
     const size_t lds = sizeof(float) * (size_t)RB * (reg_chunk(R) + 1 + (R ? F + 1 : 0));
-    with_rows(R, f.pairs.p != nullptr, [&](auto r, auto packed) {
+    with_walk(f, R, (n_rows + RB - 1) / RB, [&](auto r, auto packed, auto nt) {
+      constexpr int kThreads = decltype(nt)::value;
       for (int64_t r0 = 0; r0 < n_rows; r0 += kMaxRowBlocks * RB) {
         const int64_t rows = std::min(n_rows - r0, kMaxRowBlocks * RB);
-        hipLaunchKernelGGL((k_predict_reg<decltype(r)::value, decltype(packed)::value>),
-                           dim3((unsigned)((rows + RB - 1) / RB)), dim3(kWalkThreads), lds, s, trees_of(f),
+        hipLaunchKernelGGL((k_predict_reg<decltype(r)::value, decltype(packed)::value, kThreads>),
+                           dim3((unsigned)((rows + RB - 1) / RB)), dim3(kThreads), lds, s, trees_of(f),
                            row_major ? X + r0 * ld : X + r0, rows, ld, row_major, F, sums + r0);
       }
     });

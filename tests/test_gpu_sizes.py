@@ -508,3 +508,49 @@ def test_cached_scratch_gives_way_to_allocations_of_the_library():
         X.free()
         g.close()
         capi.release_cached_memory()
+
+
+@pytest.mark.parametrize("f", [9, 200, 600])
+@pytest.mark.parametrize("task", [capi.CLASSIFICATION, capi.REGRESSION])
+def test_predict_of_many_rows_by_a_big_model(task, f):
+    """Models of more than 6 Mi nodes under 4,096 row blocks and more walk in
+    blocks of fewer threads, with 64, 32 and no rows in LDS; the same rows, a
+    few at a time, take the others."""
+    trees, depth = 97, 15
+    per = 2 ** (depth + 1) - 1
+    rng = np.random.default_rng(f)
+    n = trees * per
+    assert n >= 6 << 20
+    k = np.arange(per)
+    inner = k < per // 2
+    where = lambda t, i: np.where(i == 0, t, trees + t * (per - 1) + i - 1)
+    nodes = np.zeros(n, capi.NODE_DTYPE)
+    for t in range(trees):
+        at = where(t, k)
+        nodes["child_start"][at] = np.where(inner, where(t, 2 * k + 1), -1)
+        nodes["child_count"][at] = np.where(inner, 2, 0)
+        nodes["attribute"][at] = np.where(inner, rng.integers(0, f, per), -1)
+        nodes["split_point"][at] = np.where(inner, 0.5, -1)
+    leaf = nodes["child_count"] == 0
+    width = 1 if task else 3
+    nodes["probability_start"] = np.where(leaf, width * (np.cumsum(leaf) - 1), -1)
+    probs = rng.integers(0, 9, width * int(leaf.sum())).astype(np.float32)  # sums are exact
+    g = capi.import_forest(nodes, probs, trees, width, f, task)
+    rows = 64 * 4096 + 33
+    X = rng.random((f, 2048), dtype=np.float32)
+    few = g.predict(X)
+    got = g.predict(_repeated(X.T, rows * f).reshape(rows, f).T.copy()).reshape(rows, -1)
+    assert np.array_equal(got, _repeated(few.reshape(2048, -1), got.size).reshape(got.shape))
+    x, total = X[:, :40], np.zeros(40)
+    for t in range(trees):
+        at = np.full(40, t)
+        for _ in range(depth):
+            d = nodes[at]
+            at = d["child_start"] + (x[d["attribute"], np.arange(40)] >= 0.5)
+        p = nodes["probability_start"][at]
+        if task:
+            total += probs[p]
+        else:
+            total += probs[p[:, None] + np.arange(3)].argmax(1) == 1
+    assert np.array_equal(few.reshape(2048, -1)[:40, 0 if task else 1], total.astype(np.float32))
+    g.close()
