@@ -822,7 +822,7 @@ __device__ __forceinline__ bool node_context(const DataArgs& d, const LevelArgs&
 // the LDS capacity is bucketed through the workgroup's scratch slab.
 template <int MAXC, int TASK>
 __device__ void rf_item(const DataArgs& d, const LevelArgs& lv, const ItemArgs& it, int f, uint32_t i, const NodeCtx& nc,
-                        TeamLds<MAXC, TASK, kBlock, kIpt>& L, const LnCtx& lx, uint32_t* s_boff) {
+                        TeamLds<MAXC, TASK, kBlock, kIpt>& L, const LnCtx& lx, uint32_t* s_boff, int slab) {
   constexpr int IPT = kIpt;
   constexpr int CAP = kCap;
   const int t = threadIdx.x;
@@ -878,9 +878,9 @@ __device__ void rf_item(const DataArgs& d, const LevelArgs& lv, const ItemArgs& 
   while (((S + (1u << wbits) - 1) >> wbits) > (uint32_t)kMaxBuckets) ++wbits;
   const int W = 1 << wbits;
   const int NB = (int)((S + (uint32_t)W - 1) >> wbits);
-  uint32_t* skey = it.scr_key + (int64_t)blockIdx.x * it.scr_stride;
-  uint32_t* saux = it.scr_aux + (int64_t)blockIdx.x * it.scr_stride;
-  int64_t* sy = TASK == 1 ? it.scr_y + (int64_t)blockIdx.x * it.scr_stride : nullptr;
+  uint32_t* skey = it.scr_key + (int64_t)slab * it.scr_stride;
+  uint32_t* saux = it.scr_aux + (int64_t)slab * it.scr_stride;
+  int64_t* sy = TASK == 1 ? it.scr_y + (int64_t)slab * it.scr_stride : nullptr;
   for (int b = t; b <= NB; b += 256) s_boff[b] = 0;
   __syncthreads();
   constexpr int U = 8;
@@ -998,7 +998,10 @@ __device__ __forceinline__ void rf_write_result(const DataArgs& d, const ItemArg
 // plain driver's nodes of any size, and the few nodes above cut_block of the
 // level graphs.  Nodes of up to 2048 entries are sorted in LDS, larger ones
 // are bucketed by dense key into a scratch slab first.  Every boundary between
-// distinct values is scored.
+// distinct values is scored.  Its speed hangs on what the compiler is told:
+// 32-bit block numbers (64-bit ones cost 4 to 8 registers) and 16-byte aligned
+// LDS (the digit counters are read 16 bytes at a time); 1M x 128, 12 trees in
+// the plain driver 2.07 s, without the first 2.21, without the second 2.10.
 template <int MAXC, int TASK>
 __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, ItemArgs it) {
   resolve_level(lv, d.C);
@@ -1006,14 +1009,14 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
   const int64_t n_items = it.n_groups * it.per_group;
   if ((int64_t)blockIdx.x >= n_items) return;
   __shared__ double s_inv[128], s_logc[128];
-  __shared__ TeamLds<MAXC, TASK, kBlock, kIpt> L;
+  __shared__ alignas(16) TeamLds<MAXC, TASK, kBlock, kIpt> L;
   __shared__ uint32_t s_boff[kMaxBuckets + 1];
   load_tables(s_inv, s_logc);
   __syncthreads();
   const LnCtx lx{s_inv, s_logc, d.T, d.Tmax, d.igF};
   const int t = threadIdx.x;
   unsigned long long my_bytes = 0;
-  for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+  for (int64_t item = (int)blockIdx.x; item < n_items; item += (int64_t)gridDim.x) {
     const int64_t grp = it.node_major ? item % it.n_groups : item / it.per_group;
     const int j = it.j0 + (int)(it.node_major ? item / it.n_groups : item % it.per_group);
     const uint32_t o = it.list ? it.list[grp] : (uint32_t)grp;
@@ -1034,7 +1037,7 @@ __global__ void __launch_bounds__(kBlock) k_search_rf(DataArgs d, LevelArgs lv, 
       continue;
     }
     if (t == 0) my_bytes += (unsigned long long)lv.m[i] * (TASK == 0 ? 12ull : 20ull);
-    rf_item<MAXC, TASK>(d, lv, it, f, i, nc, L, lx, s_boff);
+    rf_item<MAXC, TASK>(d, lv, it, f, i, nc, L, lx, s_boff, (int)blockIdx.x);
     __syncthreads();
     if (t == 0) rf_write_result<MAXC, TASK>(d, it, ridx, f, L.cr);
     __syncthreads();
