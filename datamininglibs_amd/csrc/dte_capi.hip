@@ -345,21 +345,6 @@ int64_t largest_tree(const std::vector<int64_t>& ts) {
   return m;
 }
 
-// Whether every tree's children follow in their parents' order, all in the tree.
-bool in_level_order(const std::vector<int64_t>& ts, const std::vector<int32_t>& feature,
-                    const std::vector<int32_t>& left) {
-  for (size_t t = 0; t + 1 < ts.size(); ++t) {
-    int64_t next = ts[t] + 1;
-    for (int64_t g = ts[t]; g < ts[t + 1]; ++g) {
-      if (feature[g] < 0) continue;
-      if (left[g] != next) return false;
-      next += 2;
-    }
-    if (next != ts[t + 1]) return false;
-  }
-  return true;
-}
-
 int64_t count_leaves(const std::vector<int32_t>& feature) {
   int64_t n = 0;
   for (auto v : feature) n += v < 0;
@@ -691,9 +676,18 @@ int dte_forest_import(const dte_node* nodes, int64_t n_nodes, const float* probs
           fail(DTE_ERR_INVALID_ARGUMENT, "bad child link");
       }
     }
-    for (int t = 0; t < n_trees; ++t)
+    // whether every tree's children follow in their parents' order, all in the tree
+    bool level_order = true;
+    for (int t = 0; t < n_trees; ++t) {
+      int64_t next = ts[t] + 1;
       for (int64_t g = ts[t]; g < ts[t + 1]; ++g)
-        if (feature[g] >= 0) depth[left[g]] = depth[left[g] + 1] = depth[g] + 1;
+        if (feature[g] >= 0) {
+          depth[left[g]] = depth[left[g] + 1] = depth[g] + 1;
+          level_order = level_order && left[g] == next;
+          next += 2;
+        }
+      level_order = level_order && next == ts[t + 1];
+    }
     set_device(device_id);
     hipStream_t s = library_stream(device_id);
     auto* h = new dte_forest();
@@ -706,7 +700,7 @@ int dte_forest_import(const dte_node* nodes, int64_t n_nodes, const float* probs
     f.n_trees = n_trees;
     f.n_nodes = n;
     f.n_leaves = count_leaves(feature);
-    f.level_order = in_level_order(ts, feature, left);
+    f.level_order = level_order;
     f.has_stats = false;
     f.tree_start.alloc(n_trees + 1);
     f.feature.alloc(n);
@@ -893,8 +887,10 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
     r.get(depth.data(), 4 * n);
     // structure: trees tile [0, n); children adjacent inside their tree
     if (ts[0] != 0 || ts[T] != n) fail(DTE_ERR_INVALID_ARGUMENT, "forest file tree table out of range");
+    bool level_order = true;
     for (int t = 0; t < T; ++t) {
       if (ts[t + 1] <= ts[t]) fail(DTE_ERR_INVALID_ARGUMENT, "forest file tree table out of range");
+      int64_t next = ts[t] + 1;
       if (depth[ts[t]] != 0) fail(DTE_ERR_INVALID_ARGUMENT, "forest file root depth");
       for (int64_t g = ts[t]; g < ts[t + 1]; ++g) {
         if (feature[g] < 0) {
@@ -906,7 +902,10 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
           fail(DTE_ERR_INVALID_ARGUMENT, "forest file child link out of range");
         if (depth[left[g]] != depth[g] + 1 || depth[left[g] + 1] != depth[g] + 1)
           fail(DTE_ERR_INVALID_ARGUMENT, "forest file depths inconsistent");
+        level_order = level_order && left[g] == next;
+        next += 2;
       }
+      level_order = level_order && next == ts[t + 1];
     }
     set_device(device_id);
     hipStream_t s = library_stream(device_id);
@@ -922,7 +921,7 @@ int dte_forest_load(const char* path, int32_t device_id, dte_forest** out) {
     f.algorithm = h.algorithm;
     f.n_nodes = n;
     f.n_leaves = count_leaves(feature);
-    f.level_order = in_level_order(ts, feature, left);
+    f.level_order = level_order;
     f.has_stats = h.has_stats != 0;
     f.seed = h.seed;
     f.tree_offset = h.tree_offset;

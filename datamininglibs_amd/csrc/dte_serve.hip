@@ -521,9 +521,13 @@ int dte_server_load_forest(dte_server* s, const dte_forest* forest, int32_t* slo
     f.n_nodes = src.n_nodes;
     f.pair_fbits = src.pair_fbits;
     hipStream_t ls = library_stream(s->device);
+    // one allocation for the records: three took 116 us for a forest, the two
+    // of the 16-byte records 90
+    f.slab.alloc(Forest::slab_bytes(src.tree_start.bytes()) + Forest::slab_bytes(src.pairs.bytes()) +
+                 Forest::slab_bytes(src.pair_base.bytes()) + Forest::slab_bytes(src.pnodes.bytes()));
     auto copy = [&](auto& dst, const auto& from) {
       if (!from.p) return;
-      dst.alloc(from.n);
+      f.take(dst, from.n);
       DTE_HIP(hipMemcpyAsync(dst.p, from.p, from.bytes(), hipMemcpyDeviceToDevice, ls));
     };
     copy(f.tree_start, src.tree_start);
