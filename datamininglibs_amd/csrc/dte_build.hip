@@ -3222,7 +3222,7 @@ __device__ __forceinline__ void bound_pure(const DataArgs& d, const ItemArgs& it
 }
 
 // ------------------------------------------- all draws' keys of a level ---
-// A draw's key costs the fabric a 64-byte piece of a line per entry (rows of a
+// A draw's key costs the fabric a 64-byte half of a line per entry (rows of a
 // node lie anywhere), so a level with many draws moves 64 D bytes an entry.
 // With the keys of a row side by side (KR, rows of FS words), the entry's row
 // comes over once, whole, and its D keys are written in entry order, where
@@ -7076,8 +7076,8 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     // likewise the partition tiers of a step (both algorithms)
     const PartAllFn partition_all = pick_part_all(task, C);
 
-    // One level step; par = 1 swaps the ping-pong buffers.
-    auto enqueue = [&](int par) {
+    // One level step on stream s; par = 1 swaps the ping-pong buffers.
+    auto enqueue = [&](int par, hipStream_t s) {
       DevLevel* const L = dlv.p + par;
       DevLevel* const L_next = dlv.p + (par ^ 1);
       int64_t* cs = par ? w_start_next.p : w_start.p;
@@ -7279,15 +7279,18 @@ Forest* fit_batch(FitData& fd, int t0, int T, int64_t N, int32_t F, const dte_pa
     const auto cap_t0 = std::chrono::steady_clock::now();
     for (int par = 0; par < 2; ++par) {
       hipGraph_t g = nullptr;
-      DTE_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-      try {
-        enqueue(par);
-      } catch (...) {
-        (void)hipStreamEndCapture(s, &g);
-        if (g) (void)hipGraphDestroy(g);
-        throw;
+      {
+        const RecordStream rec(s);
+        DTE_HIP(hipStreamBeginCapture(rec.stream, hipStreamCaptureModeThreadLocal));
+        try {
+          enqueue(par, rec.stream);
+        } catch (...) {
+          (void)hipStreamEndCapture(rec.stream, &g);
+          if (g) (void)hipGraphDestroy(g);
+          throw;
+        }
+        DTE_HIP(hipStreamEndCapture(rec.stream, &g));
       }
-      DTE_HIP(hipStreamEndCapture(s, &g));
       const hipError_t e = hipGraphInstantiate(&gr.e[par], g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);
       DTE_HIP(e);

@@ -289,6 +289,18 @@ hipStream_t worker_stream(int device, int k) {
   return v[k];
 }
 
+RecordStream::RecordStream(hipStream_t s) : stream(s) {
+  static std::mutex mu;                         // one recording at a time
+  static std::map<int, hipStream_t> recorders;  // device -> stream, kept for the life of the process
+  int device = 0;
+  DTE_HIP(hipGetDevice(&device));
+  if (s != library_stream(device)) return;  // a worker's own
+  lock = std::unique_lock<std::mutex>(mu);
+  hipStream_t& r = recorders[device];
+  if (!r) DTE_HIP(hipStreamCreateWithFlags(&r, hipStreamNonBlocking));
+  stream = r;
+}
+
 hipStream_t library_stream(int device) {
   std::lock_guard<std::mutex> lk(g_dev_mu);
   auto it = g_streams.find(device);

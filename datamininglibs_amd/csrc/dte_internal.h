@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -284,6 +285,14 @@ void oob_evaluate(const Forest& f, const float* X_dev, const float* targets, int
                   double out[2], hipStream_t stream);
 void device_init(int device);
 hipStream_t library_stream(int device);
+// The stream to record a graph on whose replays go to stream s, held until the
+// object ends.  A stream takes part in a recording with whatever any thread
+// sends to it, so the library stream, which all callers share, never records.
+struct RecordStream {
+  std::unique_lock<std::mutex> lock;
+  hipStream_t stream;
+  explicit RecordStream(hipStream_t s);
+};
 const LnTable& host_ln_table();
 
 constexpr int kBlock = 256;

@@ -41,17 +41,21 @@ constexpr int64_t kManyBlocks = 4096;
 constexpr int64_t kMaxRowBlocks = 0xFFFFFFFFll / kWalkThreads;
 
 // ------------------------------------------------------ node layout ----
-// Bound by the rate of cache lines that come over the fabric for the deep
-// levels (16-byte records in level order: a line per visited level, 79 GB for
-// 200 M walks of 60 M nodes, 16.0 ms).  Below kTopLevels a tree's pairs are
-// grouped by clusters of three levels -- the pair below a node at depth 9, 12,
-// .. and up to six pairs below it, 16 B each -- in slots of 1, 2, 4 or 8 pairs
-// aligned to their size, so that a cluster never straddles a 128-byte line and
-// a walk touches one line per three levels.  The top levels stay in the caches
-// whatever their order; there the lines that the 64 rows of a wave touch in one
-// step count, fewest in level order.  600,000 rows x 6, 64 trees of 8,000 nodes:
-// 0.69 ms with 16-byte records, 0.81 clustered from the root, 0.64 like this;
-// 1M x 128, 64 trees of 300,000 nodes: 5.2, 4.1, 4.1 ms.
+// Bound by read requests of the deep levels: a scattered read that misses the
+// L2 brings a 64-byte half of a line, and the fabric passes 45 to 55 G of them
+// a second (single words at random, one a line or one a half line: 48 G/s).
+// Below kTopLevels a tree's pairs are grouped by clusters of three levels --
+// the pair below a node at depth 9, 12, .. and up to six pairs below it, 16 B
+// each -- in slots of 1, 2, 4 or 8 pairs aligned to their size, so that a
+// cluster never straddles a 128-byte line and a walk takes one or two half
+// lines per three levels.  1M x 128, trees of 300,000 nodes: 2.7 requests a
+// walk with 64 trees and 2.9 with 200, at 45 G/s (16-byte records in level
+// order 4.5 and 3.1, at 51 and 39 G/s).  The top levels stay in the caches
+// whatever their order; there the lines that the 64 rows of a wave touch in
+// one step count, fewest in level order.  600,000 rows x 6, 64 trees of 8,000
+// nodes: 0.69 ms with 16-byte records, 0.81 clustered from the root, 0.64 like
+// this; 1M x 128, 64 trees of 300,000 nodes: 5.2, 4.1, 4.1 ms at 512 threads
+// a block, 3.7 like this at 256.
 constexpr int kClusterLevels = 3;
 constexpr int kTopLevels = 9;  // a multiple of kClusterLevels
 

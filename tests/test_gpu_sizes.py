@@ -1,6 +1,7 @@
 """HIP kernels at the sizes where their tiers, tiles and staging change, bit
 for bit against the CPU oracle (or a plain walk of the model)."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -554,3 +555,43 @@ def test_predict_of_many_rows_by_a_big_model(task, f):
             total += probs[p[:, None] + np.arange(3)].argmax(1) == 1
     assert np.array_equal(few.reshape(2048, -1)[:40, 0 if task else 1], total.astype(np.float32))
     g.close()
+
+
+def test_calls_of_other_threads_while_a_fit_records_its_level_steps():
+    """Fits of small data record graphs; predictions, exports and other fits
+    of the same device run beside them and share the library's stream."""
+    X, y = synth.gaussian_classes(seed=3, n=3000, f=8, n_informative=5, n_classes=3)
+    params = {a: capi.default_params(a, n_trees=6, n_classes=3, seed=4) for a in (RF, ERT)}
+    want = {a: capi.fit(X, y, params[a]) for a in (RF, ERT)}
+    canon = {a: want[a].canonical() for a in want}
+    votes = {a: want[a].predict(X) for a in want}
+    nodes = {a: want[a].export()[0].tobytes() for a in want}
+    errors = []
+
+    def fits(a):
+        for _ in range(40):
+            g = capi.fit(X, y, params[a])
+            c = g.canonical()
+            g.close()
+            if not all(np.array_equal(c[k], canon[a][k]) for k in ("feature", "threshold", "left", "rowhash")):
+                errors.append("fit")
+
+    def uses(a):
+        for _ in range(150):
+            if not np.array_equal(want[a].predict(X), votes[a]):
+                errors.append("predict")
+            if want[a].export()[0].tobytes() != nodes[a]:
+                errors.append("export")
+
+    def run(fn, a):
+        try:
+            fn(a)
+        except Exception as e:  # noqa: BLE001
+            errors.append(repr(e))
+
+    threads = [threading.Thread(target=run, args=(fn, a)) for fn in (fits, uses) for a in (RF, ERT)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[:3]
