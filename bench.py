@@ -16,8 +16,8 @@ it:
   - predict rows/s of the fitted forest on the 1M training rows;
   - `roofline`: algorithmic bytes of the dominant split-search kernel over
     its average launch time, from HIP events on the library stream;
-    `traffic` from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary
-    of the same kernel (profiles/traffic_rf_1m128.json) when present;
+    `traffic` from the committed rocprofv3 counters (L2 misses of 64 bytes
+    and writes) of the same kernel (profiles/traffic_rf_1m128.json) when present;
   - `cpu_baseline`: the CPU oracle on the host cores, one tree per core, on
     the same data (a bounded sample of the same workload).
 
@@ -99,7 +99,7 @@ def fit_steps(capi, Xd, n_rows, n_features, y, params, steps, warmup, label):
 
 def copy_calibration(nbytes=1 << 30, reps=3):
     """A plain copy kernel of known size, for scaling rocprofv3's
-    FETCH_SIZE / WRITE_SIZE counters (run under rocprofv3 --pmc)."""
+    memory counters (run under rocprofv3 --pmc)."""
     import torch
     a = torch.ones(nbytes // 4, dtype=torch.float32, device="cuda")  # fill kernel: writes nbytes
     b = torch.empty_like(a)
